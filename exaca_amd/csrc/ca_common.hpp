@@ -52,13 +52,10 @@ constexpr uint16_t kFresh = 2;  // mask built by the cell's capture; not yet loo
 // Steps ahead a cell can be scheduled; a cell with nothing to do for longer is scheduled at the
 // horizon and checks again.
 constexpr uint32_t kAlarmSlots = 64;
-// The apply pass: one workgroup per kApplyGroup capture-pass workgroups, each with a region of
-// kCandStage solidification candidates.
+// The apply pass: one workgroup per kApplyGroup capture-pass workgroups.
 constexpr uint32_t kApplyGroup = 2;
-constexpr uint32_t kCandStage = 2048;
 constexpr uint32_t apply_blocks(uint32_t claim_blocks) { return (claim_blocks + kApplyGroup - 1) / kApplyGroup; }
-// Words of one calendar slot: one bit per cell, rounded up to 32-byte rows (the list rebuild reads
-// a slot in 32-byte pieces).
+// Words of one calendar slot: one bit per cell, rounded up to 32-byte rows.
 constexpr size_t alarm_stride(long long ncell) {
     return ((static_cast<size_t>(ncell) + 31) / 32 + 7) & ~static_cast<size_t>(7);
 }
@@ -103,17 +100,16 @@ constexpr OppositeTable kOpposite = make_opposites();
 struct StepCtl {
     int32_t cycle[2];     // time step number seen by the kernels of a step of parity p
     uint32_t serial[2];   // steps executed before the step of parity p (its calendar slot)
-    uint32_t count[2];    // lengths of the steps' lists of cells to process
     uint32_t elo, ehi;    // cell-index range [elo, ehi] holding every active cell (elo > ehi: none)
-    uint32_t ncand;       // cells whose last liquid neighbour was captured in the current step
-    uint32_t rebuild_seq; // advanced before every list rebuild (its flags' tag)
     int32_t njumps;       // cycle jumps taken so far (spot-melt problems)
-    int32_t error;        // nonzero: list overflow or invalid grain
-    int32_t done;         // set by the device when a domain with autostop finishes
+    int32_t error;        // nonzero: invalid grain
+    int32_t done;         // set by the device when a domain finishes or raised an error
     int32_t final_cycle;  // the check cycle at which it finished
     int32_t last_cycle;   // the last executed step
-    int32_t next_nuc[2];  // least NucleationTime of the sites not yet decided, for the step of parity p
-    unsigned long long nactive;     // active cells at the end of the last step
+    int32_t nuc_at;       // nucleation sites of the layer decided so far (they lie in order of time)
+    int32_t nuc_next;     // the same after the nucleation of the current step
+    uint32_t serial_booked;         // steps executed before the last booking of the counters
+    unsigned long long nactive;     // active cells at the last booking
     unsigned long long nonwaiting;  // of those, past their liquidus time (the reference's numSteer)
     int32_t jump_from[kMaxJumps];  // cycle J before the jump; cycles J+1 .. T-1 were skipped
     int32_t jump_to[kMaxJumps];    // T, the first cycle executed after the jump
@@ -176,20 +172,21 @@ enum FieldKind : int {
     kFieldCentreF64 = 10,
 };
 
-// Counters of the current step, one slot per workgroup (part[row * nparts + workgroup]): every
-// workgroup overwrites its own slot, and the step's last kernel sums the rows. Same-address atomics
-// from thousands of workgroups would serialise.
+// Running counters since the last booking, one slot per workgroup (part[row * nparts + workgroup]):
+// every workgroup adds to its own slot, and the booking sums the rows. Same-address atomics from
+// thousands of workgroups would serialise. The ...At rows sum the serials of the events' steps.
 enum PartRow : int {
-    kPartClaimSol,      // solidified in the capture pass
-    kPartClaimEntered,  // first step past the liquidus time
-    kPartClaimEval,     // critical-length evaluations
-    kPartClaimMask,     // liquid masks built
-    kPartNucSol,        // solidified at nucleation (mask emptied by a nucleus)
-    kPartNucEntered,
-    kPartNucAct,        // nucleation events
-    kPartNucNn,         // nucleation events counted as the reference's nn
-    kPartCap,           // captures
-    kPartSettleSol,     // solidified in the settle pass
+    kPartEnt,    // first step past the liquidus time
+    kPartEntAt,
+    kPartSol,    // solidified
+    kPartSolAt,
+    kPartCap,    // captures
+    kPartCapAt,
+    kPartAct,    // nucleation events
+    kPartActAt,
+    kPartNn,     // nucleation events counted as the reference's nn
+    kPartEval,   // critical-length evaluations
+    kPartMask,   // liquid masks built
     kPartRows
 };
 
@@ -202,19 +199,12 @@ struct DomainView {
     long long ncell;        // X*Y*nz
     Cell *cells;
     Octa *octa;             // octahedron records (centre, critical lengths)
-    uint32_t *list[2];      // frontier of a step of parity p (list[1-p] also holds the step's
-                            // solidification candidates until the next frontier is written)
-    uint32_t *claim_cell;   // cells with claims in the current step, stored in their own frontier
-    uint32_t *claim_bits;   //   slice, and the neighbours each claimed
-    uint32_t *slice_claims; // entries of each workgroup's slice of the claim lists
-    uint32_t *cand;         // kCandStage solidification candidates per apply workgroup
-    uint32_t *cand_count;   // candidates in each region
-    uint32_t cand_cap;      // candidates staged per apply workgroup (<= kCandStage; the rest go to
-                            // the overflow list)
-    uint32_t list_cap;
+    uint32_t *claim_cell;   // cells with claims in the current step, each capture-pass workgroup's in
+    uint32_t *claim_bits;   //   a region of its own, and the neighbours each claimed
+    uint32_t *claim_count;  // entries of each workgroup's region
     int32_t nnuclei;
-    const int32_t *nloc;
-    int32_t *ntime;         // NucleationTimes; a site examined past its time is set to INT32_MAX
+    const int32_t *nloc;    // the layer's nucleation sites in ascending order of their times
+    const int32_t *ntime;   // NucleationTimes
     const float *guv;       // 10000 x 9 unit-vector components (GrainUnitVector)
     const float *seed_cdl;  // 10000 rows of kCdlStride: the 26 critical diagonal lengths of a
                             // cell-centred octahedron of each orientation
@@ -224,13 +214,10 @@ struct DomainView {
                             // 210 K saturation)
     StepCtl *ctl;
     StepStats *stats;
-    unsigned long long *part;  // kPartRows x nparts per-workgroup counters of the current step
+    unsigned long long *part;  // kPartRows x nparts per-workgroup counters
     uint32_t nparts;
     uint32_t *alarms;       // kAlarmSlots bitmaps of one bit per cell: process the cell at the step
                             // whose serial is the bitmap's slot (mod kAlarmSlots)
-    unsigned long long *chunk_flag;  // per unit of the list rebuild: tag | state | count or prefix
-    uint32_t rebuild_cap;   // list-rebuild workgroups the device holds at once (0: no limit)
-    uint32_t nchunks;
     int32_t autostop;       // end the domain on the device at the first check with no liquid left
     long long liquid0;      // liquid cells of the layer at the start
     int32_t *status;        // where the device reports the final cycle of an autostopped domain

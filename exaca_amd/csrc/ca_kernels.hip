@@ -1,17 +1,24 @@
 // ca_kernels.hip -- the CA time step as memory-bound CDNA4 kernels over the cells due this step.
 //
-// One step (reference: src/runCA.cpp:291-311) is six launches on one stream (five when no
-// nucleation site can be due):
+// One step (reference: src/runCA.cpp:291-311) is two launches on one stream (three when a nucleation
+// site can be due):
 //   k_nucleate  activates the pre-sampled nuclei whose time has come (src/CAupdate.cpp:67-200)
-//   k_claim     for every cell due this step: the growth since it was last looked at, a claim on
-//               every liquid neighbour it reaches (atomicMin of its index into the neighbour's
-//               claim word), and the step at which it is due next; a cell past its liquidus time
-//               with no liquid neighbour turns solid
-//   k_win       the claimants that won a claim (their index is in the claimed cell's word)
-//   k_apply     the winner of each claimed cell builds the new decentred octahedron, stores its
-//               26 critical lengths, and takes the cell out of its neighbours' liquid masks
-//   k_settle    a cell whose liquid neighbours were all taken by lower-indexed cells turns solid
-//   k_rebuild   the list of the cells due at the next step, in index order, from its calendar slot
+//   k_claim     for every cell due this step, gathered from the step's calendar slot: the growth
+//               since it was last looked at, a claim on every liquid neighbour it reaches (atomicMin
+//               of its index into the neighbour's claim word), and the step at which it is due next;
+//               a cell past its liquidus time with no liquid neighbour turns solid
+//   k_apply     the claimants that won a claim (their index is in the claimed cell's word) capture:
+//               each builds the new decentred octahedron, stores its 26 critical lengths, and takes
+//               the cell out of its neighbours' liquid masks
+// A cell whose liquid neighbours were all taken by lower-indexed cells in a step turns solid in that
+// step: the claim pass of the next step finds it due and gives it that step's state, and k_settle does
+// so when the caller looks at the state in between; k_book then sums the steps' counters.
+// What bounds a step of a small domain is not its work but what a launch costs before and between
+// its loads (5-14 us a kernel for a few dozen cells: caches and code are cold after each kernel
+// boundary), so a step has as few launches as its grid-wide dependences allow: claims before winners,
+// captures before the next step's claims. With separate kernels for the winners, the settling and the
+// list of due cells: 28.8, 40.5, 66.4, 76.4 us a step at 24^3, 100^3, 256^3, 400^3; with two kernels
+// 18.8, 26.4, 49.5, 60.8 us; at 800^3 (cycles 6006-6025) 0.198 and 0.180 ms.
 // A cell is due when something can happen to it: it is new, its liquidus time has passed, or its
 // half-diagonal reaches the least critical length of its liquid neighbours; a neighbour's capture
 // or nucleation that empties its mask is handled where it happens. Between those steps its growth
@@ -24,6 +31,8 @@
 // Every floating-point expression keeps the reference's operation order and float/double types;
 // the library is compiled with -ffp-contract=off and correctly rounded fp32 divide/sqrt.
 #include <hip/hip_runtime.h>
+
+#include <algorithm>
 
 #include "ca_kernels.hpp"
 #include "growth.hpp"
@@ -245,16 +254,18 @@ __device__ Octahedron new_octahedron(const float *g, double cxold, double cyold,
     return o;
 }
 
-// Wave64 inclusive prefix sum of v; returns the inclusive sum and sets total to the wave sum.
+// Wave64 inclusive prefix sum of v in registers (DPP row shifts and row broadcasts); total is the
+// wave sum. Every lane of the wave must reach the call.
 __device__ __forceinline__ uint32_t wave_inclusive_scan(uint32_t v, uint32_t &total) {
-    const int lane = threadIdx.x & 63;
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-        uint32_t n = __shfl_up(v, o, 64);
-        if (lane >= o) v += n;
-    }
-    total = __shfl(v, 63, 64);
-    return v;
+    int x = static_cast<int>(v);
+    x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, false);  // row_shr:1
+    x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, false);  // row_shr:2
+    x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xf, 0xf, false);  // row_shr:4
+    x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xf, 0xf, false);  // row_shr:8
+    x += __builtin_amdgcn_update_dpp(0, x, 0x142, 0xa, 0xf, false);  // row_bcast:15 into rows 1 and 3
+    x += __builtin_amdgcn_update_dpp(0, x, 0x143, 0xc, 0xf, false);  // row_bcast:31 into rows 2 and 3
+    total = static_cast<uint32_t>(__builtin_amdgcn_readlane(x, 63));
+    return static_cast<uint32_t>(x);
 }
 
 __device__ __forceinline__ unsigned long long block_sum(unsigned long long v, unsigned long long *sh) {
@@ -270,22 +281,8 @@ __device__ __forceinline__ unsigned long long block_sum(unsigned long long v, un
     return t;
 }
 
-// Contiguous slice of the frontier for workgroup b of the nb serving one domain. Workgroups are
-// dispatched round-robin over the 8 XCDs, so consecutive slices are given to workgroups on the
-// same XCD: neighbouring frontier cells (and their neighbour reads and claims) then share one L2.
-__device__ __forceinline__ void frontier_slice(uint32_t count, uint32_t cap, uint32_t b, uint32_t nb,
-                                               uint32_t &begin, uint32_t &end) {
-    const uint32_t n = count < cap ? count : cap;  // an overflowed list is flagged, never over-read
-    const uint32_t logical = (nb % 8 == 0) ? (b % 8) * (nb / 8) + b / 8 : b;
-    uint32_t chunk = (n + nb - 1) / nb;
-    chunk = (chunk + kBlock - 1) / kBlock * kBlock;
-    const unsigned long long b0 = static_cast<unsigned long long>(logical) * chunk;
-    begin = b0 >= n ? n : static_cast<uint32_t>(b0);
-    end = (b0 + chunk >= n) ? n : static_cast<uint32_t>(b0 + chunk);
-}
-
 // Wave-aggregated append: every lane with `want` gets its own slot of the list behind `counter`
-// (global or LDS), at one atomic per wave. Every lane of the wave must reach the call.
+// (LDS), at one atomic per wave. Every lane of the wave must reach the call.
 __device__ __forceinline__ uint32_t wave_append(bool want, uint32_t *counter) {
     const unsigned long long b = __ballot(want);
     if (b == 0) return 0;
@@ -385,10 +382,11 @@ __device__ __forceinline__ Growth growth_of(const DomainView &d) { return Growth
 // The same with the table's first ksat entries copied to the workgroup's LDS buffer when they fit
 // (the replays walk the table one dependent step at a time). Every thread of the workgroup calls it.
 constexpr int kGrowStage = 4096;  // table entries staged in LDS (32 KB)
+template <int BLOCK>
 __device__ __forceinline__ Growth staged_growth(const DomainView &d, double *lds) {
     Growth g = growth_of(d);
     if (d.ksat <= kGrowStage) {
-        for (int k = threadIdx.x; k < d.ksat; k += kBlock) lds[k] = d.grow[k];
+        for (int k = threadIdx.x; k < d.ksat; k += BLOCK) lds[k] = d.grow[k];
         g.tab = lds;
     }
     __syncthreads();
@@ -424,35 +422,40 @@ __device__ __forceinline__ void set_alarm(const DomainView &d, uint32_t serial, 
     atomicOr(&d.alarms[(serial % kAlarmSlots) * alarm_stride(d.ncell) + (q >> 5)], 1u << (q & 31));
 }
 
-struct StepCounts {
-    unsigned long long nsol, entered, neval, nmask;
-};
-// Workgroup b's value of a counter row for this step (thread 0 holds the block sum).
-__device__ __forceinline__ void put_part(const DomainView &d, int row, uint32_t b, unsigned long long v,
-                                         unsigned long long *sh) {
-    const unsigned long long t = block_sum(v, sh);
-    if (threadIdx.x == 0) d.part[static_cast<size_t>(row) * d.nparts + b] = t;
+// ---- The workgroups that serve one domain in a launch: b of nb. Every body below works for one
+// domain; the plain launches use the grid x dimension, the ensemble launches add one grid row per
+// domain slot. A finished domain (device-side termination) keeps its state: its bodies return at
+// once. ----
+
+// Events of a step counted per workgroup in LDS. A wave adds its lanes' events at once.
+enum StepCount : int { kCntEnt, kCntSol, kCntLate, kCntCap, kCntAct, kCntNn, kCntEval, kCntMask, kStepCounts };
+__device__ __forceinline__ void count_event(bool happened, uint32_t *counter) {
+    const unsigned long long m = __ballot(happened);
+    if (m && (threadIdx.x & 63) == static_cast<uint32_t>(__ffsll(static_cast<long long>(m)) - 1))
+        atomicAdd(counter, static_cast<uint32_t>(__popcll(m)));
 }
-// Four rows at once (one pair of barriers); sh holds 4 * kBlock / 64 entries.
-__device__ __forceinline__ void put_parts4(const DomainView &d, const int (&rows)[4], unsigned long long (&v)[4],
-                                           uint32_t b, unsigned long long *sh) {
-#pragma unroll
-    for (int i = 0; i < 4; i++)
-#pragma unroll
-        for (int o = 32; o > 0; o >>= 1) v[i] += __shfl_down(v[i], o, 64);
-    const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    __syncthreads();
-    if (lane == 0)
-#pragma unroll
-        for (int i = 0; i < 4; i++) sh[i * (kBlock / 64) + w] = v[i];
-    __syncthreads();
-    if (threadIdx.x == 0)
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            unsigned long long t = 0;
-            for (int q = 0; q < kBlock / 64; q++) t += sh[i * (kBlock / 64) + q];
-            d.part[static_cast<size_t>(rows[i]) * d.nparts + b] = t;
-        }
+// The step's events added to the workgroup's running totals (rows of PartRow, slot b): the counts
+// and, for what changes the number of active cells, the sums of the steps' serials, from which
+// book_totals forms the per-step sums. A late solidification belongs to the step before.
+__device__ __forceinline__ void add_parts(const DomainView &d, uint32_t b, const uint32_t *cnt, uint32_t serial) {
+    const uint32_t r = threadIdx.x;
+    if (r >= kPartRows) return;
+    unsigned long long v = 0;
+    const unsigned long long s = serial;
+    switch (r) {
+    case kPartEnt: v = cnt[kCntEnt]; break;
+    case kPartEntAt: v = cnt[kCntEnt] * s; break;
+    case kPartSol: v = static_cast<unsigned long long>(cnt[kCntSol]) + cnt[kCntLate]; break;
+    case kPartSolAt: v = cnt[kCntSol] * s + (cnt[kCntLate] ? cnt[kCntLate] * (s - 1) : 0); break;
+    case kPartCap: v = cnt[kCntCap]; break;
+    case kPartCapAt: v = cnt[kCntCap] * s; break;
+    case kPartAct: v = cnt[kCntAct]; break;
+    case kPartActAt: v = cnt[kCntAct] * s; break;
+    case kPartNn: v = cnt[kCntNn]; break;
+    case kPartEval: v = cnt[kCntEval]; break;
+    default: v = cnt[kCntMask]; break;
+    }
+    if (v) d.part[static_cast<size_t>(r) * d.nparts + b] += v;
 }
 
 // Growth index that an active cell's dl includes, at a step of growth index k. A cell not yet
@@ -465,7 +468,8 @@ __device__ __forceinline__ int growth_base(const CellWords &w, int k, bool waiti
     return static_cast<int>(w.win);
 }
 // Cell r of known mask is past its liquidus time and has no liquid neighbour left: at its visit
-// in this step's capture the reference grows it and turns it solid (src/CAupdate.cpp:722-725).
+// in the capture of the step of growth index k the reference grows it and turns it solid
+// (src/CAupdate.cpp:722-725).
 __device__ __forceinline__ void solidify(const DomainView &d, const Growth &g, uint32_t r, const CellWords &w, int k) {
     Cell &c = d.cells[r];
     c.dl = replay_growth(g, w.dl, growth_base(w, k, false), k);
@@ -474,100 +478,81 @@ __device__ __forceinline__ void solidify(const DomainView &d, const Growth &g, u
     c.ct = kSolid;
 }
 
-// Every body below works on one domain with workgroups b = 0 .. nb-1; the plain launches use the
-// grid x dimension, the ensemble launches add one grid row per domain slot. A finished domain
-// (device-side termination) keeps its state: its bodies return at once.
-
 // Nucleation (src/CAupdate.cpp:67-200). A nucleus leaves the liquid masks of its neighbours; a
 // neighbour whose mask this empties and that is past its liquidus time finds no liquid neighbour in
 // this step's capture and turns solid here.
-// Most steps have no site due: next_nuc[p], the least time of the sites not yet decided, lets every
-// workgroup return at once (its counter rows zero). A step that examines sites sets the next step's
-// value from what is left (next_nuc[1-p], reset to INT32_MAX by the capture pass of the step before);
-// for a step that does not, the capture pass passes the value on. The step's control words are
-// advanced by the capture pass too, so a step may leave this kernel out when no site can be due
-// (the host knows the sites' times).
-constexpr int kPartNucRows[4] = {kPartNucNn, kPartNucAct, kPartNucSol, kPartNucEntered};
-__device__ __forceinline__ void nucleate_body(const DomainView &d, int p, int layer, uint32_t b, uint32_t nb) {
-    __shared__ unsigned long long sh[4 * (kBlock / 64)];
-    __shared__ int smin;
-    StepCtl *ctl = d.ctl;
-    if (ctl->done) return;
-    const int cycle = ctl->cycle[p];
-    const int gate = ctl->next_nuc[p];
-    if (cycle < gate) {
-        if (threadIdx.x < 4) d.part[static_cast<size_t>(kPartNucRows[threadIdx.x]) * d.nparts + b] = 0;
-        return;
+// The sites of the layer lie in ascending order of time, so the ones due are the next few from
+// `from` on; returns how many sites were decided (a cell that is not liquid never turns liquid
+// again, so a site past its time is not looked at after). The new active cells are due in this
+// step's capture.
+template <int BLOCK>
+__device__ __forceinline__ int nucleate_body(const DomainView &d, int cycle, uint32_t serial, int layer, int from,
+                                             uint32_t b, uint32_t nb, uint32_t *cnt, uint32_t *lohi) {
+    const int i0 = from + static_cast<int>(threadIdx.x);
+    int m = __syncthreads_count(i0 < d.nnuclei && d.ntime[i0] <= cycle);
+    if (m == BLOCK) {  // more than a round of sites: the end of the run of due ones by bisection
+        int lo = from + BLOCK - 1, hi = d.nnuclei;  // ntime[lo] <= cycle < ntime[hi]
+        while (hi - lo > 1) {
+            const int mid = lo + (hi - lo) / 2;
+            if (d.ntime[mid] <= cycle)
+                lo = mid;
+            else
+                hi = mid;
+        }
+        m = hi - from;
     }
-    if (threadIdx.x == 0) smin = 0x7FFFFFFF;
-    __syncthreads();
-    int tmin = 0x7FFFFFFF;  // least time of this thread's sites left undecided
     const Grid gr = grid_of(d);
-    unsigned long long nn = 0, act = 0;
-    StepCounts n{0, 0, 0, 0};
-    for (int i = b * kBlock + threadIdx.x; i < d.nnuclei; i += nb * kBlock) {
-        const int t = d.ntime[i];
-        if (cycle < t) {
-            tmin = t < tmin ? t : tmin;
-            continue;
-        }
-        const uint32_t q = static_cast<uint32_t>(d.nloc[i]);
-        const uint32_t tail = reinterpret_cast<const uint32_t *>(d.cells + q)[7];  // lid | ct << 8 | flags
-        if (static_cast<int8_t>(tail & 0xFFu) > layer) {
-            tmin = t < tmin ? t : tmin;
-            continue;
-        }
-        // Past its time and in this layer, the site is decided now: a cell that is not liquid
-        // never turns liquid again, so the site is not looked at after this step.
-        d.ntime[i] = 0x7FFFFFFF;
-        if (((tail >> 8) & 0xFFu) != kLiquid) continue;
-        const Coord c = decode(q, gr);
-        if (c.x > 0 && c.x < d.X - 1 && c.y > 0 && c.y < d.Y - 1) nn++;
-        Cell &cq = d.cells[q];
-        cq.dl = 0.01f;
-        cq.thr = 0.0f;
-        cq.lm = kLmUnknown;
-        cq.flags = 0;
-        cq.ct = kActive | kSeedBit;
-        set_centre(d, q, (c.x + d.xoff) + 0.5, (c.y + d.yoff) + 0.5, c.z + 0.5);
-        const uint32_t valid = valid_neighbours(c, gr.X, gr.Y, gr.nzA);
-        // all updates in flight together, then the results
-        uint32_t old[26];
+    for (int k0 = static_cast<int>(b) * 64; k0 < m; k0 += static_cast<int>(nb) * BLOCK) {
+        // a wave of consecutive sites per workgroup and turn: few sites are due at once
+        const int turn = static_cast<int>(threadIdx.x >> 6) * static_cast<int>(nb) * 64;
+        const int k = k0 + turn + static_cast<int>(threadIdx.x & 63);
+        bool act = false, inner = false;
+        uint32_t nent = 0, nsol = 0;
+        if (k < m) {
+            const uint32_t q = static_cast<uint32_t>(d.nloc[from + k]);
+            const uint32_t tail = reinterpret_cast<const uint32_t *>(d.cells + q)[7];  // lid | ct << 8 | flags
+            if (static_cast<int8_t>(tail & 0xFFu) <= layer && ((tail >> 8) & 0xFFu) == kLiquid) {
+                const Coord c = decode(q, gr);
+                act = true;
+                inner = c.x > 0 && c.x < d.X - 1 && c.y > 0 && c.y < d.Y - 1;
+                Cell &cq = d.cells[q];
+                cq.dl = 0.01f;
+                cq.thr = 0.0f;
+                cq.lm = kLmUnknown;
+                cq.flags = 0;
+                cq.ct = kActive | kSeedBit;
+                set_centre(d, q, (c.x + d.xoff) + 0.5, (c.y + d.yoff) + 0.5, c.z + 0.5);
+                const uint32_t valid = valid_neighbours(c, gr.X, gr.Y, gr.nzA);
+                // all updates in flight together, then the results
+                uint32_t old[26];
 #pragma unroll
-        for (int l = 0; l < 26; l++)
-            old[l] = ((valid >> l) & 1u) ? atomicAnd(mask_word(d, q + gr.off[l]), ~(1u << kOpposite.v[l])) : 0u;
-        uint32_t emptied = 0;
+                for (int l = 0; l < 26; l++)
+                    old[l] = ((valid >> l) & 1u) ? atomicAnd(mask_word(d, q + gr.off[l]), ~(1u << kOpposite.v[l])) : 0u;
+                uint32_t emptied = 0;
 #pragma unroll
-        for (int l = 0; l < 26; l++)
-            emptied |= static_cast<uint32_t>(((valid >> l) & 1u) &&
-                                             (old[l] & (kMaskUnknown | kMaskNow)) == (1u << kOpposite.v[l])) << l;
-        for (uint32_t m = emptied; m; m &= m - 1) {
-            const uint32_t r = q + gr.offset(__builtin_ctz(m));
-            const CellWords w = load_cell(d.cells + r);
-            if ((w.ct & kTypeMask) != kActive || !(cycle > w.cts && w.lid <= layer)) continue;
-            if (!(w.flags & kCounted)) n.entered++;
-            solidify(d, growth_of(d), r, w, growth_index(d, w.cts, w.lid, r, cycle));
-            d.cells[r].flags = (w.flags & ~kFresh) | kCounted;
-            n.nsol++;
+                for (int l = 0; l < 26; l++)
+                    emptied |= static_cast<uint32_t>(((valid >> l) & 1u) &&
+                                                     (old[l] & (kMaskUnknown | kMaskNow)) == (1u << kOpposite.v[l])) << l;
+                for (uint32_t e = emptied; e; e &= e - 1) {
+                    const uint32_t r = q + gr.offset(__builtin_ctz(e));
+                    const CellWords w = load_cell(d.cells + r);
+                    if ((w.ct & kTypeMask) != kActive || !(cycle > w.cts && w.lid <= layer)) continue;
+                    if (!(w.flags & kCounted)) nent++;
+                    solidify(d, growth_of(d), r, w, growth_index(d, w.cts, w.lid, r, cycle));
+                    d.cells[r].flags = (w.flags & ~kFresh) | kCounted;
+                    nsol++;
+                }
+                atomicMin(&lohi[0], q);
+                atomicMax(&lohi[1], q);
+                set_alarm(d, serial, q);
+            }
         }
-        atomicMin(&ctl->elo, q);
-        atomicMax(&ctl->ehi, q);
-        act++;
-        const uint32_t slot = atomicAdd(&ctl->count[p], 1u);
-        if (slot < d.list_cap)
-            d.list[p][slot] = q;
-        else
-            atomicOr(&ctl->error, 1);
+        count_event(act, &cnt[kCntAct]);
+        count_event(inner, &cnt[kCntNn]);
+        if (nent) atomicAdd(&cnt[kCntEnt], nent);
+        if (nsol) atomicAdd(&cnt[kCntSol], nsol);
     }
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-        const int v = __shfl_xor(tmin, o, 64);
-        tmin = v < tmin ? v : tmin;
-    }
-    if ((threadIdx.x & 63) == 0) atomicMin(&smin, tmin);
-    unsigned long long v4[4] = {nn, act, n.nsol, n.entered};
-    put_parts4(d, {kPartNucNn, kPartNucAct, kPartNucSol, kPartNucEntered}, v4, b, sh);
-    if (threadIdx.x == 0 && smin != 0x7FFFFFFF) atomicMin(&ctl->next_nuc[1 - p], smin);
+    return m;
 }
 
 // Critical lengths of the liquid neighbours of frontier cell j (half-diagonal dlj): claims on
@@ -621,799 +606,543 @@ __device__ uint32_t evaluate_claims(const DomainView &d, const Grid &gr, uint32_
     return claimed;
 }
 
-// Pass A over the cells due this step (the step's calendar slot plus this step's nuclei), one per
-// lane: the liquidus-time gate, the growth since the cell was last looked at, and the claims.
+// ---- Units of the calendar: kUnitWords words (one wave-wide load) of a slot. The workgroups of a
+// domain share the units of the range of active cells in turn, so that the front, wherever it lies,
+// is spread over all of them. ----
+constexpr uint32_t kUnitWords = 64;
+constexpr uint32_t kUnitCells = 32 * kUnitWords;
+constexpr uint32_t kUnitsPerLane = 8;  // units whose words a wave holds at once
+
+struct UnitRange {
+    uint32_t u0, n;  // first unit, number of units
+};
+__device__ __forceinline__ uint32_t domain_units(const DomainView &d) {
+    return static_cast<uint32_t>((bitmap_words(d) + kUnitWords - 1) / kUnitWords);
+}
+// The units that may hold a due cell: all of a domain small enough for one round of its workgroups,
+// else those of the range of active cells.
+template <int BLOCK>
+__device__ __forceinline__ bool scans_all(const DomainView &d, uint32_t nb) {
+    return domain_units(d) <= nb * (BLOCK / 64) * kUnitsPerLane;
+}
+template <int BLOCK>
+__device__ __forceinline__ UnitRange unit_range(const DomainView &d, uint32_t nb) {
+    if (scans_all<BLOCK>(d, nb)) return UnitRange{0, domain_units(d)};
+    const uint32_t lo = d.ctl->elo;
+    uint32_t hi = d.ctl->ehi;
+    if (lo > hi) return UnitRange{0, 0};
+    if (hi >= static_cast<uint64_t>(d.ncell)) hi = static_cast<uint32_t>(d.ncell - 1);
+    return UnitRange{lo / kUnitCells, hi / kUnitCells - lo / kUnitCells + 1};
+}
+// The k-th unit of workgroup b. Workgroups are dispatched round-robin over the 8 XCDs; with enough
+// of them, runs of nb / 8 units go to the workgroups of one XCD, so that neighbouring cells mostly
+// share an L2.
+__device__ __forceinline__ uint32_t unit_of(uint32_t k, uint32_t b, uint32_t nb) {
+    if (nb >= 64 && nb % 8 == 0) return (k * 8 + b % 8) * (nb / 8) + b / 8;
+    return k * nb + b;
+}
+__device__ __forceinline__ uint32_t *calendar_slot(const DomainView &d, uint32_t serial) {
+    return d.alarms + (serial % kAlarmSlots) * alarm_stride(d.ncell);
+}
+// Entries of a workgroup's region of the claim lists: the cells of the most units it can hold. The
+// regions lie in the order of the workgroups' units, so that those of workgroups without any come last.
+__device__ __forceinline__ uint32_t claim_region(const DomainView &d, uint32_t nb) {
+    return (domain_units(d) + nb - 1) / nb * kUnitCells;
+}
+
+// Calls visit(has, j, record) for every cell due at the step of that serial in workgroup b's units,
+// BLOCK cells at a time in a uniform loop (has: the lane has one). The due cells are gathered in LDS
+// (`list`, CAP entries) over as many rounds of units as fit and then processed together, so that the
+// lanes are full; a round that does not fit is read again for the rest. With CLEAR the bits of a
+// finished round are cleared for the slot's next use, 64 steps on.
+template <int BLOCK, uint32_t CAP, bool CLEAR, typename F>
+__device__ __forceinline__ void for_due(const DomainView &d, uint32_t serial, uint32_t b, uint32_t nb, uint32_t *list,
+                                        uint32_t *tot, F &&visit) {
+    constexpr uint32_t kWaves = BLOCK / 64;
+    const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const UnitRange r = unit_range<BLOCK>(d, nb);
+    const uint32_t nwords = static_cast<uint32_t>(bitmap_words(d));
+    uint32_t *bits = calendar_slot(d, serial);
+    const uint32_t most = (r.n + nb - 1) / nb;  // units of the workgroup that has the most
+    uint32_t fill = 0, done = 0;                // entries in the list; cells of the round already listed
+    for (uint32_t k0 = 0; k0 < most;) {
+        uint32_t w[kUnitsPerLane], cnt = 0;
+        auto word = [&](uint32_t e) {
+            const uint32_t u = unit_of(k0 + e * kWaves + wave, b, nb);
+            const uint32_t at = (r.u0 + u) * kUnitWords + lane;
+            return u < r.n && at < nwords ? at : 0xFFFFFFFFu;
+        };
+#pragma unroll
+        for (uint32_t e = 0; e < kUnitsPerLane; e++) {
+            const uint32_t at = word(e);
+            w[e] = at != 0xFFFFFFFFu ? bits[at] : 0u;
+        }
+#pragma unroll
+        for (uint32_t e = 0; e < kUnitsPerLane; e++) cnt += __builtin_popcount(w[e]);
+        uint32_t wtot;
+        const uint32_t incl = wave_inclusive_scan(cnt, wtot);
+        if (lane == 0) tot[wave] = wtot;
+        __syncthreads();
+        uint32_t before = 0, total = 0;
+#pragma unroll
+        for (uint32_t q = 0; q < kWaves; q++) {
+            const uint32_t v = tot[q];
+            before += q < wave ? v : 0u;
+            total += v;
+        }
+        const uint32_t take = total - done < CAP - fill ? total - done : CAP - fill;
+        const bool last = done + take == total;
+        uint32_t pos = before + incl - cnt - done;  // place among the cells to list now; wraps if listed before
+#pragma unroll
+        for (uint32_t e = 0; e < kUnitsPerLane; e++) {
+            if (!w[e]) continue;
+            const uint32_t at = word(e);
+            if (CLEAR && last) bits[at] = 0u;
+            for (uint32_t m = w[e]; m; m &= m - 1, pos++)
+                if (pos < take) list[fill + pos] = at * 32u + __builtin_ctz(m);
+        }
+        fill += take;
+        done = last ? 0 : done + take;
+        if (last) k0 += kWaves * kUnitsPerLane;
+        __syncthreads();  // the list is written, tot is read
+        if (fill < CAP && k0 < most) continue;
+        // software pipeline: the next turn's record is loaded while this one's is processed
+        uint32_t jn = 0;
+        CellWords wn{};
+        if (threadIdx.x < fill) {
+            jn = list[threadIdx.x];
+            wn = load_cell(d.cells + jn);
+        }
+        for (uint32_t i0 = 0; i0 < fill; i0 += BLOCK) {
+            const uint32_t i = i0 + threadIdx.x;
+            const uint32_t j = jn;
+            const CellWords wc = wn;
+            if (i + BLOCK < fill) {
+                jn = list[i + BLOCK];
+                wn = load_cell(d.cells + jn);
+            }
+            visit(i < fill, j, wc);
+        }
+        fill = 0;
+        __syncthreads();  // the list is read
+    }
+}
+
+// A cell found with a known, empty mask at the step after the one that emptied it. The reference
+// visits cells in ascending index order with every capture visible at once, so a cell whose liquid
+// neighbours all went to lower-indexed claimants has none left at its visit and turns solid in that
+// step; a capture by itself or a later cell leaves it active for one more step (src/CAupdate.cpp:
+// 333-334, 722-725). Every capture that took a neighbour of it with a claimant of index >= its own
+// left the step's tag in its keep word. serial, cycle: the step after the one that emptied it. A cell
+// that waited for its liquidus time or its layer then was not visited in that step.
+__device__ __forceinline__ bool solid_since_last(const CellWords &w, uint32_t serial, int cycle, int layer) {
+    return !(w.lm & (kLmUnknown | kLmNow)) && !(w.flags & kFresh) && static_cast<uint32_t>(w.lm >> 32) != serial &&
+           cycle - 1 > w.cts && w.lid <= layer;
+}
+
+// Pass A over the cells due this step (the step's calendar slot), one per lane: the liquidus-time
+// gate, the growth since the cell was last looked at, and the claims.
 // The liquid neighbours come from the cell's mask (lm), kept current by the cells that leave the
 // liquid state; a new active cell builds it once from the 26 neighbour types. A cell past its
 // liquidus time with no liquid neighbour turns solid here (no capture of this step can give it
-// one).
+// one); one that the step before left without any, and that the reference turned solid in that
+// step, gets the state of that step (with follows: the step before ran just before, and its
+// solidifications are not yet settled).
 // thr is a lower bound on the critical length of every neighbour that is still liquid: the
 // smallest critical length over the liquid neighbours the cell did not claim when it last
 // evaluated them. Liquid sets only shrink and a cell's octahedron centre is
 // fixed, so no capture is possible before the half-diagonal reaches thr: the cell is scheduled for
 // that step (or for the end of its wait for the liquidus time) and not looked at before, unless a
 // neighbour's capture or nucleation empties its mask. A new active cell starts at thr = 0.
-// Cells with claims are appended to the claim lists inside the workgroup's own slice of the step's
-// list (an LDS counter, no global atomics), and the slice's count goes to slice_claims[b].
-
-__device__ __forceinline__ void claim_body(const DomainView &d, int p, int layer, uint32_t b, uint32_t nb) {
-    __shared__ unsigned long long sh[4 * (kBlock / 64)];
-    __shared__ uint32_t nclaim;
-    __shared__ double gtab[kGrowStage];
-    StepCtl *ctl = d.ctl;
-    if (ctl->done) return;
-    if (threadIdx.x == 0) nclaim = 0;
-    const Growth g = staged_growth(d, gtab);
-    const int cycle = ctl->cycle[p];
-    const uint32_t serial = ctl->serial[p];
-    if (b == 0 && threadIdx.x == 0) {
-        // the next step's control words (read only by the kernels after this one); this step's
-        // nucleation gate, passed on when no site was due, then reset for the step two on
-        ctl->cycle[1 - p] = cycle + 1;
-        ctl->serial[1 - p] = serial + 1;
-        ctl->ncand = 0;
-        ctl->rebuild_seq = ctl->rebuild_seq + 1;
-        const int gate = ctl->next_nuc[p];
-        if (cycle < gate) ctl->next_nuc[1 - p] = gate;
-        ctl->next_nuc[p] = 0x7FFFFFFF;
-    }
-    uint32_t begin, end;
-    frontier_slice(ctl->count[p], d.list_cap, b, nb, begin, end);
-    const uint32_t *list = d.list[p];
+// Cells with claims go to the workgroup's own region of the claim lists (an LDS counter, no global
+// atomics).
+template <int BLOCK, uint32_t CAP>
+__device__ __forceinline__ void claim_body(const DomainView &d, const Growth &g, int cycle, uint32_t serial, int layer,
+                                           bool follows, uint32_t b, uint32_t nb, uint32_t *list, uint32_t *tot,
+                                           uint32_t *cnt, uint32_t *nclaim) {
     const Grid gr = grid_of(d);
-    StepCounts n{0, 0, 0, 0};
-    // software pipeline: the list entry two rounds ahead and the record one round ahead are loaded
-    // while the current round is processed
-    uint32_t jn = 0, jnn = 0;
-    CellWords wn{};
-    {
-        const uint32_t i1 = begin + threadIdx.x, i2 = i1 + kBlock;
-        if (i1 < end) jn = list[i1];
-        if (i2 < end) jnn = list[i2];
-        if (i1 < end) wn = load_cell(d.cells + jn);
-    }
-    for (uint32_t i0 = begin; i0 < end; i0 += kBlock) {
-        const uint32_t i = i0 + threadIdx.x;
-        uint32_t j = 0, claimed = 0;
-        const uint32_t jc = jn;
-        const CellWords wc = wn;
-        {
-            const uint32_t i3 = i + 2 * kBlock;
-            jn = jnn;
-            if (i + kBlock < end) wn = load_cell(d.cells + jn);
-            if (i3 < end) jnn = list[i3];
-        }
-        if (i < end) {
-            j = jc;
-            const CellWords w = wc;
-            if ((w.ct & kTypeMask) == kActive) {
-                const bool waiting = !(cycle > w.cts && w.lid <= layer);
-                const int k = growth_index(d, w.cts, w.lid, j, cycle);
-                uint32_t liquid;
-                const int kdl = growth_base(w, k, waiting);
-                // the record's new words, written back as one sector at the end
-                unsigned long long lm = w.lm;
-                float dl = w.dl, thr = w.thr;
-                uint32_t win = w.win;
-                uint8_t ct = w.ct;
-                uint16_t flags = w.flags;
-                if (w.lm & kLmUnknown) {
-                    const Coord c = decode(j, gr);
-                    const uint32_t valid = valid_neighbours(c, gr.X, gr.Y, gr.nzA);
-                    liquid = 0;
+    const uint32_t region = unit_of(0, b, nb) * claim_region(d, nb);
+    for_due<BLOCK, CAP, true>(d, serial, b, nb, list, tot, [&](bool has, uint32_t j, const CellWords &w) {
+        uint32_t claimed = 0;
+        bool entered = false, sol = false, late = false, eval = false, mask = false;
+        if (has && (w.ct & kTypeMask) == kActive) {
+            const bool waiting = !(cycle > w.cts && w.lid <= layer);
+            int k = growth_index(d, w.cts, w.lid, j, cycle);
+            uint32_t liquid;
+            const int kdl = growth_base(w, k, waiting);
+            // the record's new words, written back as one sector at the end
+            unsigned long long lm = w.lm;
+            float dl = w.dl, thr = w.thr;
+            uint32_t win = w.win;
+            uint8_t ct = w.ct;
+            uint16_t flags = w.flags;
+            if (w.lm & kLmUnknown) {
+                const Coord c = decode(j, gr);
+                const uint32_t valid = valid_neighbours(c, gr.X, gr.Y, gr.nzA);
+                liquid = 0;
 #pragma unroll
-                    for (int l = 0; l < 26; l++) {
-                        const uint32_t q = ((valid >> l) & 1u) ? j + gr.off[l] : j;
-                        liquid |= static_cast<uint32_t>(d.cells[q].ct == kLiquid) << l;
-                    }
-                    lm = liquid;
-                    n.nmask++;
+                for (int l = 0; l < 26; l++) {
+                    const uint32_t q = ((valid >> l) & 1u) ? j + gr.off[l] : j;
+                    liquid |= static_cast<uint32_t>(d.cells[q].ct == kLiquid) << l;
                 }
-                else {
-                    liquid = static_cast<uint32_t>(w.lm & kLmNow);
-                }
-                if (waiting) {
-                    win = static_cast<uint32_t>(kdl);
-                    flags = w.flags & ~kFresh;
-                    const int ahead = w.cts + 1 - cycle;
-                    const uint32_t wake = ahead < 1 ? 1u
-                                                    : (ahead < static_cast<int>(kAlarmSlots) - 1 ? static_cast<uint32_t>(ahead)
-                                                                                               : kAlarmSlots - 1);
-                    set_alarm(d, serial + wake, j);
-                }
-                else {
-                    if (!(w.flags & kCounted)) n.entered++;
-                    flags = (w.flags & ~kFresh) | kCounted;
-                    dl = replay_growth(g, w.dl, kdl, k);
-                    win = static_cast<uint32_t>(k);
-                    if (!liquid) {
-                        ct = kSolid;
-                        n.nsol++;
-                    }
-                    else {
-                        if (dl >= thr) {
-                            const uint32_t at = (w.flags >> 2) & 31u;
-                            const float bound = hint_bound(thr, w.flags);
-                            if (at && !((liquid >> (at - 1)) & 1u) && dl < bound) {
-                                // the neighbour that set thr is gone and no other is reached
-                                thr = bound;
-                                flags &= ~kHintMask;
-                            }
-                            else {
-                                uint16_t hint = 0;
-                                claimed = evaluate_claims(d, gr, j, dl, liquid, w.gid, w.ct, thr, hint);
-                                flags = (flags & ~kHintMask) | hint;
-                                n.neval++;
-                            }
-                        }
-                        // No neighbour left to reach (all claimed now): the captures of this step
-                        // empty the mask and the settle pass decides the cell's fate.
-                        if (thr < __builtin_inff()) set_alarm(d, serial + steps_until(g, dl, k, thr), j);
-                    }
-                }
-                // Only this lane writes cell j in this pass (claims go to liquid cells' claim words,
-                // mask builds read liquid cells' types), so the whole sector is written back.
-                uint4 *r4 = reinterpret_cast<uint4 *>(d.cells + j);
-                r4[0] = make_uint4(static_cast<uint32_t>(lm), static_cast<uint32_t>(lm >> 32), __float_as_uint(dl),
-                                   __float_as_uint(thr));
-                r4[1] = make_uint4(static_cast<uint32_t>(w.cts), static_cast<uint32_t>(w.gid), win,
-                                   static_cast<uint32_t>(static_cast<uint8_t>(w.lid)) | (static_cast<uint32_t>(ct) << 8) |
-                                       (static_cast<uint32_t>(flags) << 16));
+                lm = liquid;
+                mask = true;
             }
+            else {
+                liquid = static_cast<uint32_t>(w.lm & kLmNow);
+            }
+            if (waiting) {
+                win = static_cast<uint32_t>(kdl);
+                flags = w.flags & ~kFresh;
+                const int ahead = w.cts + 1 - cycle;
+                const uint32_t wake = ahead < 1 ? 1u
+                                                : (ahead < static_cast<int>(kAlarmSlots) - 1 ? static_cast<uint32_t>(ahead)
+                                                                                           : kAlarmSlots - 1);
+                set_alarm(d, serial + wake, j);
+            }
+            else {
+                late = follows && solid_since_last(w, serial, cycle, layer);
+                if (late) k--;  // the step before: one executed step earlier
+                entered = !(w.flags & kCounted);
+                flags = (w.flags & ~kFresh) | kCounted;
+                dl = replay_growth(g, w.dl, kdl, k);
+                win = static_cast<uint32_t>(k);
+                if (!liquid) {
+                    ct = kSolid;
+                    sol = !late;
+                }
+                else {
+                    if (dl >= thr) {
+                        const uint32_t at = (w.flags >> 2) & 31u;
+                        const float bound = hint_bound(thr, w.flags);
+                        if (at && !((liquid >> (at - 1)) & 1u) && dl < bound) {
+                            // the neighbour that set thr is gone and no other is reached
+                            thr = bound;
+                            flags &= ~kHintMask;
+                        }
+                        else {
+                            uint16_t hint = 0;
+                            claimed = evaluate_claims(d, gr, j, dl, liquid, w.gid, w.ct, thr, hint);
+                            flags = (flags & ~kHintMask) | hint;
+                            eval = true;
+                        }
+                    }
+                    // No neighbour left to reach (all claimed now): the captures of this step
+                    // empty the mask, and the next step decides the cell's fate.
+                    if (thr < __builtin_inff()) set_alarm(d, serial + steps_until(g, dl, k, thr), j);
+                }
+            }
+            // Only this lane writes cell j in this pass (claims go to liquid cells' claim words,
+            // mask builds read liquid cells' types), so the whole sector is written back.
+            uint4 *r4 = reinterpret_cast<uint4 *>(d.cells + j);
+            r4[0] = make_uint4(static_cast<uint32_t>(lm), static_cast<uint32_t>(lm >> 32), __float_as_uint(dl),
+                               __float_as_uint(thr));
+            r4[1] = make_uint4(static_cast<uint32_t>(w.cts), static_cast<uint32_t>(w.gid), win,
+                               static_cast<uint32_t>(static_cast<uint8_t>(w.lid)) | (static_cast<uint32_t>(ct) << 8) |
+                                   (static_cast<uint32_t>(flags) << 16));
         }
-        const uint32_t slot = begin + wave_append(claimed != 0, &nclaim);
+        const uint32_t slot = wave_append(claimed != 0, nclaim);
         if (claimed) {
-            d.claim_cell[slot] = j;
-            d.claim_bits[slot] = claimed;
+            d.claim_cell[region + slot] = j;
+            d.claim_bits[region + slot] = claimed;
         }
-    }
-    __syncthreads();
-    if (threadIdx.x == 0) d.slice_claims[b] = nclaim;
-    unsigned long long v4[4] = {n.nsol, n.entered, n.neval, n.nmask};
-    put_parts4(d, {kPartClaimSol, kPartClaimEntered, kPartClaimEval, kPartClaimMask}, v4, b, sh);
+        count_event(entered, &cnt[kCntEnt]);
+        count_event(sol, &cnt[kCntSol]);
+        count_event(late, &cnt[kCntLate]);
+        count_event(eval, &cnt[kCntEval]);
+        count_event(mask, &cnt[kCntMask]);
+    });
 }
 
-// Pass B1 over the cells with claims, one workgroup per pass-A slice: a claim whose word holds the
-// claimant's own index is won (the lowest index that reached the cell). The slice's claimants that
-// won anything are compacted in place, with the claims they won, and slice_claims[b] becomes their
-// count. (Winners of a round go to positions below the round's end, whose entries every lane has
-// read before the barrier; later rounds' entries lie above.) Each claimant needs only its claim
-// words here: one round of every slice is resident at once, a short chain of dependent loads.
-__device__ __forceinline__ void win_body(const DomainView &d, int p, uint32_t b, uint32_t nb) {
-    __shared__ uint32_t nwin;
-    StepCtl *ctl = d.ctl;
-    if (ctl->done) return;
-    uint32_t beg, e;
-    frontier_slice(ctl->count[p], d.list_cap, b, nb, beg, e);
-    const uint32_t n = d.slice_claims[b];
+// The captures of a round: claimants' claims that hold the claimant's own index are won (the lowest
+// index that reached the cell). LDS of pass B.
+template <int BLOCK>
+struct ApplyLds {
+    uint32_t cell[2 * BLOCK], bits[2 * BLOCK];  // winners and the claims they won
+    int32_t gid[2 * BLOCK];
+    uint32_t item[BLOCK];  // winner << 5 | neighbour of each capture of a turn
+    uint32_t tot[BLOCK / 64];
+    uint32_t nwin;
+};
+
+// One capture (src/CAupdate.cpp:353-563, 717): the winner jc's octahedron gives that of its
+// neighbour l, the captured cell q, which is due at the next step and leaves the liquid masks of
+// its neighbours. Only masks that still hold it are updated: the masks are read first, and a cell's
+// bit is cleared by its capture alone, so the read decides exactly. A neighbour whose mask this
+// empties is due at the next step, which decides whether it turned solid in this one
+// (solid_since_last).
+__device__ __forceinline__ uint32_t capture(const DomainView &d, const Grid &gr, uint32_t serial, uint32_t jc, int l,
+                                            int h) {
+    const uint32_t q = jc + gr.offset(l);
+    const Octa &e = d.octa[jc];
+    // the winner's centre (float, as the capture uses it) and orientation, loaded with the
+    // neighbours' words below
+    const float wcx = static_cast<float>(e.x), wcy = static_cast<float>(e.y), wcz = static_cast<float>(e.z);
+    const Coord c = decode(jc, gr);
+    const Coord cqc{c.x + nb_dx(l), c.y + nb_dy(l), c.z + nb_dz(l)};
+    const uint32_t valid = valid_neighbours(cqc, gr.X, gr.Y, gr.nzA);
+    int o = orientation_of(h);
+    if (o < 0) {
+        atomicOr(&d.ctl->error, 2);
+        o = 0;
+    }
+    float gv[9];
+#pragma unroll
+    for (int m = 0; m < 9; m++) gv[m] = d.guv[9 * o + m];
+    const uint4 own = reinterpret_cast<const uint4 *>(d.cells + q)[1];  // cts, gid, win, lid | ct | flags
+    // the neighbours' words: the low word is the mask (or liquid marker), the high word
+    // of a liquid neighbour its claim word
+    unsigned long long lw[26];
+#pragma unroll
+    for (int kk = 0; kk < 26; kk++)
+        lw[kk] = ((valid >> kk) & 1u) ? *reinterpret_cast<const unsigned long long *>(&d.cells[q + gr.off[kk]].lm)
+                                      : static_cast<unsigned long long>(kMaskUnknown);
+    // The new cell's mask: its liquid neighbours at its first visit are those liquid now
+    // and not claimed in this step (every claimed cell is captured in this step, and the
+    // claims are final). Until its store below, the new cell's own words read as a
+    // claimed liquid cell, which no other capture counts.
+    uint32_t liquid = 0, mw[26];
+#pragma unroll
+    for (int kk = 0; kk < 26; kk++) {
+        liquid |= static_cast<uint32_t>(is_unclaimed_liquid(lw[kk])) << kk;
+        mw[kk] = static_cast<uint32_t>(lw[kk]);
+    }
+    // updates only where the mask still holds q, all in flight together; their results
+    // are used after the octahedron is built, which hides their round trip
+    uint32_t need = 0;
+#pragma unroll
+    for (int kk = 0; kk < 26; kk++) {
+        const uint32_t bit = 1u << kOpposite.v[kk];
+        need |= static_cast<uint32_t>((mw[kk] & (kMaskUnknown | bit)) == bit) << kk;
+    }
+#pragma unroll
+    for (int kk = 0; kk < 26; kk++)
+        if ((need >> kk) & 1u) mw[kk] = atomicAnd(mask_word(d, q + gr.off[kk]), ~(1u << kOpposite.v[kk]));
+    // a neighbour at or below the claimant's index still had q liquid at its visit
+    // in the reference's index order: its keep word gets this step's tag (every writer
+    // of a step writes the same value)
+#pragma unroll
+    for (int kk = 0; kk < 26; kk++)
+        if (((need >> kk) & 1u) && q + gr.off[kk] <= jc) keep_word(d, q + gr.off[kk])[0] = serial + 1;
+    const double xp = (c.x + d.xoff + nb_dx(l)) + 0.5;
+    const double yp = (c.y + d.yoff + nb_dy(l)) + 0.5;
+    const double zp = (c.z + nb_dz(l)) + 0.5;
+    const Octahedron oc = new_octahedron(gv, wcx, wcy, wcz, xp, yp, zp);
+    // The new cell's record, whole: nothing else writes it in this pass.
+    uint4 *r4 = reinterpret_cast<uint4 *>(d.cells + q);
+    r4[0] = make_uint4(liquid, 0u, __float_as_uint(static_cast<float>(oc.dl)), __float_as_uint(0.0f));
+    r4[1] = make_uint4(own.x, static_cast<uint32_t>(h), own.z,
+                       (own.w & 0xFFu) | (static_cast<uint32_t>(kActive) << 8) | (static_cast<uint32_t>(kFresh) << 16));
+    set_alarm(d, serial + 1, q);
+    // The new octahedron's record: its 26 critical lengths, computed once here (its
+    // evaluations read them back), and its centre; whole 16-byte pieces of one line.
+    {
+        const Faces f = faces_of(gv);
+        float4 *o4 = reinterpret_cast<float4 *>(&d.octa[q]);
+#pragma unroll
+        for (int i = 0; i < 6; i++)
+            o4[i] = make_float4(critical_length(f, xp, yp, zp, oc.cx, oc.cy, oc.cz, 4 * i),
+                                critical_length(f, xp, yp, zp, oc.cx, oc.cy, oc.cz, 4 * i + 1),
+                                critical_length(f, xp, yp, zp, oc.cx, oc.cy, oc.cz, 4 * i + 2),
+                                critical_length(f, xp, yp, zp, oc.cx, oc.cy, oc.cz, 4 * i + 3));
+        const uint2 xb = __builtin_bit_cast(uint2, oc.cx), yb = __builtin_bit_cast(uint2, oc.cy),
+                    zb = __builtin_bit_cast(uint2, oc.cz);
+        uint4 *u4 = reinterpret_cast<uint4 *>(&d.octa[q]);
+        u4[6] = make_uint4(__float_as_uint(critical_length(f, xp, yp, zp, oc.cx, oc.cy, oc.cz, 24)),
+                           __float_as_uint(critical_length(f, xp, yp, zp, oc.cx, oc.cy, oc.cz, 25)), xb.x, xb.y);
+        u4[7] = make_uint4(yb.x, yb.y, zb.x, zb.y);
+    }
+    uint32_t emptied = 0;
+#pragma unroll
+    for (int kk = 0; kk < 26; kk++) {
+        const uint32_t bit = 1u << kOpposite.v[kk];
+        emptied |= static_cast<uint32_t>(((need >> kk) & 1u) && (mw[kk] & (kMaskUnknown | kMaskNow)) == bit) << kk;
+    }
+    for (uint32_t m = emptied; m; m &= m - 1) set_alarm(d, serial + 1, q + gr.offset(__builtin_ctz(m)));
+    return q;
+}
+
+// Pass B over the n claimants that claimant(k, cell, bits) gives: the winners of up to two rounds
+// are gathered in LDS with the claims they won, their captures numbered by a block scan and built
+// one per lane (a winner mostly has one; one lane per capture keeps every lane's chain of dependent
+// accesses to one capture).
+template <int BLOCK, typename F>
+__device__ __forceinline__ void apply_body(const DomainView &d, uint32_t serial, uint32_t n, F &&claimant,
+                                           ApplyLds<BLOCK> &s, uint32_t *cnt, uint32_t *lohi) {
+    constexpr uint32_t kWaves = BLOCK / 64;
+    const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const Grid gr = grid_of(d);
-    if (threadIdx.x == 0) nwin = 0;
-    // two claimants per thread and round, their loads in flight together (a slice holds a little
-    // more than one workgroup's worth)
-    constexpr uint32_t kPer = 2;
-    for (uint32_t k0 = 0; k0 < n; k0 += kPer * kBlock) {
-        uint32_t j[kPer], cb[kPer], won[kPer];
-#pragma unroll
-        for (uint32_t e = 0; e < kPer; e++) {
-            const uint32_t k = k0 + e * kBlock + threadIdx.x;
-            j[e] = 0;
-            cb[e] = 0;
-            won[e] = 0;
-            if (k < n) {
-                j[e] = d.claim_cell[beg + k];
-                cb[e] = d.claim_bits[beg + k];
-            }
-        }
-#pragma unroll
-        for (uint32_t e = 0; e < kPer; e++) {
+    uint32_t qlo = 0xFFFFFFFFu, qhi = 0;
+    if (threadIdx.x == 0) s.nwin = 0;
+    __syncthreads();
+    for (uint32_t k0 = 0; k0 < n; k0 += BLOCK) {
+        const uint32_t k = k0 + threadIdx.x;
+        uint32_t j = 0, cb = 0, won = 0;
+        int32_t gid = 0;
+        if (k < n) {
+            claimant(k, j, cb);
+            gid = d.cells[j].gid;
             uint32_t cw[26];
 #pragma unroll
-            for (int l = 0; l < 26; l++) cw[l] = ((cb[e] >> l) & 1u) ? *claim_word(d, j[e] + gr.off[l]) : kClaimNone;
+            for (int l = 0; l < 26; l++) cw[l] = ((cb >> l) & 1u) ? *claim_word(d, j + gr.off[l]) : kClaimNone;
 #pragma unroll
-            for (int l = 0; l < 26; l++) won[e] |= static_cast<uint32_t>(cw[l] == j[e]) << l;
+            for (int l = 0; l < 26; l++) won |= static_cast<uint32_t>(cw[l] == j) << l;
+        }
+        const uint32_t slot = wave_append(won != 0, &s.nwin);
+        if (won) {
+            s.cell[slot] = j;
+            s.bits[slot] = won;
+            s.gid[slot] = gid;
         }
         __syncthreads();
-#pragma unroll
-        for (uint32_t e = 0; e < kPer; e++) {
-            const uint32_t slot = wave_append(won[e] != 0, &nwin);
-            if (won[e]) {
-                d.claim_cell[beg + slot] = j[e];
-                d.claim_bits[beg + slot] = won[e];
-            }
-        }
-    }
-    __syncthreads();
-    if (threadIdx.x == 0) d.slice_claims[b] = nwin;
-}
-
-// Pass B2 over the winners: workgroup a takes the winners of the kApplyGroup slices a*kApplyGroup ..
-// (a few dozen each). The captures of a round of winners are numbered by a block scan and built one
-// per lane (a winner mostly has one; one lane per capture keeps every lane's chain of dependent
-// accesses to one capture): the winner's octahedron gives the captured cell's
-// (src/CAupdate.cpp:353-563, 717), the new cell is due at the next step, and the captured cell
-// leaves the liquid masks of its neighbours. Only masks that still hold it are updated: the masks
-// are read first, and a cell's bit is cleared by its capture alone, so the read decides exactly.
-// A neighbour whose mask this empties is a solidification candidate of this step, staged per
-// workgroup in LDS and written to the workgroup's own region of the candidate buffer (no shared
-// counter); a wave that finds the stage full appends to the overflow list in the other list buffer.
-__device__ __forceinline__ void apply_body(const DomainView &d, int p, uint32_t a, uint32_t nbc) {
-    __shared__ unsigned long long sh[kBlock / 64];
-    __shared__ uint32_t wave_tot[kBlock / 64];
-    __shared__ uint32_t pre[kBlock + 1];
-    __shared__ uint32_t won_cell[kBlock], won_bits[kBlock];
-    __shared__ uint32_t cstage[kCandStage];
-    __shared__ uint32_t ncstage, stage_end;
-    StepCtl *ctl = d.ctl;
-    if (ctl->done) return;
-    // stage capacity in use (kCandStage; less only when a caller narrows it)
-    const uint32_t cap = d.cand_cap < kCandStage ? d.cand_cap : kCandStage;
-    if (threadIdx.x == 0) {
-        ncstage = 0;
-        stage_end = cap;
-    }
-    uint32_t *overflow = d.list[1 - p];
-    uint32_t beg[kApplyGroup], upto[kApplyGroup], n = 0;
-#pragma unroll
-    for (uint32_t g = 0; g < kApplyGroup; g++) {
-        const uint32_t b = a * kApplyGroup + g;
-        uint32_t e = 0, cnt = 0;
-        beg[g] = 0;
-        if (b < nbc) {
-            frontier_slice(ctl->count[p], d.list_cap, b, nbc, beg[g], e);
-            cnt = d.slice_claims[b];
-        }
-        n += cnt;
-        upto[g] = n;
-    }
-    const uint32_t serial = ctl->serial[p];
-    const Grid gr = grid_of(d);
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    unsigned long long ncap = 0;
-    uint32_t qlo = 0xFFFFFFFFu, qhi = 0;
-    for (uint32_t k0 = 0; k0 < n; k0 += kBlock) {
-        // This round's winners in LDS, and the block-wide exclusive prefix of their capture counts.
-        const uint32_t k = k0 + threadIdx.x;
-        uint32_t j = 0, won = 0;
-        if (k < n) {
-            uint32_t i = beg[0] + k;
-#pragma unroll
-            for (uint32_t g = 1; g < kApplyGroup; g++)
-                if (k >= upto[g - 1]) i = beg[g] + (k - upto[g - 1]);
-            j = d.claim_cell[i];
-            won = d.claim_bits[i];
-        }
-        const uint32_t cnt = __builtin_popcount(won);
+        const uint32_t nwin = s.nwin;
+        __syncthreads();
+        if (k0 + BLOCK < n && nwin <= BLOCK) continue;  // room for another round
+        // the captures of the winners gathered so far: thread t numbers those of winners 2t, 2t + 1
+        const uint32_t w0 = 2 * threadIdx.x;
+        const uint32_t b0 = w0 < nwin ? s.bits[w0] : 0u, b1 = w0 + 1 < nwin ? s.bits[w0 + 1] : 0u;
+        const uint32_t c0 = __builtin_popcount(b0), mine = c0 + __builtin_popcount(b1);
         uint32_t wtot;
-        const uint32_t incl = wave_inclusive_scan(cnt, wtot);
-        if (lane == 63) wave_tot[wave] = wtot;
-        won_cell[threadIdx.x] = j;
-        won_bits[threadIdx.x] = won;
+        const uint32_t incl = wave_inclusive_scan(mine, wtot);
+        if (lane == 0) s.tot[wave] = wtot;
         __syncthreads();
-        uint32_t base = 0, total = 0;
-        for (int w = 0; w < kBlock / 64; w++) {
-            if (w < wave) base += wave_tot[w];
-            total += wave_tot[w];
+        uint32_t first = incl - mine, total = 0;
+#pragma unroll
+        for (uint32_t q = 0; q < kWaves; q++) {
+            const uint32_t v = s.tot[q];
+            first += q < wave ? v : 0u;
+            total += v;
         }
-        pre[threadIdx.x] = base + incl - cnt;
-        if (threadIdx.x == 0) pre[kBlock] = total;
-        __syncthreads();
-        // One capture per lane: item t belongs to the winner s with pre[s] <= t < pre[s + 1].
-        for (uint32_t t0 = 0; t0 < total; t0 += kBlock) {
-            const uint32_t t = t0 + threadIdx.x;
-            uint32_t q = 0, emptied = 0;
-            if (t < total) {
-                uint32_t lo = 0, hi = kBlock;  // pre[lo] <= t < pre[hi]
-                while (hi - lo > 1) {
-                    const uint32_t mid = (lo + hi) >> 1;
-                    if (pre[mid] <= t)
-                        lo = mid;
-                    else
-                        hi = mid;
-                }
-                const uint32_t jc = won_cell[lo];
-                uint32_t bits = won_bits[lo];
-                for (uint32_t r = t - pre[lo]; r; r--) bits &= bits - 1;
-                const int l = __builtin_ctz(bits);
-                q = jc + gr.offset(l);
-                // the winner's grain and centre (float, as the capture uses it), loaded with the
-                // neighbours' words below
-                const int h = d.cells[jc].gid;
-                const Octa &e = d.octa[jc];
-                const float wcx = static_cast<float>(e.x), wcy = static_cast<float>(e.y), wcz = static_cast<float>(e.z);
-                const Coord c = decode(jc, gr);
-                const Coord cqc{c.x + nb_dx(l), c.y + nb_dy(l), c.z + nb_dz(l)};
-                const uint32_t valid = valid_neighbours(cqc, gr.X, gr.Y, gr.nzA);
-                // the grain's orientation, loaded with the neighbours' words below rather than
-                // after the mask atomics
-                int o = orientation_of(h);
-                if (o < 0) {
-                    atomicOr(&ctl->error, 2);
-                    o = 0;
-                }
-                float gv[9];
-#pragma unroll
-                for (int m = 0; m < 9; m++) gv[m] = d.guv[9 * o + m];
-                // the neighbours' words: the low word is the mask (or liquid marker), the high word
-                // of a liquid neighbour its claim word
-                unsigned long long lw[26];
-#pragma unroll
-                for (int kk = 0; kk < 26; kk++)
-                    lw[kk] = ((valid >> kk) & 1u) ? *reinterpret_cast<const unsigned long long *>(&d.cells[q + gr.off[kk]].lm)
-                                                  : static_cast<unsigned long long>(kMaskUnknown);
-                // The new cell's mask: its liquid neighbours at its first visit are those liquid now
-                // and not claimed in this step (every claimed cell is captured in this step, and the
-                // claims are final). Until its store below, the new cell's own words read as a
-                // claimed liquid cell, which no other capture counts.
-                uint32_t liquid = 0, mw[26];
-#pragma unroll
-                for (int kk = 0; kk < 26; kk++) {
-                    liquid |= static_cast<uint32_t>(is_unclaimed_liquid(lw[kk])) << kk;
-                    mw[kk] = static_cast<uint32_t>(lw[kk]);
-                }
-                // updates only where the mask still holds q, all in flight together; their results
-                // are used after the octahedron is built, which hides their round trip
-                uint32_t need = 0;
-#pragma unroll
-                for (int kk = 0; kk < 26; kk++) {
-                    const uint32_t bit = 1u << kOpposite.v[kk];
-                    need |= static_cast<uint32_t>((mw[kk] & (kMaskUnknown | bit)) == bit) << kk;
-                }
-#pragma unroll
-                for (int kk = 0; kk < 26; kk++)
-                    if ((need >> kk) & 1u) mw[kk] = atomicAnd(mask_word(d, q + gr.off[kk]), ~(1u << kOpposite.v[kk]));
-                // a neighbour at or below the claimant's index still had q liquid at its visit
-                // in the reference's index order: its keep word gets this step's tag (every writer
-                // of a step writes the same value)
-#pragma unroll
-                for (int kk = 0; kk < 26; kk++)
-                    if (((need >> kk) & 1u) && q + gr.off[kk] <= jc) keep_word(d, q + gr.off[kk])[0] = serial + 1;
-                const double xp = (c.x + d.xoff + nb_dx(l)) + 0.5;
-                const double yp = (c.y + d.yoff + nb_dy(l)) + 0.5;
-                const double zp = (c.z + nb_dz(l)) + 0.5;
-                const Octahedron oc = new_octahedron(gv, wcx, wcy, wcz, xp, yp, zp);
-                Cell &cq = d.cells[q];
-                cq.gid = h;
-                cq.dl = static_cast<float>(oc.dl);
-                cq.thr = 0.0f;
-                cq.flags = kFresh;
-                cq.ct = kActive;
-                set_alarm(d, serial + 1, q);
-                ncap++;
+        for (uint32_t t0 = 0; t0 < total; t0 += BLOCK) {
+            uint32_t pos = first - t0;  // wraps below the turn: not in [0, BLOCK)
+            for (uint32_t m = b0; m; m &= m - 1, pos++)
+                if (pos < BLOCK) s.item[pos] = (w0 << 5) | static_cast<uint32_t>(__builtin_ctz(m));
+            for (uint32_t m = b1; m; m &= m - 1, pos++)
+                if (pos < BLOCK) s.item[pos] = ((w0 + 1) << 5) | static_cast<uint32_t>(__builtin_ctz(m));
+            __syncthreads();
+            const bool has = t0 + threadIdx.x < total;
+            if (has) {
+                const uint32_t it = s.item[threadIdx.x];
+                const uint32_t q = capture(d, gr, serial, s.cell[it >> 5], static_cast<int>(it & 31u), s.gid[it >> 5]);
                 qlo = q < qlo ? q : qlo;
                 qhi = q > qhi ? q : qhi;
-#pragma unroll
-                for (int kk = 0; kk < 26; kk++) {
-                    const uint32_t bit = 1u << kOpposite.v[kk];
-                    emptied |= static_cast<uint32_t>(((need >> kk) & 1u) && (mw[kk] & (kMaskUnknown | kMaskNow)) == bit) << kk;
-                }
-                cq.lm = liquid;
-                // The new octahedron's record: its 26 critical lengths, computed once here (its
-                // evaluations read them back), and its centre; whole 16-byte pieces of one line.
-                {
-                    const Faces f = faces_of(gv);
-                    float4 *o4 = reinterpret_cast<float4 *>(&d.octa[q]);
-#pragma unroll
-                    for (int i = 0; i < 6; i++)
-                        o4[i] = make_float4(critical_length(f, xp, yp, zp, oc.cx, oc.cy, oc.cz, 4 * i),
-                                            critical_length(f, xp, yp, zp, oc.cx, oc.cy, oc.cz, 4 * i + 1),
-                                            critical_length(f, xp, yp, zp, oc.cx, oc.cy, oc.cz, 4 * i + 2),
-                                            critical_length(f, xp, yp, zp, oc.cx, oc.cy, oc.cz, 4 * i + 3));
-                    const uint2 xb = __builtin_bit_cast(uint2, oc.cx), yb = __builtin_bit_cast(uint2, oc.cy),
-                                zb = __builtin_bit_cast(uint2, oc.cz);
-                    uint4 *u4 = reinterpret_cast<uint4 *>(&d.octa[q]);
-                    u4[6] = make_uint4(__float_as_uint(critical_length(f, xp, yp, zp, oc.cx, oc.cy, oc.cz, 24)),
-                                       __float_as_uint(critical_length(f, xp, yp, zp, oc.cx, oc.cy, oc.cz, 25)), xb.x, xb.y);
-                    u4[7] = make_uint4(yb.x, yb.y, zb.x, zb.y);
-                }
             }
-            // Candidates: staged in LDS (one LDS atomic per wave); a wave that finds the stage
-            // full appends to the global list directly. Waves reserve disjoint stage ranges in
-            // the order of their atomics, so every wave after the first that does not fit does
-            // not fit either, and every range below that wave's base is filled: stage_end (the
-            // least base of a wave that did not fit) bounds the entries copied out below.
-            const uint32_t ce = __builtin_popcount(emptied);
-            uint32_t ctot;
-            const uint32_t cincl = wave_inclusive_scan(ce, ctot);
-            if (ctot) {
-                uint32_t cbase = 0;
-                if (lane == 63) cbase = atomicAdd(&ncstage, ctot);
-                cbase = __shfl(cbase, 63, 64);
-                const bool staged = cbase + ctot <= cap;
-                if (!staged) {
-                    if (lane == 63) {
-                        atomicMin(&stage_end, cbase);
-                        cbase = atomicAdd(&ctl->ncand, ctot);
-                    }
-                    cbase = __shfl(cbase, 63, 64);
-                }
-                uint32_t pos = cbase + cincl - ce;
-                for (uint32_t r = emptied; r; r &= r - 1, pos++) {
-                    const uint32_t cell = q + gr.offset(__builtin_ctz(r));
-                    if (staged)
-                        cstage[pos] = cell;
-                    else if (pos < d.list_cap)
-                        overflow[pos] = cell;
-                }
-            }
+            count_event(has, &cnt[kCntCap]);
+            __syncthreads();
         }
+        if (threadIdx.x == 0) s.nwin = 0;
         __syncthreads();
     }
-    // The staged candidates go to this workgroup's region (the barrier orders thread 0's
-    // initialisation before these reads when the workgroup had no winners).
-    __syncthreads();
-    const uint32_t staged = ncstage < stage_end ? ncstage : stage_end;
-    for (uint32_t i = threadIdx.x; i < staged; i += kBlock) d.cand[a * kCandStage + i] = cstage[i];
-    if (threadIdx.x == 0) d.cand_count[a] = staged;
-    put_part(d, kPartCap, a, ncap, sh);
-    // New cells widen the range of active cells (least and greatest index of this workgroup).
-    __shared__ uint32_t lohi[2 * (kBlock / 64)];
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-        const uint32_t a2 = __shfl_down(qlo, o, 64), b2 = __shfl_down(qhi, o, 64);
-        qlo = a2 < qlo ? a2 : qlo;
-        qhi = b2 > qhi ? b2 : qhi;
-    }
-    if (lane == 0) {
-        lohi[2 * wave] = qlo;
-        lohi[2 * wave + 1] = qhi;
-    }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        for (int w = 1; w < kBlock / 64; w++) {
-            qlo = lohi[2 * w] < qlo ? lohi[2 * w] : qlo;
-            qhi = lohi[2 * w + 1] > qhi ? lohi[2 * w + 1] : qhi;
-        }
-        // the range rarely grows: most workgroups need no atomic
-        if (qlo <= qhi) {
-            if (qlo < ctl->elo) atomicMin(&ctl->elo, qlo);
-            if (qhi > ctl->ehi) atomicMax(&ctl->ehi, qhi);
-        }
+    if (qlo <= qhi) {
+        atomicMin(&lohi[0], qlo);
+        atomicMax(&lohi[1], qhi);
     }
 }
 
-// The settle pass has one workgroup per apply workgroup: workgroup b takes the candidates of
-// region b and a share of the overflow list.
-__host__ __device__ constexpr uint32_t settle_blocks(uint32_t claim_blocks) { return apply_blocks(claim_blocks); }
+// The range of active cells widened by a workgroup's new ones (lohi in LDS; every thread calls it).
+// It rarely grows: most workgroups need no atomic.
+__device__ __forceinline__ void widen_range(const DomainView &d, const uint32_t *lohi) {
+    __syncthreads();
+    if (threadIdx.x == 0 && lohi[0] <= lohi[1]) {
+        if (lohi[0] < d.ctl->elo) atomicMin(&d.ctl->elo, lohi[0]);
+        if (lohi[1] > d.ctl->ehi) atomicMax(&d.ctl->ehi, lohi[1]);
+    }
+}
 
-// Pass C over the candidates: a cell whose every claim-time liquid neighbour was captured in this
-// step by a lower-indexed cell has no liquid neighbour left when the reference visits it in index
-// order, so it grows and turns solid now (src/CAupdate.cpp:333-334, 722-725); a capture by itself
-// or by a later cell leaves it active, with no liquid neighbour: it turns solid at the next step. A
-// cell not past its liquidus time is not visited this step.
-// A candidate's mask was emptied by this step's captures, each of which tagged the candidate's
-// keep word with this step when its claimant's index is >= the candidate's: the tag decides.
-__device__ __forceinline__ void settle_body(const DomainView &d, int p, int layer, uint32_t b, uint32_t nb) {
-    __shared__ unsigned long long sh[kBlock / 64];
+// The solidifications that the last executed step left to the next one (solid_since_last), made now
+// that a caller looks at the state. The cells are due at the next step, whose calendar slot stays
+// as it is. due: the cells due at the next step.
+template <int BLOCK, uint32_t CAP>
+__device__ __forceinline__ void settle_body(const DomainView &d, const Growth &g, int next_cycle, uint32_t next_serial,
+                                            int layer, uint32_t b, uint32_t nb, uint32_t *list, uint32_t *tot,
+                                            uint32_t *cnt) {
+    for_due<BLOCK, CAP, false>(d, next_serial, b, nb, list, tot, [&](bool has, uint32_t j, const CellWords &w) {
+        const bool late = has && (w.ct & kTypeMask) == kActive && solid_since_last(w, next_serial, next_cycle, layer);
+        if (late) solidify(d, g, j, w, growth_index(d, w.cts, w.lid, j, next_cycle - 1));
+        count_event(late, &cnt[kCntLate]);
+    });
+}
+
+// The running totals since the last booking, summed by one workgroup over the rows of every
+// workgroup and added to the run's statistics; the rows start at zero again. With S0 .. S - 1 the
+// serials of the steps since then, an event of serial s that adds a cell to a step's count from the
+// same step on adds it to S - s steps, one that does so from the step after to S - 1 - s. The
+// reference's numSteer of a step: active cells past their liquidus time at the start of its capture
+// pass.
+template <int BLOCK>
+__device__ __forceinline__ void book_totals(const DomainView &d, uint32_t serial_now, unsigned long long (*red)[BLOCK / 64]) {
     StepCtl *ctl = d.ctl;
-    if (ctl->done) return;
-    const int cycle = ctl->cycle[p];
-    const uint32_t serial = ctl->serial[p];
-    const uint32_t nown = d.cand_count[b];
-    const uint32_t nover = ctl->ncand < d.list_cap ? ctl->ncand : d.list_cap;
-    const uint32_t *own = d.cand + b * kCandStage;
-    const uint32_t *overflow = d.list[1 - p];
-    unsigned long long nsol = 0;
-    // the growth table is read from global memory: a candidate has mostly been growing on the
-    // plateau, where the replay needs no table entry, so staging it would cost more than it saves
-    const Growth g = growth_of(d);
-    auto settle = [&](uint32_t r) {
-        const CellWords w = load_cell(d.cells + r);
-        if ((w.ct & kTypeMask) != kActive || !(cycle > w.cts && w.lid <= layer)) return;
-        if (static_cast<uint32_t>(w.lm >> 32) == serial + 1) {
-            set_alarm(d, serial + 1, r);
-        }
-        else {
-            solidify(d, g, r, w, growth_index(d, w.cts, w.lid, r, cycle));
-            nsol++;
-        }
-    };
-    for (uint32_t i = threadIdx.x; i < nown; i += kBlock) settle(own[i]);
-    for (uint32_t i = b * kBlock + threadIdx.x; i < nover; i += nb * kBlock) settle(overflow[i]);
-    put_part(d, kPartSettleSol, b, nsol, sh);
-}
-
-
-// The list of the next step is every set bit of its calendar slot, in ascending cell index, over
-// the chunks of the range of active cells; the slot is cleared as it is read. One pass: workgroup
-// b of nbw - 1 takes units b, b + nbw - 1, ... of kUnitChunks chunks, counts a unit's bits, and
-// finds the unit's offset by decoupled look-back over the units before it (each unit publishes its
-// count, then its inclusive prefix, as one tagged 64-bit word); then it writes the unit's cells.
-// A unit's count never waits on anything, and a unit waits only for lower units, of workgroups
-// dispatched before it or of earlier rounds of workgroups that are resident with it (the plain
-// launch has at most 513 workgroups, and at 3 workgroups per CU all are resident); each wait is
-// bounded all the same (error 8). The last workgroup books the step meanwhile. (The range is a few
-// thousand chunks at 800^3: several hundred units, one to two per CU; measured there, units of
-// 4, 8, 16 chunks with up to 512, 256, 128 workgroups: 23.9, 29.5, 65.9 us.)
-constexpr uint32_t kChunkWords = 8 * kBlock;  // thread t of a chunk holds its words 8t .. 8t + 7
-constexpr uint32_t kChunkCells = 32 * kChunkWords;
-constexpr uint32_t kUnitChunks = 4;
-constexpr uint32_t kRebuildStage = 8192;  // list entries of a unit staged in LDS (32 KB)
-constexpr unsigned long long kFlagCount = 1ull << 32;   // value = the chunk's own count
-constexpr unsigned long long kFlagPrefix = 2ull << 32;  // value = count of the chunk and all before it
-constexpr unsigned long long kFlagState = 3ull << 32;
-constexpr unsigned long long kFlagTag = ~((1ull << 34) - 1);
-constexpr uint32_t kLookBackSpins = 1u << 20;  // bound on the waits of one look-back (error 8 past it)
-
-__device__ __forceinline__ bool chunk_range(const DomainView &d, uint32_t &c0, uint32_t &c1) {
-    const uint32_t lo = d.ctl->elo;
-    uint32_t hi = d.ctl->ehi;
-    if (lo > hi) return false;
-    if (hi >= static_cast<uint64_t>(d.ncell)) hi = static_cast<uint32_t>(d.ncell - 1);
-    c0 = lo / kChunkCells;
-    c1 = hi / kChunkCells;
-    return true;
-}
-__device__ __forceinline__ uint32_t *next_slot(const DomainView &d, int p) {
-    return d.alarms + ((d.ctl->serial[p] + 1) % kAlarmSlots) * alarm_stride(d.ncell);
-}
-// Flags of one rebuild carry its tag (the rebuild sequence number, advanced by the kernels that
-// precede a rebuild: the capture pass, rewake and layer setup; tags cycle through 2^30 - 1 nonzero values), so the
-// flags of earlier rebuilds need no clearing.
-__device__ __forceinline__ unsigned long long flag_tag(uint32_t seq) {
-    return static_cast<unsigned long long>(seq % ((1u << 30) - 1) + 1) << 34;
-}
-__device__ __forceinline__ void publish(unsigned long long *f, unsigned long long v) {
-    __hip_atomic_store(f, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-__device__ __forceinline__ unsigned long long peek(unsigned long long *f) {
-    return __hip_atomic_load(f, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-
-// Cells before unit u (u > 0), by one wave: windows of 64 predecessors, nearest first, summed up
-// to the nearest one holding a prefix; unit 0 always holds one.
-__device__ uint32_t look_back(const DomainView &d, uint32_t u, unsigned long long tag) {
-    const int lane = threadIdx.x & 63;
-    uint32_t excl = 0, spins = 0;
-    long long j0 = static_cast<long long>(u) - 1;
-    for (;;) {
-        const long long j = j0 - lane;
-        const unsigned long long f = j >= 0 ? peek(d.chunk_flag + j) : (tag | kFlagPrefix);
-        const bool valid = (f & kFlagTag) == tag && (f & kFlagState) != 0;
-        const unsigned long long pm = __ballot((f & kFlagTag) == tag && (f & kFlagState) == kFlagPrefix);
-        const unsigned long long vm = __ballot(valid);
-        const int np = pm ? __builtin_ctzll(pm) : 63;
-        const unsigned long long need = np >= 63 ? ~0ull : ((2ull << np) - 1);
-        if ((vm & need) != need) {
-            if (++spins > kLookBackSpins) {
-                if (lane == 0) atomicOr(&d.ctl->error, 8);
-                return excl;
-            }
-            __builtin_amdgcn_s_sleep(2);
-            continue;
-        }
-        uint32_t v = lane <= np ? static_cast<uint32_t>(f) : 0u;
-#pragma unroll
-        for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-        excl += v;
-        if (pm) return excl;
-        j0 -= 64;
-    }
-}
-
-// The step's counters: the per-workgroup slots of each row summed over the grids that wrote them
-// (nb capture workgroups, the apply and settle workgroups that go with them, nnb nucleation
-// workgroups).
-constexpr uint32_t kMaxPartsPerThread = 8;  // nparts <= 8 * kBlock
-struct StepSums {
-    unsigned long long v[kPartRows];
-};
-__device__ __forceinline__ StepSums sum_parts(const DomainView &d, uint32_t nb, uint32_t nnb) {
-    __shared__ unsigned long long red[kPartRows][kBlock / 64];
-    const uint32_t na = apply_blocks(nb);
-    StepSums s;
-#pragma unroll
+#pragma unroll 1
     for (int r = 0; r < kPartRows; r++) {
-        const uint32_t n = (r >= kPartNucSol && r <= kPartNucNn) ? nnb
-                           : (r == kPartCap ? na : (r == kPartSettleSol ? settle_blocks(nb) : nb));
-        const unsigned long long *row = d.part + static_cast<size_t>(r) * d.nparts;
+        unsigned long long *row = d.part + static_cast<size_t>(r) * d.nparts;
         unsigned long long v = 0;
-#pragma unroll
-        for (uint32_t k = 0; k < kMaxPartsPerThread; k++) {
-            const uint32_t i = threadIdx.x + k * kBlock;
-            if (i < n) v += row[i];
+        for (uint32_t i = threadIdx.x; i < d.nparts; i += BLOCK) {
+            const unsigned long long x = row[i];
+            v += x;
+            if (x) row[i] = 0;
         }
 #pragma unroll
         for (int o = 32; o > 0; o >>= 1) v += __shfl_down(v, o, 64);
         if ((threadIdx.x & 63) == 0) red[r][threadIdx.x >> 6] = v;
     }
     __syncthreads();
+    if (threadIdx.x != 0) return;
+    unsigned long long v[kPartRows];
 #pragma unroll
     for (int r = 0; r < kPartRows; r++) {
-        unsigned long long v = 0;
-        for (int w = 0; w < kBlock / 64; w++) v += red[r][w];
-        s.v[r] = v;
+        v[r] = 0;
+        for (int w = 0; w < BLOCK / 64; w++) v[r] += red[r][w];
     }
-    return s;
+    StepStats st = *d.stats;
+    const unsigned long long S = serial_now, n = S - ctl->serial_booked;
+    const unsigned long long ent = S * v[kPartEnt] - v[kPartEntAt];          // from the same step on
+    const unsigned long long sol = (S - 1) * v[kPartSol] - v[kPartSolAt];    // from the next step on
+    const unsigned long long act = S * v[kPartAct] - v[kPartActAt];          // from the same step on
+    const unsigned long long cap = (S - 1) * v[kPartCap] - v[kPartCapAt];    // from the next step on
+    const unsigned long long frontier = n * ctl->nonwaiting + ent - sol;
+    st.frontier += frontier;
+    st.waiting += n * ctl->nactive + act + cap - sol - frontier;
+    st.solidified += v[kPartSol];
+    st.captures += v[kPartCap];
+    st.activated += v[kPartAct];
+    st.nucleated += v[kPartNn];
+    st.evaluated += v[kPartEval];
+    st.masks += v[kPartMask];
+    *d.stats = st;
+    ctl->nonwaiting += v[kPartEnt] - v[kPartSol];
+    ctl->nactive += v[kPartAct] + v[kPartCap] - v[kPartSol];
+    ctl->serial_booked = serial_now;
 }
 
-// Closing a rebuild (the list's length is set by the last unit, or here when there is none): with
-// account the step's counters are booked and a domain with autostop ends at a check step (cycle a
+// The end of a domain: stopped by an error flag (its later steps would work on a broken state; the
+// host learns of it at its next check or poll), or, with autostop, at a check step (cycle a
 // multiple of 1000) with no liquid left: liquid cells only ever leave the liquid state by capture
 // or nucleation, so the reference's superheated + undercooled count (src/CAupdate.cpp:738-783) is
-// the initial liquid count minus both. A rebuild between steps passes account 0.
-__device__ __forceinline__ void set_count(const DomainView &d, int p, uint32_t total) {
-    d.ctl->count[1 - p] = total < d.list_cap ? total : d.list_cap;
-    if (total > d.list_cap) atomicOr(&d.ctl->error, 1);
-}
-__device__ __forceinline__ void close_rebuild(const DomainView &d, int p, int account, uint32_t nb, uint32_t nnb,
-                                              uint32_t nunits) {
+// the initial liquid count minus both.
+__device__ __forceinline__ void end_domain(const DomainView &d, int cycle) {
     StepCtl *ctl = d.ctl;
-    StepSums sums;
-    if (account) sums = sum_parts(d, nb, nnb);
-    if (threadIdx.x != 0) return;
-    if (!nunits) set_count(d, p, 0);
-    if (!account) return;
-    // Counters are read once and written once (every access is a dependent round trip for this
-    // single thread).
-    const unsigned long long *v = sums.v;
-    const unsigned long long sol = v[kPartClaimSol] + v[kPartNucSol] + v[kPartSettleSol];
-    StepStats st = *d.stats;
-    const unsigned long long nonwaiting = ctl->nonwaiting + v[kPartClaimEntered] + v[kPartNucEntered];
-    const unsigned long long active = ctl->nactive + v[kPartNucAct];
-    st.solidified += sol;
-    st.evaluated += v[kPartClaimEval];
-    st.masks += v[kPartClaimMask];
-    st.captures += v[kPartCap];
-    st.nucleated += v[kPartNucNn];
-    st.activated += v[kPartNucAct];
-    // The reference's numSteer of this step: active cells past their liquidus time at the start of
-    // its capture pass.
-    st.frontier += nonwaiting;
-    st.waiting += active - nonwaiting;
-    *d.stats = st;
-    ctl->nonwaiting = nonwaiting - sol;
-    ctl->nactive = active + v[kPartCap] - sol;
-    const int cycle = ctl->cycle[p];
-    ctl->last_cycle = cycle;
-    // A domain whose kernels raised an error flag stops here: its later steps would work on a
-    // truncated list. The host learns of it at its next check (plain path) or poll (ensemble).
     const int32_t err = ctl->error;
-    if (err) {
-        ctl->done = 1;
-        ctl->final_cycle = cycle;
-        if (d.status_err) *d.status_err = err;
-        if (d.status) *d.status = cycle;
-        return;
-    }
-    if (d.autostop && cycle % 1000 == 0 &&
-        d.liquid0 - static_cast<long long>(st.captures) - static_cast<long long>(st.activated) == 0) {
-        ctl->done = 1;
-        ctl->final_cycle = cycle;
-        if (d.status) *d.status = cycle;
-    }
-}
-
-__device__ __forceinline__ void rebuild_body(const DomainView &d, int p, int account, uint32_t nb, uint32_t nnb,
-                                             uint32_t b, uint32_t nbw) {
-    __shared__ uint32_t sh_excl;
-    __shared__ uint32_t wave_tot[kUnitChunks][kBlock / 64];
-    __shared__ uint32_t stage[kRebuildStage];
-    StepCtl *ctl = d.ctl;
-    if (ctl->done) return;
-    uint32_t c0 = 1, c1 = 0;
-    const bool any = chunk_range(d, c0, c1);
-    const uint32_t nunits = any ? (c1 - c0) / kUnitChunks + 1 : 0;
-    if (b == nbw - 1) {
-        close_rebuild(d, p, account, nb, nnb, nunits);
-        return;
-    }
-    const unsigned long long tag = flag_tag(ctl->rebuild_seq);
-    const uint32_t nwords = static_cast<uint32_t>(bitmap_words(d));
-    uint32_t *bits = next_slot(d, p);
-    uint32_t *next = d.list[1 - p];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    for (uint32_t t = b; t < nunits; t += nbw - 1) {
-        // the unit's words, all loads in flight together
-        uint32_t w[kUnitChunks][8];
-#pragma unroll
-        for (uint32_t k = 0; k < kUnitChunks; k++) {
-            const uint32_t c = c0 + t * kUnitChunks + k;
-            const uint32_t w0 = c * kChunkWords + 8 * threadIdx.x;
-            if (c <= c1 && w0 + 8 <= nwords) {
-                const uint4 a = reinterpret_cast<const uint4 *>(bits + w0)[0];
-                const uint4 b = reinterpret_cast<const uint4 *>(bits + w0)[1];
-                w[k][0] = a.x, w[k][1] = a.y, w[k][2] = a.z, w[k][3] = a.w;
-                w[k][4] = b.x, w[k][5] = b.y, w[k][6] = b.z, w[k][7] = b.w;
-            }
-            else {
-#pragma unroll
-                for (int i = 0; i < 8; i++) w[k][i] = (c <= c1 && w0 + i < nwords) ? bits[w0 + i] : 0u;
-            }
-        }
-        uint32_t cnt[kUnitChunks], incl[kUnitChunks];
-#pragma unroll
-        for (uint32_t k = 0; k < kUnitChunks; k++) {
-            cnt[k] = 0;
-#pragma unroll
-            for (int i = 0; i < 8; i++) cnt[k] += __builtin_popcount(w[k][i]);
-            uint32_t wtot;
-            incl[k] = wave_inclusive_scan(cnt[k], wtot);
-            if (lane == 63) wave_tot[k][wave] = wtot;
-        }
-        __syncthreads();
-        // offset of this thread's cells within the unit (chunk by chunk, thread by thread)
-        uint32_t off[kUnitChunks], agg = 0;
-#pragma unroll
-        for (uint32_t k = 0; k < kUnitChunks; k++) {
-            uint32_t before = 0, tot = 0;
-            for (int q = 0; q < kBlock / 64; q++) {
-                if (q < wave) before += wave_tot[k][q];
-                tot += wave_tot[k][q];
-            }
-            off[k] = agg + before + incl[k] - cnt[k];
-            agg += tot;
-        }
-        if (wave == 0) {
-            uint32_t excl = 0;
-            if (t == 0) {
-                if (lane == 0) publish(d.chunk_flag + t, tag | kFlagPrefix | agg);
-            }
-            else {
-                if (lane == 0) publish(d.chunk_flag + t, tag | kFlagCount | agg);
-                excl = look_back(d, t, tag);
-                if (lane == 0) publish(d.chunk_flag + t, tag | kFlagPrefix | (excl + agg));
-            }
-            if (lane == 0) {
-                sh_excl = excl;
-                // the last unit knows the list's length
-                if (t == nunits - 1) set_count(d, p, excl + agg);
-            }
-        }
-        // the slot is cleared where it held bits; the cells go to LDS in list order when they fit
-        const bool staged = agg <= kRebuildStage;
-#pragma unroll
-        for (uint32_t k = 0; k < kUnitChunks; k++) {
-            const uint32_t c = c0 + t * kUnitChunks + k;
-            const uint32_t w0 = c * kChunkWords + 8 * threadIdx.x;
-            if (c <= c1 && w0 + 8 <= nwords) {
-                if (w[k][0] | w[k][1] | w[k][2] | w[k][3]) reinterpret_cast<uint4 *>(bits + w0)[0] = make_uint4(0, 0, 0, 0);
-                if (w[k][4] | w[k][5] | w[k][6] | w[k][7]) reinterpret_cast<uint4 *>(bits + w0)[1] = make_uint4(0, 0, 0, 0);
-            }
-            else {
-#pragma unroll
-                for (int i = 0; i < 8; i++)
-                    if (w[k][i]) bits[w0 + i] = 0u;
-            }
-            if (staged) {
-                uint32_t o = off[k];
-#pragma unroll
-                for (int i = 0; i < 8; i++)
-                    for (uint32_t m = w[k][i]; m; m &= m - 1) stage[o++] = (w0 + i) * 32u + __builtin_ctz(m);
-            }
-        }
-        __syncthreads();
-        const uint32_t excl = sh_excl;
-        if (staged) {
-            for (uint32_t i = threadIdx.x; i < agg; i += kBlock)
-                if (excl + i < d.list_cap) next[excl + i] = stage[i];
-        }
-        else {
-#pragma unroll
-            for (uint32_t k = 0; k < kUnitChunks; k++) {
-                const uint32_t w0 = (c0 + t * kUnitChunks + k) * kChunkWords + 8 * threadIdx.x;
-                uint32_t pos = excl + off[k];
-#pragma unroll
-                for (int i = 0; i < 8; i++)
-                    for (uint32_t m = w[k][i]; m; m &= m - 1, pos++)
-                        if (pos < d.list_cap) next[pos] = (w0 + i) * 32u + __builtin_ctz(m);
-            }
-        }
-        __syncthreads();  // the stage and the scan words are reused by the next unit
-    }
+    const bool finished = d.autostop && cycle % 1000 == 0 &&
+                          d.liquid0 - static_cast<long long>(d.stats->captures) -
+                                  static_cast<long long>(d.stats->activated) == 0;
+    if (!err && !finished) return;
+    ctl->done = 1;
+    ctl->final_cycle = cycle;
+    if (err && d.status_err) *d.status_err = err;
+    if (d.status) *d.status = cycle;
 }
 
 // Every active cell of the window due at the next step (after a cycle jump, whose skipped steps the
 // calendar did not count). Active cells above the window (substrate cells next to a later layer's
 // melt pool) are never stepped, as the reference's pass 1 never visits them.
-__device__ __forceinline__ void rewake_body(const DomainView &d, int p_next, uint32_t b, uint32_t nb) {
-    StepCtl *ctl = d.ctl;
-    if (b == 0 && threadIdx.x == 0) ctl->rebuild_seq = ctl->rebuild_seq + 1;
+__global__ __launch_bounds__(kBlock) void k_rewake(DomainView d, int p_next) {
+    const StepCtl *ctl = d.ctl;
     const uint32_t lo = ctl->elo, hi = ctl->ehi;
     if (lo > hi) return;
     const unsigned long long end = static_cast<unsigned long long>(d.X) * d.Y * d.nzA;
     const uint32_t serial = ctl->serial[p_next];
-    for (unsigned long long q = lo + static_cast<unsigned long long>(b) * kBlock + threadIdx.x; q <= hi && q < end;
-         q += static_cast<unsigned long long>(nb) * kBlock)
+    for (unsigned long long q = lo + static_cast<unsigned long long>(blockIdx.x) * kBlock + threadIdx.x; q <= hi && q < end;
+         q += static_cast<unsigned long long>(gridDim.x) * kBlock)
         if ((d.cells[q].ct & kTypeMask) == kActive) set_alarm(d, serial, static_cast<uint32_t>(q));
 }
 
@@ -1445,13 +1174,12 @@ __global__ __launch_bounds__(kBlock) void k_layer_bounds(DomainView d, int next_
 // window [zlo, nzA) gets a cell-centred octahedron (half-diagonal 0.01, centre at the cell centre,
 // critical lengths from its orientation) and an unknown liquid mask (its neighbours changed with the
 // layer), is counted afresh, and is due at the first step of the layer (the step of parity p_next).
-// The calendar was cleared before; the list is rebuilt after. ctl->nactive and the range of active
+// The calendar was cleared before. ctl->nactive and the range of active
 // cells (ctl->elo, ctl->ehi, reset by the host) are accumulated here.
 __global__ __launch_bounds__(kBlock) void k_layer_setup(DomainView d, int p_next) {
     __shared__ unsigned long long sh[kBlock / 64];
     StepCtl *ctl = d.ctl;
     const uint32_t serial = ctl->serial[p_next];
-    if (blockIdx.x == 0 && threadIdx.x == 0) ctl->rebuild_seq = ctl->rebuild_seq + 1;
     const Grid gr = grid_of(d);
     const long long begin = static_cast<long long>(d.X) * d.Y * d.zlo;
     const long long end = static_cast<long long>(d.X) * d.Y * d.nzA;
@@ -1488,54 +1216,142 @@ __global__ __launch_bounds__(kBlock) void k_layer_setup(DomainView d, int p_next
     }
 }
 
+// LDS of a workgroup's step counters and of the range of its new active cells.
+struct StepTally {
+    uint32_t cnt[kStepCounts];
+    uint32_t lohi[2];
+};
+__device__ __forceinline__ void clear_tally(StepTally &t) {
+    if (threadIdx.x < kStepCounts) t.cnt[threadIdx.x] = 0;
+    if (threadIdx.x < 2) t.lohi[threadIdx.x] = threadIdx.x == 0 ? 0xFFFFFFFFu : 0u;
+    __syncthreads();
+}
+// Whether the step at `cycle` directly follows the last executed one (no cycle jump, same layer).
+__device__ __forceinline__ bool follows_last(const StepCtl *ctl, int cycle) {
+    return cycle > 1 && ctl->last_cycle == cycle - 1;
+}
+constexpr uint32_t kDueStage = 1024;  // due cells of a turn staged in LDS
+
+__device__ __forceinline__ void nucleate_step(const DomainView &d, int p, int layer, uint32_t b, uint32_t nb) {
+    __shared__ StepTally t;
+    StepCtl *ctl = d.ctl;
+    if (ctl->done) return;
+    const int cycle = ctl->cycle[p];
+    const uint32_t serial = ctl->serial[p];
+    const int from = ctl->nuc_at;
+    clear_tally(t);
+    const int m = nucleate_body<kBlock>(d, cycle, serial, layer, from, b, nb, t.cnt, t.lohi);
+    if (b == 0 && threadIdx.x == 0) ctl->nuc_next = from + m;
+    if (!m) return;
+    widen_range(d, t.lohi);
+    add_parts(d, b, t.cnt, serial);
+}
+__device__ __forceinline__ void claim_step(const DomainView &d, int p, int layer, uint32_t b, uint32_t nb) {
+    __shared__ StepTally t;
+    __shared__ uint32_t nclaim;
+    __shared__ double gtab[kGrowStage];
+    __shared__ uint32_t list[kDueStage], tot[kBlock / 64];
+    StepCtl *ctl = d.ctl;
+    if (ctl->done) return;
+    if (threadIdx.x == 0) nclaim = 0;
+    clear_tally(t);
+    const Growth g = staged_growth<kBlock>(d, gtab);
+    const int cycle = ctl->cycle[p];
+    const uint32_t serial = ctl->serial[p];
+    if (b == 0 && threadIdx.x == 0) {
+        // the next step's control words (read only by the kernels after this one)
+        ctl->cycle[1 - p] = cycle + 1;
+        ctl->serial[1 - p] = serial + 1;
+        ctl->nuc_at = max(ctl->nuc_at, ctl->nuc_next);
+    }
+    claim_body<kBlock, kDueStage>(d, g, cycle, serial, layer, follows_last(ctl, cycle), b, nb, list, tot, t.cnt, &nclaim);
+    __syncthreads();
+    if (threadIdx.x == 0) d.claim_count[b] = nclaim;
+    add_parts(d, b, t.cnt, serial);
+}
+__device__ __forceinline__ void apply_step(const DomainView &d, int p, uint32_t a, uint32_t nbc) {
+    __shared__ StepTally t;
+    __shared__ ApplyLds<kBlock> s;
+    StepCtl *ctl = d.ctl;
+    if (ctl->done) return;
+    const uint32_t serial = ctl->serial[p];
+    if (a == 0 && threadIdx.x == 0) ctl->last_cycle = ctl->cycle[p];
+    // the claimants of kApplyGroup capture-pass workgroups
+    uint32_t n0 = 0, n = 0, r0 = 0, r1 = 0;
+    static_assert(kApplyGroup == 2, "two regions");
+    const uint32_t region = claim_region(d, nbc);
+    n0 = n = d.claim_count[2 * a];
+    r0 = unit_of(0, 2 * a, nbc) * region;
+    if (2 * a + 1 < nbc) {
+        n += d.claim_count[2 * a + 1];
+        r1 = unit_of(0, 2 * a + 1, nbc) * region;
+    }
+    clear_tally(t);
+    apply_body<kBlock>(
+        d, serial, n,
+        [&](uint32_t k, uint32_t &j, uint32_t &bits) {
+            const uint32_t i = k < n0 ? r0 + k : r1 + (k - n0);
+            j = d.claim_cell[i];
+            bits = d.claim_bits[i];
+        },
+        s, t.cnt, t.lohi);
+    widen_range(d, t.lohi);
+    add_parts(d, a, t.cnt, serial);
+}
+__device__ __forceinline__ void settle_step(const DomainView &d, int p_next, int layer, uint32_t b, uint32_t nb) {
+    __shared__ StepTally t;
+    __shared__ uint32_t list[kDueStage], tot[kBlock / 64];
+    StepCtl *ctl = d.ctl;
+    if (ctl->done || !follows_last(ctl, ctl->cycle[p_next])) return;
+    clear_tally(t);
+    const uint32_t serial = ctl->serial[p_next];
+    settle_body<kBlock, kDueStage>(d, growth_of(d), ctl->cycle[p_next], serial, layer, b, nb, list, tot, t.cnt);
+    __syncthreads();
+    add_parts(d, b, t.cnt, serial);
+}
+__device__ __forceinline__ void book_step(const DomainView &d, int p_next) {
+    __shared__ unsigned long long red[kPartRows][kBlock / 64];
+    if (d.ctl->done) return;
+    book_totals<kBlock>(d, d.ctl->serial[p_next], red);
+    if (threadIdx.x == 0) end_domain(d, d.ctl->last_cycle);
+}
+
 // Plain launches: one domain, passed by value.
 __global__ __launch_bounds__(kBlock) void k_nucleate(DomainView d, int p, int layer) {
-    nucleate_body(d, p, layer, blockIdx.x, gridDim.x);
+    nucleate_step(d, p, layer, blockIdx.x, gridDim.x);
 }
 __global__ __launch_bounds__(kBlock) void k_claim(DomainView d, int p, int layer) {
-    claim_body(d, p, layer, blockIdx.x, gridDim.x);
-}
-__global__ __launch_bounds__(kBlock) void k_win(DomainView d, int p) {
-    win_body(d, p, blockIdx.x, gridDim.x);
+    claim_step(d, p, layer, blockIdx.x, gridDim.x);
 }
 __global__ __launch_bounds__(kBlock) void k_apply(DomainView d, int p, int nbc) {
-    apply_body(d, p, blockIdx.x, static_cast<uint32_t>(nbc));
+    apply_step(d, p, blockIdx.x, static_cast<uint32_t>(nbc));
 }
-__global__ __launch_bounds__(kBlock) void k_settle(DomainView d, int p, int layer) {
-    settle_body(d, p, layer, blockIdx.x, gridDim.x);
+__global__ __launch_bounds__(kBlock) void k_settle(DomainView d, int p_next, int layer) {
+    settle_step(d, p_next, layer, blockIdx.x, gridDim.x);
 }
-__global__ __launch_bounds__(kBlock) void k_rebuild(DomainView d, int p, int account, int nb, int nnb) {
-    rebuild_body(d, p, account, static_cast<uint32_t>(nb), static_cast<uint32_t>(nnb), blockIdx.x, gridDim.x);
-}
-__global__ __launch_bounds__(kBlock) void k_rewake(DomainView d, int p_next) {
-    rewake_body(d, p_next, blockIdx.x, gridDim.x);
-}
+__global__ __launch_bounds__(kBlock) void k_book(DomainView d, int p_next) { book_step(d, p_next); }
 
 // Ensemble launches: grid row y serves domain slot y of a device-resident table; an empty slot has
 // no control block.
 __global__ __launch_bounds__(kBlock) void k_nucleate_n(const DomainView *v, int p, int layer) {
     const DomainView &d = v[blockIdx.y];
-    if (d.ctl) nucleate_body(d, p, layer, blockIdx.x, gridDim.x);
+    if (d.ctl) nucleate_step(d, p, layer, blockIdx.x, gridDim.x);
 }
 __global__ __launch_bounds__(kBlock) void k_claim_n(const DomainView *v, int p, int layer) {
     const DomainView &d = v[blockIdx.y];
-    if (d.ctl) claim_body(d, p, layer, blockIdx.x, gridDim.x);
-}
-__global__ __launch_bounds__(kBlock) void k_win_n(const DomainView *v, int p) {
-    const DomainView &d = v[blockIdx.y];
-    if (d.ctl) win_body(d, p, blockIdx.x, gridDim.x);
+    if (d.ctl) claim_step(d, p, layer, blockIdx.x, gridDim.x);
 }
 __global__ __launch_bounds__(kBlock) void k_apply_n(const DomainView *v, int p, int nbc) {
     const DomainView &d = v[blockIdx.y];
-    if (d.ctl) apply_body(d, p, blockIdx.x, static_cast<uint32_t>(nbc));
+    if (d.ctl) apply_step(d, p, blockIdx.x, static_cast<uint32_t>(nbc));
 }
-__global__ __launch_bounds__(kBlock) void k_settle_n(const DomainView *v, int p, int layer) {
+__global__ __launch_bounds__(kBlock) void k_settle_n(const DomainView *v, int p_next, int layer) {
     const DomainView &d = v[blockIdx.y];
-    if (d.ctl) settle_body(d, p, layer, blockIdx.x, gridDim.x);
+    if (d.ctl) settle_step(d, p_next, layer, blockIdx.x, gridDim.x);
 }
-__global__ __launch_bounds__(kBlock) void k_rebuild_n(const DomainView *v, int p, int nb, int nnb) {
+__global__ __launch_bounds__(kBlock) void k_book_n(const DomainView *v, int p_next) {
     const DomainView &d = v[blockIdx.y];
-    if (d.ctl) rebuild_body(d, p, 1, static_cast<uint32_t>(nb), static_cast<uint32_t>(nnb), blockIdx.x, gridDim.x);
+    if (d.ctl) book_step(d, p_next);
 }
 
 __global__ __launch_bounds__(kBlock) void k_check(DomainView d, int cycle, int layer, CheckResult *out) {
@@ -1607,6 +1423,7 @@ __global__ __launch_bounds__(kBlock) void k_seed_init(DomainView d, const uint32
         const Coord c = decode(q, d.X, d.Y);
         d.cells[q].dl = 0.01f;
         set_centre(d, q, (c.x + d.xoff) + 0.5, (c.y + d.yoff) + 0.5, c.z + 0.5);
+        set_alarm(d, 0, q);
     }
 }
 
@@ -1701,6 +1518,7 @@ __global__ __launch_bounds__(kBlock) void k_init_substrate(DomainView d, const u
         r.gid = static_cast<int32_t>(i + 1);
         r.ct = kActive | kSeedBit;
         set_centre(d, q, (c.x + d.xoff) + 0.5, (c.y + d.yoff) + 0.5, c.z + 0.5);
+        set_alarm(d, 0, q);
     }
 }
 __global__ __launch_bounds__(kBlock) void k_init_sites(DomainView d, const int32_t *sites, uint32_t n) {
@@ -1780,6 +1598,18 @@ __global__ __launch_bounds__(kBlock) void k_geometry_probe(const float *guv, con
     for (int l = 0; l < 26; l++) b[4 + l] = critical_length(f, a[4], a[5], a[6], o.cx, o.cy, o.cz, l);
 }
 
+// Cells due at the step of that serial, added to *out.
+__global__ __launch_bounds__(kBlock) void k_count_due(DomainView d, uint32_t serial, unsigned long long *out) {
+    __shared__ unsigned long long sh[kBlock / 64];
+    const uint32_t *bits = calendar_slot(d, serial);
+    unsigned long long c = 0;
+    for (size_t i = static_cast<size_t>(blockIdx.x) * kBlock + threadIdx.x; i < bitmap_words(d);
+         i += static_cast<size_t>(gridDim.x) * kBlock)
+        c += __builtin_popcount(bits[i]);
+    const unsigned long long t = block_sum(c, sh);
+    if (threadIdx.x == 0 && t) atomicAdd(out, t);
+}
+
 // Unique GrainIDs of a region: the flags k_grain_stats set, counted into *out.
 __global__ __launch_bounds__(kBlock) void k_count_flags(const uint32_t *gflag, uint32_t n, unsigned long long *out) {
     __shared__ unsigned long long sh[kBlock / 64];
@@ -1810,88 +1640,57 @@ inline int grid_for(long long n, int cap) {
 
 }  // namespace
 
-int nucleation_blocks(const DomainView &d) { return grid_for(d.nnuclei, 1024); }
+int nucleation_blocks(const DomainView &d) { return grid_for(d.nnuclei, 64); }
+uint32_t calendar_units(long long ncell) {
+    return static_cast<uint32_t>(((ncell + 31) / 32 + kUnitWords - 1) / kUnitWords);
+}
+size_t claim_entries(long long ncell, uint32_t most_blocks) {
+    const size_t units = calendar_units(ncell);
+    return (units + std::min<size_t>(units, most_blocks)) * kUnitCells;
+}
 void launch_nucleation(const DomainView &d, int parity, int layer, hipStream_t s) {
     k_nucleate<<<nucleation_blocks(d), kBlock, 0, s>>>(d, parity, layer);
 }
-void launch_claim(const DomainView &d, int parity, int layer, int blocks, hipStream_t s) {
+void launch_capture(const DomainView &d, int parity, int layer, int blocks, hipStream_t s) {
     k_claim<<<blocks, kBlock, 0, s>>>(d, parity, layer);
-}
-// Workgroups of the list rebuild: at most one per unit of the whole domain, 512, and as many as
-// the device holds at once (each takes every (n-1)-th unit: a unit of a second round waits for a
-// unit of a higher workgroup of the first, which must then be resident), plus the one that books
-// the step.
-int rebuild_blocks(const DomainView &d, int blocks) {
-    const uint32_t units = (d.nchunks + kUnitChunks - 1) / kUnitChunks;
-    uint32_t cap = static_cast<uint32_t>(blocks < 512 ? blocks : 512);
-    if (d.rebuild_cap && d.rebuild_cap < cap) cap = d.rebuild_cap;
-    return static_cast<int>(units < cap ? units : cap) + 1;
-}
-uint32_t rebuild_resident(int cus) {
-    int per_cu = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_rebuild, kBlock, 0) != hipSuccess || per_cu < 1)
-        per_cu = 1;
-    return static_cast<uint32_t>(per_cu) * static_cast<uint32_t>(cus);
-}
-uint32_t rebuild_units(long long ncell) {
-    const unsigned long long words = (static_cast<unsigned long long>(ncell) + 31) / 32;
-    const unsigned long long chunks = (words + kChunkWords - 1) / kChunkWords;
-    return static_cast<uint32_t>((chunks + kUnitChunks - 1) / kUnitChunks);
-}
-void launch_apply(const DomainView &d, int parity, int layer, int blocks, bool nucleated, hipStream_t s) {
-    const int cb = rebuild_blocks(d, blocks);
-    k_win<<<blocks, kBlock, 0, s>>>(d, parity);
     k_apply<<<apply_blocks(blocks), kBlock, 0, s>>>(d, parity, blocks);
-    k_settle<<<settle_blocks(blocks), kBlock, 0, s>>>(d, parity, layer);
-    k_rebuild<<<cb, kBlock, 0, s>>>(d, parity, 1, blocks, nucleated ? grid_for(d.nnuclei, 1024) : 0);
+}
+void launch_settle(const DomainView &d, int parity_next, int layer, int blocks, hipStream_t s) {
+    k_settle<<<blocks, kBlock, 0, s>>>(d, parity_next, layer);
+    k_book<<<1, kBlock, 0, s>>>(d, parity_next);
 }
 void launch_layer_bounds(const DomainView &d, int next_layer, int *out, hipStream_t s) {
     k_layer_bounds<<<grid_for(d.ncell, 4096), kBlock, 0, s>>>(d, next_layer, out);
 }
-void launch_layer_setup(const DomainView &d, int parity_next, int blocks, hipStream_t s) {
-    const int cb = rebuild_blocks(d, blocks);
+void launch_layer_setup(const DomainView &d, int parity_next, hipStream_t s) {
     const long long n = static_cast<long long>(d.X) * d.Y * (d.nzA - d.zlo);
     k_layer_setup<<<grid_for(n, 4096), kBlock, 0, s>>>(d, parity_next);
-    k_rebuild<<<cb, kBlock, 0, s>>>(d, 1 - parity_next, 0, blocks, 0);
 }
 void launch_rewake(const DomainView &d, int parity_next, int blocks, hipStream_t s) {
-    const int cb = rebuild_blocks(d, blocks);
     k_rewake<<<blocks, kBlock, 0, s>>>(d, parity_next);
-    k_rebuild<<<cb, kBlock, 0, s>>>(d, 1 - parity_next, 0, blocks, 0);
 }
 void launch_step_timed(const DomainView &d, int parity, int layer, int blocks, hipStream_t s, hipEvent_t *ev) {
-    const int cb = rebuild_blocks(d, blocks);
     int e = 0;
     auto rec = [&]() { (void)hipEventRecord(ev[e++], s); };
     rec();
-    k_nucleate<<<grid_for(d.nnuclei, 1024), kBlock, 0, s>>>(d, parity, layer);
+    k_nucleate<<<nucleation_blocks(d), kBlock, 0, s>>>(d, parity, layer);
     rec();
     rec();
     k_claim<<<blocks, kBlock, 0, s>>>(d, parity, layer);
     rec();
     rec();
-    k_win<<<blocks, kBlock, 0, s>>>(d, parity);
-    rec();
-    rec();
     k_apply<<<apply_blocks(blocks), kBlock, 0, s>>>(d, parity, blocks);
     rec();
-    rec();
-    k_settle<<<settle_blocks(blocks), kBlock, 0, s>>>(d, parity, layer);
-    rec();
-    rec();
-    k_rebuild<<<cb, kBlock, 0, s>>>(d, parity, 1, blocks, grid_for(d.nnuclei, 1024));
-    rec();
 }
-void launch_step_n(const DomainView *views, int slots, int parity, int layer, int nuc_blocks, int blocks,
-                   hipStream_t s) {
-    k_nucleate_n<<<dim3(nuc_blocks, slots), kBlock, 0, s>>>(views, parity, layer);
-    k_claim_n<<<dim3(blocks, slots), kBlock, 0, s>>>(views, parity, layer);
-    k_win_n<<<dim3(blocks, slots), kBlock, 0, s>>>(views, parity);
-    k_apply_n<<<dim3(apply_blocks(blocks), slots), kBlock, 0, s>>>(views, parity, blocks);
-    k_settle_n<<<dim3(settle_blocks(blocks), slots), kBlock, 0, s>>>(views, parity, layer);
-    // one round of workgroups covers every unit of an ensemble domain (at most kEnsembleUnits):
-    // each waits only for workgroups of its row dispatched before it; plus the booking workgroup
-    k_rebuild_n<<<dim3(kEnsembleUnits + 1, slots), kBlock, 0, s>>>(views, parity, blocks, nuc_blocks);
+void launch_steps_n(const DomainView *views, int slots, int steps, int layer, int nuc_blocks, int blocks,
+                    hipStream_t s) {
+    for (int k = 0; k < steps; k++) {
+        k_nucleate_n<<<dim3(nuc_blocks, slots), kBlock, 0, s>>>(views, k & 1, layer);
+        k_claim_n<<<dim3(blocks, slots), kBlock, 0, s>>>(views, k & 1, layer);
+        k_apply_n<<<dim3(apply_blocks(blocks), slots), kBlock, 0, s>>>(views, k & 1, blocks);
+    }
+    k_settle_n<<<dim3(blocks, slots), kBlock, 0, s>>>(views, steps & 1, layer);
+    k_book_n<<<dim3(1, slots), kBlock, 0, s>>>(views, steps & 1);
 }
 void launch_check(const DomainView &d, int cycle, int layer, CheckResult *out, hipStream_t s) {
     k_check<<<grid_for(d.ncell, 4096), kBlock, 0, s>>>(d, cycle, layer, out);
@@ -1921,6 +1720,9 @@ void launch_extract(const DomainView &d, int field, void *out, hipStream_t s) {
 }
 void launch_count_flags(const uint32_t *gflag, uint32_t n, unsigned long long *out, hipStream_t s) {
     k_count_flags<<<grid_for(n, 1024), kBlock, 0, s>>>(gflag, n, out);
+}
+void launch_count_due(const DomainView &d, uint32_t serial, unsigned long long *out, hipStream_t s) {
+    k_count_due<<<grid_for((d.ncell + 31) / 32, 1024), kBlock, 0, s>>>(d, serial, out);
 }
 void launch_fill(uint32_t *p, size_t n, uint32_t v, hipStream_t s) {
     k_fill<<<grid_for(static_cast<long long>(n), 4096), kBlock, 0, s>>>(p, n, v);

@@ -36,7 +36,6 @@ StepCtl initial_ctl(const HostDomain &hd) {
     StepCtl c;
     std::memset(&c, 0, sizeof c);
     c.cycle[0] = 1;
-    c.count[0] = static_cast<uint32_t>(hd.active.size());
     c.elo = 0xFFFFFFFFu;
     c.ehi = 0;
     for (uint32_t q : hd.active) {
@@ -46,34 +45,48 @@ StepCtl initial_ctl(const HostDomain &hd) {
     c.nactive = hd.active.size();
     c.layer_zlo[0] = hd.zlow;
     c.layer_zhi[0] = hd.zhigh;
-    c.next_nuc[0] = 0x7FFFFFFF;
-    c.next_nuc[1] = 0x7FFFFFFF;
-    for (int32_t t : hd.ntime) c.next_nuc[0] = std::min(c.next_nuc[0], t);
     return c;
 }
 
+// The nucleation sites that a layer's steps can activate (LayerID up to the layer's), in ascending
+// order of their times, so that the sites due at a step are the next few of the list. A site of an
+// earlier layer that was decided there is not liquid any more and changes nothing.
+void layer_sites(const HostDomain &hd, int layer, std::vector<int32_t> &loc, std::vector<int32_t> &time) {
+    std::vector<uint32_t> order;
+    order.reserve(hd.nloc.size());
+    for (uint32_t i = 0; i < hd.nloc.size(); i++)
+        if (hd.sparse || hd.lid[hd.nloc[i]] <= layer) order.push_back(i);
+    std::stable_sort(order.begin(), order.end(), [&](uint32_t a, uint32_t b) { return hd.ntime[a] < hd.ntime[b]; });
+    loc.resize(order.size());
+    time.resize(order.size());
+    for (size_t k = 0; k < order.size(); k++) {
+        loc[k] = hd.nloc[order[k]];
+        time[k] = hd.ntime[order[k]];
+    }
+}
+
 // Initial cell records of a domain: the compact host arrays are staged in device buffers that are
-// free until the first step (the claim lists and the second list: at least 12 bytes per cell) and
-// packed on the device. The initially active cells are the first step's list (list[0]), with their
-// cell-centred octahedra; the calendar starts empty. Synchronises the stream (the host sources
-// are temporaries).
+// free until the first step (the claim lists and the calendar: at least 16 bytes per cell) and packed
+// on the device. The initially active cells get their cell-centred octahedra and are due at the
+// first step; the calendar holds nothing else. Synchronises the stream (the host sources are
+// temporaries).
 void upload_cells(const DomainView &d, const HostDomain &hd, uint8_t *melted, hipStream_t s) {
     const size_t n = static_cast<size_t>(hd.ncell);
+    const size_t calendar = 4 * kAlarmSlots * alarm_stride(d.ncell);
     if (hd.sparse) {
-        // built on the device from the per-plane CritTimeStep and the draws' lists, staged in
-        // buffers that are free until the first step; the active list is the first step's list
+        // built on the device from the per-plane CritTimeStep and the draws' lists
         int32_t *plane_cts = reinterpret_cast<int32_t *>(d.claim_bits);
         int32_t *sites = reinterpret_cast<int32_t *>(d.claim_cell);
+        uint32_t *active = d.claim_bits + hd.plane_cts.size();
+        HIP_OK(hipMemsetAsync(d.alarms, 0, calendar, s));
         HIP_OK(hipMemcpyAsync(plane_cts, hd.plane_cts.data(), 4 * hd.plane_cts.size(), hipMemcpyHostToDevice, s));
         if (!hd.nloc.empty())
             HIP_OK(hipMemcpyAsync(sites, hd.nloc.data(), 4 * hd.nloc.size(), hipMemcpyHostToDevice, s));
         if (!hd.active.empty())
-            HIP_OK(hipMemcpyAsync(d.list[0], hd.active.data(), 4 * hd.active.size(), hipMemcpyHostToDevice, s));
-        launch_init_directional(d, plane_cts, hd.nx, hd.ny, melted, d.list[0], static_cast<uint32_t>(hd.active.size()),
+            HIP_OK(hipMemcpyAsync(active, hd.active.data(), 4 * hd.active.size(), hipMemcpyHostToDevice, s));
+        launch_init_directional(d, plane_cts, hd.nx, hd.ny, melted, active, static_cast<uint32_t>(hd.active.size()),
                                 sites, static_cast<uint32_t>(hd.nloc.size()), s);
         HIP_OK(hipGetLastError());
-        HIP_OK(hipMemsetAsync(d.alarms, 0, 4 * kAlarmSlots * alarm_stride(d.ncell), s));
-        HIP_OK(hipMemsetAsync(d.chunk_flag, 0, 8ull * d.nchunks, s));
         HIP_OK(hipStreamSynchronize(s));
         return;
     }
@@ -82,7 +95,7 @@ void upload_cells(const DomainView &d, const HostDomain &hd, uint8_t *melted, hi
     for (uint32_t q : hd.active) ct[q] |= kSeedBit;
     uint8_t *ct_d = reinterpret_cast<uint8_t *>(d.claim_cell);
     int8_t *lid_d = reinterpret_cast<int8_t *>(ct_d + n);
-    int32_t *gid_d = reinterpret_cast<int32_t *>(d.list[1]);
+    int32_t *gid_d = reinterpret_cast<int32_t *>(d.alarms);
     int32_t *cts_d = reinterpret_cast<int32_t *>(d.claim_bits);
     HIP_OK(hipMemcpyAsync(ct_d, ct.data(), n, hipMemcpyHostToDevice, s));
     HIP_OK(hipMemcpyAsync(lid_d, hd.lid.data(), n, hipMemcpyHostToDevice, s));
@@ -90,11 +103,10 @@ void upload_cells(const DomainView &d, const HostDomain &hd, uint8_t *melted, hi
     HIP_OK(hipMemcpyAsync(cts_d, hd.cts.data(), 4 * n, hipMemcpyHostToDevice, s));
     launch_pack(d, ct_d, lid_d, gid_d, cts_d, s);
     HIP_OK(hipGetLastError());
-    HIP_OK(hipMemsetAsync(d.alarms, 0, 4 * kAlarmSlots * alarm_stride(d.ncell), s));
-    HIP_OK(hipMemsetAsync(d.chunk_flag, 0, 8ull * d.nchunks, s));
+    HIP_OK(hipMemsetAsync(d.alarms, 0, calendar, s));
     if (!hd.active.empty()) {
-        HIP_OK(hipMemcpyAsync(d.list[0], hd.active.data(), 4 * hd.active.size(), hipMemcpyHostToDevice, s));
-        launch_seed_init(d, d.list[0], static_cast<uint32_t>(hd.active.size()), s);
+        HIP_OK(hipMemcpyAsync(d.claim_cell, hd.active.data(), 4 * hd.active.size(), hipMemcpyHostToDevice, s));
+        launch_seed_init(d, d.claim_cell, static_cast<uint32_t>(hd.active.size()), s);
         HIP_OK(hipGetLastError());
     }
     HIP_OK(hipStreamSynchronize(s));
@@ -150,13 +162,13 @@ struct exaca_state {
     hipGraphExec_t graph = nullptr;       // kGraphSteps steps
     hipGraphExec_t graph_quiet = nullptr; // the same without the nucleation kernels
     int graph_layer = -1;
-    // Nucleation times in ascending order, and the last step whose nucleation kernel ran: a step
-    // may leave the kernel out when no time falls after that step and up to it (every site of a
-    // time at or before a step where the kernel ran is decided there). Single-layer decks only: a
-    // site of a later layer waits past its time.
+    // The layer's nucleation times in ascending order, and the last step whose nucleation kernel
+    // ran: a step may leave the kernel out when no time falls after that step and up to it (every
+    // site of a time at or before a step where the kernel ran is decided there).
     std::vector<int32_t> nuc_times;
     int nuc_through = 0;
     bool nuc_skip = false;
+    int32_t *nloc = nullptr, *ntime = nullptr;  // device copies of the layer's sites
     double init_seconds = 0;
     int device = 0;
     int layer = 0;              // the layer being solidified
@@ -182,6 +194,22 @@ struct exaca_state {
 
 namespace {
 
+// The layer's nucleation sites to the device; its steps start with none decided. Synchronises the
+// stream.
+void upload_sites(exaca_state *h, int layer) {
+    std::vector<int32_t> loc;
+    exaca::layer_sites(h->host, layer, loc, h->nuc_times);
+    if (!loc.empty()) {
+        HIP_OK(hipMemcpyAsync(h->nloc, loc.data(), 4 * loc.size(), hipMemcpyHostToDevice, h->stream));
+        HIP_OK(hipMemcpyAsync(h->ntime, h->nuc_times.data(), 4 * loc.size(), hipMemcpyHostToDevice, h->stream));
+    }
+    HIP_OK(hipStreamSynchronize(h->stream));
+    h->dv.nloc = h->nloc;
+    h->dv.ntime = h->ntime;
+    h->dv.nnuclei = static_cast<int32_t>(loc.size());
+    h->nuc_through = std::numeric_limits<int>::min();
+}
+
 void build_device_state(exaca_state *h) {
     using namespace exaca;
     const HostDomain &hd = h->host;
@@ -194,8 +222,7 @@ void build_device_state(exaca_state *h) {
     // Frontier kernels: up to 4 workgroups per CU (the capture pass is then resident in one round;
     // measured at 800^3: 2, 3, 4, 6, 8 per CU give 110, 101, 96, 102, 118 us), fewer for small
     // domains (the frontier never exceeds the cell count, and a slice is at least one workgroup of
-    // cells). (At most 2048: the per-workgroup step counters are summed by one workgroup, 8 slots
-    // a thread.)
+    // cells).
     const long long cap = std::min<long long>(2048, ((prop.multiProcessorCount * 4 + 7) / 8) * 8);
     const long long want = ((hd.ncell / 4096 + 7) / 8) * 8;
     h->blocks = static_cast<int>(std::max<long long>(8, std::min(cap, want)));
@@ -212,25 +239,12 @@ void build_device_state(exaca_state *h) {
     const size_t n = static_cast<size_t>(hd.ncell);
     d.cells = h->alloc<Cell>(n);
     d.octa = h->alloc<Octa>(n);
-    d.list_cap = static_cast<uint32_t>(n);
-    d.list[0] = h->alloc<uint32_t>(n);
-    d.list[1] = h->alloc<uint32_t>(n);
-    d.claim_cell = h->alloc<uint32_t>(n);
-    d.claim_bits = h->alloc<uint32_t>(n);
-    d.slice_claims = h->alloc<uint32_t>(h->blocks);
-    d.cand = h->alloc<uint32_t>(static_cast<size_t>(apply_blocks(h->blocks)) * kCandStage);
-    d.cand_count = h->alloc<uint32_t>(apply_blocks(h->blocks));
-    d.cand_cap = cand_stage_cap();
-    const size_t nwords = (n + 31) / 32;
-    d.nchunks = static_cast<uint32_t>((nwords + 2047) / 2048);
+    d.claim_cell = h->alloc<uint32_t>(claim_entries(hd.ncell, h->blocks));
+    d.claim_bits = h->alloc<uint32_t>(claim_entries(hd.ncell, h->blocks));
+    d.claim_count = h->alloc<uint32_t>(h->blocks);
     d.alarms = h->alloc<uint32_t>(kAlarmSlots * alarm_stride(d.ncell));
-    d.chunk_flag = h->alloc<unsigned long long>(d.nchunks);
-    d.rebuild_cap = exaca::rebuild_resident(prop.multiProcessorCount);
-    d.nnuclei = static_cast<int32_t>(hd.nloc.size());
-    int32_t *nloc = h->alloc<int32_t>(hd.nloc.size());
-    int32_t *ntime = h->alloc<int32_t>(hd.ntime.size());
-    d.nloc = nloc;
-    d.ntime = ntime;
+    h->nloc = h->alloc<int32_t>(hd.nloc.size());
+    h->ntime = h->alloc<int32_t>(hd.ntime.size());
     float *guv = h->alloc<float>(hd.guv.size());
     d.guv = guv;
     std::vector<float> seed(static_cast<size_t>(kCdlStride) * kNumOrientations, 0.0f);
@@ -248,16 +262,13 @@ void build_device_state(exaca_state *h) {
     h->check = h->alloc<CheckResult>(1);
     d.ctl = h->ctl;
     d.stats = h->stats;
-    d.nparts = 2048;  // the capture grid (<= 2048) and the nucleation grid (<= 1024)
+    d.nparts = static_cast<uint32_t>(std::max(h->blocks, 64));  // the capture grid and the nucleation grid (<= 64)
     d.part = h->alloc<unsigned long long>(static_cast<size_t>(kPartRows) * d.nparts);
 
     // Initial state; per-cell undercooling is not stored (it is a function of the steps executed
     // below the liquidus time).
     hipStream_t s = h->stream;
-    if (!hd.nloc.empty()) {
-        HIP_OK(hipMemcpyAsync(nloc, hd.nloc.data(), hd.nloc.size() * 4, hipMemcpyHostToDevice, s));
-        HIP_OK(hipMemcpyAsync(ntime, hd.ntime.data(), hd.ntime.size() * 4, hipMemcpyHostToDevice, s));
-    }
+    upload_sites(h, 0);
     HIP_OK(hipMemcpyAsync(guv, hd.guv.data(), hd.guv.size() * 4, hipMemcpyHostToDevice, s));
     HIP_OK(hipMemcpyAsync(seed_d, seed.data(), seed.size() * 4, hipMemcpyHostToDevice, s));
     HIP_OK(hipMemcpyAsync(grow_d, grow.data(), grow.size() * 8, hipMemcpyHostToDevice, s));
@@ -327,7 +338,8 @@ void next_layer(exaca_state *h, int layer_done, int verbose) {
         }
     // the layer's record, the new layer's first cycle, and fresh counts of the active cells
     StepCtl *c = h->ctl;
-    const int32_t end = h->cycle, j0 = h->njumps, layer = layer_done + 1, one = 1, zero = 0, open = 0;
+    const int32_t end = h->cycle, j0 = h->njumps, layer = layer_done + 1, one = 1, zero = 0;
+    const int32_t none_decided[2] = {0, 0};  // nuc_at, nuc_next
     const uint32_t range[2] = {0xFFFFFFFFu, 0};
     const unsigned long long none[2] = {0, 0};
     HIP_OK(hipMemcpyAsync(&c->layer_end[layer_done], &end, 4, hipMemcpyHostToDevice, h->stream));
@@ -337,12 +349,13 @@ void next_layer(exaca_state *h, int layer_done, int verbose) {
     HIP_OK(hipMemcpyAsync(&c->layer_zhi[layer], &zhigh, 4, hipMemcpyHostToDevice, h->stream));
     HIP_OK(hipMemcpyAsync(&c->cycle[h->parity], &one, 4, hipMemcpyHostToDevice, h->stream));
     HIP_OK(hipMemcpyAsync(&c->last_cycle, &zero, 4, hipMemcpyHostToDevice, h->stream));
-    HIP_OK(hipMemcpyAsync(&c->next_nuc[h->parity], &open, 4, hipMemcpyHostToDevice, h->stream));
+    HIP_OK(hipMemcpyAsync(&c->nuc_at, none_decided, sizeof none_decided, hipMemcpyHostToDevice, h->stream));
+    upload_sites(h, layer);
     HIP_OK(hipMemcpyAsync(&c->elo, range, sizeof range, hipMemcpyHostToDevice, h->stream));
     HIP_OK(hipMemcpyAsync(&c->nactive, none, sizeof none, hipMemcpyHostToDevice, h->stream));
     // the calendar starts empty: every active cell of the window is due at the first step
     launch_fill(h->dv.alarms, static_cast<size_t>(kAlarmSlots) * alarm_stride(h->dv.ncell), 0u, h->stream);
-    launch_layer_setup(h->dv, h->parity, h->blocks, h->stream);
+    launch_layer_setup(h->dv, h->parity, h->stream);
     HIP_OK(hipGetLastError());
     HIP_OK(hipStreamSynchronize(h->stream));  // host values above are stack temporaries
     h->layer = layer;
@@ -352,9 +365,13 @@ void next_layer(exaca_state *h, int layer_done, int verbose) {
 void step_nucleation(exaca_state *h, int layer) {
     exaca::launch_nucleation(h->dv, h->parity, layer, h->stream);
 }
-void step_capture(exaca_state *h, int layer, bool nucleated = true) {
-    exaca::launch_claim(h->dv, h->parity, layer, h->blocks, h->stream);
-    exaca::launch_apply(h->dv, h->parity, layer, h->blocks, nucleated, h->stream);
+void step_capture(exaca_state *h, int layer) {
+    exaca::launch_capture(h->dv, h->parity, layer, h->blocks, h->stream);
+}
+// After the last step of a call: its state and statistics complete.
+void finish_steps(exaca_state *h, int layer) {
+    exaca::launch_settle(h->dv, h->parity, layer, h->blocks, h->stream);
+    HIP_OK(hipGetLastError());
 }
 // Whether steps h->cycle + 1 .. last need the nucleation kernel.
 bool nucleation_due(const exaca_state *h, int last) {
@@ -376,8 +393,7 @@ void ensure_graph(exaca_state *h, int layer) {
         for (int k = 0; k < kGraphSteps; k++) {
             const int p = k & 1;
             if (nucleate) exaca::launch_nucleation(h->dv, p, layer, h->stream);
-            exaca::launch_claim(h->dv, p, layer, h->blocks, h->stream);
-            exaca::launch_apply(h->dv, p, layer, h->blocks, nucleate, h->stream);
+            exaca::launch_capture(h->dv, p, layer, h->blocks, h->stream);
         }
         HIP_OK(hipStreamEndCapture(h->stream, &g));
         HIP_OK(hipGraphInstantiate(nucleate ? &h->graph : &h->graph_quiet, g, nullptr, nullptr, 0));
@@ -387,6 +403,7 @@ void ensure_graph(exaca_state *h, int layer) {
 }
 
 void run_steps(exaca_state *h, int layer, int n, bool use_graph) {
+    if (n <= 0) return;
     while (n > 0) {
         if (use_graph && h->parity == 0 && n >= kGraphSteps) {
             ensure_graph(h, layer);
@@ -403,13 +420,13 @@ void run_steps(exaca_state *h, int layer, int n, bool use_graph) {
                 step_nucleation(h, layer);
                 h->nuc_through = h->cycle + 1;
             }
-            step_capture(h, layer, nucleate);
+            step_capture(h, layer);
             h->parity ^= 1;
             h->cycle += 1;
             n -= 1;
         }
     }
-    HIP_OK(hipGetLastError());
+    finish_steps(h, layer);
 }
 
 void device_check(exaca_state *h, int *cycle, int layer, uint64_t counts[5], int *xswitch, int verbose) {
@@ -509,16 +526,13 @@ exaca_state *create_state(const std::string &input, const std::string &dd, bool 
     h->deck.seed = seed;
     h->host = exaca::initialize_sparse(h->deck, verbose);
     build_device_state(h.get());
-    h->nuc_times = h->host.ntime;
-    std::sort(h->nuc_times.begin(), h->nuc_times.end());
-    h->nuc_through = std::numeric_limits<int>::min();
-    h->nuc_skip = h->deck.num_layers == 1 && std::getenv("EXACA_NUCLEATE_EVERY_STEP") == nullptr;
+    h->nuc_skip = std::getenv("EXACA_NUCLEATE_EVERY_STEP") == nullptr;
     h->init_seconds = std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
     return h.release();
 }
 
 // Steps one at a time with HIP events around every kernel (no graphs): per-kernel device time of
-// nucleation, claim, apply, settle and the frontier rebuild (bitmap count / scan / write).
+// nucleation, claim and apply.
 void profile(exaca_state *h, int layer, int nsteps, double *ms, int64_t counts[5], int64_t *launches) {
     using exaca::kTimedKernels;
     exaca::StepStats before, after;
@@ -542,6 +556,7 @@ void profile(exaca_state *h, int layer, int nsteps, double *ms, int64_t counts[5
                 break;
             }
         }
+        finish_steps(h, layer);
         HIP_OK(hipStreamSynchronize(h->stream));
         for (int q = 0; q < k; q++)
             for (int r = 0; r < kTimedKernels; r++) {
@@ -743,7 +758,7 @@ int exaca_nucleation_nn(exaca_state *h, int cycle, int layer, int32_t *nn) {
         const int nb = exaca::nucleation_blocks(h->dv);
         std::vector<unsigned long long> row(static_cast<size_t>(nb));
         exaca::StepStats st;
-        HIP_OK(hipMemcpyAsync(row.data(), h->dv.part + static_cast<size_t>(exaca::kPartNucNn) * h->dv.nparts,
+        HIP_OK(hipMemcpyAsync(row.data(), h->dv.part + static_cast<size_t>(exaca::kPartNn) * h->dv.nparts,
                               row.size() * sizeof(unsigned long long), hipMemcpyDeviceToHost, h->stream));
         HIP_OK(hipMemcpyAsync(&st, h->stats, sizeof st, hipMemcpyDeviceToHost, h->stream));
         HIP_OK(hipStreamSynchronize(h->stream));
@@ -758,8 +773,8 @@ int exaca_cell_capture(exaca_state *h, int cycle, int layer) {
         if (!h) throw std::invalid_argument("null handle");
         if (h->pending != cycle) throw StateError("capture requires nucleation of the same cycle first");
         step_capture(h, layer);
-        HIP_OK(hipGetLastError());
         h->parity ^= 1;
+        finish_steps(h, layer);
         h->cycle = cycle;
         h->pending = -1;
     });
@@ -891,8 +906,17 @@ int exaca_query(const exaca_state *h, int64_t out[20]) {
         out[10] = static_cast<int64_t>(st.captures);
         out[11] = static_cast<int64_t>(st.solidified);
         out[12] = static_cast<int64_t>(st.waiting);
-        out[13] = c.count[h->parity];
-        out[14] = h->dv.list_cap;
+        {  // the check's result block is free between steps
+            unsigned long long due = 0;
+            HIP_OK(hipMemcpyAsync(h->check, &due, sizeof due, hipMemcpyHostToDevice, h->stream));
+            exaca::launch_count_due(h->dv, c.serial[h->parity], reinterpret_cast<unsigned long long *>(h->check),
+                                    h->stream);
+            HIP_OK(hipGetLastError());
+            HIP_OK(hipMemcpyAsync(&due, h->check, sizeof due, hipMemcpyDeviceToHost, h->stream));
+            HIP_OK(hipStreamSynchronize(h->stream));
+            out[13] = static_cast<int64_t>(due);
+        }
+        out[14] = hd.ncell;
         out[15] = static_cast<int64_t>(h->bytes);
         out[16] = static_cast<int64_t>(st.evaluated);
         out[17] = static_cast<int64_t>(st.masks);
@@ -912,10 +936,7 @@ int exaca_profile_steps(exaca_state *h, int layer, int nsteps, double ms[3], int
         double all[exaca::kTimedKernels];
         int64_t launches = 0;
         profile(h, layer, nsteps, all, counts, &launches);
-        ms[0] = all[0];
-        ms[1] = all[1];
-        ms[2] = 0;
-        for (int k = 2; k < exaca::kTimedKernels; k++) ms[2] += all[k];
+        for (int k = 0; k < exaca::kTimedKernels; k++) ms[k] = all[k];
     });
 }
 
@@ -924,7 +945,12 @@ int exaca_profile_kernels(exaca_state *h, int layer, int nsteps, double ms[6], i
         if (!h || !ms || !counts || nsteps < 0) throw std::invalid_argument("bad argument");
         if (h->pending >= 0) throw StateError("profile_kernels called between nucleation and capture");
         int64_t launches = 0;
-        profile(h, layer, nsteps, ms, counts, &launches);
+        double all[exaca::kTimedKernels];
+        profile(h, layer, nsteps, all, counts, &launches);
+        ms[0] = all[0];
+        ms[1] = all[1];
+        ms[3] = all[2];
+        ms[2] = ms[4] = ms[5] = 0;  // the winners are decided in apply, the next step's list in claim
     });
 }
 

@@ -1,9 +1,9 @@
 // ensemble.hip -- many CA domains resident on one GPU, stepped together.
 //
 // Each domain occupies one slot: its state lives in a sub-range of a single device arena, and its
-// DomainView sits in a device-resident slot table. One step of every slot is four launches whose
-// grid row y serves slot y (launch_step_n); 50-step chunks of those launches are captured once in a
-// HIP graph and replayed. Every domain keeps its own cycle, control block and frontier, and stops
+// DomainView sits in a device-resident slot table. One step of every slot is three launches
+// whose grid row y serves slot y (launch_steps_n); 50-step chunks of those launches are captured once in
+// a HIP graph and replayed. Every domain keeps its own cycle, control block and frontier, and stops
 // itself on the device at the first 1000-step check with no liquid left, so each one evolves
 // exactly as it would alone on the plain path. The host admits new domains into free slots
 // between chunks (continuous batching) and polls the per-slot status words after each chunk.
@@ -27,6 +27,7 @@ namespace exaca {
 void upload_cells(const DomainView &d, const HostDomain &hd, uint8_t *melted, hipStream_t s);
 StepCtl initial_ctl(const HostDomain &hd);
 void download_field(const DomainView &d, int field, void *dst, size_t dst_bytes, hipStream_t s);
+void layer_sites(const HostDomain &hd, int layer, std::vector<int32_t> &loc, std::vector<int32_t> &time);
 }  // namespace exaca
 
 namespace {
@@ -84,12 +85,10 @@ size_t domain_bytes(const exaca::HostDomain &h, size_t ngrow) {
     const size_t n = static_cast<size_t>(h.ncell);
     size_t b = 0;
     b += up(sizeof(exaca::Cell) * n) + up(sizeof(exaca::Octa) * n);  // cell records
-    b += 4 * up(4 * n) + up(4 * kMaxSlices);                            // frontier, claim lists
-    b += up(4ull * exaca::apply_blocks(kMaxSlices) * exaca::kCandStage) + up(4 * exaca::apply_blocks(kMaxSlices));
+    b += 2 * up(4 * exaca::claim_entries(h.ncell, kMaxSlices)) + up(4 * kMaxSlices);  // claim lists
     b += 2 * up(4 * std::max<size_t>(h.nloc.size(), 1)) + up(8 * ngrow);
     b += up(sizeof(exaca::StepCtl)) + up(sizeof(exaca::StepStats)) + up(8ull * exaca::kPartRows * kMaxSlices);
-    const size_t nwords = (n + 31) / 32;
-    b += up(4 * exaca::kAlarmSlots * exaca::alarm_stride(h.ncell)) + up(8 * ((nwords + 2047) / 2048));  // calendar, chunk flags
+    b += up(4 * exaca::kAlarmSlots * exaca::alarm_stride(h.ncell));  // calendar
     return b;
 }
 
@@ -157,8 +156,7 @@ hipGraphExec_t graph_for(exaca_ensemble *e, int blocks) {
     if (it != e->graphs.end()) return it->second;
     hipGraph_t g;
     HIP_OK(hipStreamBeginCapture(e->stream, hipStreamCaptureModeThreadLocal));
-    for (int k = 0; k < kChunk; k++)
-        exaca::launch_step_n(e->views_d, e->slots, k & 1, 0, e->nuc_blocks, blocks, e->stream);
+    exaca::launch_steps_n(e->views_d, e->slots, kChunk, 0, e->nuc_blocks, blocks, e->stream);
     HIP_OK(hipStreamEndCapture(e->stream, &g));
     hipGraphExec_t x;
     HIP_OK(hipGraphInstantiate(&x, g, nullptr, nullptr, 0));
@@ -187,6 +185,8 @@ void admit(exaca_ensemble *e, const exaca_prepared *pr, int *slot_out) {
         p += up(bytes);
         return q;
     };
+    std::vector<int32_t> loc, time;
+    exaca::layer_sites(hd, 0, loc, time);
     DomainView d{};
     d.X = hd.X;
     d.Y = hd.Y;
@@ -197,27 +197,18 @@ void admit(exaca_ensemble *e, const exaca_prepared *pr, int *slot_out) {
     d.ncell = hd.ncell;
     d.cells = reinterpret_cast<Cell *>(carve(sizeof(Cell) * n));
     d.octa = reinterpret_cast<Octa *>(carve(sizeof(Octa) * n));
-    d.list[0] = reinterpret_cast<uint32_t *>(carve(4 * n));
-    d.list[1] = reinterpret_cast<uint32_t *>(carve(4 * n));
-    d.claim_cell = reinterpret_cast<uint32_t *>(carve(4 * n));
-    d.claim_bits = reinterpret_cast<uint32_t *>(carve(4 * n));
-    d.slice_claims = reinterpret_cast<uint32_t *>(carve(4 * kMaxSlices));
-    d.cand = reinterpret_cast<uint32_t *>(carve(4ull * exaca::apply_blocks(kMaxSlices) * exaca::kCandStage));
-    d.cand_count = reinterpret_cast<uint32_t *>(carve(4 * exaca::apply_blocks(kMaxSlices)));
-    d.cand_cap = exaca::cand_stage_cap();
-    d.list_cap = static_cast<uint32_t>(n);
+    d.claim_cell = reinterpret_cast<uint32_t *>(carve(4 * exaca::claim_entries(hd.ncell, kMaxSlices)));
+    d.claim_bits = reinterpret_cast<uint32_t *>(carve(4 * exaca::claim_entries(hd.ncell, kMaxSlices)));
+    d.claim_count = reinterpret_cast<uint32_t *>(carve(4 * kMaxSlices));
     int32_t *nloc = reinterpret_cast<int32_t *>(carve(4 * std::max<size_t>(hd.nloc.size(), 1)));
     int32_t *ntime = reinterpret_cast<int32_t *>(carve(4 * std::max<size_t>(hd.nloc.size(), 1)));
     double *grow = reinterpret_cast<double *>(carve(8 * pr->grow.size()));
-    const size_t nwords = (n + 31) / 32;
-    d.nchunks = static_cast<uint32_t>((nwords + 2047) / 2048);
     d.alarms = reinterpret_cast<uint32_t *>(carve(4 * kAlarmSlots * alarm_stride(d.ncell)));
-    d.chunk_flag = reinterpret_cast<unsigned long long *>(carve(8ull * d.nchunks));
     d.ctl = reinterpret_cast<StepCtl *>(carve(sizeof(StepCtl)));
     d.stats = reinterpret_cast<StepStats *>(carve(sizeof(StepStats)));
     d.nparts = kMaxSlices;
     d.part = reinterpret_cast<unsigned long long *>(carve(8ull * kPartRows * kMaxSlices));
-    d.nnuclei = static_cast<int32_t>(hd.nloc.size());
+    d.nnuclei = static_cast<int32_t>(loc.size());
     d.nloc = nloc;
     d.ntime = ntime;
     d.guv = e->guv;
@@ -231,9 +222,9 @@ void admit(exaca_ensemble *e, const exaca_prepared *pr, int *slot_out) {
     d.status_err = e->status_d + e->slots + slot;
 
     hipStream_t s = e->stream;
-    if (!hd.nloc.empty()) {
-        HIP_OK(hipMemcpyAsync(nloc, hd.nloc.data(), 4 * hd.nloc.size(), hipMemcpyHostToDevice, s));
-        HIP_OK(hipMemcpyAsync(ntime, hd.ntime.data(), 4 * hd.ntime.size(), hipMemcpyHostToDevice, s));
+    if (!loc.empty()) {
+        HIP_OK(hipMemcpyAsync(nloc, loc.data(), 4 * loc.size(), hipMemcpyHostToDevice, s));
+        HIP_OK(hipMemcpyAsync(ntime, time.data(), 4 * time.size(), hipMemcpyHostToDevice, s));
     }
     HIP_OK(hipMemcpyAsync(grow, pr->grow.data(), 8 * pr->grow.size(), hipMemcpyHostToDevice, s));
     exaca::upload_cells(d, hd, nullptr, s);
@@ -313,10 +304,9 @@ int exaca_prepare(const char *input_file, const char *data_dir, uint64_t seed, e
         const exaca::HostDomain &h = pr->host;
         pr->grow = exaca::growth_table(h.A, h.B, h.C, h.D, h.dU, 1 << 25);
         if (pr->grow.size() >= (1u << 25)) throw std::runtime_error("undercooling never saturates within 2^25 steps");
-        if (exaca::rebuild_units(h.ncell) > exaca::kEnsembleUnits)
+        if (h.ncell > exaca::kEnsembleCells)
             throw std::invalid_argument("domain too large for an ensemble slot (at most " +
-                                        std::to_string(exaca::kEnsembleUnits) +
-                                        " list-rebuild units, about 33 M cells); run it on the plain path");
+                                        std::to_string(exaca::kEnsembleCells) + " cells); run it on the plain path");
         if (h.sparse)  // every cell inside the walls is liquid but the substrate's active cells
             pr->liquid0 = static_cast<long long>(h.nx) * h.ny * (h.nz - 2) - static_cast<long long>(h.active.size());
         else

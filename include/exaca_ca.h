@@ -185,7 +185,8 @@ const char *exaca_last_error(void);
 int exaca_profile_steps(exaca_state *h, int layer, int nsteps, double ms[3], int64_t counts[5]);
 
 /* As exaca_profile_steps with every kernel timed on its own: ms[0..5] = nucleation, claim, the
- * claims' winners, apply, settle and the rebuild of the next step's list. */
+ * claims' winners, apply, settle and the rebuild of the next step's list (the winners are decided in
+ * the apply kernel and the list is gathered in the claim kernel: ms[2], ms[4] and ms[5] are 0). */
 int exaca_profile_kernels(exaca_state *h, int layer, int nsteps, double ms[6], int64_t counts[5]);
 
 /* HBM calibration (no reference counterpart): a plain device copy of `bytes` bytes repeated
