@@ -59,6 +59,10 @@ constexpr uint32_t apply_blocks(uint32_t claim_blocks) { return (claim_blocks + 
 constexpr size_t alarm_stride(long long ncell) {
     return ((static_cast<size_t>(ncell) + 31) / 32 + 7) & ~static_cast<size_t>(7);
 }
+// Workgroups of a team that steps a domain in one launch. A CU holds one of them, so the teams of the
+// four hardware queues a process has always find room beside each other in 256 CUs, however their
+// workgroups are dispatched: no team waits for one of its own that waits for room.
+constexpr int kMaxTeam = 64;
 constexpr int kMaxJumps = 4096;
 constexpr int kMaxLayers = 256;
 
@@ -102,12 +106,13 @@ struct StepCtl {
     uint32_t serial[2];   // steps executed before the step of parity p (its calendar slot)
     uint32_t elo, ehi;    // cell-index range [elo, ehi] holding every active cell (elo > ehi: none)
     int32_t njumps;       // cycle jumps taken so far (spot-melt problems)
-    int32_t error;        // nonzero: invalid grain
+    int32_t error;        // flags: 2 invalid grain, 16 a barrier wait past its bound
     int32_t done;         // set by the device when a domain finishes or raised an error
     int32_t final_cycle;  // the check cycle at which it finished
     int32_t last_cycle;   // the last executed step
     int32_t nuc_at;       // nucleation sites of the layer decided so far (they lie in order of time)
     int32_t nuc_next;     // the same after the nucleation of the current step
+    uint32_t barrier;     // barriers passed by the teams of the launches before
     uint32_t serial_booked;         // steps executed before the last booking of the counters
     unsigned long long nactive;     // active cells at the last booking
     unsigned long long nonwaiting;  // of those, past their liquidus time (the reference's numSteer)
@@ -218,6 +223,7 @@ struct DomainView {
     uint32_t nparts;
     uint32_t *alarms;       // kAlarmSlots bitmaps of one bit per cell: process the cell at the step
                             // whose serial is the bitmap's slot (mod kAlarmSlots)
+    uint32_t *sync;         // the team barrier's words, one per workgroup
     int32_t autostop;       // end the domain on the device at the first check with no liquid left
     long long liquid0;      // liquid cells of the layer at the start
     int32_t *status;        // where the device reports the final cycle of an autostopped domain

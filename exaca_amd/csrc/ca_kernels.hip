@@ -91,7 +91,7 @@ __device__ __forceinline__ int nb_dz(int l) { return static_cast<int>((kPackZ >>
 struct Grid {
     Divisor xy, y;
     int X, Y, nzA;
-    int off[26];  // linear offsets of the 26 neighbours, for loops unrolled over l
+    int row[9];  // linear offsets of the rows of neighbours, (dz + 1) * 3 + dx + 1
     // linear offset of neighbour l for a per-lane l
     __device__ __forceinline__ int offset(int l) const {
         return nb_dz(l) * static_cast<int>(xy.d) + nb_dx(l) * Y + nb_dy(l);
@@ -105,8 +105,31 @@ __device__ __forceinline__ Grid grid_of(const DomainView &d) {
     g.xy = Divisor::make(static_cast<uint32_t>(d.X) * static_cast<uint32_t>(d.Y));
     g.y = Divisor::make(static_cast<uint32_t>(d.Y));
 #pragma unroll
-    for (int l = 0; l < 26; l++) g.off[l] = (kNbZ[l] * d.X + kNbX[l]) * d.Y + kNbY[l];
+    for (int r = 0; r < 9; r++) g.row[r] = ((r / 3 - 1) * d.X + (r % 3 - 1)) * d.Y;
     return g;
+}
+// The neighbours of cell q by rows: neighbour l is one of three consecutive cells of a row, so the
+// nine row addresses and constant offsets reach all 26 (26 addresses of their own would cost the
+// capture pass 34 more registers).
+struct Rows {
+    Cell *row[9];
+    __device__ __forceinline__ Cell &cell(int l) const { return row[(kNbZ[l] + 1) * 3 + kNbX[l] + 1][kNbY[l]]; }
+    // the low word of a cell's liquid-neighbour mask (bits 0-25 and the not-yet-known bit), and the high word
+    __device__ __forceinline__ uint32_t *low(int l) const { return reinterpret_cast<uint32_t *>(&cell(l).lm); }
+    __device__ __forceinline__ uint32_t *high(int l) const { return low(l) + 1; }
+};
+// A cell that is active or was liquid lies off the bottom and top planes (walls), so all 26 of its
+// linear neighbours lie in the array, whatever its x and y: they can be read without a test each,
+// and masked by `valid` after. A cell that did not (there is none) would read those of the nearest
+// one that does, with no valid neighbour.
+__device__ __forceinline__ Rows rows_of(const DomainView &d, const Grid &g, uint32_t q, uint32_t &valid) {
+    const uint32_t reach = g.xy.d + g.y.d + 1, last = static_cast<uint32_t>(d.ncell) - 1 - reach;
+    const uint32_t at = q < reach ? reach : (q > last ? last : q);
+    valid = at == q ? valid : 0u;
+    Rows r;
+#pragma unroll
+    for (int i = 0; i < 9; i++) r.row[i] = d.cells + static_cast<uint32_t>(at + g.row[i]);
+    return r;
 }
 __device__ __forceinline__ Coord decode(uint32_t p, const Grid &g) {
     Coord c;
@@ -320,16 +343,9 @@ __device__ __forceinline__ CellWords load_cell(const Cell *c) {
     return w;
 }
 
-// The low word of a cell's liquid-neighbour mask: bits 0-25 and the not-yet-known bit.
-__device__ __forceinline__ uint32_t *mask_word(const DomainView &d, uint32_t q) {
-    return reinterpret_cast<uint32_t *>(&d.cells[q].lm);
-}
-// The high word: serial + 1 of the last step in which a capture by a cell of index >= q took one
-// of q's liquid neighbours (0: none yet). Written by the capture pass only where the low word is
-// known, so the 64-bit stores of a mask build (which clear it) never meet it in one step.
-__device__ __forceinline__ uint32_t *keep_word(const DomainView &d, uint32_t q) {
-    return reinterpret_cast<uint32_t *>(&d.cells[q].lm) + 1;
-}
+// The high word of an active cell: serial + 1 of the last step in which a capture by a cell of index
+// >= q took one of q's liquid neighbours (0: none yet). Written by the capture pass only where the low
+// word is known, so the 64-bit stores of a mask build (which clear it) never meet it in one step.
 constexpr uint32_t kMaskUnknown = static_cast<uint32_t>(kLmUnknown);
 constexpr uint32_t kMaskNow = static_cast<uint32_t>(kLmNow);
 // A liquid cell's words: the low word keeps bits 26-31 of its initial all-ones value (only bits
@@ -338,7 +354,9 @@ constexpr uint32_t kMaskNow = static_cast<uint32_t>(kLmNow);
 // cell is captured in the same step and never turns liquid again, so a claim word is read only in
 // the step that wrote it, and the capture overwrites both words.
 constexpr uint32_t kLiquidMark = 1u << 30;
-__device__ __forceinline__ uint32_t *claim_word(const DomainView &d, uint32_t q) { return keep_word(d, q); }
+__device__ __forceinline__ uint32_t *claim_word(const DomainView &d, uint32_t q) {
+    return reinterpret_cast<uint32_t *>(&d.cells[q].lm) + 1;
+}
 __device__ __forceinline__ bool is_unclaimed_liquid(unsigned long long lm) {
     return (static_cast<uint32_t>(lm) & kLiquidMark) && static_cast<uint32_t>(lm >> 32) == kClaimNone;
 }
@@ -434,27 +452,31 @@ __device__ __forceinline__ void count_event(bool happened, uint32_t *counter) {
     if (m && (threadIdx.x & 63) == static_cast<uint32_t>(__ffsll(static_cast<long long>(m)) - 1))
         atomicAdd(counter, static_cast<uint32_t>(__popcll(m)));
 }
-// The step's events added to the workgroup's running totals (rows of PartRow, slot b): the counts
-// and, for what changes the number of active cells, the sums of the steps' serials, from which
-// book_totals forms the per-step sums. A late solidification belongs to the step before.
+// A step's contribution to counter row r: the counts and, for what changes the number of active
+// cells, the sums of the steps' serials, from which book_totals forms the per-step sums. A late
+// solidification belongs to the step before.
+__device__ __forceinline__ unsigned long long part_value(uint32_t r, const uint32_t *cnt, uint32_t serial) {
+    const unsigned long long s = serial;
+    switch (r) {
+    case kPartEnt: return cnt[kCntEnt];
+    case kPartEntAt: return cnt[kCntEnt] * s;
+    case kPartSol: return static_cast<unsigned long long>(cnt[kCntSol]) + cnt[kCntLate];
+    case kPartSolAt: return cnt[kCntSol] * s + (cnt[kCntLate] ? cnt[kCntLate] * (s - 1) : 0);
+    case kPartCap: return cnt[kCntCap];
+    case kPartCapAt: return cnt[kCntCap] * s;
+    case kPartAct: return cnt[kCntAct];
+    case kPartActAt: return cnt[kCntAct] * s;
+    case kPartNn: return cnt[kCntNn];
+    case kPartEval: return cnt[kCntEval];
+    case kPartMask: return cnt[kCntMask];
+    default: return 0;
+    }
+}
+// The step's events added to workgroup b's running totals.
 __device__ __forceinline__ void add_parts(const DomainView &d, uint32_t b, const uint32_t *cnt, uint32_t serial) {
     const uint32_t r = threadIdx.x;
     if (r >= kPartRows) return;
-    unsigned long long v = 0;
-    const unsigned long long s = serial;
-    switch (r) {
-    case kPartEnt: v = cnt[kCntEnt]; break;
-    case kPartEntAt: v = cnt[kCntEnt] * s; break;
-    case kPartSol: v = static_cast<unsigned long long>(cnt[kCntSol]) + cnt[kCntLate]; break;
-    case kPartSolAt: v = cnt[kCntSol] * s + (cnt[kCntLate] ? cnt[kCntLate] * (s - 1) : 0); break;
-    case kPartCap: v = cnt[kCntCap]; break;
-    case kPartCapAt: v = cnt[kCntCap] * s; break;
-    case kPartAct: v = cnt[kCntAct]; break;
-    case kPartActAt: v = cnt[kCntAct] * s; break;
-    case kPartNn: v = cnt[kCntNn]; break;
-    case kPartEval: v = cnt[kCntEval]; break;
-    default: v = cnt[kCntMask]; break;
-    }
+    const unsigned long long v = part_value(r, cnt, serial);
     if (v) d.part[static_cast<size_t>(r) * d.nparts + b] += v;
 }
 
@@ -522,12 +544,13 @@ __device__ __forceinline__ int nucleate_body(const DomainView &d, int cycle, uin
                 cq.flags = 0;
                 cq.ct = kActive | kSeedBit;
                 set_centre(d, q, (c.x + d.xoff) + 0.5, (c.y + d.yoff) + 0.5, c.z + 0.5);
-                const uint32_t valid = valid_neighbours(c, gr.X, gr.Y, gr.nzA);
+                uint32_t valid = valid_neighbours(c, gr.X, gr.Y, gr.nzA);
+                const Rows rows = rows_of(d, gr, q, valid);
                 // all updates in flight together, then the results
                 uint32_t old[26];
 #pragma unroll
                 for (int l = 0; l < 26; l++)
-                    old[l] = ((valid >> l) & 1u) ? atomicAnd(mask_word(d, q + gr.off[l]), ~(1u << kOpposite.v[l])) : 0u;
+                    old[l] = ((valid >> l) & 1u) ? atomicAnd(rows.low(l), ~(1u << kOpposite.v[l])) : 0u;
                 uint32_t emptied = 0;
 #pragma unroll
                 for (int l = 0; l < 26; l++)
@@ -586,20 +609,27 @@ __device__ uint32_t evaluate_claims(const DomainView &d, const Grid &gr, uint32_
     const float2 v2 = reinterpret_cast<const float2 *>(row)[12];
     cdl[24] = v2.x;
     cdl[25] = v2.y;
-    uint32_t claimed = 0;
+    // In integer and min/max operations on the lengths, a neighbour that is not liquid (or, for the
+    // threshold, reached) counting as infinitely far: conditions of 26 neighbours at once would need
+    // more scalar registers than there are. dlj - len has its sign bit set exactly when dlj < len.
+    constexpr uint32_t kInf = 0x7F800000u;
+    uint32_t beyond = 0;
     float next = __builtin_inff(), next2 = __builtin_inff();
     int at = -1;
 #pragma unroll
     for (int l = 0; l < 26; l++) {
-        const bool liq = (liquid >> l) & 1u;
-        const bool reach = dlj >= cdl[l];
-        claimed |= static_cast<uint32_t>(liq && reach) << l;
-        const bool open = liq && !reach;
-        const bool lower = open && cdl[l] < next;
-        next2 = lower ? next : ((open && cdl[l] < next2) ? cdl[l] : next2);
-        at = lower ? l : at;
-        next = lower ? cdl[l] : next;
+        const uint32_t liq = static_cast<uint32_t>(static_cast<int32_t>(liquid << (31 - l)) >> 31);
+        const uint32_t len = (__float_as_uint(cdl[l]) & liq) | (kInf & ~liq);
+        const uint32_t sign = __float_as_uint(dlj - __uint_as_float(len));
+        beyond |= (sign >> 31) << l;
+        const uint32_t open = static_cast<uint32_t>(static_cast<int32_t>(sign) >> 31);
+        const float v = __uint_as_float((len & open) | (kInf & ~open));
+        next2 = fminf(next2, fmaxf(next, v));
+        at = v < next ? l : at;
+        next = fminf(next, v);
+        if (l % 4 == 3) __builtin_amdgcn_sched_barrier(0);  // the masked lengths of four neighbours at a time
     }
+    const uint32_t claimed = ~beyond & liquid;
     for (uint32_t m = claimed; m; m &= m - 1) atomicMin(claim_word(d, j + gr.offset(__builtin_ctz(m))), j);
     thr = next;
     hint = threshold_hint(at, next, next2);
@@ -634,12 +664,11 @@ __device__ __forceinline__ UnitRange unit_range(const DomainView &d, uint32_t nb
     if (hi >= static_cast<uint64_t>(d.ncell)) hi = static_cast<uint32_t>(d.ncell - 1);
     return UnitRange{lo / kUnitCells, hi / kUnitCells - lo / kUnitCells + 1};
 }
-// The k-th unit of workgroup b. Workgroups are dispatched round-robin over the 8 XCDs; with enough
-// of them, runs of nb / 8 units go to the workgroups of one XCD, so that neighbouring cells mostly
-// share an L2.
-__device__ __forceinline__ uint32_t unit_of(uint32_t k, uint32_t b, uint32_t nb) {
-    if (nb >= 64 && nb % 8 == 0) return (k * 8 + b % 8) * (nb / 8) + b / 8;
-    return k * nb + b;
+// Workgroup b's place among the nb: its k-th unit is unit k * nb + its place. Workgroups are
+// dispatched round-robin over the 8 XCDs; with enough of them, runs of nb / 8 units go to the
+// workgroups of one XCD, so that neighbouring cells mostly share an L2.
+__device__ __forceinline__ uint32_t place_of(uint32_t b, uint32_t nb) {
+    return nb >= 64 && nb % 8 == 0 ? (b % 8) * (nb / 8) + b / 8 : b;
 }
 __device__ __forceinline__ uint32_t *calendar_slot(const DomainView &d, uint32_t serial) {
     return d.alarms + (serial % kAlarmSlots) * alarm_stride(d.ncell);
@@ -661,22 +690,21 @@ __device__ __forceinline__ void for_due(const DomainView &d, uint32_t serial, ui
     constexpr uint32_t kWaves = BLOCK / 64;
     const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const UnitRange r = unit_range<BLOCK>(d, nb);
-    const uint32_t nwords = static_cast<uint32_t>(bitmap_words(d));
     uint32_t *bits = calendar_slot(d, serial);
     const uint32_t most = (r.n + nb - 1) / nb;  // units of the workgroup that has the most
+    // this lane's word of its wave's first unit, and the end of the range's words
+    const uint32_t first = (r.u0 + wave * nb + place_of(b, nb)) * kUnitWords + lane;
+    const uint32_t nwords = static_cast<uint32_t>(bitmap_words(d));
+    const uint32_t end = (r.u0 + r.n) * kUnitWords < nwords ? (r.u0 + r.n) * kUnitWords : nwords;
     uint32_t fill = 0, done = 0;                // entries in the list; cells of the round already listed
     for (uint32_t k0 = 0; k0 < most;) {
         uint32_t w[kUnitsPerLane], cnt = 0;
-        auto word = [&](uint32_t e) {
-            const uint32_t u = unit_of(k0 + e * kWaves + wave, b, nb);
-            const uint32_t at = (r.u0 + u) * kUnitWords + lane;
-            return u < r.n && at < nwords ? at : 0xFFFFFFFFu;
-        };
+        auto word = [&](uint32_t e) { return first + (k0 + e * kWaves) * nb * kUnitWords; };
+        // all loads in flight together (no test around each: a word past the end reads the last one)
 #pragma unroll
-        for (uint32_t e = 0; e < kUnitsPerLane; e++) {
-            const uint32_t at = word(e);
-            w[e] = at != 0xFFFFFFFFu ? bits[at] : 0u;
-        }
+        for (uint32_t e = 0; e < kUnitsPerLane; e++) w[e] = bits[word(e) < end ? word(e) : end - 1];
+#pragma unroll
+        for (uint32_t e = 0; e < kUnitsPerLane; e++) w[e] = word(e) < end ? w[e] : 0u;
 #pragma unroll
         for (uint32_t e = 0; e < kUnitsPerLane; e++) cnt += __builtin_popcount(w[e]);
         uint32_t wtot;
@@ -696,10 +724,9 @@ __device__ __forceinline__ void for_due(const DomainView &d, uint32_t serial, ui
 #pragma unroll
         for (uint32_t e = 0; e < kUnitsPerLane; e++) {
             if (!w[e]) continue;
-            const uint32_t at = word(e);
-            if (CLEAR && last) bits[at] = 0u;
+            if (CLEAR && last) bits[word(e)] = 0u;
             for (uint32_t m = w[e]; m; m &= m - 1, pos++)
-                if (pos < take) list[fill + pos] = at * 32u + __builtin_ctz(m);
+                if (pos < take) list[fill + pos] = word(e) * 32u + __builtin_ctz(m);
         }
         fill += take;
         done = last ? 0 : done + take;
@@ -754,14 +781,13 @@ __device__ __forceinline__ bool solid_since_last(const CellWords &w, uint32_t se
 // fixed, so no capture is possible before the half-diagonal reaches thr: the cell is scheduled for
 // that step (or for the end of its wait for the liquidus time) and not looked at before, unless a
 // neighbour's capture or nucleation empties its mask. A new active cell starts at thr = 0.
-// Cells with claims go to the workgroup's own region of the claim lists (an LDS counter, no global
-// atomics).
-template <int BLOCK, uint32_t CAP>
+// Cells with claims are numbered by an LDS counter (no global atomics) and handed to put(number, cell,
+// claimed neighbours).
+template <int BLOCK, uint32_t CAP, typename F>
 __device__ __forceinline__ void claim_body(const DomainView &d, const Growth &g, int cycle, uint32_t serial, int layer,
                                            bool follows, uint32_t b, uint32_t nb, uint32_t *list, uint32_t *tot,
-                                           uint32_t *cnt, uint32_t *nclaim) {
+                                           uint32_t *cnt, uint32_t *nclaim, F &&put) {
     const Grid gr = grid_of(d);
-    const uint32_t region = unit_of(0, b, nb) * claim_region(d, nb);
     for_due<BLOCK, CAP, true>(d, serial, b, nb, list, tot, [&](bool has, uint32_t j, const CellWords &w) {
         uint32_t claimed = 0;
         bool entered = false, sol = false, late = false, eval = false, mask = false;
@@ -778,13 +804,12 @@ __device__ __forceinline__ void claim_body(const DomainView &d, const Growth &g,
             uint16_t flags = w.flags;
             if (w.lm & kLmUnknown) {
                 const Coord c = decode(j, gr);
-                const uint32_t valid = valid_neighbours(c, gr.X, gr.Y, gr.nzA);
+                uint32_t valid = valid_neighbours(c, gr.X, gr.Y, gr.nzA);
+                const Rows rows = rows_of(d, gr, j, valid);
                 liquid = 0;
 #pragma unroll
-                for (int l = 0; l < 26; l++) {
-                    const uint32_t q = ((valid >> l) & 1u) ? j + gr.off[l] : j;
-                    liquid |= static_cast<uint32_t>(d.cells[q].ct == kLiquid) << l;
-                }
+                for (int l = 0; l < 26; l++) liquid |= static_cast<uint32_t>(rows.cell(l).ct == kLiquid) << l;
+                liquid &= valid;
                 lm = liquid;
                 mask = true;
             }
@@ -842,10 +867,7 @@ __device__ __forceinline__ void claim_body(const DomainView &d, const Growth &g,
                                    (static_cast<uint32_t>(flags) << 16));
         }
         const uint32_t slot = wave_append(claimed != 0, nclaim);
-        if (claimed) {
-            d.claim_cell[region + slot] = j;
-            d.claim_bits[region + slot] = claimed;
-        }
+        if (claimed) put(slot, j, claimed);
         count_event(entered, &cnt[kCntEnt]);
         count_event(sol, &cnt[kCntSol]);
         count_event(late, &cnt[kCntLate]);
@@ -880,7 +902,7 @@ __device__ __forceinline__ uint32_t capture(const DomainView &d, const Grid &gr,
     const float wcx = static_cast<float>(e.x), wcy = static_cast<float>(e.y), wcz = static_cast<float>(e.z);
     const Coord c = decode(jc, gr);
     const Coord cqc{c.x + nb_dx(l), c.y + nb_dy(l), c.z + nb_dz(l)};
-    const uint32_t valid = valid_neighbours(cqc, gr.X, gr.Y, gr.nzA);
+    uint32_t valid = valid_neighbours(cqc, gr.X, gr.Y, gr.nzA);
     int o = orientation_of(h);
     if (o < 0) {
         atomicOr(&d.ctl->error, 2);
@@ -892,11 +914,11 @@ __device__ __forceinline__ uint32_t capture(const DomainView &d, const Grid &gr,
     const uint4 own = reinterpret_cast<const uint4 *>(d.cells + q)[1];  // cts, gid, win, lid | ct | flags
     // the neighbours' words: the low word is the mask (or liquid marker), the high word
     // of a liquid neighbour its claim word
+    const Rows rows = rows_of(d, gr, q, valid);
     unsigned long long lw[26];
 #pragma unroll
     for (int kk = 0; kk < 26; kk++)
-        lw[kk] = ((valid >> kk) & 1u) ? *reinterpret_cast<const unsigned long long *>(&d.cells[q + gr.off[kk]].lm)
-                                      : static_cast<unsigned long long>(kMaskUnknown);
+        lw[kk] = rows.cell(kk).lm;
     // The new cell's mask: its liquid neighbours at its first visit are those liquid now
     // and not claimed in this step (every claimed cell is captured in this step, and the
     // claims are final). Until its store below, the new cell's own words read as a
@@ -907,27 +929,32 @@ __device__ __forceinline__ uint32_t capture(const DomainView &d, const Grid &gr,
         liquid |= static_cast<uint32_t>(is_unclaimed_liquid(lw[kk])) << kk;
         mw[kk] = static_cast<uint32_t>(lw[kk]);
     }
-    // updates only where the mask still holds q, all in flight together; their results
-    // are used after the octahedron is built, which hides their round trip
     uint32_t need = 0;
 #pragma unroll
     for (int kk = 0; kk < 26; kk++) {
         const uint32_t bit = 1u << kOpposite.v[kk];
         need |= static_cast<uint32_t>((mw[kk] & (kMaskUnknown | bit)) == bit) << kk;
     }
+    liquid &= valid;
+    need &= valid;
+    const double xp = (c.x + d.xoff + nb_dx(l)) + 0.5;
+    const double yp = (c.y + d.yoff + nb_dy(l)) + 0.5;
+    const double zp = (c.z + nb_dz(l)) + 0.5;
+    const Octahedron oc = new_octahedron(gv, wcx, wcy, wcz, xp, yp, zp);
+    // updates only where the mask still holds q, all in flight together; their results are used
+    // after the critical lengths are computed, which hides their round trip (before the octahedron
+    // is built, the 26 results would take more registers than there are)
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int kk = 0; kk < 26; kk++)
-        if ((need >> kk) & 1u) mw[kk] = atomicAnd(mask_word(d, q + gr.off[kk]), ~(1u << kOpposite.v[kk]));
+        if ((need >> kk) & 1u) mw[kk] = atomicAnd(rows.low(kk), ~(1u << kOpposite.v[kk]));
     // a neighbour at or below the claimant's index still had q liquid at its visit
     // in the reference's index order: its keep word gets this step's tag (every writer
     // of a step writes the same value)
 #pragma unroll
     for (int kk = 0; kk < 26; kk++)
-        if (((need >> kk) & 1u) && q + gr.off[kk] <= jc) keep_word(d, q + gr.off[kk])[0] = serial + 1;
-    const double xp = (c.x + d.xoff + nb_dx(l)) + 0.5;
-    const double yp = (c.y + d.yoff + nb_dy(l)) + 0.5;
-    const double zp = (c.z + nb_dz(l)) + 0.5;
-    const Octahedron oc = new_octahedron(gv, wcx, wcy, wcz, xp, yp, zp);
+        if (((need >> kk) & 1u) && q + gr.row[(kNbZ[kk] + 1) * 3 + kNbX[kk] + 1] + kNbY[kk] <= jc)
+            *rows.high(kk) = serial + 1;
     // The new cell's record, whole: nothing else writes it in this pass.
     uint4 *r4 = reinterpret_cast<uint4 *>(d.cells + q);
     r4[0] = make_uint4(liquid, 0u, __float_as_uint(static_cast<float>(oc.dl)), __float_as_uint(0.0f));
@@ -982,11 +1009,18 @@ __device__ __forceinline__ void apply_body(const DomainView &d, uint32_t serial,
         if (k < n) {
             claimant(k, j, cb);
             gid = d.cells[j].gid;
-            uint32_t cw[26];
+            // a claimant mostly has one or two claims: four words in flight at a time
+            for (uint32_t m = cb; m;) {
+                uint32_t bit[4], cw[4];
 #pragma unroll
-            for (int l = 0; l < 26; l++) cw[l] = ((cb >> l) & 1u) ? *claim_word(d, j + gr.off[l]) : kClaimNone;
+                for (int e = 0; e < 4; e++) {
+                    bit[e] = m & (0u - m);
+                    m &= m - 1;
+                    cw[e] = *claim_word(d, bit[e] ? j + gr.offset(__builtin_ctz(bit[e])) : j);
+                }
 #pragma unroll
-            for (int l = 0; l < 26; l++) won |= static_cast<uint32_t>(cw[l] == j) << l;
+                for (int e = 0; e < 4; e++) won |= cw[e] == j ? bit[e] : 0u;
+            }
         }
         const uint32_t slot = wave_append(won != 0, &s.nwin);
         if (won) {
@@ -1070,29 +1104,24 @@ __device__ __forceinline__ void settle_body(const DomainView &d, const Growth &g
 // reference's numSteer of a step: active cells past their liquidus time at the start of its capture
 // pass.
 template <int BLOCK>
-__device__ __forceinline__ void book_totals(const DomainView &d, uint32_t serial_now, unsigned long long (*red)[BLOCK / 64]) {
+__device__ __forceinline__ void book_totals(const DomainView &d, uint32_t serial_now, unsigned long long *red) {
     StepCtl *ctl = d.ctl;
-#pragma unroll 1
-    for (int r = 0; r < kPartRows; r++) {
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    for (int r = wave; r < kPartRows; r += BLOCK / 64) {
         unsigned long long *row = d.part + static_cast<size_t>(r) * d.nparts;
         unsigned long long v = 0;
-        for (uint32_t i = threadIdx.x; i < d.nparts; i += BLOCK) {
+        for (uint32_t i = lane; i < d.nparts; i += 64) {
             const unsigned long long x = row[i];
             v += x;
             if (x) row[i] = 0;
         }
 #pragma unroll
         for (int o = 32; o > 0; o >>= 1) v += __shfl_down(v, o, 64);
-        if ((threadIdx.x & 63) == 0) red[r][threadIdx.x >> 6] = v;
+        if (lane == 0) red[r] = v;
     }
     __syncthreads();
     if (threadIdx.x != 0) return;
-    unsigned long long v[kPartRows];
-#pragma unroll
-    for (int r = 0; r < kPartRows; r++) {
-        v[r] = 0;
-        for (int w = 0; w < BLOCK / 64; w++) v[r] += red[r][w];
-    }
+    const unsigned long long *v = red;
     StepStats st = *d.stats;
     const unsigned long long S = serial_now, n = S - ctl->serial_booked;
     const unsigned long long ent = S * v[kPartEnt] - v[kPartEntAt];          // from the same step on
@@ -1264,7 +1293,12 @@ __device__ __forceinline__ void claim_step(const DomainView &d, int p, int layer
         ctl->serial[1 - p] = serial + 1;
         ctl->nuc_at = max(ctl->nuc_at, ctl->nuc_next);
     }
-    claim_body<kBlock, kDueStage>(d, g, cycle, serial, layer, follows_last(ctl, cycle), b, nb, list, tot, t.cnt, &nclaim);
+    const uint32_t region = place_of(b, nb) * claim_region(d, nb);
+    claim_body<kBlock, kDueStage>(d, g, cycle, serial, layer, follows_last(ctl, cycle), b, nb, list, tot, t.cnt, &nclaim,
+                                  [&](uint32_t k, uint32_t j, uint32_t claimed) {
+                                      d.claim_cell[region + k] = j;
+                                      d.claim_bits[region + k] = claimed;
+                                  });
     __syncthreads();
     if (threadIdx.x == 0) d.claim_count[b] = nclaim;
     add_parts(d, b, t.cnt, serial);
@@ -1281,10 +1315,10 @@ __device__ __forceinline__ void apply_step(const DomainView &d, int p, uint32_t 
     static_assert(kApplyGroup == 2, "two regions");
     const uint32_t region = claim_region(d, nbc);
     n0 = n = d.claim_count[2 * a];
-    r0 = unit_of(0, 2 * a, nbc) * region;
+    r0 = place_of(2 * a, nbc) * region;
     if (2 * a + 1 < nbc) {
         n += d.claim_count[2 * a + 1];
-        r1 = unit_of(0, 2 * a + 1, nbc) * region;
+        r1 = place_of(2 * a + 1, nbc) * region;
     }
     clear_tally(t);
     apply_body<kBlock>(
@@ -1310,10 +1344,156 @@ __device__ __forceinline__ void settle_step(const DomainView &d, int p_next, int
     add_parts(d, b, t.cnt, serial);
 }
 __device__ __forceinline__ void book_step(const DomainView &d, int p_next) {
-    __shared__ unsigned long long red[kPartRows][kBlock / 64];
+    __shared__ unsigned long long red[kPartRows];
     if (d.ctl->done) return;
     book_totals<kBlock>(d, d.ctl->serial[p_next], red);
     if (threadIdx.x == 0) end_domain(d, d.ctl->last_cycle);
+}
+
+// ---- A team of workgroups that runs many steps of one domain in one launch. ----
+
+// The team's barrier: every workgroup posts the barrier's number in its own word and waits for all
+// the others' words (each polls all of them: one hop, 1.7 us for 8 workgroups and 2.6 us for 32,
+// against 2.0 and 2.7 us with a workgroup that gathers and releases). What the team wrote before it
+// is visible to the team after it (agent-scope release and acquire by one wave, ordered with the rest
+// of the workgroup by its own barriers). A team of one needs the workgroup's barrier alone.
+// Teams are small enough that their workgroups always find room beside each other (kMaxTeam); the wait
+// is bounded all the same, by the 100 MHz clock: false (with error 16) past it, for every thread.
+constexpr unsigned long long kTeamWait = 2000000000ull;  // 20 s
+struct Team {
+    uint32_t b, nb;
+    uint32_t number;  // of the last barrier passed
+};
+__device__ __forceinline__ bool team_sync(const DomainView &d, Team &t) {
+    __syncthreads();
+    if (t.nb == 1) return true;
+    t.number++;
+    bool late = false;
+    if (threadIdx.x < 64) {
+        if (threadIdx.x == 0) {
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+            __hip_atomic_store(d.sync + t.b, t.number, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+        if (threadIdx.x < t.nb) {
+            const unsigned long long t0 = wall_clock64();
+            while (static_cast<int32_t>(__hip_atomic_load(d.sync + threadIdx.x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) -
+                                        t.number) < 0) {
+                if (wall_clock64() - t0 > kTeamWait) {
+                    atomicOr(&d.ctl->error, 16);
+                    late = true;
+                    break;
+                }
+            }
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+    }
+    return !__syncthreads_or(late);
+}
+
+constexpr uint32_t kTeamDue = 2048;     // due cells of a turn staged in LDS
+constexpr uint32_t kTeamClaims = 1024;  // claimants staged in LDS; the rest go to the claim lists
+
+struct TeamLds {
+    double grow[kGrowStage];
+    ApplyLds<kTeamBlock> apply;
+    uint32_t list[kTeamDue];
+    uint32_t claim_cell[kTeamClaims], claim_bits[kTeamClaims];
+    uint32_t tot[kTeamBlock / 64];
+    uint32_t nclaim;
+    StepTally tally[2];
+    unsigned long long red[kPartRows];
+};
+
+// nsteps steps of one domain (nucleate: their nucleation too), settled and booked at the end. Two
+// barriers a step: the claims of a step before its winners, its captures before the next step's due
+// cells; a step with a nucleation site due has one more. Control words and counters stay in registers
+// and LDS, the growth table in LDS, and caches and code stay warm from step to step.
+__device__ __forceinline__ void steps_body(const DomainView &d, int p, int layer, int nsteps, bool nucleate, uint32_t b,
+                                           uint32_t nb, TeamLds &s) {
+    StepCtl *ctl = d.ctl;
+    if (ctl->done) return;
+    Team team{b, nb, ctl->barrier};
+    int cycle = ctl->cycle[p];
+    uint32_t serial = ctl->serial[p];
+    bool follows = follows_last(ctl, cycle);
+    int site = max(ctl->nuc_at, ctl->nuc_next);
+    int next_site = nucleate && site < d.nnuclei ? d.ntime[site] : 0x7FFFFFFF;
+    const Growth g = staged_growth<kTeamBlock>(d, s.grow);
+    const uint32_t region = place_of(b, nb) * claim_region(d, nb);
+    const bool whole = scans_all<kTeamBlock>(d, nb);
+    clear_tally(s.tally[0]);
+    clear_tally(s.tally[1]);
+    unsigned long long acc = 0;  // thread r: counter row r
+    const int p_end = (p + nsteps) & 1;
+    while (nsteps > 0) {
+        // a domain with autostop is looked at after every step whose cycle is a multiple of 1000
+        int n = nsteps;
+        if (d.autostop && n > 1000 - (cycle - 1) % 1000) n = 1000 - (cycle - 1) % 1000;
+        nsteps -= n;
+        for (; n > 0; n--) {
+            StepTally &t = s.tally[serial & 1], &before = s.tally[(serial & 1) ^ 1];
+            if (cycle >= next_site) {
+                site += nucleate_body<kTeamBlock>(d, cycle, serial, layer, site, b, nb, t.cnt, t.lohi);
+                next_site = site < d.nnuclei ? d.ntime[site] : 0x7FFFFFFF;
+                if (!whole) widen_range(d, t.lohi);
+                if (!team_sync(d, team)) return;
+            }
+            if (threadIdx.x == 0) s.nclaim = 0;
+            __syncthreads();
+            claim_body<kTeamBlock, kTeamDue>(d, g, cycle, serial, layer, follows, b, nb, s.list, s.tot, t.cnt, &s.nclaim,
+                                             [&](uint32_t k, uint32_t j, uint32_t claimed) {
+                                                 if (k < kTeamClaims) {
+                                                     s.claim_cell[k] = j;
+                                                     s.claim_bits[k] = claimed;
+                                                 }
+                                                 else {
+                                                     d.claim_cell[region + k] = j;
+                                                     d.claim_bits[region + k] = claimed;
+                                                 }
+                                             });
+            if (!team_sync(d, team)) return;
+            if (threadIdx.x < kStepCounts) before.cnt[threadIdx.x] = 0;
+            apply_body<kTeamBlock>(
+                d, serial, s.nclaim,
+                [&](uint32_t k, uint32_t &j, uint32_t &bits) {
+                    j = k < kTeamClaims ? s.claim_cell[k] : d.claim_cell[region + k];
+                    bits = k < kTeamClaims ? s.claim_bits[k] : d.claim_bits[region + k];
+                },
+                s.apply, t.cnt, t.lohi);
+            if (!whole) widen_range(d, t.lohi);
+            if (!team_sync(d, team)) return;
+            acc += part_value(threadIdx.x, t.cnt, serial);
+            follows = true;
+            cycle++;
+            serial++;
+        }
+        StepTally &t = s.tally[serial & 1], &before = s.tally[(serial & 1) ^ 1];
+        settle_body<kTeamBlock, kTeamDue>(d, g, cycle, serial, layer, b, nb, s.list, s.tot, t.cnt);
+        widen_range(d, t.lohi);
+        widen_range(d, before.lohi);
+        acc += part_value(threadIdx.x, t.cnt, serial);
+        if (threadIdx.x < kPartRows && acc) d.part[static_cast<size_t>(threadIdx.x) * d.nparts + b] += acc;
+        acc = 0;
+        if (!team_sync(d, team)) return;
+        clear_tally(s.tally[0]);
+        clear_tally(s.tally[1]);
+        if (b == 0) {
+            book_totals<kTeamBlock>(d, serial, s.red);
+            if (threadIdx.x == 0) {
+                ctl->last_cycle = cycle - 1;
+                ctl->nuc_at = site;
+                end_domain(d, cycle - 1);
+                ctl->cycle[p_end] = cycle;
+                ctl->serial[p_end] = serial;
+                ctl->barrier = team.number + (nsteps > 0);  // with the barrier below
+            }
+        }
+        follows = false;  // settled
+        if (nsteps > 0) {
+            if (!team_sync(d, team)) return;
+            if (ctl->done) return;
+        }
+    }
 }
 
 // Plain launches: one domain, passed by value.
@@ -1330,6 +1510,10 @@ __global__ __launch_bounds__(kBlock) void k_settle(DomainView d, int p_next, int
     settle_step(d, p_next, layer, blockIdx.x, gridDim.x);
 }
 __global__ __launch_bounds__(kBlock) void k_book(DomainView d, int p_next) { book_step(d, p_next); }
+__global__ __launch_bounds__(kTeamBlock) void k_steps(DomainView d, int p, int layer, int nsteps, int nucleate) {
+    __shared__ TeamLds s;
+    steps_body(d, p, layer, nsteps, nucleate != 0, blockIdx.x, gridDim.x, s);
+}
 
 // Ensemble launches: grid row y serves domain slot y of a device-resident table; an empty slot has
 // no control block.
@@ -1658,6 +1842,9 @@ void launch_capture(const DomainView &d, int parity, int layer, int blocks, hipS
 void launch_settle(const DomainView &d, int parity_next, int layer, int blocks, hipStream_t s) {
     k_settle<<<blocks, kBlock, 0, s>>>(d, parity_next, layer);
     k_book<<<1, kBlock, 0, s>>>(d, parity_next);
+}
+void launch_steps(const DomainView &d, int parity, int layer, int steps, bool nucleate, int team, hipStream_t s) {
+    k_steps<<<team, kTeamBlock, 0, s>>>(d, parity, layer, steps, nucleate ? 1 : 0);
 }
 void launch_layer_bounds(const DomainView &d, int next_layer, int *out, hipStream_t s) {
     k_layer_bounds<<<grid_for(d.ncell, 4096), kBlock, 0, s>>>(d, next_layer, out);

@@ -20,6 +20,10 @@ void launch_capture(const DomainView &d, int parity, int layer, int blocks, hipS
 // The solidifications the last step left to the next one, and the counters booked: before the state
 // or the statistics are looked at. parity_next is the parity of the next step.
 void launch_settle(const DomainView &d, int parity_next, int layer, int blocks, hipStream_t s);
+// `steps` steps in one launch of a team of workgroups (at most kMaxTeam), settled and booked;
+// nucleate: with their nucleation (else none of their sites may be due).
+constexpr int kTeamBlock = 512;
+void launch_steps(const DomainView &d, int parity, int layer, int steps, bool nucleate, int team, hipStream_t s);
 // Units of a calendar slot, and entries of the claim lists for up to most_blocks capture-pass
 // workgroups.
 uint32_t calendar_units(long long ncell);

@@ -158,6 +158,7 @@ struct exaca_state {
     int cycle = 0;         // last executed step
     int pending = -1;      // cycle whose nucleation ran but whose capture has not
     int blocks = 2048;     // workgroups of the frontier kernels
+    int team = 0;          // workgroups of the resident kernel that runs many steps (0: two launches a step)
     int njumps = 0;
     hipGraphExec_t graph = nullptr;       // kGraphSteps steps
     hipGraphExec_t graph_quiet = nullptr; // the same without the nucleation kernels
@@ -194,6 +195,18 @@ struct exaca_state {
 
 namespace {
 
+// Workgroups of the team that steps a domain in one launch, by the cross-section X * Y that its front
+// spreads over; 0: too wide, two launches a step over the whole device are faster. Measured, us a
+// step with a team of the size chosen and with two launches: 24^3 13.4 (1) and 17.0; 64^3 20.7 (16)
+// and 22.0; 100^3 22.8 (32) and 23.4; 200^3 33.5 (64) and 45.1; 256^3 44.7 (64) and 44.5.
+int team_size(const exaca::HostDomain &hd) {
+    const long long area = static_cast<long long>(hd.X) * hd.Y;
+    if (area <= 48 * 48) return 1;
+    if (area <= 80 * 80) return 16;
+    if (area <= 128 * 128) return 32;
+    return area <= 240 * 240 ? 64 : 0;
+}
+
 // The layer's nucleation sites to the device; its steps start with none decided. Synchronises the
 // stream.
 void upload_sites(exaca_state *h, int layer) {
@@ -226,7 +239,11 @@ void build_device_state(exaca_state *h) {
     const long long cap = std::min<long long>(2048, ((prop.multiProcessorCount * 4 + 7) / 8) * 8);
     const long long want = ((hd.ncell / 4096 + 7) / 8) * 8;
     h->blocks = static_cast<int>(std::max<long long>(8, std::min(cap, want)));
-    if (const int forced = exaca::frontier_blocks_override()) h->blocks = forced;
+    h->team = std::min(team_size(hd), prop.multiProcessorCount / 4);
+    if (const int forced = exaca::frontier_blocks_override()) {
+        h->blocks = forced;
+        h->team = 0;
+    }
 
     DomainView &d = h->dv;
     d.X = hd.X;
@@ -239,8 +256,8 @@ void build_device_state(exaca_state *h) {
     const size_t n = static_cast<size_t>(hd.ncell);
     d.cells = h->alloc<Cell>(n);
     d.octa = h->alloc<Octa>(n);
-    d.claim_cell = h->alloc<uint32_t>(claim_entries(hd.ncell, h->blocks));
-    d.claim_bits = h->alloc<uint32_t>(claim_entries(hd.ncell, h->blocks));
+    d.claim_cell = h->alloc<uint32_t>(claim_entries(hd.ncell, static_cast<uint32_t>(std::max(h->blocks, kMaxTeam))));
+    d.claim_bits = h->alloc<uint32_t>(claim_entries(hd.ncell, static_cast<uint32_t>(std::max(h->blocks, kMaxTeam))));
     d.claim_count = h->alloc<uint32_t>(h->blocks);
     d.alarms = h->alloc<uint32_t>(kAlarmSlots * alarm_stride(d.ncell));
     h->nloc = h->alloc<int32_t>(hd.nloc.size());
@@ -257,12 +274,13 @@ void build_device_state(exaca_state *h) {
     d.grow = grow_d;
     d.ngrow = static_cast<int32_t>(grow.size());
     d.ksat = growth_plateau(grow);
+    d.sync = h->alloc<uint32_t>(kMaxTeam);
     h->ctl = h->alloc<StepCtl>(1);
     h->stats = h->alloc<StepStats>(1);
     h->check = h->alloc<CheckResult>(1);
     d.ctl = h->ctl;
     d.stats = h->stats;
-    d.nparts = static_cast<uint32_t>(std::max(h->blocks, 64));  // the capture grid and the nucleation grid (<= 64)
+    d.nparts = static_cast<uint32_t>(std::max(h->blocks, kMaxTeam));  // the capture grid, the team and the nucleation grid (<= 64)
     d.part = h->alloc<unsigned long long>(static_cast<size_t>(kPartRows) * d.nparts);
 
     // Initial state; per-cell undercooling is not stored (it is a function of the steps executed
@@ -277,6 +295,7 @@ void build_device_state(exaca_state *h) {
     StepCtl c = initial_ctl(hd);
     HIP_OK(hipMemcpyAsync(h->ctl, &c, sizeof c, hipMemcpyHostToDevice, s));
     HIP_OK(hipMemsetAsync(h->stats, 0, sizeof(StepStats), s));
+    HIP_OK(hipMemsetAsync(d.sync, 0, 4 * kMaxTeam, s));
     HIP_OK(hipMemsetAsync(d.part, 0, 8ull * kPartRows * d.nparts, s));
     HIP_OK(hipStreamSynchronize(s));
 }
@@ -404,6 +423,14 @@ void ensure_graph(exaca_state *h, int layer) {
 
 void run_steps(exaca_state *h, int layer, int n, bool use_graph) {
     if (n <= 0) return;
+    if (h->team) {
+        exaca::launch_steps(h->dv, h->parity, layer, n, true, h->team, h->stream);
+        HIP_OK(hipGetLastError());
+        h->cycle += n;
+        h->parity ^= n & 1;
+        h->nuc_through = h->cycle;
+        return;
+    }
     while (n > 0) {
         if (use_graph && h->parity == 0 && n >= kGraphSteps) {
             ensure_graph(h, layer);
@@ -772,9 +799,16 @@ int exaca_cell_capture(exaca_state *h, int cycle, int layer) {
     return guarded([&] {
         if (!h) throw std::invalid_argument("null handle");
         if (h->pending != cycle) throw StateError("capture requires nucleation of the same cycle first");
-        step_capture(h, layer);
-        h->parity ^= 1;
-        finish_steps(h, layer);
+        if (h->team) {
+            exaca::launch_steps(h->dv, h->parity, layer, 1, false, h->team, h->stream);
+            HIP_OK(hipGetLastError());
+            h->parity ^= 1;
+        }
+        else {
+            step_capture(h, layer);
+            h->parity ^= 1;
+            finish_steps(h, layer);
+        }
         h->cycle = cycle;
         h->pending = -1;
     });

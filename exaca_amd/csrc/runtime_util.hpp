@@ -30,13 +30,14 @@ inline std::string device_error_text(int flags) {
     std::string s = "device error flag " + std::to_string(flags) + " (";
     const char *sep = "";
     if (flags & 2) s += sep, s += "2: an active cell with GrainID 0", sep = ", ";
-    if (flags & ~2) s += sep, s += "unknown bits";
+    if (flags & 16) s += sep, s += "16: a barrier wait that did not end within its bound", sep = ", ";
+    if (flags & ~18) s += sep, s += "unknown bits";
     return s + ")";
 }
 
 // Workgroups of the frontier kernels of a plain-path handle: EXACA_BLOCKS (8 .. 2048, a multiple
-// of 8) overrides the size-based choice. Tests narrow it so that slices hold many claimants and
-// the kernels' multi-round paths run.
+// of 8) overrides the size-based choice, with two launches a step whatever the size. Tests narrow it
+// so that a workgroup holds many claimants and the kernels' multi-round paths run.
 inline int frontier_blocks_override() {
     const char *env = std::getenv("EXACA_BLOCKS");
     if (!env) return 0;
