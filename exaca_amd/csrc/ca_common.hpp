@@ -52,9 +52,6 @@ constexpr uint16_t kFresh = 2;  // mask built by the cell's capture; not yet loo
 // Steps ahead a cell can be scheduled; a cell with nothing to do for longer is scheduled at the
 // horizon and checks again.
 constexpr uint32_t kAlarmSlots = 64;
-// The apply pass: one workgroup per kApplyGroup capture-pass workgroups.
-constexpr uint32_t kApplyGroup = 2;
-constexpr uint32_t apply_blocks(uint32_t claim_blocks) { return (claim_blocks + kApplyGroup - 1) / kApplyGroup; }
 // Words of one calendar slot: one bit per cell, rounded up to 32-byte rows.
 constexpr size_t alarm_stride(long long ncell) {
     return ((static_cast<size_t>(ncell) + 31) / 32 + 7) & ~static_cast<size_t>(7);
@@ -177,23 +174,49 @@ enum FieldKind : int {
     kFieldCentreF64 = 10,
 };
 
-// Running counters since the last booking, one slot per workgroup (part[row * nparts + workgroup]):
-// every workgroup adds to its own slot, and the booking sums the rows. Same-address atomics from
-// thousands of workgroups would serialise. The ...At rows sum the serials of the events' steps.
-enum PartRow : int {
-    kPartEnt,    // first step past the liquidus time
-    kPartEntAt,
-    kPartSol,    // solidified
-    kPartSolAt,
-    kPartCap,    // captures
-    kPartCapAt,
-    kPartAct,    // nucleation events
-    kPartActAt,
-    kPartNn,     // nucleation events counted as the reference's nn
-    kPartEval,   // critical-length evaluations
-    kPartMask,   // liquid masks built
-    kPartRows
+// Events of a step that the workgroups count.
+enum StepCount : int {
+    kCntEnt,   // first step past the liquidus time
+    kCntSol,   // solidified
+    kCntLate,  // solidified in the step before
+    kCntCap,   // captures
+    kCntAct,   // nucleation events
+    kCntNn,    // nucleation events counted as the reference's nn
+    kCntEval,  // critical-length evaluations
+    kCntMask,  // liquid masks built
+    kStepCounts
 };
+// Running counters since the last booking, one slot per workgroup (part[row * nparts + workgroup]), two
+// rows per kind of event: their number, and the sum of the serials of their steps. Every workgroup
+// adds to its own slot, and the booking sums the rows. Same-address atomics from thousands of
+// workgroups would serialise.
+constexpr int kPartRows = 2 * kStepCounts;
+
+// Unsigned division by a constant of the domain as a multiply-high and shifts (the round-up method;
+// exact for every 32-bit dividend). Made on the host: its two 64-bit divisions take a wave a
+// microsecond.
+struct Divisor {
+    uint32_t d, mul, sh1, sh2;
+    static Divisor make(uint32_t d) {
+        Divisor r;
+        r.d = d;
+        uint32_t l = 0;
+        while ((1ull << l) < d) l++;
+        r.mul = static_cast<uint32_t>(((1ull << 32) * ((1ull << l) - d)) / d + 1);
+        r.sh1 = l > 0 ? 1 : 0;
+        r.sh2 = l > 0 ? l - 1 : 0;
+        return r;
+    }
+#ifdef __HIPCC__
+    __device__ __forceinline__ uint32_t div(uint32_t n) const {
+        const uint32_t t = __umulhi(n, mul);
+        return (t + ((n - t) >> sh1)) >> sh2;
+    }
+#endif
+};
+// Units of the calendar: kUnitWords words of a slot, one wave-wide load.
+constexpr uint32_t kUnitWords = 64;
+constexpr uint32_t kUnitCells = 32 * kUnitWords;
 
 // Everything a kernel needs to address one CA domain.
 struct DomainView {
@@ -202,6 +225,8 @@ struct DomainView {
     int zlo;                // ZBound_Low, the window's bottom plane (0 in the first layer)
     int xoff, yoff;         // MyXOffset, MyYOffset (-1 for one rank)
     long long ncell;        // X*Y*nz
+    Divisor by_xy, by_y;    // division by X*Y and by Y
+    uint32_t nwords, units; // words of a calendar slot that hold cells, and its units
     Cell *cells;
     Octa *octa;             // octahedron records (centre, critical lengths)
     uint32_t *claim_cell;   // cells with claims in the current step, each capture-pass workgroup's in
@@ -214,6 +239,8 @@ struct DomainView {
     const float *seed_cdl;  // 10000 rows of kCdlStride: the 26 critical diagonal lengths of a
                             // cell-centred octahedron of each orientation
     const double *grow;     // growth increment after k executed steps below the liquidus
+    const uint32_t *grow_sums;  // rows of sums of the increments' deltas (growth_sums), of ksat + 2 entries
+    uint32_t sums_usable;   // the rows that hold
     int32_t ngrow;          // table length; the last entry holds for every larger k
     int32_t ksat;           // from this k on every increment is the last entry (the 0.045 cap or the
                             // 210 K saturation)
@@ -229,5 +256,18 @@ struct DomainView {
     int32_t *status;        // where the device reports the final cycle of an autostopped domain
     int32_t *status_err;    // where it reports the error flags of a domain stopped by an error
 };
+
+// The view's sizes for a domain of X x Y x nz cells, the top of its active window at nzA.
+inline void set_geometry(DomainView &d, int X, int Y, int nz, int nzA) {
+    d.X = X;
+    d.Y = Y;
+    d.nz = nz;
+    d.nzA = nzA;
+    d.ncell = static_cast<long long>(X) * Y * nz;
+    d.by_xy = Divisor::make(static_cast<uint32_t>(X) * static_cast<uint32_t>(Y));
+    d.by_y = Divisor::make(static_cast<uint32_t>(Y));
+    d.nwords = static_cast<uint32_t>((d.ncell + 31) / 32);
+    d.units = (d.nwords + kUnitWords - 1) / kUnitWords;
+}
 
 }  // namespace exaca

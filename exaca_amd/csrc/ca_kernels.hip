@@ -63,26 +63,6 @@ __device__ __forceinline__ int executed_in(int t, int cycle, const StepCtl *ctl,
 struct Coord {
     int x, y, z;
 };
-// Unsigned division by a runtime-uniform divisor as a multiply-high and shifts (the round-up
-// method; exact for every 32-bit dividend). mul/shift come from Divisor::make on the host side of
-// the kernel (uniform, so they live in scalar registers).
-struct Divisor {
-    uint32_t d, mul, sh1, sh2;
-    __host__ __device__ static Divisor make(uint32_t d) {
-        Divisor r;
-        r.d = d;
-        uint32_t l = 0;
-        while ((1ull << l) < d) l++;
-        r.mul = static_cast<uint32_t>(((1ull << 32) * ((1ull << l) - d)) / d + 1);
-        r.sh1 = l > 0 ? 1 : 0;
-        r.sh2 = l > 0 ? l - 1 : 0;
-        return r;
-    }
-    __device__ __forceinline__ uint32_t div(uint32_t n) const {
-        const uint32_t t = __umulhi(n, mul);
-        return (t + ((n - t) >> sh1)) >> sh2;
-    }
-};
 // Offsets of neighbour l (a per-lane value) decoded from the packed constants.
 __device__ __forceinline__ int nb_dx(int l) { return static_cast<int>((kPackX >> (2 * l)) & 3u) - 1; }
 __device__ __forceinline__ int nb_dy(int l) { return static_cast<int>((kPackY >> (2 * l)) & 3u) - 1; }
@@ -102,8 +82,8 @@ __device__ __forceinline__ Grid grid_of(const DomainView &d) {
     g.X = d.X;
     g.Y = d.Y;
     g.nzA = d.nzA;
-    g.xy = Divisor::make(static_cast<uint32_t>(d.X) * static_cast<uint32_t>(d.Y));
-    g.y = Divisor::make(static_cast<uint32_t>(d.Y));
+    g.xy = d.by_xy;
+    g.y = d.by_y;
 #pragma unroll
     for (int r = 0; r < 9; r++) g.row[r] = ((r / 3 - 1) * d.X + (r % 3 - 1)) * d.Y;
     return g;
@@ -118,14 +98,17 @@ struct Rows {
     __device__ __forceinline__ uint32_t *low(int l) const { return reinterpret_cast<uint32_t *>(&cell(l).lm); }
     __device__ __forceinline__ uint32_t *high(int l) const { return low(l) + 1; }
 };
-// A cell that is active or was liquid lies off the bottom and top planes (walls), so all 26 of its
-// linear neighbours lie in the array, whatever its x and y: they can be read without a test each,
-// and masked by `valid` after. A cell that did not (there is none) would read those of the nearest
-// one that does, with no valid neighbour.
-__device__ __forceinline__ Rows rows_of(const DomainView &d, const Grid &g, uint32_t q, uint32_t &valid) {
+// A cell that is active or was liquid lies inside the walls, so all 26 of its linear neighbours lie
+// in the array: they can be read without a test each, and masked by the valid ones after. For a cell
+// that did not (there is none), the nearest one that does, and no valid neighbour.
+__device__ __forceinline__ uint32_t inner_cell(const DomainView &d, const Grid &g, uint32_t q, uint32_t &valid) {
     const uint32_t reach = g.xy.d + g.y.d + 1, last = static_cast<uint32_t>(d.ncell) - 1 - reach;
     const uint32_t at = q < reach ? reach : (q > last ? last : q);
     valid = at == q ? valid : 0u;
+    return at;
+}
+__device__ __forceinline__ Rows rows_of(const DomainView &d, const Grid &g, uint32_t q, uint32_t &valid) {
+    const uint32_t at = inner_cell(d, g, q, valid);
     Rows r;
 #pragma unroll
     for (int i = 0; i < 9; i++) r.row[i] = d.cells + static_cast<uint32_t>(at + g.row[i]);
@@ -189,8 +172,8 @@ __device__ __forceinline__ Faces faces_of(const float *g) {
 // (xp, yp, zp): the largest |F_q . (x_l - c)| (src/CAupdate.cpp:553-563), rounded to float as
 // the reference stores it.
 __device__ __forceinline__ float critical_length(const Faces &f, double xp, double yp, double zp, double cx,
-                                                 double cy, double cz, int l) {
-    const double ex = xp + nb_dx(l) - cx, ey = yp + nb_dy(l) - cy, ez = zp + nb_dz(l) - cz;
+                                                 double cy, double cz, int dx, int dy, int dz) {
+    const double ex = xp + dx - cx, ey = yp + dy - cy, ez = zp + dz - cz;
     const double d0 = ex * f.fx[0] + ey * f.fy[0] + ez * f.fz[0];
     const double d1 = ex * f.fx[1] + ey * f.fy[1] + ez * f.fz[1];
     const double d2 = ex * f.fx[2] + ey * f.fy[2] + ez * f.fz[2];
@@ -218,10 +201,11 @@ __device__ __forceinline__ double sel3(int i, double a, double b, double c) { re
 __device__ Octahedron new_octahedron(const float *g, double cxold, double cyold, double czold, double xp, double yp,
                                      double zp) {
     const double x0 = xp - cxold, y0 = yp - cyold, z0 = zp - czold;
-    const double mag0 = sqrtf(static_cast<float>(x0 * x0 + y0 * y0 + z0 * z0));
-    const double a1 = (g[0] * x0 + g[1] * y0 + g[2] * z0) / mag0;
-    const double a2 = (g[3] * x0 + g[4] * y0 + g[5] * z0) / mag0;
-    const double a3 = (g[6] * x0 + g[7] * y0 + g[8] * z0) / mag0;
+    // the reference divides these by the distance of the centres; only their signs are used, and
+    // the quotient's sign is the dividend's
+    const double a1 = g[0] * x0 + g[1] * y0 + g[2] * z0;
+    const double a2 = g[3] * x0 + g[4] * y0 + g[5] * z0;
+    const double a3 = g[6] * x0 + g[7] * y0 + g[8] * z0;
     const float s1 = (a1 < 0) ? 1.0f : -1.0f, s2 = (a2 < 0) ? 1.0f : -1.0f, s3 = (a3 < 0) ? 1.0f : -1.0f;
     const double d1x = g[0] * s1, d1y = g[1] * s1, d1z = g[2] * s1;
     const double d2x = g[3] * s2, d2y = g[4] * s2, d2z = g[5] * s2;
@@ -289,6 +273,18 @@ __device__ __forceinline__ uint32_t wave_inclusive_scan(uint32_t v, uint32_t &to
     x += __builtin_amdgcn_update_dpp(0, x, 0x143, 0xc, 0xf, false);  // row_bcast:31 into rows 2 and 3
     total = static_cast<uint32_t>(__builtin_amdgcn_readlane(x, 63));
     return static_cast<uint32_t>(x);
+}
+
+// Wave64 maximum of v, in lane 63 (the same steps; 0 where a lane has no source).
+__device__ __forceinline__ uint32_t wave_max(uint32_t v) {
+    auto step = [&](int x) { v = static_cast<uint32_t>(x) > v ? static_cast<uint32_t>(x) : v; };
+    step(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), 0x111, 0xf, 0xf, false));
+    step(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), 0x112, 0xf, 0xf, false));
+    step(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), 0x114, 0xf, 0xf, false));
+    step(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), 0x118, 0xf, 0xf, false));
+    step(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), 0x142, 0xa, 0xf, false));
+    step(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), 0x143, 0xc, 0xf, false));
+    return v;
 }
 
 __device__ __forceinline__ unsigned long long block_sum(unsigned long long v, unsigned long long *sh) {
@@ -371,15 +367,23 @@ __device__ __forceinline__ bool is_unclaimed_liquid(unsigned long long lm) {
 // (pass 1 visits the window only and accumulates only while LayerID <= layer, and the undercooling
 // is never reset between layers; src/CAupdate.cpp:217-237, src/runCA.cpp:283-418). 0 while the cell
 // waits for its liquidus time or its layer.
-__device__ __forceinline__ int growth_index(const DomainView &d, int cts, int lid, uint32_t q, int cycle) {
-    const StepCtl *c = d.ctl;
+// The layer and its cycle jumps, read once.
+struct LayerAt {
+    int layer, j0, j1;
+};
+__device__ __forceinline__ LayerAt layer_at(const StepCtl *c) {
     const int L = c->layer;
-    if (lid > L) return 0;
-    int k = executed_in(cts, cycle, c, c->layer_jump0[L], c->njumps);
+    return LayerAt{L, c->layer_jump0[L], c->njumps};
+}
+__device__ __forceinline__ int growth_index(const DomainView &d, const LayerAt &at, int cts, int lid, uint32_t q, int cycle) {
+    const StepCtl *c = d.ctl;
+    if (lid > at.layer) return 0;
+    int k = executed_in(cts, cycle, c, at.j0, at.j1);
     k = k < 0 ? 0 : k;
-    if (L > 0) {
-        const int z = static_cast<int>(q / (static_cast<uint32_t>(d.X) * static_cast<uint32_t>(d.Y)));
-        for (int l = lid < 0 ? 0 : lid; l < L; l++) {
+    const int first = lid < 0 ? 0 : lid;
+    if (first < at.layer) {
+        const int z = static_cast<int>(d.by_xy.div(q));
+        for (int l = first; l < at.layer; l++) {
             if (z < c->layer_zlo[l] || z > c->layer_zhi[l]) continue;
             const int e = executed_in(cts, c->layer_end[l], c, c->layer_jump0[l], c->layer_jump0[l + 1]);
             k += e < 0 ? 0 : e;
@@ -387,55 +391,55 @@ __device__ __forceinline__ int growth_index(const DomainView &d, int cts, int li
     }
     return k;
 }
-// The growth increments: grow[k] below the plateau index ksat, the plateau value from there on.
-// tab is the table or a copy of its first ksat entries in LDS (the capture pass stages one, as its
-// replays walk the table one dependent step at a time).
+// The growth table as growth.hpp takes it: increments (a step across a binade's boundary reads one)
+// and the sums of their deltas, whose first rows a kernel that looks at many cells holds in LDS.
+// The chain of a cell's lane is a few reads whatever the number of steps; rounding them one
+// after another, up to 63 to catch up and 63 to find the next step due, was the longest part
+// of a step of a small domain (50^3 of the finest time step: 23 -> 16 us a step).
 struct Growth {
     const double *tab;
-    int ksat;
+    const uint32_t *sums;
+    const __attribute__((address_space(3))) uint32_t *staged;  // in LDS (a generic pointer would be read through flat loads)
+    int ksat, nstaged;  // rows staged
     double gsat;
+    uint32_t usable;
     __device__ __forceinline__ double inc(int k) const { return k < ksat ? tab[k] : gsat; }
-};
-__device__ __forceinline__ Growth growth_of(const DomainView &d) { return Growth{d.grow, d.ksat, d.grow[d.ngrow - 1]}; }
-// The same with the table's first ksat entries copied to the workgroup's LDS buffer when they fit
-// (the replays walk the table one dependent step at a time). Every thread of the workgroup calls it.
-constexpr int kGrowStage = 4096;  // table entries staged in LDS (32 KB)
-template <int BLOCK>
-__device__ __forceinline__ Growth staged_growth(const DomainView &d, double *lds) {
-    Growth g = growth_of(d);
-    if (d.ksat <= kGrowStage) {
-        for (int k = threadIdx.x; k < d.ksat; k += BLOCK) lds[k] = d.grow[k];
-        g.tab = lds;
+    template <typename F>
+    __device__ __forceinline__ void with_row(int r, F &&f) const {
+        const int at = r * (ksat + 2);
+        if (r < nstaged) f(sum_row_at(staged + at, ksat));
+        else f(sum_row_at(sums + at, ksat));
     }
+};
+__device__ __forceinline__ Growth growth_of(const DomainView &d) {
+    return Growth{d.grow, d.grow_sums, nullptr, d.ksat, 0, d.grow[d.ngrow - 1], d.sums_usable};
+}
+// The same with as many rows of the sums as fit copied to the workgroup's LDS buffer of N entries.
+// Every thread of the workgroup calls it.
+template <int BLOCK, int N>
+__device__ __forceinline__ Growth staged_growth(const DomainView &d, uint32_t (&lds)[N]) {
+    Growth g = growth_of(d);
+    const int len = d.ksat + 2;
+    g.staged = (const __attribute__((address_space(3))) uint32_t *)lds;
+    g.nstaged = N / len < kSumRows ? N / len : kSumRows;
+    for (int i = threadIdx.x; i < g.nstaged * len; i += BLOCK) lds[i] = d.grow_sums[i];
     __syncthreads();
     return g;
 }
 
 // dl after the growth of the steps with index k0+1 .. k1, one float rounding per step exactly as
 // the reference stores it.
-__device__ float replay_growth(const Growth &g, float dl, int k0, int k1) {
-    int k = k0;
-    for (; k < k1 && k + 1 < g.ksat; k++) dl = grow_step(dl, g.inc(k + 1));
-    if (k < k1) dl = advance_const(dl, k1 - k, g.gsat);
-    return dl;
+__device__ __forceinline__ float replay_growth(const Growth &g, float dl, int k0, int k1) {
+    return advance_steps(g, dl, k0, k1);
 }
 // Steps ahead (1 .. kAlarmSlots - 1) at which dl, now at growth index k, first reaches thr; the
 // horizon when it does not get there before.
-__device__ uint32_t steps_until(const Growth &g, float dl, int k, float thr) {
-    const int horizon = static_cast<int>(kAlarmSlots) - 1;
-    int n = 0;
-    while (n < horizon && k + n + 1 < g.ksat) {
-        n++;
-        dl = grow_step(dl, g.inc(k + n));
-        if (dl >= thr) return static_cast<uint32_t>(n);
-    }
-    if (n == horizon) return static_cast<uint32_t>(horizon);
-    return static_cast<uint32_t>(n + reach_const(dl, g.gsat, thr, horizon - n));
+__device__ __forceinline__ uint32_t steps_until(const Growth &g, float dl, int k, float thr) {
+    return static_cast<uint32_t>(reach_steps(g, dl, k, thr, static_cast<int>(kAlarmSlots) - 1));
 }
 
 // ---- The calendar: cell q is processed at the step of serial s when bit q of slot s mod
 // kAlarmSlots is set. ----
-__device__ __forceinline__ size_t bitmap_words(const DomainView &d) { return static_cast<size_t>((d.ncell + 31) / 32); }
 __device__ __forceinline__ void set_alarm(const DomainView &d, uint32_t serial, uint32_t q) {
     atomicOr(&d.alarms[(serial % kAlarmSlots) * alarm_stride(d.ncell) + (q >> 5)], 1u << (q & 31));
 }
@@ -446,38 +450,33 @@ __device__ __forceinline__ void set_alarm(const DomainView &d, uint32_t serial, 
 // once. ----
 
 // Events of a step counted per workgroup in LDS. A wave adds its lanes' events at once.
-enum StepCount : int { kCntEnt, kCntSol, kCntLate, kCntCap, kCntAct, kCntNn, kCntEval, kCntMask, kStepCounts };
 __device__ __forceinline__ void count_event(bool happened, uint32_t *counter) {
     const unsigned long long m = __ballot(happened);
     if (m && (threadIdx.x & 63) == static_cast<uint32_t>(__ffsll(static_cast<long long>(m)) - 1))
         atomicAdd(counter, static_cast<uint32_t>(__popcll(m)));
 }
-// A step's contribution to counter row r: the counts and, for what changes the number of active
-// cells, the sums of the steps' serials, from which book_totals forms the per-step sums. A late
-// solidification belongs to the step before.
-__device__ __forceinline__ unsigned long long part_value(uint32_t r, const uint32_t *cnt, uint32_t serial) {
-    const unsigned long long s = serial;
-    switch (r) {
-    case kPartEnt: return cnt[kCntEnt];
-    case kPartEntAt: return cnt[kCntEnt] * s;
-    case kPartSol: return static_cast<unsigned long long>(cnt[kCntSol]) + cnt[kCntLate];
-    case kPartSolAt: return cnt[kCntSol] * s + (cnt[kCntLate] ? cnt[kCntLate] * (s - 1) : 0);
-    case kPartCap: return cnt[kCntCap];
-    case kPartCapAt: return cnt[kCntCap] * s;
-    case kPartAct: return cnt[kCntAct];
-    case kPartActAt: return cnt[kCntAct] * s;
-    case kPartNn: return cnt[kCntNn];
-    case kPartEval: return cnt[kCntEval];
-    case kPartMask: return cnt[kCntMask];
-    default: return 0;
+// A workgroup's events over some steps, thread e holding those of kind e: their number and the sum of
+// the serials of their steps, from which book_totals forms the per-step sums.
+struct Tally {
+    unsigned long long n = 0, at = 0;
+    __device__ __forceinline__ void add(const uint32_t *cnt, uint32_t serial) {
+        if (threadIdx.x >= kStepCounts) return;
+        const uint32_t c = cnt[threadIdx.x];
+        n += c;
+        at += static_cast<unsigned long long>(c) * serial;
     }
-}
-// The step's events added to workgroup b's running totals.
+    // to workgroup b's running totals
+    __device__ __forceinline__ void put(const DomainView &d, uint32_t b) {
+        if (threadIdx.x >= kStepCounts || !n) return;
+        d.part[static_cast<size_t>(2 * threadIdx.x) * d.nparts + b] += n;
+        d.part[static_cast<size_t>(2 * threadIdx.x + 1) * d.nparts + b] += at;
+        n = at = 0;
+    }
+};
 __device__ __forceinline__ void add_parts(const DomainView &d, uint32_t b, const uint32_t *cnt, uint32_t serial) {
-    const uint32_t r = threadIdx.x;
-    if (r >= kPartRows) return;
-    const unsigned long long v = part_value(r, cnt, serial);
-    if (v) d.part[static_cast<size_t>(r) * d.nparts + b] += v;
+    Tally t;
+    t.add(cnt, serial);
+    t.put(d, b);
 }
 
 // Growth index that an active cell's dl includes, at a step of growth index k. A cell not yet
@@ -561,7 +560,7 @@ __device__ __forceinline__ int nucleate_body(const DomainView &d, int cycle, uin
                     const CellWords w = load_cell(d.cells + r);
                     if ((w.ct & kTypeMask) != kActive || !(cycle > w.cts && w.lid <= layer)) continue;
                     if (!(w.flags & kCounted)) nent++;
-                    solidify(d, growth_of(d), r, w, growth_index(d, w.cts, w.lid, r, cycle));
+                    solidify(d, growth_of(d), r, w, growth_index(d, layer_at(d.ctl), w.cts, w.lid, r, cycle));
                     d.cells[r].flags = (w.flags & ~kFresh) | kCounted;
                     nsol++;
                 }
@@ -627,7 +626,9 @@ __device__ uint32_t evaluate_claims(const DomainView &d, const Grid &gr, uint32_
         next2 = fminf(next2, fmaxf(next, v));
         at = v < next ? l : at;
         next = fminf(next, v);
-        if (l % 4 == 3) __builtin_amdgcn_sched_barrier(0);  // the masked lengths of four neighbours at a time
+        // four neighbours at a time: their masked lengths and conditions all at once would take 20
+        // registers more, and a workgroup a CU less
+        if (l % 4 == 3) asm volatile("" : "+v"(liquid), "+v"(dlj), "+v"(beyond), "+v"(next), "+v"(next2), "+v"(at));
     }
     const uint32_t claimed = ~beyond & liquid;
     for (uint32_t m = claimed; m; m &= m - 1) atomicMin(claim_word(d, j + gr.offset(__builtin_ctz(m))), j);
@@ -636,28 +637,23 @@ __device__ uint32_t evaluate_claims(const DomainView &d, const Grid &gr, uint32_
     return claimed;
 }
 
-// ---- Units of the calendar: kUnitWords words (one wave-wide load) of a slot. The workgroups of a
+// ---- The workgroups of a
 // domain share the units of the range of active cells in turn, so that the front, wherever it lies,
 // is spread over all of them. ----
-constexpr uint32_t kUnitWords = 64;
-constexpr uint32_t kUnitCells = 32 * kUnitWords;
 constexpr uint32_t kUnitsPerLane = 8;  // units whose words a wave holds at once
 
 struct UnitRange {
     uint32_t u0, n;  // first unit, number of units
 };
-__device__ __forceinline__ uint32_t domain_units(const DomainView &d) {
-    return static_cast<uint32_t>((bitmap_words(d) + kUnitWords - 1) / kUnitWords);
-}
 // The units that may hold a due cell: all of a domain small enough for one round of its workgroups,
 // else those of the range of active cells.
 template <int BLOCK>
 __device__ __forceinline__ bool scans_all(const DomainView &d, uint32_t nb) {
-    return domain_units(d) <= nb * (BLOCK / 64) * kUnitsPerLane;
+    return d.units <= nb * (BLOCK / 64) * kUnitsPerLane;
 }
 template <int BLOCK>
 __device__ __forceinline__ UnitRange unit_range(const DomainView &d, uint32_t nb) {
-    if (scans_all<BLOCK>(d, nb)) return UnitRange{0, domain_units(d)};
+    if (scans_all<BLOCK>(d, nb)) return UnitRange{0, d.units};
     const uint32_t lo = d.ctl->elo;
     uint32_t hi = d.ctl->ehi;
     if (lo > hi) return UnitRange{0, 0};
@@ -676,7 +672,7 @@ __device__ __forceinline__ uint32_t *calendar_slot(const DomainView &d, uint32_t
 // Entries of a workgroup's region of the claim lists: the cells of the most units it can hold. The
 // regions lie in the order of the workgroups' units, so that those of workgroups without any come last.
 __device__ __forceinline__ uint32_t claim_region(const DomainView &d, uint32_t nb) {
-    return (domain_units(d) + nb - 1) / nb * kUnitCells;
+    return (d.units + nb - 1) / nb * kUnitCells;
 }
 
 // Calls visit(has, j, record) for every cell due at the step of that serial in workgroup b's units,
@@ -691,22 +687,25 @@ __device__ __forceinline__ void for_due(const DomainView &d, uint32_t serial, ui
     const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const UnitRange r = unit_range<BLOCK>(d, nb);
     uint32_t *bits = calendar_slot(d, serial);
-    const uint32_t most = (r.n + nb - 1) / nb;  // units of the workgroup that has the most
     // this lane's word of its wave's first unit, and the end of the range's words
     const uint32_t first = (r.u0 + wave * nb + place_of(b, nb)) * kUnitWords + lane;
-    const uint32_t nwords = static_cast<uint32_t>(bitmap_words(d));
-    const uint32_t end = (r.u0 + r.n) * kUnitWords < nwords ? (r.u0 + r.n) * kUnitWords : nwords;
+    const uint32_t end = (r.u0 + r.n) * kUnitWords < d.nwords ? (r.u0 + r.n) * kUnitWords : d.nwords;
     uint32_t fill = 0, done = 0;                // entries in the list; cells of the round already listed
-    for (uint32_t k0 = 0; k0 < most;) {
+    for (uint32_t k0 = 0; k0 * nb < r.n;) {
         uint32_t w[kUnitsPerLane], cnt = 0;
         auto word = [&](uint32_t e) { return first + (k0 + e * kWaves) * nb * kUnitWords; };
         // all loads in flight together (no test around each: a word past the end reads the last one)
+        const uint32_t turns = (r.n - k0 * nb + kWaves * nb - 1) / (kWaves * nb);  // that have a unit at all
 #pragma unroll
-        for (uint32_t e = 0; e < kUnitsPerLane; e++) w[e] = bits[word(e) < end ? word(e) : end - 1];
+        for (uint32_t e = 0; e < kUnitsPerLane; e++) {
+            w[e] = 0;
+            if (e < turns) w[e] = bits[word(e) < end ? word(e) : end - 1];
+        }
 #pragma unroll
-        for (uint32_t e = 0; e < kUnitsPerLane; e++) w[e] = word(e) < end ? w[e] : 0u;
-#pragma unroll
-        for (uint32_t e = 0; e < kUnitsPerLane; e++) cnt += __builtin_popcount(w[e]);
+        for (uint32_t e = 0; e < kUnitsPerLane; e++) {
+            w[e] = word(e) < end ? w[e] : 0u;
+            cnt += __builtin_popcount(w[e]);
+        }
         uint32_t wtot;
         const uint32_t incl = wave_inclusive_scan(cnt, wtot);
         if (lane == 0) tot[wave] = wtot;
@@ -723,7 +722,7 @@ __device__ __forceinline__ void for_due(const DomainView &d, uint32_t serial, ui
         uint32_t pos = before + incl - cnt - done;  // place among the cells to list now; wraps if listed before
 #pragma unroll
         for (uint32_t e = 0; e < kUnitsPerLane; e++) {
-            if (!w[e]) continue;
+            if (e >= turns || !w[e]) continue;
             if (CLEAR && last) bits[word(e)] = 0u;
             for (uint32_t m = w[e]; m; m &= m - 1, pos++)
                 if (pos < take) list[fill + pos] = word(e) * 32u + __builtin_ctz(m);
@@ -732,7 +731,7 @@ __device__ __forceinline__ void for_due(const DomainView &d, uint32_t serial, ui
         done = last ? 0 : done + take;
         if (last) k0 += kWaves * kUnitsPerLane;
         __syncthreads();  // the list is written, tot is read
-        if (fill < CAP && k0 < most) continue;
+        if (fill < CAP && k0 * nb < r.n) continue;
         // software pipeline: the next turn's record is loaded while this one's is processed
         uint32_t jn = 0;
         CellWords wn{};
@@ -767,6 +766,25 @@ __device__ __forceinline__ bool solid_since_last(const CellWords &w, uint32_t se
            cycle - 1 > w.cts && w.lid <= layer;
 }
 
+// The liquid ones among the 26 neighbours of active cell j, from their types: a plane of nine at a time
+// (only a nucleus or a seed asks, once, and 26 reads in flight would cost the claim pass registers).
+__device__ __forceinline__ uint32_t liquid_neighbours(const DomainView &d, const Grid &gr, uint32_t j) {
+    uint32_t raw = 0;  // bit 9 (dz + 1) + 3 (dx + 1) + dy + 1
+#pragma unroll 1
+    for (int z = 0; z < 3; z++) {
+        const Cell *row = d.cells + static_cast<uint32_t>(j + (z - 1) * static_cast<int>(gr.xy.d));
+        uint32_t nine = 0;
+#pragma unroll
+        for (int i = 0; i < 9; i++)
+            nine |= static_cast<uint32_t>(row[(i / 3 - 1) * gr.Y + i % 3 - 1].ct == kLiquid) << i;
+        raw |= nine << (9 * z);
+    }
+    uint32_t liquid = 0;
+#pragma unroll
+    for (int l = 0; l < 26; l++) liquid |= ((raw >> (9 * (kNbZ[l] + 1) + 3 * (kNbX[l] + 1) + kNbY[l] + 1)) & 1u) << l;
+    return liquid;
+}
+
 // Pass A over the cells due this step (the step's calendar slot), one per lane: the liquidus-time
 // gate, the growth since the cell was last looked at, and the claims.
 // The liquid neighbours come from the cell's mask (lm), kept current by the cells that leave the
@@ -784,16 +802,16 @@ __device__ __forceinline__ bool solid_since_last(const CellWords &w, uint32_t se
 // Cells with claims are numbered by an LDS counter (no global atomics) and handed to put(number, cell,
 // claimed neighbours).
 template <int BLOCK, uint32_t CAP, typename F>
-__device__ __forceinline__ void claim_body(const DomainView &d, const Growth &g, int cycle, uint32_t serial, int layer,
-                                           bool follows, uint32_t b, uint32_t nb, uint32_t *list, uint32_t *tot,
-                                           uint32_t *cnt, uint32_t *nclaim, F &&put) {
-    const Grid gr = grid_of(d);
+__device__ __forceinline__ void claim_body(const DomainView &d, const Grid &gr, const Growth &g, const LayerAt &at,
+                                           int cycle, uint32_t serial, bool follows, uint32_t b, uint32_t nb,
+                                           uint32_t *list, uint32_t *tot, uint32_t *cnt, uint32_t *nclaim, F &&put) {
+    const int layer = at.layer;
     for_due<BLOCK, CAP, true>(d, serial, b, nb, list, tot, [&](bool has, uint32_t j, const CellWords &w) {
         uint32_t claimed = 0;
         bool entered = false, sol = false, late = false, eval = false, mask = false;
         if (has && (w.ct & kTypeMask) == kActive) {
             const bool waiting = !(cycle > w.cts && w.lid <= layer);
-            int k = growth_index(d, w.cts, w.lid, j, cycle);
+            int k = growth_index(d, at, w.cts, w.lid, j, cycle);
             uint32_t liquid;
             const int kdl = growth_base(w, k, waiting);
             // the record's new words, written back as one sector at the end
@@ -805,11 +823,7 @@ __device__ __forceinline__ void claim_body(const DomainView &d, const Growth &g,
             if (w.lm & kLmUnknown) {
                 const Coord c = decode(j, gr);
                 uint32_t valid = valid_neighbours(c, gr.X, gr.Y, gr.nzA);
-                const Rows rows = rows_of(d, gr, j, valid);
-                liquid = 0;
-#pragma unroll
-                for (int l = 0; l < 26; l++) liquid |= static_cast<uint32_t>(rows.cell(l).ct == kLiquid) << l;
-                liquid &= valid;
+                liquid = liquid_neighbours(d, gr, inner_cell(d, gr, j, valid)) & valid;
                 lm = liquid;
                 mask = true;
             }
@@ -838,9 +852,9 @@ __device__ __forceinline__ void claim_body(const DomainView &d, const Growth &g,
                 }
                 else {
                     if (dl >= thr) {
-                        const uint32_t at = (w.flags >> 2) & 31u;
+                        const uint32_t set_by = (w.flags >> 2) & 31u;
                         const float bound = hint_bound(thr, w.flags);
-                        if (at && !((liquid >> (at - 1)) & 1u) && dl < bound) {
+                        if (set_by && !((liquid >> (set_by - 1)) & 1u) && dl < bound) {
                             // the neighbour that set thr is gone and no other is reached
                             thr = bound;
                             flags &= ~kHintMask;
@@ -876,33 +890,31 @@ __device__ __forceinline__ void claim_body(const DomainView &d, const Growth &g,
     });
 }
 
-// The captures of a round: claimants' claims that hold the claimant's own index are won (the lowest
-// index that reached the cell). LDS of pass B.
+// A capture's new octahedron, built by one lane and read by the 32 that give the captured cell its
+// place among its neighbours.
+struct Capture {
+    double cx, cy, cz;
+    float gv[9];  // the grain's unit vectors
+    float dl;
+    uint32_t from, q;  // the winner and the captured cell
+    int32_t gid;
+};
+// LDS of pass B.
 template <int BLOCK>
 struct ApplyLds {
     uint32_t cell[2 * BLOCK], bits[2 * BLOCK];  // winners and the claims they won
     int32_t gid[2 * BLOCK];
     uint32_t item[BLOCK];  // winner << 5 | neighbour of each capture of a turn
+    Capture made[BLOCK];
     uint32_t tot[BLOCK / 64];
     uint32_t nwin;
 };
 
-// One capture (src/CAupdate.cpp:353-563, 717): the winner jc's octahedron gives that of its
-// neighbour l, the captured cell q, which is due at the next step and leaves the liquid masks of
-// its neighbours. Only masks that still hold it are updated: the masks are read first, and a cell's
-// bit is cleared by its capture alone, so the read decides exactly. A neighbour whose mask this
-// empties is due at the next step, which decides whether it turned solid in this one
-// (solid_since_last).
-__device__ __forceinline__ uint32_t capture(const DomainView &d, const Grid &gr, uint32_t serial, uint32_t jc, int l,
-                                            int h) {
-    const uint32_t q = jc + gr.offset(l);
+// The octahedron of the winner jc's capture of its neighbour l (src/CAupdate.cpp:353-515).
+__device__ __forceinline__ void build_capture(const DomainView &d, const Grid &gr, uint32_t jc, int l, int h, Capture &m) {
     const Octa &e = d.octa[jc];
-    // the winner's centre (float, as the capture uses it) and orientation, loaded with the
-    // neighbours' words below
+    // the winner's centre, float as the capture uses it
     const float wcx = static_cast<float>(e.x), wcy = static_cast<float>(e.y), wcz = static_cast<float>(e.z);
-    const Coord c = decode(jc, gr);
-    const Coord cqc{c.x + nb_dx(l), c.y + nb_dy(l), c.z + nb_dz(l)};
-    uint32_t valid = valid_neighbours(cqc, gr.X, gr.Y, gr.nzA);
     int o = orientation_of(h);
     if (o < 0) {
         atomicOr(&d.ctl->error, 2);
@@ -910,103 +922,131 @@ __device__ __forceinline__ uint32_t capture(const DomainView &d, const Grid &gr,
     }
     float gv[9];
 #pragma unroll
-    for (int m = 0; m < 9; m++) gv[m] = d.guv[9 * o + m];
-    const uint4 own = reinterpret_cast<const uint4 *>(d.cells + q)[1];  // cts, gid, win, lid | ct | flags
-    // the neighbours' words: the low word is the mask (or liquid marker), the high word
-    // of a liquid neighbour its claim word
-    const Rows rows = rows_of(d, gr, q, valid);
-    unsigned long long lw[26];
-#pragma unroll
-    for (int kk = 0; kk < 26; kk++)
-        lw[kk] = rows.cell(kk).lm;
-    // The new cell's mask: its liquid neighbours at its first visit are those liquid now
-    // and not claimed in this step (every claimed cell is captured in this step, and the
-    // claims are final). Until its store below, the new cell's own words read as a
-    // claimed liquid cell, which no other capture counts.
-    uint32_t liquid = 0, mw[26];
-#pragma unroll
-    for (int kk = 0; kk < 26; kk++) {
-        liquid |= static_cast<uint32_t>(is_unclaimed_liquid(lw[kk])) << kk;
-        mw[kk] = static_cast<uint32_t>(lw[kk]);
-    }
-    uint32_t need = 0;
-#pragma unroll
-    for (int kk = 0; kk < 26; kk++) {
-        const uint32_t bit = 1u << kOpposite.v[kk];
-        need |= static_cast<uint32_t>((mw[kk] & (kMaskUnknown | bit)) == bit) << kk;
-    }
-    liquid &= valid;
-    need &= valid;
+    for (int i = 0; i < 9; i++) gv[i] = d.guv[9 * o + i];
+    const Coord c = decode(jc, gr);
     const double xp = (c.x + d.xoff + nb_dx(l)) + 0.5;
     const double yp = (c.y + d.yoff + nb_dy(l)) + 0.5;
     const double zp = (c.z + nb_dz(l)) + 0.5;
+#pragma unroll
+    for (int i = 0; i < 9; i++) m.gv[i] = gv[i];
+    m.from = jc;
+    m.q = jc + gr.offset(l);
+    m.gid = h;
+    __builtin_amdgcn_sched_barrier(0);  // stored before the octahedron is built: fewer registers live
     const Octahedron oc = new_octahedron(gv, wcx, wcy, wcz, xp, yp, zp);
-    // updates only where the mask still holds q, all in flight together; their results are used
-    // after the critical lengths are computed, which hides their round trip (before the octahedron
-    // is built, the 26 results would take more registers than there are)
-    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int kk = 0; kk < 26; kk++)
-        if ((need >> kk) & 1u) mw[kk] = atomicAnd(rows.low(kk), ~(1u << kOpposite.v[kk]));
-    // a neighbour at or below the claimant's index still had q liquid at its visit
-    // in the reference's index order: its keep word gets this step's tag (every writer
-    // of a step writes the same value)
-#pragma unroll
-    for (int kk = 0; kk < 26; kk++)
-        if (((need >> kk) & 1u) && q + gr.row[(kNbZ[kk] + 1) * 3 + kNbX[kk] + 1] + kNbY[kk] <= jc)
-            *rows.high(kk) = serial + 1;
-    // The new cell's record, whole: nothing else writes it in this pass.
-    uint4 *r4 = reinterpret_cast<uint4 *>(d.cells + q);
-    r4[0] = make_uint4(liquid, 0u, __float_as_uint(static_cast<float>(oc.dl)), __float_as_uint(0.0f));
-    r4[1] = make_uint4(own.x, static_cast<uint32_t>(h), own.z,
-                       (own.w & 0xFFu) | (static_cast<uint32_t>(kActive) << 8) | (static_cast<uint32_t>(kFresh) << 16));
-    set_alarm(d, serial + 1, q);
-    // The new octahedron's record: its 26 critical lengths, computed once here (its
-    // evaluations read them back), and its centre; whole 16-byte pieces of one line.
-    {
-        const Faces f = faces_of(gv);
-        float4 *o4 = reinterpret_cast<float4 *>(&d.octa[q]);
-#pragma unroll
-        for (int i = 0; i < 6; i++)
-            o4[i] = make_float4(critical_length(f, xp, yp, zp, oc.cx, oc.cy, oc.cz, 4 * i),
-                                critical_length(f, xp, yp, zp, oc.cx, oc.cy, oc.cz, 4 * i + 1),
-                                critical_length(f, xp, yp, zp, oc.cx, oc.cy, oc.cz, 4 * i + 2),
-                                critical_length(f, xp, yp, zp, oc.cx, oc.cy, oc.cz, 4 * i + 3));
-        const uint2 xb = __builtin_bit_cast(uint2, oc.cx), yb = __builtin_bit_cast(uint2, oc.cy),
-                    zb = __builtin_bit_cast(uint2, oc.cz);
-        uint4 *u4 = reinterpret_cast<uint4 *>(&d.octa[q]);
-        u4[6] = make_uint4(__float_as_uint(critical_length(f, xp, yp, zp, oc.cx, oc.cy, oc.cz, 24)),
-                           __float_as_uint(critical_length(f, xp, yp, zp, oc.cx, oc.cy, oc.cz, 25)), xb.x, xb.y);
-        u4[7] = make_uint4(yb.x, yb.y, zb.x, zb.y);
-    }
-    uint32_t emptied = 0;
-#pragma unroll
-    for (int kk = 0; kk < 26; kk++) {
-        const uint32_t bit = 1u << kOpposite.v[kk];
-        emptied |= static_cast<uint32_t>(((need >> kk) & 1u) && (mw[kk] & (kMaskUnknown | kMaskNow)) == bit) << kk;
-    }
-    for (uint32_t m = emptied; m; m &= m - 1) set_alarm(d, serial + 1, q + gr.offset(__builtin_ctz(m)));
-    return q;
+    m.cx = oc.cx;
+    m.cy = oc.cy;
+    m.cz = oc.cz;
+    m.dl = static_cast<float>(oc.dl);
 }
 
-// Pass B over the n claimants that claimant(k, cell, bits) gives: the winners of up to two rounds
-// are gathered in LDS with the claims they won, their captures numbered by a block scan and built
-// one per lane (a winner mostly has one; one lane per capture keeps every lane's chain of dependent
-// accesses to one capture).
+// A lane's neighbour number within its half-wave (26 .. 31: none), its offsets, and the number that the
+// cell has as the neighbour's neighbour.
+struct NeighbourLane {
+    int l, dx, dy, dz, off, back;
+};
+__device__ __forceinline__ NeighbourLane neighbour_lane(const Grid &gr) {
+    NeighbourLane n;
+    n.l = static_cast<int>(threadIdx.x & 31u);
+    const int l = n.l < 26 ? n.l : 0;
+    n.dx = nb_dx(l);
+    n.dy = nb_dy(l);
+    n.dz = nb_dz(l);
+    n.off = gr.offset(l);
+    n.back = 0;
+#pragma unroll
+    for (int i = 0; i < 26; i++) n.back = l == i ? kOpposite.v[i] : n.back;
+    return n;
+}
+
+// The captured cell's place (src/CAupdate.cpp:553-563, 717), by a half-wave, one lane per neighbour: the
+// cell is active, due at the next step and leaves the liquid masks of its neighbours, and its 26
+// critical lengths and its centre are written as one line. Only masks that still hold the cell are
+// updated: a mask is read first, and a cell's bit is cleared by its capture alone, so the read decides
+// exactly. A neighbour whose mask this empties is due at the next step, which decides whether it turned
+// solid in this one (solid_since_last). word was read beforehand: the neighbour's lm, and in lanes 26 and
+// 27 the last two words of the cell's own record.
+__device__ __forceinline__ bool has_neighbour(const DomainView &d, const NeighbourLane &n, const Coord &c) {
+    const int x = c.x + n.dx, y = c.y + n.dy, z = c.z + n.dz;
+    return n.l < 26 && x >= 0 && x < d.X && y >= 0 && y < d.Y && z >= 0 && z < d.nzA;
+}
+__device__ __forceinline__ void place_capture(const DomainView &d, const NeighbourLane &n, uint32_t serial,
+                                              const Capture &m, const Coord &c, bool valid, unsigned long long word) {
+    const uint32_t q = m.q, nb = q + n.off, low = static_cast<uint32_t>(word), bit = 1u << n.back;
+    // The new cell's mask: its liquid neighbours at its first visit are those liquid now and not claimed
+    // in this step (every claimed cell is captured in this step, and the claims are final). Until it is
+    // stored, the new cell's own words read as a claimed liquid cell, which no other capture counts.
+    const unsigned long long ballot = __ballot(valid && is_unclaimed_liquid(word));
+    const uint32_t liquid = static_cast<uint32_t>(threadIdx.x & 32u ? ballot >> 32 : ballot);
+    const bool need = valid && (low & (kMaskUnknown | bit)) == bit;
+    uint32_t old = 0;
+    uint32_t *words = reinterpret_cast<uint32_t *>(&d.cells[nb].lm);
+    if (need) {
+        old = atomicAnd(words, ~bit);
+        // a neighbour at or below the claimant's index still had q liquid at its visit in the reference's
+        // index order: its keep word gets this step's tag (every writer of a step writes the same value)
+        if (nb <= m.from) words[1] = serial + 1;
+    }
+    const double xp = (c.x + d.xoff) + 0.5, yp = (c.y + d.yoff) + 0.5, zp = c.z + 0.5;
+    const float len = critical_length(faces_of(m.gv), xp, yp, zp, m.cx, m.cy, m.cz, n.dx, n.dy, n.dz);
+    const uint32_t i = n.l < 26 ? 0u : static_cast<uint32_t>(n.l - 26);
+    const double centre = i < 2 ? m.cx : (i < 4 ? m.cy : m.cz);
+    const unsigned long long cb = __builtin_bit_cast(unsigned long long, centre);
+    const uint32_t half = static_cast<uint32_t>(i & 1u ? cb >> 32 : cb);
+    reinterpret_cast<uint32_t *>(&d.octa[q])[n.l] = n.l < 26 ? __float_as_uint(len) : half;
+    // The new cell's record, whole: nothing else writes it in this pass.
+    if (n.l >= 26 && n.l < 30) {
+        unsigned long long w = liquid;  // lm (lane 28)
+        if (n.l == 26) w = (word & 0xFFFFFFFFull) | static_cast<unsigned long long>(static_cast<uint32_t>(m.gid)) << 32;  // cts, gid
+        if (n.l == 27) w = (word & 0xFFFFFFFFFFull) | static_cast<unsigned long long>(kActive) << 40 | static_cast<unsigned long long>(kFresh) << 48;  // win, lid, ct, flags
+        if (n.l == 29) w = __float_as_uint(m.dl);  // dl, thr
+        reinterpret_cast<unsigned long long *>(d.cells + q)[n.l < 28 ? n.l - 24 : n.l - 28] = w;
+    }
+    if (n.l == 30) set_alarm(d, serial + 1, q);
+    if (need && (old & (kMaskUnknown | kMaskNow)) == bit) set_alarm(d, serial + 1, nb);
+}
+
+// The range of active cells widened by a workgroup's new ones: those of nucleation in lohi (LDS) and
+// the captures' least and greatest index per thread. Every thread calls it. The range rarely grows: most
+// workgroups need no atomic.
+struct NewCells {
+    uint32_t lo = 0xFFFFFFFFu, hi = 0;
+};
+__device__ __forceinline__ void widen_range(const DomainView &d, uint32_t *lohi, const NewCells &n = NewCells{}) {
+    const uint32_t lo = ~wave_max(~n.lo), hi = wave_max(n.hi);  // in lane 63
+    if ((threadIdx.x & 63) == 63 && lo <= hi) {
+        atomicMin(&lohi[0], lo);
+        atomicMax(&lohi[1], hi);
+    }
+    __syncthreads();
+    if (threadIdx.x == 0 && lohi[0] <= lohi[1]) {
+        if (lohi[0] < d.ctl->elo) atomicMin(&d.ctl->elo, lohi[0]);
+        if (lohi[1] > d.ctl->ehi) atomicMax(&d.ctl->ehi, lohi[1]);
+    }
+}
+
+// Pass B over the claimants that claimant(k, cell, bits) gives. A claim whose word holds the claimant's
+// own index is won (the lowest index that reached the cell). The winners of up to two rounds are
+// gathered in LDS with the claims they won and their captures numbered by a block scan (a winner mostly
+// has one). A capture's octahedron is built by one lane; its neighbours are then visited by the 26
+// lanes of a half-wave, so that the words of three consecutive neighbours are read together, its
+// lengths are one store of one line, and its chain is one length and one mask long instead of 26.
+// One lane per capture took 242 registers (two waves a SIMD) and about 10 000 cycles for one
+// capture, this 123 registers and half the cycles (24^3 9.3 -> 7.4 us a step); at 800^3, 63 000 captures a
+// step, the pass takes 72 us against 83 us.
 template <int BLOCK, typename F>
-__device__ __forceinline__ void apply_body(const DomainView &d, uint32_t serial, uint32_t n, F &&claimant,
-                                           ApplyLds<BLOCK> &s, uint32_t *cnt, uint32_t *lohi) {
+__device__ __forceinline__ void apply_body(const DomainView &d, const Grid &gr, uint32_t serial, uint32_t nclaimants,
+                                           F &&claimant, ApplyLds<BLOCK> &s, uint32_t *cnt, NewCells &made) {
     constexpr uint32_t kWaves = BLOCK / 64;
     const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const Grid gr = grid_of(d);
-    uint32_t qlo = 0xFFFFFFFFu, qhi = 0;
+    const NeighbourLane n = neighbour_lane(gr);
     if (threadIdx.x == 0) s.nwin = 0;
     __syncthreads();
-    for (uint32_t k0 = 0; k0 < n; k0 += BLOCK) {
+    for (uint32_t k0 = 0; k0 < nclaimants; k0 += BLOCK) {
         const uint32_t k = k0 + threadIdx.x;
         uint32_t j = 0, cb = 0, won = 0;
         int32_t gid = 0;
-        if (k < n) {
+        if (k < nclaimants) {
             claimant(k, j, cb);
             gid = d.cells[j].gid;
             // a claimant mostly has one or two claims: four words in flight at a time
@@ -1031,7 +1071,7 @@ __device__ __forceinline__ void apply_body(const DomainView &d, uint32_t serial,
         __syncthreads();
         const uint32_t nwin = s.nwin;
         __syncthreads();
-        if (k0 + BLOCK < n && nwin <= BLOCK) continue;  // room for another round
+        if (k0 + BLOCK < nclaimants && nwin <= BLOCK) continue;  // room for another round
         // the captures of the winners gathered so far: thread t numbers those of winners 2t, 2t + 1
         const uint32_t w0 = 2 * threadIdx.x;
         const uint32_t b0 = w0 < nwin ? s.bits[w0] : 0u, b1 = w0 + 1 < nwin ? s.bits[w0 + 1] : 0u;
@@ -1054,32 +1094,44 @@ __device__ __forceinline__ void apply_body(const DomainView &d, uint32_t serial,
             for (uint32_t m = b1; m; m &= m - 1, pos++)
                 if (pos < BLOCK) s.item[pos] = ((w0 + 1) << 5) | static_cast<uint32_t>(__builtin_ctz(m));
             __syncthreads();
-            const bool has = t0 + threadIdx.x < total;
-            if (has) {
+            const uint32_t turn = total - t0 < BLOCK ? total - t0 : BLOCK;
+            // the neighbours' words of a half-wave's first capture are on their way while the octahedra
+            // are built, and those of its next one while it places one
+            uint32_t i = threadIdx.x >> 5;
+            Coord c{};
+            bool valid = false;
+            unsigned long long word = 0;
+            auto fetch = [&]() {
+                if (i >= turn) return;
+                const uint32_t it = s.item[i];
+                const uint32_t q = s.cell[it >> 5] + gr.offset(static_cast<int>(it & 31u));
+                c = decode(q, gr);
+                valid = has_neighbour(d, n, c);
+                const unsigned long long *at = &d.cells[n.l < 26 ? q + n.off : q].lm + (n.l < 26 ? 0 : n.l - 24);
+                if (valid || n.l == 26 || n.l == 27) word = *at;
+            };
+            fetch();
+            if (threadIdx.x < turn) {
                 const uint32_t it = s.item[threadIdx.x];
-                const uint32_t q = capture(d, gr, serial, s.cell[it >> 5], static_cast<int>(it & 31u), s.gid[it >> 5]);
-                qlo = q < qlo ? q : qlo;
-                qhi = q > qhi ? q : qhi;
+                build_capture(d, gr, s.cell[it >> 5], static_cast<int>(it & 31u), s.gid[it >> 5], s.made[threadIdx.x]);
             }
-            count_event(has, &cnt[kCntCap]);
+            if (threadIdx.x == 0) cnt[kCntCap] += turn;
+            __syncthreads();
+            while (i < turn) {
+                const Capture &m = s.made[i];
+                const Coord at = c;
+                const bool ok = valid;
+                const unsigned long long w = word;
+                made.lo = m.q < made.lo ? m.q : made.lo;
+                made.hi = m.q > made.hi ? m.q : made.hi;
+                i += BLOCK / 32;
+                fetch();
+                place_capture(d, n, serial, m, at, ok, w);
+            }
             __syncthreads();
         }
         if (threadIdx.x == 0) s.nwin = 0;
         __syncthreads();
-    }
-    if (qlo <= qhi) {
-        atomicMin(&lohi[0], qlo);
-        atomicMax(&lohi[1], qhi);
-    }
-}
-
-// The range of active cells widened by a workgroup's new ones (lohi in LDS; every thread calls it).
-// It rarely grows: most workgroups need no atomic.
-__device__ __forceinline__ void widen_range(const DomainView &d, const uint32_t *lohi) {
-    __syncthreads();
-    if (threadIdx.x == 0 && lohi[0] <= lohi[1]) {
-        if (lohi[0] < d.ctl->elo) atomicMin(&d.ctl->elo, lohi[0]);
-        if (lohi[1] > d.ctl->ehi) atomicMax(&d.ctl->ehi, lohi[1]);
     }
 }
 
@@ -1087,12 +1139,12 @@ __device__ __forceinline__ void widen_range(const DomainView &d, const uint32_t 
 // that a caller looks at the state. The cells are due at the next step, whose calendar slot stays
 // as it is. due: the cells due at the next step.
 template <int BLOCK, uint32_t CAP>
-__device__ __forceinline__ void settle_body(const DomainView &d, const Growth &g, int next_cycle, uint32_t next_serial,
-                                            int layer, uint32_t b, uint32_t nb, uint32_t *list, uint32_t *tot,
+__device__ __forceinline__ void settle_body(const DomainView &d, const Growth &g, const LayerAt &at, int next_cycle,
+                                            uint32_t next_serial, uint32_t b, uint32_t nb, uint32_t *list, uint32_t *tot,
                                             uint32_t *cnt) {
     for_due<BLOCK, CAP, false>(d, next_serial, b, nb, list, tot, [&](bool has, uint32_t j, const CellWords &w) {
-        const bool late = has && (w.ct & kTypeMask) == kActive && solid_since_last(w, next_serial, next_cycle, layer);
-        if (late) solidify(d, g, j, w, growth_index(d, w.cts, w.lid, j, next_cycle - 1));
+        const bool late = has && (w.ct & kTypeMask) == kActive && solid_since_last(w, next_serial, next_cycle, at.layer);
+        if (late) solidify(d, g, j, w, growth_index(d, at, w.cts, w.lid, j, next_cycle - 1));
         count_event(late, &cnt[kCntLate]);
     });
 }
@@ -1121,25 +1173,27 @@ __device__ __forceinline__ void book_totals(const DomainView &d, uint32_t serial
     }
     __syncthreads();
     if (threadIdx.x != 0) return;
-    const unsigned long long *v = red;
-    StepStats st = *d.stats;
     const unsigned long long S = serial_now, n = S - ctl->serial_booked;
-    const unsigned long long ent = S * v[kPartEnt] - v[kPartEntAt];          // from the same step on
-    const unsigned long long sol = (S - 1) * v[kPartSol] - v[kPartSolAt];    // from the next step on
-    const unsigned long long act = S * v[kPartAct] - v[kPartActAt];          // from the same step on
-    const unsigned long long cap = (S - 1) * v[kPartCap] - v[kPartCapAt];    // from the next step on
-    const unsigned long long frontier = n * ctl->nonwaiting + ent - sol;
+    const unsigned long long *v = red;
+    auto count = [&](int e) { return v[2 * e]; };
+    // an event counted in the step of its serial and all later ones, and one from the step after on
+    auto from_same = [&](int e) { return S * v[2 * e] - v[2 * e + 1]; };
+    auto from_next = [&](int e) { return (S - 1) * v[2 * e] - v[2 * e + 1]; };
+    // a late solidification belongs to the step before the one that found it
+    const unsigned long long sols = count(kCntSol) + count(kCntLate), sol = from_next(kCntSol) + from_same(kCntLate);
+    const unsigned long long frontier = n * ctl->nonwaiting + from_same(kCntEnt) - sol;
+    StepStats st = *d.stats;
     st.frontier += frontier;
-    st.waiting += n * ctl->nactive + act + cap - sol - frontier;
-    st.solidified += v[kPartSol];
-    st.captures += v[kPartCap];
-    st.activated += v[kPartAct];
-    st.nucleated += v[kPartNn];
-    st.evaluated += v[kPartEval];
-    st.masks += v[kPartMask];
+    st.waiting += n * ctl->nactive + from_same(kCntAct) + from_next(kCntCap) - sol - frontier;
+    st.solidified += sols;
+    st.captures += count(kCntCap);
+    st.activated += count(kCntAct);
+    st.nucleated += count(kCntNn);
+    st.evaluated += count(kCntEval);
+    st.masks += count(kCntMask);
     *d.stats = st;
-    ctl->nonwaiting += v[kPartEnt] - v[kPartSol];
-    ctl->nactive += v[kPartAct] + v[kPartCap] - v[kPartSol];
+    ctl->nonwaiting += count(kCntEnt) - sols;
+    ctl->nactive += count(kCntAct) + count(kCntCap) - sols;
     ctl->serial_booked = serial_now;
 }
 
@@ -1260,6 +1314,7 @@ __device__ __forceinline__ bool follows_last(const StepCtl *ctl, int cycle) {
     return cycle > 1 && ctl->last_cycle == cycle - 1;
 }
 constexpr uint32_t kDueStage = 1024;  // due cells of a turn staged in LDS
+constexpr int kClaimSums = 2048;      // entries of the growth sums staged in LDS by every claim workgroup
 
 __device__ __forceinline__ void nucleate_step(const DomainView &d, int p, int layer, uint32_t b, uint32_t nb) {
     __shared__ StepTally t;
@@ -1275,16 +1330,16 @@ __device__ __forceinline__ void nucleate_step(const DomainView &d, int p, int la
     widen_range(d, t.lohi);
     add_parts(d, b, t.cnt, serial);
 }
-__device__ __forceinline__ void claim_step(const DomainView &d, int p, int layer, uint32_t b, uint32_t nb) {
+__device__ __forceinline__ void claim_step(const DomainView &d, int p, uint32_t b, uint32_t nb) {
     __shared__ StepTally t;
     __shared__ uint32_t nclaim;
-    __shared__ double gtab[kGrowStage];
+    __shared__ uint32_t gsums[kClaimSums];
     __shared__ uint32_t list[kDueStage], tot[kBlock / 64];
     StepCtl *ctl = d.ctl;
     if (ctl->done) return;
     if (threadIdx.x == 0) nclaim = 0;
     clear_tally(t);
-    const Growth g = staged_growth<kBlock>(d, gtab);
+    const Growth g = staged_growth<kBlock>(d, gsums);
     const int cycle = ctl->cycle[p];
     const uint32_t serial = ctl->serial[p];
     if (b == 0 && threadIdx.x == 0) {
@@ -1294,8 +1349,8 @@ __device__ __forceinline__ void claim_step(const DomainView &d, int p, int layer
         ctl->nuc_at = max(ctl->nuc_at, ctl->nuc_next);
     }
     const uint32_t region = place_of(b, nb) * claim_region(d, nb);
-    claim_body<kBlock, kDueStage>(d, g, cycle, serial, layer, follows_last(ctl, cycle), b, nb, list, tot, t.cnt, &nclaim,
-                                  [&](uint32_t k, uint32_t j, uint32_t claimed) {
+    claim_body<kBlock, kDueStage>(d, grid_of(d), g, layer_at(ctl), cycle, serial, follows_last(ctl, cycle), b, nb, list,
+                                  tot, t.cnt, &nclaim, [&](uint32_t k, uint32_t j, uint32_t claimed) {
                                       d.claim_cell[region + k] = j;
                                       d.claim_bits[region + k] = claimed;
                                   });
@@ -1310,36 +1365,28 @@ __device__ __forceinline__ void apply_step(const DomainView &d, int p, uint32_t 
     if (ctl->done) return;
     const uint32_t serial = ctl->serial[p];
     if (a == 0 && threadIdx.x == 0) ctl->last_cycle = ctl->cycle[p];
-    // the claimants of kApplyGroup capture-pass workgroups
-    uint32_t n0 = 0, n = 0, r0 = 0, r1 = 0;
-    static_assert(kApplyGroup == 2, "two regions");
-    const uint32_t region = claim_region(d, nbc);
-    n0 = n = d.claim_count[2 * a];
-    r0 = place_of(2 * a, nbc) * region;
-    if (2 * a + 1 < nbc) {
-        n += d.claim_count[2 * a + 1];
-        r1 = place_of(2 * a + 1, nbc) * region;
-    }
+    const uint32_t n = d.claim_count[a];
+    const uint32_t region = place_of(a, nbc) * claim_region(d, nbc);
     clear_tally(t);
+    NewCells made;
     apply_body<kBlock>(
-        d, serial, n,
+        d, grid_of(d), serial, n,
         [&](uint32_t k, uint32_t &j, uint32_t &bits) {
-            const uint32_t i = k < n0 ? r0 + k : r1 + (k - n0);
-            j = d.claim_cell[i];
-            bits = d.claim_bits[i];
+            j = d.claim_cell[region + k];
+            bits = d.claim_bits[region + k];
         },
-        s, t.cnt, t.lohi);
-    widen_range(d, t.lohi);
+        s, t.cnt, made);
+    widen_range(d, t.lohi, made);
     add_parts(d, a, t.cnt, serial);
 }
-__device__ __forceinline__ void settle_step(const DomainView &d, int p_next, int layer, uint32_t b, uint32_t nb) {
+__device__ __forceinline__ void settle_step(const DomainView &d, int p_next, uint32_t b, uint32_t nb) {
     __shared__ StepTally t;
     __shared__ uint32_t list[kDueStage], tot[kBlock / 64];
     StepCtl *ctl = d.ctl;
     if (ctl->done || !follows_last(ctl, ctl->cycle[p_next])) return;
     clear_tally(t);
     const uint32_t serial = ctl->serial[p_next];
-    settle_body<kBlock, kDueStage>(d, growth_of(d), ctl->cycle[p_next], serial, layer, b, nb, list, tot, t.cnt);
+    settle_body<kBlock, kDueStage>(d, growth_of(d), layer_at(ctl), ctl->cycle[p_next], serial, b, nb, list, tot, t.cnt);
     __syncthreads();
     add_parts(d, b, t.cnt, serial);
 }
@@ -1390,11 +1437,12 @@ __device__ __forceinline__ bool team_sync(const DomainView &d, Team &t) {
     return !__syncthreads_or(late);
 }
 
+constexpr int kTeamSums = 12288;        // entries of the growth sums staged in LDS
 constexpr uint32_t kTeamDue = 2048;     // due cells of a turn staged in LDS
-constexpr uint32_t kTeamClaims = 1024;  // claimants staged in LDS; the rest go to the claim lists
+constexpr uint32_t kTeamClaims = 512;   // claimants staged in LDS; the rest go to the claim lists
 
 struct TeamLds {
-    double grow[kGrowStage];
+    uint32_t sums[kTeamSums];
     ApplyLds<kTeamBlock> apply;
     uint32_t list[kTeamDue];
     uint32_t claim_cell[kTeamClaims], claim_bits[kTeamClaims];
@@ -1418,12 +1466,15 @@ __device__ __forceinline__ void steps_body(const DomainView &d, int p, int layer
     bool follows = follows_last(ctl, cycle);
     int site = max(ctl->nuc_at, ctl->nuc_next);
     int next_site = nucleate && site < d.nnuclei ? d.ntime[site] : 0x7FFFFFFF;
-    const Growth g = staged_growth<kTeamBlock>(d, s.grow);
+    const Growth g = staged_growth<kTeamBlock>(d, s.sums);
     const uint32_t region = place_of(b, nb) * claim_region(d, nb);
     const bool whole = scans_all<kTeamBlock>(d, nb);
+    const Grid gr = grid_of(d);
+    const LayerAt at = layer_at(ctl);
     clear_tally(s.tally[0]);
     clear_tally(s.tally[1]);
-    unsigned long long acc = 0;  // thread r: counter row r
+    Tally acc;
+    NewCells made;
     const int p_end = (p + nsteps) & 1;
     while (nsteps > 0) {
         // a domain with autostop is looked at after every step whose cycle is a multiple of 1000
@@ -1440,7 +1491,7 @@ __device__ __forceinline__ void steps_body(const DomainView &d, int p, int layer
             }
             if (threadIdx.x == 0) s.nclaim = 0;
             __syncthreads();
-            claim_body<kTeamBlock, kTeamDue>(d, g, cycle, serial, layer, follows, b, nb, s.list, s.tot, t.cnt, &s.nclaim,
+            claim_body<kTeamBlock, kTeamDue>(d, gr, g, at, cycle, serial, follows, b, nb, s.list, s.tot, t.cnt, &s.nclaim,
                                              [&](uint32_t k, uint32_t j, uint32_t claimed) {
                                                  if (k < kTeamClaims) {
                                                      s.claim_cell[k] = j;
@@ -1454,26 +1505,25 @@ __device__ __forceinline__ void steps_body(const DomainView &d, int p, int layer
             if (!team_sync(d, team)) return;
             if (threadIdx.x < kStepCounts) before.cnt[threadIdx.x] = 0;
             apply_body<kTeamBlock>(
-                d, serial, s.nclaim,
+                d, gr, serial, s.nclaim,
                 [&](uint32_t k, uint32_t &j, uint32_t &bits) {
                     j = k < kTeamClaims ? s.claim_cell[k] : d.claim_cell[region + k];
                     bits = k < kTeamClaims ? s.claim_bits[k] : d.claim_bits[region + k];
                 },
-                s.apply, t.cnt, t.lohi);
-            if (!whole) widen_range(d, t.lohi);
+                s.apply, t.cnt, made);
+            if (!whole) widen_range(d, t.lohi, made);
             if (!team_sync(d, team)) return;
-            acc += part_value(threadIdx.x, t.cnt, serial);
+            acc.add(t.cnt, serial);
             follows = true;
             cycle++;
             serial++;
         }
         StepTally &t = s.tally[serial & 1], &before = s.tally[(serial & 1) ^ 1];
-        settle_body<kTeamBlock, kTeamDue>(d, g, cycle, serial, layer, b, nb, s.list, s.tot, t.cnt);
-        widen_range(d, t.lohi);
+        settle_body<kTeamBlock, kTeamDue>(d, g, at, cycle, serial, b, nb, s.list, s.tot, t.cnt);
+        widen_range(d, t.lohi, made);
         widen_range(d, before.lohi);
-        acc += part_value(threadIdx.x, t.cnt, serial);
-        if (threadIdx.x < kPartRows && acc) d.part[static_cast<size_t>(threadIdx.x) * d.nparts + b] += acc;
-        acc = 0;
+        acc.add(t.cnt, serial);
+        acc.put(d, b);
         if (!team_sync(d, team)) return;
         clear_tally(s.tally[0]);
         clear_tally(s.tally[1]);
@@ -1500,14 +1550,14 @@ __device__ __forceinline__ void steps_body(const DomainView &d, int p, int layer
 __global__ __launch_bounds__(kBlock) void k_nucleate(DomainView d, int p, int layer) {
     nucleate_step(d, p, layer, blockIdx.x, gridDim.x);
 }
-__global__ __launch_bounds__(kBlock) void k_claim(DomainView d, int p, int layer) {
-    claim_step(d, p, layer, blockIdx.x, gridDim.x);
+__global__ __launch_bounds__(kBlock) void k_claim(DomainView d, int p) {
+    claim_step(d, p, blockIdx.x, gridDim.x);
 }
 __global__ __launch_bounds__(kBlock) void k_apply(DomainView d, int p, int nbc) {
     apply_step(d, p, blockIdx.x, static_cast<uint32_t>(nbc));
 }
-__global__ __launch_bounds__(kBlock) void k_settle(DomainView d, int p_next, int layer) {
-    settle_step(d, p_next, layer, blockIdx.x, gridDim.x);
+__global__ __launch_bounds__(kBlock) void k_settle(DomainView d, int p_next) {
+    settle_step(d, p_next, blockIdx.x, gridDim.x);
 }
 __global__ __launch_bounds__(kBlock) void k_book(DomainView d, int p_next) { book_step(d, p_next); }
 __global__ __launch_bounds__(kTeamBlock) void k_steps(DomainView d, int p, int layer, int nsteps, int nucleate) {
@@ -1521,17 +1571,17 @@ __global__ __launch_bounds__(kBlock) void k_nucleate_n(const DomainView *v, int 
     const DomainView &d = v[blockIdx.y];
     if (d.ctl) nucleate_step(d, p, layer, blockIdx.x, gridDim.x);
 }
-__global__ __launch_bounds__(kBlock) void k_claim_n(const DomainView *v, int p, int layer) {
+__global__ __launch_bounds__(kBlock) void k_claim_n(const DomainView *v, int p) {
     const DomainView &d = v[blockIdx.y];
-    if (d.ctl) claim_step(d, p, layer, blockIdx.x, gridDim.x);
+    if (d.ctl) claim_step(d, p, blockIdx.x, gridDim.x);
 }
 __global__ __launch_bounds__(kBlock) void k_apply_n(const DomainView *v, int p, int nbc) {
     const DomainView &d = v[blockIdx.y];
     if (d.ctl) apply_step(d, p, blockIdx.x, static_cast<uint32_t>(nbc));
 }
-__global__ __launch_bounds__(kBlock) void k_settle_n(const DomainView *v, int p_next, int layer) {
+__global__ __launch_bounds__(kBlock) void k_settle_n(const DomainView *v, int p_next) {
     const DomainView &d = v[blockIdx.y];
-    if (d.ctl) settle_step(d, p_next, layer, blockIdx.x, gridDim.x);
+    if (d.ctl) settle_step(d, p_next, blockIdx.x, gridDim.x);
 }
 __global__ __launch_bounds__(kBlock) void k_book_n(const DomainView *v, int p_next) {
     const DomainView &d = v[blockIdx.y];
@@ -1738,7 +1788,7 @@ __global__ __launch_bounds__(kBlock) void k_extract(DomainView d, int field, voi
         case kFieldDiagonal: {  // float, with the growth of the steps since the cell was last looked at
             float dl = c.dl;
             if ((c.ct & kTypeMask) == kActive && !(c.lm & kLmUnknown) && !(c.flags & kFresh))
-                dl = replay_growth(growth_of(d), dl, static_cast<int>(c.win), growth_index(d, c.cts, c.lid, static_cast<uint32_t>(q), d.ctl->last_cycle));
+                dl = replay_growth(growth_of(d), dl, static_cast<int>(c.win), growth_index(d, layer_at(d.ctl), c.cts, c.lid, static_cast<uint32_t>(q), d.ctl->last_cycle));
             static_cast<float *>(out)[q] = dl;
             break;
         }
@@ -1779,7 +1829,7 @@ __global__ __launch_bounds__(kBlock) void k_geometry_probe(const float *guv, con
     b[2] = o.cz;
     b[3] = static_cast<float>(o.dl);
     const Faces f = faces_of(g);
-    for (int l = 0; l < 26; l++) b[4 + l] = critical_length(f, a[4], a[5], a[6], o.cx, o.cy, o.cz, l);
+    for (int l = 0; l < 26; l++) b[4 + l] = critical_length(f, a[4], a[5], a[6], o.cx, o.cy, o.cz, nb_dx(l), nb_dy(l), nb_dz(l));
 }
 
 // Cells due at the step of that serial, added to *out.
@@ -1787,7 +1837,7 @@ __global__ __launch_bounds__(kBlock) void k_count_due(DomainView d, uint32_t ser
     __shared__ unsigned long long sh[kBlock / 64];
     const uint32_t *bits = calendar_slot(d, serial);
     unsigned long long c = 0;
-    for (size_t i = static_cast<size_t>(blockIdx.x) * kBlock + threadIdx.x; i < bitmap_words(d);
+    for (size_t i = static_cast<size_t>(blockIdx.x) * kBlock + threadIdx.x; i < d.nwords;
          i += static_cast<size_t>(gridDim.x) * kBlock)
         c += __builtin_popcount(bits[i]);
     const unsigned long long t = block_sum(c, sh);
@@ -1825,22 +1875,23 @@ inline int grid_for(long long n, int cap) {
 }  // namespace
 
 int nucleation_blocks(const DomainView &d) { return grid_for(d.nnuclei, 64); }
-uint32_t calendar_units(long long ncell) {
-    return static_cast<uint32_t>(((ncell + 31) / 32 + kUnitWords - 1) / kUnitWords);
+int claim_per_cu() {
+    int n = 0;
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, k_claim, kBlock, 0) != hipSuccess) n = 1;
+    return n < 1 ? 1 : n;
 }
-size_t claim_entries(long long ncell, uint32_t most_blocks) {
-    const size_t units = calendar_units(ncell);
-    return (units + std::min<size_t>(units, most_blocks)) * kUnitCells;
+size_t claim_entries(const DomainView &d, uint32_t most_blocks) {
+    return static_cast<size_t>(d.units + std::min(d.units, most_blocks)) * kUnitCells;
 }
 void launch_nucleation(const DomainView &d, int parity, int layer, hipStream_t s) {
     k_nucleate<<<nucleation_blocks(d), kBlock, 0, s>>>(d, parity, layer);
 }
-void launch_capture(const DomainView &d, int parity, int layer, int blocks, hipStream_t s) {
-    k_claim<<<blocks, kBlock, 0, s>>>(d, parity, layer);
-    k_apply<<<apply_blocks(blocks), kBlock, 0, s>>>(d, parity, blocks);
+void launch_capture(const DomainView &d, int parity, int blocks, hipStream_t s) {
+    k_claim<<<blocks, kBlock, 0, s>>>(d, parity);
+    k_apply<<<blocks, kBlock, 0, s>>>(d, parity, blocks);
 }
-void launch_settle(const DomainView &d, int parity_next, int layer, int blocks, hipStream_t s) {
-    k_settle<<<blocks, kBlock, 0, s>>>(d, parity_next, layer);
+void launch_settle(const DomainView &d, int parity_next, int blocks, hipStream_t s) {
+    k_settle<<<blocks, kBlock, 0, s>>>(d, parity_next);
     k_book<<<1, kBlock, 0, s>>>(d, parity_next);
 }
 void launch_steps(const DomainView &d, int parity, int layer, int steps, bool nucleate, int team, hipStream_t s) {
@@ -1863,20 +1914,20 @@ void launch_step_timed(const DomainView &d, int parity, int layer, int blocks, h
     k_nucleate<<<nucleation_blocks(d), kBlock, 0, s>>>(d, parity, layer);
     rec();
     rec();
-    k_claim<<<blocks, kBlock, 0, s>>>(d, parity, layer);
+    k_claim<<<blocks, kBlock, 0, s>>>(d, parity);
     rec();
     rec();
-    k_apply<<<apply_blocks(blocks), kBlock, 0, s>>>(d, parity, blocks);
+    k_apply<<<blocks, kBlock, 0, s>>>(d, parity, blocks);
     rec();
 }
 void launch_steps_n(const DomainView *views, int slots, int steps, int layer, int nuc_blocks, int blocks,
                     hipStream_t s) {
     for (int k = 0; k < steps; k++) {
         k_nucleate_n<<<dim3(nuc_blocks, slots), kBlock, 0, s>>>(views, k & 1, layer);
-        k_claim_n<<<dim3(blocks, slots), kBlock, 0, s>>>(views, k & 1, layer);
-        k_apply_n<<<dim3(apply_blocks(blocks), slots), kBlock, 0, s>>>(views, k & 1, blocks);
+        k_claim_n<<<dim3(blocks, slots), kBlock, 0, s>>>(views, k & 1);
+        k_apply_n<<<dim3(blocks, slots), kBlock, 0, s>>>(views, k & 1, blocks);
     }
-    k_settle_n<<<dim3(blocks, slots), kBlock, 0, s>>>(views, steps & 1, layer);
+    k_settle_n<<<dim3(blocks, slots), kBlock, 0, s>>>(views, steps & 1);
     k_book_n<<<dim3(1, slots), kBlock, 0, s>>>(views, steps & 1);
 }
 void launch_check(const DomainView &d, int cycle, int layer, CheckResult *out, hipStream_t s) {

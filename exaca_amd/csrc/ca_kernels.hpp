@@ -16,18 +16,18 @@ int nucleation_blocks(const DomainView &d);
 // CellCapture (src/CAupdate.cpp:204-728) in two kernels: the liquidus-time gate, growth, neighbour
 // scan and claims of the cells due this step (also prepares the control slot of the next step);
 // then claims decided and winners' captures.
-void launch_capture(const DomainView &d, int parity, int layer, int blocks, hipStream_t s);
+void launch_capture(const DomainView &d, int parity, int blocks, hipStream_t s);
 // The solidifications the last step left to the next one, and the counters booked: before the state
 // or the statistics are looked at. parity_next is the parity of the next step.
-void launch_settle(const DomainView &d, int parity_next, int layer, int blocks, hipStream_t s);
+void launch_settle(const DomainView &d, int parity_next, int blocks, hipStream_t s);
 // `steps` steps in one launch of a team of workgroups (at most kMaxTeam), settled and booked;
 // nucleate: with their nucleation (else none of their sites may be due).
 constexpr int kTeamBlock = 512;
 void launch_steps(const DomainView &d, int parity, int layer, int steps, bool nucleate, int team, hipStream_t s);
-// Units of a calendar slot, and entries of the claim lists for up to most_blocks capture-pass
-// workgroups.
-uint32_t calendar_units(long long ncell);
-size_t claim_entries(long long ncell, uint32_t most_blocks);
+// Capture-pass workgroups that a CU holds at once.
+int claim_per_cu();
+// Entries of the claim lists for up to most_blocks capture-pass workgroups.
+size_t claim_entries(const DomainView &d, uint32_t most_blocks);
 // Every active cell due at the next step: after a cycle jump, whose skipped steps the calendar did
 // not count. parity_next is the parity of the next step.
 void launch_rewake(const DomainView &d, int parity_next, int blocks, hipStream_t s);

@@ -21,6 +21,7 @@
 #include "ca_common.hpp"
 #include "ca_kernels.hpp"
 #include "deck.hpp"
+#include "growth.hpp"
 #include "init.hpp"
 #include "output.hpp"
 #include "runtime_util.hpp"
@@ -195,16 +196,25 @@ struct exaca_state {
 
 namespace {
 
-// Workgroups of the team that steps a domain in one launch, by the cross-section X * Y that its front
-// spreads over; 0: too wide, two launches a step over the whole device are faster. Measured, us a
-// step with a team of the size chosen and with two launches: 24^3 13.4 (1) and 17.0; 64^3 20.7 (16)
-// and 22.0; 100^3 22.8 (32) and 23.4; 200^3 33.5 (64) and 45.1; 256^3 44.7 (64) and 44.5.
-int team_size(const exaca::HostDomain &hd) {
-    const long long area = static_cast<long long>(hd.X) * hd.Y;
-    if (area <= 48 * 48) return 1;
-    if (area <= 80 * 80) return 16;
-    if (area <= 128 * 128) return 32;
-    return area <= 240 * 240 ? 64 : 0;
+// Workgroups of the team that steps a domain in one launch, by the cross-section that its front
+// spreads over (X * Y; of a spot melt, one spot's: the spots solidify after one another, and about
+// 1.5 radius^2 cells are due together). 0: two launches a step over the whole device are faster. Measured,
+// us a step, with teams of 1, 8, 16, 32, 64 workgroups and two launches (-: not run):
+//   24^3 7.4, 9.5, 10.0, -, -, 13.1      44^3 17.8, 13.1, 13.5, 13.9, 15.1, 17.9
+//   56^3 31.6, 15.5, 15.4, 15.8, 16.9, 19.9      64^3 29.8, 13.6, 13.3, 13.8, 15.5, 16.5
+//   100^3 84.6, 20.8, 16.4, 15.3, 16.5, 17.9     150^3 -, -, 26.4, 20.2, 19.6, 21.6
+//   176^3 -, -, 40.2, 26.4, 22.3, 23.8           200^3 -, 55.5, 35.0, 26.1, 23.9, 23.6
+//   256^3 -, 168, 91.5, 55.0, 36.3, 31.1
+//   spots of radius 20 8.4, 9.2, 9.5, 10.0, -, 11.6; 25 5.1, 5.2, 5.4, 5.4, -, 6.2; 50 49.4, 15.3,
+//   13.0, 13.0, 14.9, 14.7; 6 x 6 of radius 75 (456 x 456 cells) -, -, 32.4, 23.4, 20.5, 18.6
+int team_size(const exaca::Deck &deck, const exaca::HostDomain &hd) {
+    const long long plane = static_cast<long long>(hd.X) * hd.Y;
+    if (plane > 190 * 190) return 0;
+    const double area = deck.sim_type == "S" ? 1.5 * deck.spot_radius * deck.spot_radius : static_cast<double>(plane);
+    if (area <= 34 * 34) return 1;
+    if (area <= 60 * 60) return 8;
+    if (area <= 84 * 84) return 16;
+    return area <= 150 * 150 ? 32 : 64;
 }
 
 // The layer's nucleation sites to the device; its steps start with none decided. Synchronises the
@@ -236,28 +246,25 @@ void build_device_state(exaca_state *h) {
     // measured at 800^3: 2, 3, 4, 6, 8 per CU give 110, 101, 96, 102, 118 us), fewer for small
     // domains (the frontier never exceeds the cell count, and a slice is at least one workgroup of
     // cells).
-    const long long cap = std::min<long long>(2048, ((prop.multiProcessorCount * 4 + 7) / 8) * 8);
+    const int per_cu = std::min(4, exaca::claim_per_cu());
+    const long long cap = std::min<long long>(2048, ((prop.multiProcessorCount * per_cu + 7) / 8) * 8);
     const long long want = ((hd.ncell / 4096 + 7) / 8) * 8;
     h->blocks = static_cast<int>(std::max<long long>(8, std::min(cap, want)));
-    h->team = std::min(team_size(hd), prop.multiProcessorCount / 4);
+    h->team = std::min(team_size(h->deck, hd), prop.multiProcessorCount / 4);
     if (const int forced = exaca::frontier_blocks_override()) {
         h->blocks = forced;
         h->team = 0;
     }
 
     DomainView &d = h->dv;
-    d.X = hd.X;
-    d.Y = hd.Y;
-    d.nz = hd.nz;
-    d.nzA = hd.nzA;
+    set_geometry(d, hd.X, hd.Y, hd.nz, hd.nzA);
     d.xoff = hd.xoff;
     d.yoff = hd.yoff;
-    d.ncell = hd.ncell;
     const size_t n = static_cast<size_t>(hd.ncell);
     d.cells = h->alloc<Cell>(n);
     d.octa = h->alloc<Octa>(n);
-    d.claim_cell = h->alloc<uint32_t>(claim_entries(hd.ncell, static_cast<uint32_t>(std::max(h->blocks, kMaxTeam))));
-    d.claim_bits = h->alloc<uint32_t>(claim_entries(hd.ncell, static_cast<uint32_t>(std::max(h->blocks, kMaxTeam))));
+    d.claim_cell = h->alloc<uint32_t>(claim_entries(d, static_cast<uint32_t>(std::max(h->blocks, kMaxTeam))));
+    d.claim_bits = h->alloc<uint32_t>(claim_entries(d, static_cast<uint32_t>(std::max(h->blocks, kMaxTeam))));
     d.claim_count = h->alloc<uint32_t>(h->blocks);
     d.alarms = h->alloc<uint32_t>(kAlarmSlots * alarm_stride(d.ncell));
     h->nloc = h->alloc<int32_t>(hd.nloc.size());
@@ -274,6 +281,10 @@ void build_device_state(exaca_state *h) {
     d.grow = grow_d;
     d.ngrow = static_cast<int32_t>(grow.size());
     d.ksat = growth_plateau(grow);
+    const GrowthSums sums = growth_sums(grow, d.ksat);
+    uint32_t *sums_d = h->alloc<uint32_t>(sums.sums.size());
+    d.grow_sums = sums_d;
+    d.sums_usable = sums.usable;
     d.sync = h->alloc<uint32_t>(kMaxTeam);
     h->ctl = h->alloc<StepCtl>(1);
     h->stats = h->alloc<StepStats>(1);
@@ -290,6 +301,7 @@ void build_device_state(exaca_state *h) {
     HIP_OK(hipMemcpyAsync(guv, hd.guv.data(), hd.guv.size() * 4, hipMemcpyHostToDevice, s));
     HIP_OK(hipMemcpyAsync(seed_d, seed.data(), seed.size() * 4, hipMemcpyHostToDevice, s));
     HIP_OK(hipMemcpyAsync(grow_d, grow.data(), grow.size() * 8, hipMemcpyHostToDevice, s));
+    HIP_OK(hipMemcpyAsync(sums_d, sums.sums.data(), sums.sums.size() * 4, hipMemcpyHostToDevice, s));
     h->melted = h->alloc<uint8_t>(n);
     upload_cells(d, hd, h->melted, s);
     StepCtl c = initial_ctl(hd);
@@ -384,12 +396,12 @@ void next_layer(exaca_state *h, int layer_done, int verbose) {
 void step_nucleation(exaca_state *h, int layer) {
     exaca::launch_nucleation(h->dv, h->parity, layer, h->stream);
 }
-void step_capture(exaca_state *h, int layer) {
-    exaca::launch_capture(h->dv, h->parity, layer, h->blocks, h->stream);
+void step_capture(exaca_state *h) {
+    exaca::launch_capture(h->dv, h->parity, h->blocks, h->stream);
 }
 // After the last step of a call: its state and statistics complete.
-void finish_steps(exaca_state *h, int layer) {
-    exaca::launch_settle(h->dv, h->parity, layer, h->blocks, h->stream);
+void finish_steps(exaca_state *h) {
+    exaca::launch_settle(h->dv, h->parity, h->blocks, h->stream);
     HIP_OK(hipGetLastError());
 }
 // Whether steps h->cycle + 1 .. last need the nucleation kernel.
@@ -412,7 +424,7 @@ void ensure_graph(exaca_state *h, int layer) {
         for (int k = 0; k < kGraphSteps; k++) {
             const int p = k & 1;
             if (nucleate) exaca::launch_nucleation(h->dv, p, layer, h->stream);
-            exaca::launch_capture(h->dv, p, layer, h->blocks, h->stream);
+            exaca::launch_capture(h->dv, p, h->blocks, h->stream);
         }
         HIP_OK(hipStreamEndCapture(h->stream, &g));
         HIP_OK(hipGraphInstantiate(nucleate ? &h->graph : &h->graph_quiet, g, nullptr, nullptr, 0));
@@ -447,13 +459,13 @@ void run_steps(exaca_state *h, int layer, int n, bool use_graph) {
                 step_nucleation(h, layer);
                 h->nuc_through = h->cycle + 1;
             }
-            step_capture(h, layer);
+            step_capture(h);
             h->parity ^= 1;
             h->cycle += 1;
             n -= 1;
         }
     }
-    finish_steps(h, layer);
+    finish_steps(h);
 }
 
 void device_check(exaca_state *h, int *cycle, int layer, uint64_t counts[5], int *xswitch, int verbose) {
@@ -583,7 +595,7 @@ void profile(exaca_state *h, int layer, int nsteps, double *ms, int64_t counts[5
                 break;
             }
         }
-        finish_steps(h, layer);
+        finish_steps(h);
         HIP_OK(hipStreamSynchronize(h->stream));
         for (int q = 0; q < k; q++)
             for (int r = 0; r < kTimedKernels; r++) {
@@ -785,7 +797,7 @@ int exaca_nucleation_nn(exaca_state *h, int cycle, int layer, int32_t *nn) {
         const int nb = exaca::nucleation_blocks(h->dv);
         std::vector<unsigned long long> row(static_cast<size_t>(nb));
         exaca::StepStats st;
-        HIP_OK(hipMemcpyAsync(row.data(), h->dv.part + static_cast<size_t>(exaca::kPartNn) * h->dv.nparts,
+        HIP_OK(hipMemcpyAsync(row.data(), h->dv.part + static_cast<size_t>(2 * exaca::kCntNn) * h->dv.nparts,
                               row.size() * sizeof(unsigned long long), hipMemcpyDeviceToHost, h->stream));
         HIP_OK(hipMemcpyAsync(&st, h->stats, sizeof st, hipMemcpyDeviceToHost, h->stream));
         HIP_OK(hipStreamSynchronize(h->stream));
@@ -805,9 +817,9 @@ int exaca_cell_capture(exaca_state *h, int cycle, int layer) {
             h->parity ^= 1;
         }
         else {
-            step_capture(h, layer);
+            step_capture(h);
             h->parity ^= 1;
-            finish_steps(h, layer);
+            finish_steps(h);
         }
         h->cycle = cycle;
         h->pending = -1;

@@ -20,6 +20,7 @@
 #include "ca_common.hpp"
 #include "ca_kernels.hpp"
 #include "deck.hpp"
+#include "growth.hpp"
 #include "init.hpp"
 #include "runtime_util.hpp"
 
@@ -81,12 +82,14 @@ struct Arena {
 };
 
 // Device bytes one domain needs (state, frontier lists, tables, control).
-size_t domain_bytes(const exaca::HostDomain &h, size_t ngrow) {
+size_t domain_bytes(const exaca::HostDomain &h, size_t ngrow, size_t nsums) {
     const size_t n = static_cast<size_t>(h.ncell);
+    exaca::DomainView v{};
+    exaca::set_geometry(v, h.X, h.Y, h.nz, h.nzA);
     size_t b = 0;
     b += up(sizeof(exaca::Cell) * n) + up(sizeof(exaca::Octa) * n);  // cell records
-    b += 2 * up(4 * exaca::claim_entries(h.ncell, kMaxSlices)) + up(4 * kMaxSlices);  // claim lists
-    b += 2 * up(4 * std::max<size_t>(h.nloc.size(), 1)) + up(8 * ngrow);
+    b += 2 * up(4 * exaca::claim_entries(v, kMaxSlices)) + up(4 * kMaxSlices);  // claim lists
+    b += 2 * up(4 * std::max<size_t>(h.nloc.size(), 1)) + up(8 * ngrow) + up(4 * nsums);
     b += up(sizeof(exaca::StepCtl)) + up(sizeof(exaca::StepStats)) + up(8ull * exaca::kPartRows * kMaxSlices);
     b += up(4 * exaca::kAlarmSlots * exaca::alarm_stride(h.ncell));  // calendar
     return b;
@@ -99,6 +102,8 @@ struct exaca_prepared {
     exaca::Deck deck;
     exaca::HostDomain host;
     std::vector<double> grow;
+    int ksat = 0;
+    exaca::GrowthSums sums;
     long long liquid0 = 0;
     size_t bytes = 0;
 };
@@ -188,21 +193,18 @@ void admit(exaca_ensemble *e, const exaca_prepared *pr, int *slot_out) {
     std::vector<int32_t> loc, time;
     exaca::layer_sites(hd, 0, loc, time);
     DomainView d{};
-    d.X = hd.X;
-    d.Y = hd.Y;
-    d.nz = hd.nz;
-    d.nzA = hd.nzA;
+    exaca::set_geometry(d, hd.X, hd.Y, hd.nz, hd.nzA);
     d.xoff = hd.xoff;
     d.yoff = hd.yoff;
-    d.ncell = hd.ncell;
     d.cells = reinterpret_cast<Cell *>(carve(sizeof(Cell) * n));
     d.octa = reinterpret_cast<Octa *>(carve(sizeof(Octa) * n));
-    d.claim_cell = reinterpret_cast<uint32_t *>(carve(4 * exaca::claim_entries(hd.ncell, kMaxSlices)));
-    d.claim_bits = reinterpret_cast<uint32_t *>(carve(4 * exaca::claim_entries(hd.ncell, kMaxSlices)));
+    d.claim_cell = reinterpret_cast<uint32_t *>(carve(4 * exaca::claim_entries(d, kMaxSlices)));
+    d.claim_bits = reinterpret_cast<uint32_t *>(carve(4 * exaca::claim_entries(d, kMaxSlices)));
     d.claim_count = reinterpret_cast<uint32_t *>(carve(4 * kMaxSlices));
     int32_t *nloc = reinterpret_cast<int32_t *>(carve(4 * std::max<size_t>(hd.nloc.size(), 1)));
     int32_t *ntime = reinterpret_cast<int32_t *>(carve(4 * std::max<size_t>(hd.nloc.size(), 1)));
     double *grow = reinterpret_cast<double *>(carve(8 * pr->grow.size()));
+    uint32_t *sums = reinterpret_cast<uint32_t *>(carve(4 * pr->sums.sums.size()));
     d.alarms = reinterpret_cast<uint32_t *>(carve(4 * kAlarmSlots * alarm_stride(d.ncell)));
     d.ctl = reinterpret_cast<StepCtl *>(carve(sizeof(StepCtl)));
     d.stats = reinterpret_cast<StepStats *>(carve(sizeof(StepStats)));
@@ -215,7 +217,9 @@ void admit(exaca_ensemble *e, const exaca_prepared *pr, int *slot_out) {
     d.seed_cdl = e->seed_cdl;
     d.grow = grow;
     d.ngrow = static_cast<int32_t>(pr->grow.size());
-    d.ksat = exaca::growth_plateau(pr->grow);
+    d.ksat = pr->ksat;
+    d.grow_sums = sums;
+    d.sums_usable = pr->sums.usable;
     d.autostop = 1;
     d.liquid0 = pr->liquid0;
     d.status = e->status_d + slot;
@@ -227,6 +231,7 @@ void admit(exaca_ensemble *e, const exaca_prepared *pr, int *slot_out) {
         HIP_OK(hipMemcpyAsync(ntime, time.data(), 4 * time.size(), hipMemcpyHostToDevice, s));
     }
     HIP_OK(hipMemcpyAsync(grow, pr->grow.data(), 8 * pr->grow.size(), hipMemcpyHostToDevice, s));
+    HIP_OK(hipMemcpyAsync(sums, pr->sums.sums.data(), 4 * pr->sums.sums.size(), hipMemcpyHostToDevice, s));
     exaca::upload_cells(d, hd, nullptr, s);
     // Chunks end on parity 0, so a new domain always starts in slot 0 of its control block.
     StepCtl c = exaca::initial_ctl(hd);
@@ -304,6 +309,8 @@ int exaca_prepare(const char *input_file, const char *data_dir, uint64_t seed, e
         const exaca::HostDomain &h = pr->host;
         pr->grow = exaca::growth_table(h.A, h.B, h.C, h.D, h.dU, 1 << 25);
         if (pr->grow.size() >= (1u << 25)) throw std::runtime_error("undercooling never saturates within 2^25 steps");
+        pr->ksat = exaca::growth_plateau(pr->grow);
+        pr->sums = exaca::growth_sums(pr->grow, pr->ksat);
         if (h.ncell > exaca::kEnsembleCells)
             throw std::invalid_argument("domain too large for an ensemble slot (at most " +
                                         std::to_string(exaca::kEnsembleCells) + " cells); run it on the plain path");
@@ -311,7 +318,7 @@ int exaca_prepare(const char *input_file, const char *data_dir, uint64_t seed, e
             pr->liquid0 = static_cast<long long>(h.nx) * h.ny * (h.nz - 2) - static_cast<long long>(h.active.size());
         else
             for (long long q = 0; q < h.ncell; q++) pr->liquid0 += (h.ct[q] == exaca::kLiquid && h.lid[q] == 0);
-        pr->bytes = domain_bytes(h, pr->grow.size());
+        pr->bytes = domain_bytes(h, pr->grow.size(), pr->sums.sums.size());
         *out = pr.release();
     });
 }

@@ -1,7 +1,8 @@
 """GPU: the kernel that runs many steps of a domain in one launch, at the cross-sections where the
 number of its workgroups changes (the last of a size and the first of the next, to the first domain
 that takes two launches a step), against the oracle, cell for cell. One workgroup also gets a
-bottom plane full of grains, whose claimants exceed what it stages in LDS. Each domain is run three
+domain where a third of the cells are nuclei: about 740 captures a step, more claimants than it
+stages in LDS. Each domain is run three
 ways: in one call, in calls of odd lengths (each settles and books its own last step), and through
 the time-step functions with their check."""
 import numpy as np
@@ -14,15 +15,18 @@ from conftest import DATA, c_deck
 pytestmark = pytest.mark.gpu
 
 CASES = {
-    "46x46x9_full": dict(n=9, nx=46, ny=46, density=2000, fraction=1.0),
-    "46x46x9": dict(n=9, nx=46, ny=46, density=2000, fraction=0.05),
-    "47x47x9": dict(n=9, nx=47, ny=47, density=2000, fraction=0.05),
-    "78x78x7": dict(n=7, nx=78, ny=78, density=1000, fraction=0.05),
-    "79x79x7": dict(n=7, nx=79, ny=79, density=1000, fraction=0.05),
-    "126x126x5": dict(n=5, nx=126, ny=126, density=500, fraction=0.05),
-    "127x127x5": dict(n=5, nx=127, ny=127, density=500, fraction=0.05),
-    "238x238x4": dict(n=4, nx=238, ny=238, density=200, fraction=0.05),
-    "239x239x4": dict(n=4, nx=239, ny=239, density=200, fraction=0.05),
+    "32x32x9_full": dict(n=9, nx=32, ny=32, density=2000, fraction=1.0),
+    "32x32x60_third_nuclei": dict(n=60, nx=32, ny=32, density=300000, fraction=1.0, N=1, G=1e5),
+    "32x32x9": dict(n=9, nx=32, ny=32, density=2000, fraction=0.05),
+    "33x33x9": dict(n=9, nx=33, ny=33, density=2000, fraction=0.05),
+    "58x58x7_full": dict(n=7, nx=58, ny=58, density=1000, fraction=1.0),
+    "59x59x7": dict(n=7, nx=59, ny=59, density=1000, fraction=0.05),
+    "82x82x5": dict(n=5, nx=82, ny=82, density=1000, fraction=0.05),
+    "83x83x5": dict(n=5, nx=83, ny=83, density=500, fraction=0.05),
+    "148x148x4": dict(n=4, nx=148, ny=148, density=500, fraction=0.05),
+    "149x149x4": dict(n=4, nx=149, ny=149, density=200, fraction=0.05),
+    "188x188x4": dict(n=4, nx=188, ny=188, density=200, fraction=0.05),
+    "189x189x4": dict(n=4, nx=189, ny=189, density=200, fraction=0.05),
 }
 
 
