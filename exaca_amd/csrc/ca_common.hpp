@@ -257,6 +257,11 @@ struct DomainView {
     int32_t *status_err;    // where it reports the error flags of a domain stopped by an error
 };
 
+// A workgroup of an ensemble's launch: workgroup b of the nb that serve the domain of a slot.
+struct TeamPlace {
+    uint32_t slot, b, nb;
+};
+
 // The view's sizes for a domain of X x Y x nz cells, the top of its active window at nzA.
 inline void set_geometry(DomainView &d, int X, int Y, int nz, int nzA) {
     d.X = X;

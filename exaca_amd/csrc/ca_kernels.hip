@@ -1565,27 +1565,26 @@ __global__ __launch_bounds__(kTeamBlock) void k_steps(DomainView d, int p, int l
     steps_body(d, p, layer, nsteps, nucleate != 0, blockIdx.x, gridDim.x, s);
 }
 
-// Ensemble launches: grid row y serves domain slot y of a device-resident table; an empty slot has
-// no control block.
-__global__ __launch_bounds__(kBlock) void k_nucleate_n(const DomainView *v, int p, int layer) {
-    const DomainView &d = v[blockIdx.y];
-    if (d.ctl) nucleate_step(d, p, layer, blockIdx.x, gridDim.x);
+// Ensemble launches: workgroup i is workgroup b of the team of nb that serves the domain of one slot
+// (its TeamPlace); a team's workgroups follow one another. Views and places lie in tables that no
+// kernel writes, read as constants so that a view is kept in scalar registers like an argument.
+template <typename T>
+__device__ __forceinline__ T load_constant(const T *table, uint32_t i) {
+    static_assert(sizeof(T) % 4 == 0, "whole words");
+    struct Words {
+        uint32_t w[sizeof(T) / 4];
+    } v;
+    const auto *src = (const __attribute__((address_space(4))) uint32_t *)(table + i);
+#pragma unroll
+    for (uint32_t k = 0; k < sizeof(T) / 4; k++) v.w[k] = src[k];
+    return __builtin_bit_cast(T, v);
 }
-__global__ __launch_bounds__(kBlock) void k_claim_n(const DomainView *v, int p) {
-    const DomainView &d = v[blockIdx.y];
-    if (d.ctl) claim_step(d, p, blockIdx.x, gridDim.x);
-}
-__global__ __launch_bounds__(kBlock) void k_apply_n(const DomainView *v, int p, int nbc) {
-    const DomainView &d = v[blockIdx.y];
-    if (d.ctl) apply_step(d, p, blockIdx.x, static_cast<uint32_t>(nbc));
-}
-__global__ __launch_bounds__(kBlock) void k_settle_n(const DomainView *v, int p_next) {
-    const DomainView &d = v[blockIdx.y];
-    if (d.ctl) settle_step(d, p_next, blockIdx.x, gridDim.x);
-}
-__global__ __launch_bounds__(kBlock) void k_book_n(const DomainView *v, int p_next) {
-    const DomainView &d = v[blockIdx.y];
-    if (d.ctl) book_step(d, p_next);
+__global__ __launch_bounds__(kTeamBlock) void k_steps_n(const DomainView *views, const TeamPlace *places, int layer,
+                                                        int nsteps) {
+    __shared__ TeamLds s;
+    const TeamPlace at = load_constant(places, blockIdx.x);
+    const DomainView d = load_constant(views, at.slot);
+    steps_body(d, 0, layer, nsteps, true, at.b, at.nb, s);
 }
 
 __global__ __launch_bounds__(kBlock) void k_check(DomainView d, int cycle, int layer, CheckResult *out) {
@@ -1920,15 +1919,9 @@ void launch_step_timed(const DomainView &d, int parity, int layer, int blocks, h
     k_apply<<<blocks, kBlock, 0, s>>>(d, parity, blocks);
     rec();
 }
-void launch_steps_n(const DomainView *views, int slots, int steps, int layer, int nuc_blocks, int blocks,
+void launch_steps_n(const DomainView *views, const TeamPlace *places, uint32_t workgroups, int steps, int layer,
                     hipStream_t s) {
-    for (int k = 0; k < steps; k++) {
-        k_nucleate_n<<<dim3(nuc_blocks, slots), kBlock, 0, s>>>(views, k & 1, layer);
-        k_claim_n<<<dim3(blocks, slots), kBlock, 0, s>>>(views, k & 1);
-        k_apply_n<<<dim3(blocks, slots), kBlock, 0, s>>>(views, k & 1, blocks);
-    }
-    k_settle_n<<<dim3(blocks, slots), kBlock, 0, s>>>(views, steps & 1);
-    k_book_n<<<dim3(1, slots), kBlock, 0, s>>>(views, steps & 1);
+    k_steps_n<<<workgroups, kTeamBlock, 0, s>>>(views, places, layer, steps);
 }
 void launch_check(const DomainView &d, int cycle, int layer, CheckResult *out, hipStream_t s) {
     k_check<<<grid_for(d.ncell, 4096), kBlock, 0, s>>>(d, cycle, layer, out);

@@ -36,9 +36,9 @@ void launch_rewake(const DomainView &d, int parity_next, int blocks, hipStream_t
 void launch_layer_bounds(const DomainView &d, int next_layer, int *out, hipStream_t s);
 // LayerSetup on the resident state for the window [d.zlo, d.nzA).
 void launch_layer_setup(const DomainView &d, int parity_next, hipStream_t s);
-// `steps` steps (from parity 0) of every domain in a device-resident table of `slots` views (grid
-// row = slot), then their settling and booking.
-void launch_steps_n(const DomainView *views, int slots, int steps, int layer, int nuc_blocks, int blocks,
+// `steps` steps (an even number, from parity 0) of the domains of a device-resident table of views,
+// settled and booked: one workgroup per entry of `places`.
+void launch_steps_n(const DomainView *views, const TeamPlace *places, uint32_t workgroups, int steps, int layer,
                     hipStream_t s);
 // IntermediateOutputAndCheck's reduction (src/CAupdate.cpp:738-758, 792-808).
 void launch_check(const DomainView &d, int cycle, int layer, CheckResult *out, hipStream_t s);

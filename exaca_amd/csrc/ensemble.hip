@@ -1,16 +1,18 @@
 // ensemble.hip -- many CA domains resident on one GPU, stepped together.
 //
 // Each domain occupies one slot: its state lives in a sub-range of a single device arena, and its
-// DomainView sits in a device-resident slot table. One step of every slot is three launches
-// whose grid row y serves slot y (launch_steps_n); 50-step chunks of those launches are captured once in
-// a HIP graph and replayed. Every domain keeps its own cycle, control block and frontier, and stops
-// itself on the device at the first 1000-step check with no liquid left, so each one evolves
-// exactly as it would alone on the plain path. The host admits new domains into free slots
-// between chunks (continuous batching) and polls the per-slot status words after each chunk.
+// DomainView sits in a device-resident slot table. A launch runs many steps of every domain: a team of
+// workgroups takes each domain through them on its own (k_steps_n), so no domain waits for another
+// within a launch, and the larger a domain, the larger its team (share_out). Every domain keeps its
+// own cycle, control block and calendar, and stops itself on the device at the first 1000-step check
+// with no liquid left, so each one evolves exactly as it would alone on the plain path. The host
+// admits new domains into free slots between launches (continuous batching) and polls the
+// per-slot status words after each.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
 #include <chrono>
+#include <cmath>
 #include <cstring>
 #include <map>
 #include <memory>
@@ -37,8 +39,9 @@ using exaca::DeviceError;
 using exaca::StateError;
 using exaca::guarded;
 
-constexpr int kChunk = 50;         // steps per graph replay (even: parity 0 at chunk boundaries)
-constexpr int kMaxSlices = 256;    // largest workgroups-per-slot candidate
+constexpr int kChunk = 50;         // steps are rounded up to this (even: parity 0 at launch boundaries)
+constexpr int kMaxLaunch = 1000;   // most steps of one launch (a multiple of kChunk)
+constexpr int kMaxBlocks = 256;    // largest workgroups-per-slot setting
 constexpr size_t kAlign = 256;
 
 size_t up(size_t n) { return (n + kAlign - 1) / kAlign * kAlign; }
@@ -88,9 +91,9 @@ size_t domain_bytes(const exaca::HostDomain &h, size_t ngrow, size_t nsums) {
     exaca::set_geometry(v, h.X, h.Y, h.nz, h.nzA);
     size_t b = 0;
     b += up(sizeof(exaca::Cell) * n) + up(sizeof(exaca::Octa) * n);  // cell records
-    b += 2 * up(4 * exaca::claim_entries(v, kMaxSlices)) + up(4 * kMaxSlices);  // claim lists
+    b += 2 * up(4 * exaca::claim_entries(v, exaca::kMaxTeam)) + up(4 * exaca::kMaxTeam);  // claim lists, barrier words
     b += 2 * up(4 * std::max<size_t>(h.nloc.size(), 1)) + up(8 * ngrow) + up(4 * nsums);
-    b += up(sizeof(exaca::StepCtl)) + up(sizeof(exaca::StepStats)) + up(8ull * exaca::kPartRows * kMaxSlices);
+    b += up(sizeof(exaca::StepCtl)) + up(sizeof(exaca::StepStats)) + up(8ull * exaca::kPartRows * exaca::kMaxTeam);
     b += up(4 * exaca::kAlarmSlots * exaca::alarm_stride(h.ncell));  // calendar
     return b;
 }
@@ -111,8 +114,8 @@ struct exaca_prepared {
 struct exaca_ensemble {
     hipStream_t stream = nullptr;
     int slots = 0;
-    int blocks = 64;      // workgroups per slot (frontier kernels)
-    int nuc_blocks = 4;   // workgroups per slot (nucleation)
+    int blocks = 64;      // workgroups per slot, at most
+    int cus = 0;          // compute units, each of which holds one workgroup of a team
     Arena arena;
     exaca::DomainView *views_d = nullptr;
     std::vector<exaca::DomainView> views;
@@ -124,13 +127,17 @@ struct exaca_ensemble {
     // tables shared by every slot (one orientation file per ensemble)
     std::string orientation_file;
     float *guv = nullptr, *seed_cdl = nullptr;
-    std::map<int, hipGraphExec_t> graphs;  // per workgroups-per-slot setting
+    // The workgroups of a launch, for the domains that run now (dirty: to be shared out afresh)
+    exaca::TeamPlace *places_d = nullptr;
+    std::vector<exaca::TeamPlace> places;
+    size_t places_cap = 0;
+    bool dirty = true;
     long long steps = 0;
 
     ~exaca_ensemble() {
-        for (auto &kv : graphs) (void)hipGraphExecDestroy(kv.second);
         if (arena.base) (void)hipFree(arena.base);
         if (views_d) (void)hipFree(views_d);
+        if (places_d) (void)hipFree(places_d);
         if (status_d) (void)hipFree(status_d);
         if (guv) (void)hipFree(guv);
         if (seed_cdl) (void)hipFree(seed_cdl);
@@ -156,18 +163,90 @@ void ensure_tables(exaca_ensemble *e, const exaca::HostDomain &h, const std::str
     HIP_OK(hipMemcpy(e->seed_cdl, seed.data(), seed.size() * 4, hipMemcpyHostToDevice));
 }
 
-hipGraphExec_t graph_for(exaca_ensemble *e, int blocks) {
-    auto it = e->graphs.find(blocks);
-    if (it != e->graphs.end()) return it->second;
-    hipGraph_t g;
-    HIP_OK(hipStreamBeginCapture(e->stream, hipStreamCaptureModeThreadLocal));
-    exaca::launch_steps_n(e->views_d, e->slots, kChunk, 0, e->nuc_blocks, blocks, e->stream);
-    HIP_OK(hipStreamEndCapture(e->stream, &g));
-    hipGraphExec_t x;
-    HIP_OK(hipGraphInstantiate(&x, g, nullptr, nullptr, 0));
-    HIP_OK(hipGraphDestroy(g));
-    e->graphs[blocks] = x;
-    return x;
+// Estimated time of a step (us) of a domain with that cross-section and team: a chain that grows
+// with the team's barriers, and the front's cells by the team, dearer in a large domain, whose records
+// the caches don't hold. Single domains measured, us: 24^3 7.4
+// with 1 workgroup, 44^3 17.8 with 1 and 13.1 with 8, 100^3 84.6 with 1, 20.8 with 8 and 15.3 with 32,
+// 256^3 168 with 8 and 36.3 with 64.
+double step_estimate(const exaca::DomainView &d, int team) {
+    const double chain = team == 1 ? 3.0 : 7.0 + std::log2(static_cast<double>(team));
+    const double per_cell = 0.0075 + 0.0125 * std::min(1.0, static_cast<double>(d.ncell) / 1.6e7);
+    return chain + per_cell * static_cast<double>(d.X) * d.Y / team;
+}
+
+// The workgroups of a launch. A launch lasts as long as its slowest domain, and no less than all
+// domains' workgroup time over the device's CUs (a workgroup takes a CU; those that find none wait for
+// the domains before them to finish their steps). Every running domain starts with a team of one, and
+// the slowest one's team is doubled, up to the workgroups-per-slot setting, while CUs are spare and
+// it gains from it; beyond the CUs only while it would take half as long again as its share of them
+// (its larger team costs the others time). The largest teams come first, so that the small domains
+// fill in behind them. Measured, ms for all solves (at most 32 workgroups a slot) within the CUs only,
+// beyond them while the estimate of the launch falls, and by this rule: 256 domains of sides 32-256
+// 4892, 3016, 3491; 64 of 32-64 254, 267, 252; 16 of 64-192 303, 329, 302. (Every slot's row of the same
+// number of workgroups, with kernel boundaries between the passes: 5872, 1045, 738.)
+void share_out(exaca_ensemble *e) {
+    if (!e->dirty) return;
+    std::vector<std::pair<double, int>> running;  // estimate, slot
+    std::vector<int> team(e->slots, 0);
+    double area = 0;  // workgroup time of all
+    int total = 0;    // workgroups
+    for (int s = 0; s < e->slots; s++)
+        if (e->used[s] && e->status[s] == 0) {
+            team[s] = 1;
+            running.emplace_back(step_estimate(e->views[s], 1), s);
+            area += running.back().first;
+            total++;
+        }
+    const int most = std::min(e->blocks, exaca::kMaxTeam);
+    std::make_heap(running.begin(), running.end());
+    while (!running.empty()) {
+        std::pop_heap(running.begin(), running.end());
+        const auto [t, s] = running.back();
+        running.pop_back();
+        if (2 * team[s] > most) break;
+        const double less = step_estimate(e->views[s], 2 * team[s]);
+        const double grown = area + 2 * team[s] * less - team[s] * t;
+        if (less > 0.95 * t) break;  // the slowest domain gains nothing from more
+        if (total + team[s] > e->cus && t < 1.5 * grown / e->cus) break;
+        area = grown;
+        total += team[s];
+        team[s] *= 2;
+        running.emplace_back(less, s);
+        std::push_heap(running.begin(), running.end());
+    }
+    e->places.clear();
+    for (int nb = exaca::kMaxTeam; nb >= 1; nb /= 2)
+        for (int s = 0; s < e->slots; s++)
+            if (team[s] == nb)
+                for (int b = 0; b < nb; b++)
+                    e->places.push_back(exaca::TeamPlace{static_cast<uint32_t>(s), static_cast<uint32_t>(b),
+                                                         static_cast<uint32_t>(nb)});
+    if (!e->places.empty()) {
+        if (e->places.size() > e->places_cap) {
+            HIP_OK(hipStreamSynchronize(e->stream));
+            if (e->places_d) HIP_OK(hipFree(e->places_d));
+            e->places_d = nullptr;
+            e->places_cap = 0;
+            HIP_OK(hipMalloc(&e->places_d, sizeof(exaca::TeamPlace) * 2 * e->places.size()));
+            e->places_cap = 2 * e->places.size();
+        }
+        HIP_OK(hipMemcpyAsync(e->places_d, e->places.data(), sizeof(exaca::TeamPlace) * e->places.size(),
+                              hipMemcpyHostToDevice, e->stream));
+        HIP_OK(hipStreamSynchronize(e->stream));  // e->places may change
+    }
+    e->dirty = false;
+}
+
+// Enqueues `steps` steps (a multiple of kChunk) of every running domain.
+void launch(exaca_ensemble *e, int steps) {
+    share_out(e);
+    e->steps += steps;
+    if (e->places.empty()) return;
+    for (int n; steps > 0; steps -= n) {
+        n = std::min(steps, kMaxLaunch);
+        exaca::launch_steps_n(e->views_d, e->places_d, static_cast<uint32_t>(e->places.size()), n, 0, e->stream);
+        HIP_OK(hipGetLastError());
+    }
 }
 
 void admit(exaca_ensemble *e, const exaca_prepared *pr, int *slot_out) {
@@ -198,9 +277,9 @@ void admit(exaca_ensemble *e, const exaca_prepared *pr, int *slot_out) {
     d.yoff = hd.yoff;
     d.cells = reinterpret_cast<Cell *>(carve(sizeof(Cell) * n));
     d.octa = reinterpret_cast<Octa *>(carve(sizeof(Octa) * n));
-    d.claim_cell = reinterpret_cast<uint32_t *>(carve(4 * exaca::claim_entries(d, kMaxSlices)));
-    d.claim_bits = reinterpret_cast<uint32_t *>(carve(4 * exaca::claim_entries(d, kMaxSlices)));
-    d.claim_count = reinterpret_cast<uint32_t *>(carve(4 * kMaxSlices));
+    d.claim_cell = reinterpret_cast<uint32_t *>(carve(4 * exaca::claim_entries(d, exaca::kMaxTeam)));
+    d.claim_bits = reinterpret_cast<uint32_t *>(carve(4 * exaca::claim_entries(d, exaca::kMaxTeam)));
+    d.sync = reinterpret_cast<uint32_t *>(carve(4 * kMaxTeam));
     int32_t *nloc = reinterpret_cast<int32_t *>(carve(4 * std::max<size_t>(hd.nloc.size(), 1)));
     int32_t *ntime = reinterpret_cast<int32_t *>(carve(4 * std::max<size_t>(hd.nloc.size(), 1)));
     double *grow = reinterpret_cast<double *>(carve(8 * pr->grow.size()));
@@ -208,8 +287,8 @@ void admit(exaca_ensemble *e, const exaca_prepared *pr, int *slot_out) {
     d.alarms = reinterpret_cast<uint32_t *>(carve(4 * kAlarmSlots * alarm_stride(d.ncell)));
     d.ctl = reinterpret_cast<StepCtl *>(carve(sizeof(StepCtl)));
     d.stats = reinterpret_cast<StepStats *>(carve(sizeof(StepStats)));
-    d.nparts = kMaxSlices;
-    d.part = reinterpret_cast<unsigned long long *>(carve(8ull * kPartRows * kMaxSlices));
+    d.nparts = kMaxTeam;
+    d.part = reinterpret_cast<unsigned long long *>(carve(8ull * kPartRows * kMaxTeam));
     d.nnuclei = static_cast<int32_t>(loc.size());
     d.nloc = nloc;
     d.ntime = ntime;
@@ -237,7 +316,8 @@ void admit(exaca_ensemble *e, const exaca_prepared *pr, int *slot_out) {
     StepCtl c = exaca::initial_ctl(hd);
     HIP_OK(hipMemcpyAsync(d.ctl, &c, sizeof c, hipMemcpyHostToDevice, s));
     HIP_OK(hipMemsetAsync(d.stats, 0, sizeof(StepStats), s));
-    HIP_OK(hipMemsetAsync(d.part, 0, 8ull * kPartRows * kMaxSlices, s));
+    HIP_OK(hipMemsetAsync(d.part, 0, 8ull * kPartRows * kMaxTeam, s));
+    HIP_OK(hipMemsetAsync(d.sync, 0, 4 * kMaxTeam, s));
     const int32_t zero = 0;
     HIP_OK(hipMemcpyAsync(e->status_d + slot, &zero, 4, hipMemcpyHostToDevice, s));
     HIP_OK(hipMemcpyAsync(e->status_d + e->slots + slot, &zero, 4, hipMemcpyHostToDevice, s));
@@ -249,6 +329,7 @@ void admit(exaca_ensemble *e, const exaca_prepared *pr, int *slot_out) {
     e->used[slot] = 1;
     e->status[slot] = 0;
     e->status[e->slots + slot] = 0;
+    e->dirty = true;
     *slot_out = slot;
 }
 
@@ -262,14 +343,10 @@ void release(exaca_ensemble *e, int slot) {
     e->used[slot] = 0;
     e->status[slot] = -1;
     e->status[e->slots + slot] = 0;
+    e->dirty = true;
 }
 
-void advance(exaca_ensemble *e, int steps) {
-    const int chunks = (steps + kChunk - 1) / kChunk;
-    hipGraphExec_t g = graph_for(e, e->blocks);
-    for (int c = 0; c < chunks; c++) HIP_OK(hipGraphLaunch(g, e->stream));
-    e->steps += static_cast<long long>(chunks) * kChunk;
-}
+void advance(exaca_ensemble *e, int steps) { launch(e, (steps + kChunk - 1) / kChunk * kChunk); }
 
 void poll(exaca_ensemble *e) {
     HIP_OK(hipMemcpyAsync(e->status.data(), e->status_d, 8 * e->slots, hipMemcpyDeviceToHost, e->stream));
@@ -279,6 +356,8 @@ void poll(exaca_ensemble *e) {
             e->status[s] = -1;
             e->status[e->slots + s] = 0;
         }
+    for (const exaca::TeamPlace &p : e->places)
+        if (p.b == 0 && e->status[p.slot] != 0) e->dirty = true;  // finished: its workgroups serve the others
 }
 
 unsigned long long frontier_total(exaca_ensemble *e) {
@@ -351,6 +430,9 @@ int exaca_ensemble_create(int slots, size_t arena_bytes, exaca_ensemble **out) {
         HIP_OK(hipMemset(e->views_d, 0, sizeof(exaca::DomainView) * slots));
         HIP_OK(hipMalloc(&e->status_d, 8 * slots));
         HIP_OK(hipMemset(e->status_d, 0, 8 * slots));
+        int dev = 0;
+        HIP_OK(hipGetDevice(&dev));
+        HIP_OK(hipDeviceGetAttribute(&e->cus, hipDeviceAttributeMultiprocessorCount, dev));
         e->views.assign(slots, exaca::DomainView{});
         e->status.assign(2 * static_cast<size_t>(slots), -1);
         std::fill(e->status.begin() + slots, e->status.end(), 0);
@@ -393,8 +475,9 @@ int exaca_ensemble_poll(exaca_ensemble *e, int32_t *final_cycles, int32_t *error
 
 int exaca_ensemble_set_blocks(exaca_ensemble *e, int blocks) {
     return guarded([&] {
-        if (!e || blocks < 8 || blocks > kMaxSlices || blocks % 8) throw std::invalid_argument("bad workgroup count");
+        if (!e || blocks < 8 || blocks > kMaxBlocks || blocks % 8) throw std::invalid_argument("bad workgroup count");
         e->blocks = blocks;
+        e->dirty = true;
     });
 }
 
@@ -406,19 +489,20 @@ int exaca_ensemble_autotune(exaca_ensemble *e, int chunks_per_candidate, int *ch
         // device time per active-cell update.
         const int candidates[] = {16, 32, 64, 128, 256};
         double best = 1e300;
-        int best_b = e->blocks;
+        int best_b = candidates[0];
         hipEvent_t e0, e1;
         HIP_OK(hipEventCreate(&e0));
         HIP_OK(hipEventCreate(&e1));
         for (int b : candidates) {
-            hipGraphExec_t g = graph_for(e, b);
+            e->blocks = b;
+            e->dirty = true;
+            share_out(e);
             HIP_OK(hipStreamSynchronize(e->stream));
             const unsigned long long f0 = frontier_total(e);
             HIP_OK(hipEventRecord(e0, e->stream));
-            for (int c = 0; c < chunks_per_candidate; c++) HIP_OK(hipGraphLaunch(g, e->stream));
+            for (int c = 0; c < chunks_per_candidate; c++) launch(e, kChunk);
             HIP_OK(hipEventRecord(e1, e->stream));
             HIP_OK(hipEventSynchronize(e1));
-            e->steps += static_cast<long long>(chunks_per_candidate) * kChunk;
             float ms = 0;
             HIP_OK(hipEventElapsedTime(&ms, e0, e1));
             const unsigned long long f1 = frontier_total(e);
@@ -431,6 +515,7 @@ int exaca_ensemble_autotune(exaca_ensemble *e, int chunks_per_candidate, int *ch
         (void)hipEventDestroy(e0);
         (void)hipEventDestroy(e1);
         e->blocks = best_b;
+        e->dirty = true;
         *chosen = best_b;
     });
 }

@@ -155,14 +155,15 @@ int exaca_ensemble_create(int slots, size_t arena_bytes, exaca_ensemble **out);
 int exaca_ensemble_admit(exaca_ensemble *e, const exaca_prepared *pr, int *slot);
 /* Frees a slot and its memory. */
 int exaca_ensemble_release(exaca_ensemble *e, int slot);
-/* Enqueues `steps` more steps of every slot (rounded up to 50-step graph replays; asynchronous). */
+/* Enqueues `steps` more steps of every slot (rounded up to a multiple of 50; asynchronous). */
 int exaca_ensemble_advance(exaca_ensemble *e, int steps);
 /* Waits for the queued steps; final_cycles[slots] receives each slot's final cycle, 0 while it
  * runs, -1 when empty. errors[slots] (may be NULL) receives each slot's device error flags (the
  * flags of exaca_last_error's device messages; 0: none). A domain that raises one is stopped on
  * the device at the end of that step: its final cycle is then that step and its result is void. */
 int exaca_ensemble_poll(exaca_ensemble *e, int32_t *final_cycles, int32_t *errors);
-/* Workgroups per slot for the frontier kernels (multiple of 8, 8..256). */
+/* Workgroups per slot, at most (multiple of 8, 8..256; the device shares its compute units out among
+ * the running domains by their size). */
 int exaca_ensemble_set_blocks(exaca_ensemble *e, int blocks);
 /* Online autotuner: runs chunks_per_candidate chunks per workgroup-count candidate on the live
  * ensemble and keeps the one with the least device time per active-cell update. */
