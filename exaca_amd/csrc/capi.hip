@@ -271,8 +271,7 @@ void build_device_state(exaca_state *h) {
     h->ntime = h->alloc<int32_t>(hd.ntime.size());
     float *guv = h->alloc<float>(hd.guv.size());
     d.guv = guv;
-    std::vector<float> seed(static_cast<size_t>(kCdlStride) * kNumOrientations, 0.0f);
-    for (int o = 0; o < kNumOrientations; o++) seed_critical_lengths(&hd.guv[9 * o], &seed[kCdlStride * o]);
+    const std::vector<float> seed = seed_table(hd.guv, seed_rows(hd));
     float *seed_d = h->alloc<float>(seed.size());
     d.seed_cdl = seed_d;
     std::vector<double> grow = growth_table(hd.A, hd.B, hd.C, hd.D, hd.dU, 1 << 25);

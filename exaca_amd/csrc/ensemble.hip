@@ -155,8 +155,7 @@ void ensure_tables(exaca_ensemble *e, const exaca::HostDomain &h, const std::str
         return;
     }
     e->orientation_file = orientation_file;
-    std::vector<float> seed(static_cast<size_t>(kCdlStride) * kNumOrientations, 0.0f);
-    for (int o = 0; o < kNumOrientations; o++) seed_critical_lengths(&h.guv[9 * o], &seed[kCdlStride * o]);
+    const std::vector<float> seed = seed_table(h.guv, kNumOrientations);
     HIP_OK(hipMalloc(&e->guv, h.guv.size() * 4));
     HIP_OK(hipMalloc(&e->seed_cdl, seed.size() * 4));
     HIP_OK(hipMemcpy(e->guv, h.guv.data(), h.guv.size() * 4, hipMemcpyHostToDevice));

@@ -10,6 +10,7 @@
 #include <cmath>
 #include <cstdio>
 #include <cstdlib>
+#include <cstring>
 #include <fstream>
 #include <iostream>
 #include <random>
@@ -468,29 +469,100 @@ void nuclei(const Deck &d, HostDomain &h, const std::vector<uint32_t> &sites) {
 
 }  // namespace
 
+namespace {
+// std::atof of the text [b, e): a sign, up to 15 digits and a point are an integer below 2^53 over a
+// power of ten below 10^16, both exact, so their quotient is the correctly rounded value; anything
+// else goes through atof itself. (10 ns a value; atof on a string of its own takes 100.)
+double decimal(const char *b, const char *e) {
+    static constexpr double kTen[16] = {1e0, 1e1, 1e2, 1e3, 1e4, 1e5, 1e6, 1e7, 1e8, 1e9, 1e10, 1e11, 1e12, 1e13, 1e14, 1e15};
+    const char *p = b;
+    const bool minus = p < e && *p == '-';
+    p += minus;
+    uint64_t digits = 0;
+    int n = 0, frac = -1;
+    for (; p < e; p++) {
+        if (*p >= '0' && *p <= '9') {
+            digits = 10 * digits + static_cast<uint64_t>(*p - '0');
+            n++;
+            frac += frac >= 0;
+        }
+        else if (*p == '.' && frac < 0)
+            frac = 0;
+        else
+            break;
+        if (n > 15) break;
+    }
+    if (p == e && n > 0 && n <= 15) {
+        const double v = static_cast<double>(digits) / kTen[frac > 0 ? frac : 0];
+        return minus ? -v : v;
+    }
+    return std::atof(std::string(b, e).c_str());
+}
+}  // namespace
+
 std::vector<float> read_orientations(const std::string &path) {
     std::vector<float> guv(9 * kNumOrientations, 0.0f);
-    std::ifstream in(path);
+    std::ifstream in(path, std::ios::binary);
     if (!in.is_open()) throw std::runtime_error("Could not locate/open Substrate file");
-    std::string line;
-    std::getline(in, line);
-    for (int i = 0; i < kNumOrientations; i++) {
-        if (!std::getline(in, line)) break;
-        std::istringstream ss(line);
-        std::string tok;
-        int slot = 0;
-        while (slot < 9 && std::getline(ss, tok, ',')) guv[9 * i + slot++] = static_cast<float>(std::atof(tok.c_str()));
+    in.seekg(0, std::ios::end);
+    const std::streamoff size = in.tellg();
+    std::string text(size > 0 ? static_cast<size_t>(size) : 0, '\0');
+    in.seekg(0);
+    in.read(&text[0], static_cast<std::streamsize>(text.size()));
+    const char *p = text.data(), *end = p + std::max<std::streamsize>(in.gcount(), 0);
+    auto line_end = [&] {
+        const void *q = p < end ? std::memchr(p, '\n', static_cast<size_t>(end - p)) : nullptr;
+        return q ? static_cast<const char *>(q) : end;
+    };
+    p = std::min(line_end() + 1, end);  // the number of orientations
+    for (int i = 0; i < kNumOrientations && p < end; i++) {
+        const char *le = line_end();
+        for (int slot = 0; slot < 9 && p < le; slot++) {
+            const void *q = std::memchr(p, ',', static_cast<size_t>(le - p));
+            const char *te = q ? static_cast<const char *>(q) : le;
+            // a carriage return before the line's end ends the number, as atof would take it
+            const char *ve = te > p && te == le && te[-1] == '\r' ? te - 1 : te;
+            guv[9 * i + slot] = static_cast<float>(decimal(p, ve));
+            p = std::min(te + 1, le);
+        }
+        p = std::min(le + 1, end);
     }
     return guv;
+}
+
+std::vector<float> seed_table(const std::vector<float> &guv, int rows) {
+    std::vector<float> t(static_cast<size_t>(kCdlStride) * rows, 0.0f);
+    auto some = [&](int a, int b) {
+        for (int o = a; o < b; o++) seed_critical_lengths(&guv[9 * o], &t[static_cast<size_t>(kCdlStride) * o]);
+    };
+    const int n = std::min<int>(8, std::max(1, std::min<int>(rows / 1000, std::thread::hardware_concurrency())));
+    std::vector<std::thread> th;
+    try {
+        for (int k = 1; k < n; k++) th.emplace_back(some, rows / n * k, k + 1 < n ? rows / n * (k + 1) : rows);
+    }
+    catch (...) {  // no more threads: the rest here
+    }
+    some(0, n > 1 ? rows / n : rows);
+    for (int k = static_cast<int>(th.size()) + 1; k < n; k++) some(rows / n * k, k + 1 < n ? rows / n * (k + 1) : rows);
+    for (std::thread &x : th) x.join();
+    return t;
+}
+
+int seed_rows(const HostDomain &h) {
+    int most = 0;  // the greatest |GrainID|
+    if (h.sparse)
+        most = static_cast<int>(std::min<size_t>(std::max(h.active.size(), h.nloc.size()), kNumOrientations));
+    for (int32_t g : h.gid) most = std::max(most, std::abs(g));
+    return std::max(1, std::min(most, kNumOrientations));
 }
 
 void seed_critical_lengths(const float *g, float out[26]) {
     for (int n = 0; n < 26; n++) {
         const double x0 = kNbX[n], y0 = kNbY[n], z0 = kNbZ[n];
-        const double mag0 = std::pow(std::pow(x0, 2.0) + std::pow(y0, 2.0) + std::pow(z0, 2.0), 0.5);
         double diag[3][3];
         for (int a = 0; a < 3; a++) {
-            const double ang = (g[3 * a] * x0 + g[3 * a + 1] * y0 + g[3 * a + 2] * z0) / mag0;
+            // the reference divides by the neighbour's distance; only the sign is used
+            const double ang = g[3 * a] * x0 + g[3 * a + 1] * y0 + g[3 * a + 2] * z0;
             for (int c = 0; c < 3; c++) diag[a][c] = (ang < 0) ? g[3 * a + c] : -g[3 * a + c];
         }
         const double u1[3] = {diag[1][0] - diag[0][0], diag[1][1] - diag[0][1], diag[1][2] - diag[0][2]};

@@ -76,6 +76,11 @@ HostDomain initialize_sparse(const Deck &deck, bool verbose);
 // (src/CAupdate.cpp:112-194), evaluated with the host libm exactly as the reference does.
 void seed_critical_lengths(const float *guv9, float out26[26]);
 
+// The table of them by orientation, rows of kCdlStride floats, for the first `rows` orientations; and the
+// orientations that a grain of the domain can have (a cell-centred octahedron belongs to a grain).
+std::vector<float> seed_table(const std::vector<float> &guv, int rows);
+int seed_rows(const HostDomain &h);
+
 // Growth increment per step after k executed steps below the liquidus, k = 0 .. n-1; the last
 // entry is the saturated value (undercooling clamped at 210 K or no longer increasing).
 std::vector<double> growth_table(double A, double B, double C, double D, float dU, int max_entries);
