@@ -414,17 +414,15 @@ struct Growth {
 __device__ __forceinline__ Growth growth_of(const DomainView &d) {
     return Growth{d.grow, d.grow_sums, nullptr, d.ksat, 0, d.grow[d.ngrow - 1], d.sums_usable};
 }
-// The same with as many rows of the sums as fit copied to the workgroup's LDS buffer of N entries.
-// Every thread of the workgroup calls it.
+// Copies as many rows of the sums as fit to the workgroup's LDS buffer of N entries. Every thread of the
+// workgroup calls it.
 template <int BLOCK, int N>
-__device__ __forceinline__ Growth staged_growth(const DomainView &d, uint32_t (&lds)[N]) {
-    Growth g = growth_of(d);
+__device__ __forceinline__ void stage_sums(const DomainView &d, Growth &g, uint32_t (&lds)[N]) {
     const int len = d.ksat + 2;
     g.staged = (const __attribute__((address_space(3))) uint32_t *)lds;
     g.nstaged = N / len < kSumRows ? N / len : kSumRows;
     for (int i = threadIdx.x; i < g.nstaged * len; i += BLOCK) lds[i] = d.grow_sums[i];
     __syncthreads();
-    return g;
 }
 
 // dl after the growth of the steps with index k0+1 .. k1, one float rounding per step exactly as
@@ -902,12 +900,12 @@ struct Capture {
 // LDS of pass B.
 template <int BLOCK>
 struct ApplyLds {
-    uint32_t cell[2 * BLOCK], bits[2 * BLOCK];  // winners and the claims they won
-    int32_t gid[2 * BLOCK];
-    uint32_t item[BLOCK];  // winner << 5 | neighbour of each capture of a turn
+    // captures to make: the winner, its grain, and the neighbour of it that it captures
+    uint32_t from[BLOCK];
+    int32_t gid[BLOCK];
+    uint8_t which[BLOCK];
     Capture made[BLOCK];
-    uint32_t tot[BLOCK / 64];
-    uint32_t nwin;
+    uint32_t n;
 };
 
 // The octahedron of the winner jc's capture of its neighbour l (src/CAupdate.cpp:353-515).
@@ -1026,9 +1024,8 @@ __device__ __forceinline__ void widen_range(const DomainView &d, uint32_t *lohi,
 }
 
 // Pass B over the claimants that claimant(k, cell, bits) gives. A claim whose word holds the claimant's
-// own index is won (the lowest index that reached the cell). The winners of up to two rounds are
-// gathered in LDS with the claims they won and their captures numbered by a block scan (a winner mostly
-// has one). A capture's octahedron is built by one lane; its neighbours are then visited by the 26
+// own index is won (the lowest index that reached the cell). The captures won are gathered in LDS over
+// as many rounds as fit. A capture's octahedron is built by one lane; its neighbours are then visited by the 26
 // lanes of a half-wave, so that the words of three consecutive neighbours are read together, its
 // lengths are one store of one line, and its chain is one length and one mask long instead of 26.
 // One lane per capture took 242 registers (two waves a SIMD) and about 10 000 cycles for one
@@ -1037,10 +1034,9 @@ __device__ __forceinline__ void widen_range(const DomainView &d, uint32_t *lohi,
 template <int BLOCK, typename F>
 __device__ __forceinline__ void apply_body(const DomainView &d, const Grid &gr, uint32_t serial, uint32_t nclaimants,
                                            F &&claimant, ApplyLds<BLOCK> &s, uint32_t *cnt, NewCells &made) {
-    constexpr uint32_t kWaves = BLOCK / 64;
-    const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const uint32_t lane = threadIdx.x & 63;
     const NeighbourLane n = neighbour_lane(gr);
-    if (threadIdx.x == 0) s.nwin = 0;
+    if (threadIdx.x == 0) s.n = 0;
     __syncthreads();
     for (uint32_t k0 = 0; k0 < nclaimants; k0 += BLOCK) {
         const uint32_t k = k0 + threadIdx.x;
@@ -1062,76 +1058,59 @@ __device__ __forceinline__ void apply_body(const DomainView &d, const Grid &gr, 
                 for (int e = 0; e < 4; e++) won |= cw[e] == j ? bit[e] : 0u;
             }
         }
-        const uint32_t slot = wave_append(won != 0, &s.nwin);
-        if (won) {
-            s.cell[slot] = j;
-            s.bits[slot] = won;
-            s.gid[slot] = gid;
-        }
-        __syncthreads();
-        const uint32_t nwin = s.nwin;
-        __syncthreads();
-        if (k0 + BLOCK < nclaimants && nwin <= BLOCK) continue;  // room for another round
-        // the captures of the winners gathered so far: thread t numbers those of winners 2t, 2t + 1
-        const uint32_t w0 = 2 * threadIdx.x;
-        const uint32_t b0 = w0 < nwin ? s.bits[w0] : 0u, b1 = w0 + 1 < nwin ? s.bits[w0 + 1] : 0u;
-        const uint32_t c0 = __builtin_popcount(b0), mine = c0 + __builtin_popcount(b1);
-        uint32_t wtot;
-        const uint32_t incl = wave_inclusive_scan(mine, wtot);
-        if (lane == 0) s.tot[wave] = wtot;
-        __syncthreads();
-        uint32_t first = incl - mine, total = 0;
-#pragma unroll
-        for (uint32_t q = 0; q < kWaves; q++) {
-            const uint32_t v = s.tot[q];
-            first += q < wave ? v : 0u;
-            total += v;
-        }
-        for (uint32_t t0 = 0; t0 < total; t0 += BLOCK) {
-            uint32_t pos = first - t0;  // wraps below the turn: not in [0, BLOCK)
-            for (uint32_t m = b0; m; m &= m - 1, pos++)
-                if (pos < BLOCK) s.item[pos] = (w0 << 5) | static_cast<uint32_t>(__builtin_ctz(m));
-            for (uint32_t m = b1; m; m &= m - 1, pos++)
-                if (pos < BLOCK) s.item[pos] = ((w0 + 1) << 5) | static_cast<uint32_t>(__builtin_ctz(m));
+        // the captures won go to the list; those that no longer fit wait until it is empty again
+        for (bool all = false; !all;) {
+            uint32_t wtot, base = 0;
+            const uint32_t c = __builtin_popcount(won), incl = wave_inclusive_scan(c, wtot);
+            if (lane == 63 && wtot) base = atomicAdd(&s.n, wtot);
+            uint32_t pos = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(base), 63)) + incl - c;
+            for (; won && pos < BLOCK; won &= won - 1, pos++) {
+                s.from[pos] = j;
+                s.gid[pos] = gid;
+                s.which[pos] = static_cast<uint8_t>(__builtin_ctz(won));
+            }
             __syncthreads();
-            const uint32_t turn = total - t0 < BLOCK ? total - t0 : BLOCK;
+            const uint32_t total = s.n;
+            all = total <= BLOCK;
+            const uint32_t turn = all ? total : BLOCK;
+            __syncthreads();
+            if (all && k0 + BLOCK < nclaimants) continue;  // with the next round's
             // the neighbours' words of a half-wave's first capture are on their way while the octahedra
             // are built, and those of its next one while it places one
             uint32_t i = threadIdx.x >> 5;
-            Coord c{};
+            Coord at{};
             bool valid = false;
             unsigned long long word = 0;
             auto fetch = [&]() {
                 if (i >= turn) return;
-                const uint32_t it = s.item[i];
-                const uint32_t q = s.cell[it >> 5] + gr.offset(static_cast<int>(it & 31u));
-                c = decode(q, gr);
-                valid = has_neighbour(d, n, c);
-                const unsigned long long *at = &d.cells[n.l < 26 ? q + n.off : q].lm + (n.l < 26 ? 0 : n.l - 24);
-                if (valid || n.l == 26 || n.l == 27) word = *at;
+                const uint32_t q = s.from[i] + gr.offset(static_cast<int>(s.which[i]));
+                at = decode(q, gr);
+                valid = has_neighbour(d, n, at);
+                const unsigned long long *p = &d.cells[n.l < 26 ? q + n.off : q].lm + (n.l < 26 ? 0 : n.l - 24);
+                if (valid || n.l == 26 || n.l == 27) word = *p;
             };
             fetch();
-            if (threadIdx.x < turn) {
-                const uint32_t it = s.item[threadIdx.x];
-                build_capture(d, gr, s.cell[it >> 5], static_cast<int>(it & 31u), s.gid[it >> 5], s.made[threadIdx.x]);
+            if (threadIdx.x < turn)
+                build_capture(d, gr, s.from[threadIdx.x], static_cast<int>(s.which[threadIdx.x]), s.gid[threadIdx.x],
+                              s.made[threadIdx.x]);
+            if (threadIdx.x == 0) {
+                cnt[kCntCap] += turn;
+                s.n = 0;
             }
-            if (threadIdx.x == 0) cnt[kCntCap] += turn;
             __syncthreads();
             while (i < turn) {
                 const Capture &m = s.made[i];
-                const Coord at = c;
+                const Coord c0 = at;
                 const bool ok = valid;
                 const unsigned long long w = word;
                 made.lo = m.q < made.lo ? m.q : made.lo;
                 made.hi = m.q > made.hi ? m.q : made.hi;
                 i += BLOCK / 32;
                 fetch();
-                place_capture(d, n, serial, m, at, ok, w);
+                place_capture(d, n, serial, m, c0, ok, w);
             }
             __syncthreads();
         }
-        if (threadIdx.x == 0) s.nwin = 0;
-        __syncthreads();
     }
 }
 
@@ -1339,7 +1318,8 @@ __device__ __forceinline__ void claim_step(const DomainView &d, int p, uint32_t 
     if (ctl->done) return;
     if (threadIdx.x == 0) nclaim = 0;
     clear_tally(t);
-    const Growth g = staged_growth<kBlock>(d, gsums);
+    Growth g = growth_of(d);
+    stage_sums<kBlock>(d, g, gsums);
     const int cycle = ctl->cycle[p];
     const uint32_t serial = ctl->serial[p];
     if (b == 0 && threadIdx.x == 0) {
@@ -1466,7 +1446,9 @@ __device__ __forceinline__ void steps_body(const DomainView &d, int p, int layer
     bool follows = follows_last(ctl, cycle);
     int site = max(ctl->nuc_at, ctl->nuc_next);
     int next_site = nucleate && site < d.nnuclei ? d.ntime[site] : 0x7FFFFFFF;
-    const Growth g = staged_growth<kTeamBlock>(d, s.sums);
+    // a launch of a few steps would not earn back what it stages
+    Growth g = growth_of(d);
+    if (nsteps >= 8) stage_sums<kTeamBlock>(d, g, s.sums);
     const uint32_t region = place_of(b, nb) * claim_region(d, nb);
     const bool whole = scans_all<kTeamBlock>(d, nb);
     const Grid gr = grid_of(d);

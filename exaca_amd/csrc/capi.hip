@@ -1,5 +1,5 @@
 // capi.hip -- the C ABI (include/exaca_ca.h): device state of one CA domain, the per-step entry
-// points, the device-resident layer loop replayed from HIP graphs, and the RunProgram_Reduced
+// points, the device-resident layer loop, and the RunProgram_Reduced
 // drop-in.
 #include <hip/hip_runtime.h>
 
@@ -141,7 +141,6 @@ using exaca::StateError;
 using exaca::guarded;
 using exaca::g_last_error;
 
-constexpr int kGraphSteps = 50;  // even: a graph starts and ends on parity 0
 
 }  // namespace
 
@@ -161,9 +160,6 @@ struct exaca_state {
     int blocks = 2048;     // workgroups of the frontier kernels
     int team = 0;          // workgroups of the resident kernel that runs many steps (0: two launches a step)
     int njumps = 0;
-    hipGraphExec_t graph = nullptr;       // kGraphSteps steps
-    hipGraphExec_t graph_quiet = nullptr; // the same without the nucleation kernels
-    int graph_layer = -1;
     // The layer's nucleation times in ascending order, and the last step whose nucleation kernel
     // ran: a step may leave the kernel out when no time falls after that step and up to it (every
     // site of a time at or before a step where the kernel ran is decided there).
@@ -187,8 +183,6 @@ struct exaca_state {
         return static_cast<T *>(p);
     }
     ~exaca_state() {
-        if (graph) (void)hipGraphExecDestroy(graph);
-        if (graph_quiet) (void)hipGraphExecDestroy(graph_quiet);
         for (void *p : buffers) (void)hipFree(p);
         if (stream) (void)hipStreamDestroy(stream);
     }
@@ -361,11 +355,6 @@ void next_layer(exaca_state *h, int layer_done, int verbose) {
     }
     h->dv.zlo = zlo;
     h->dv.nzA = zhigh + 1;
-    for (hipGraphExec_t *ge : {&h->graph, &h->graph_quiet})  // they hold the old window in their arguments
-        if (*ge) {
-            HIP_OK(hipGraphExecDestroy(*ge));
-            *ge = nullptr;
-        }
     // the layer's record, the new layer's first cycle, and fresh counts of the active cells
     StepCtl *c = h->ctl;
     const int32_t end = h->cycle, j0 = h->njumps, layer = layer_done + 1, one = 1, zero = 0;
@@ -392,9 +381,6 @@ void next_layer(exaca_state *h, int layer_done, int verbose) {
     h->cycle = 0;
 }
 
-void step_nucleation(exaca_state *h, int layer) {
-    exaca::launch_nucleation(h->dv, h->parity, layer, h->stream);
-}
 void step_capture(exaca_state *h) {
     exaca::launch_capture(h->dv, h->parity, h->blocks, h->stream);
 }
@@ -403,36 +389,19 @@ void finish_steps(exaca_state *h) {
     exaca::launch_settle(h->dv, h->parity, h->blocks, h->stream);
     HIP_OK(hipGetLastError());
 }
-// Whether steps h->cycle + 1 .. last need the nucleation kernel.
-bool nucleation_due(const exaca_state *h, int last) {
-    if (!h->nuc_skip) return true;
+// The nucleation of the step at `cycle`, where a site is due.
+void step_nucleation(exaca_state *h, int layer, int cycle) {
     const auto it = std::upper_bound(h->nuc_times.begin(), h->nuc_times.end(), h->nuc_through);
-    return it != h->nuc_times.end() && *it <= last;
+    if (h->nuc_skip && (it == h->nuc_times.end() || *it > cycle)) return;
+    exaca::launch_nucleation(h->dv, h->parity, layer, h->stream);
+    h->nuc_through = cycle;
 }
 
-void ensure_graph(exaca_state *h, int layer) {
-    if (h->graph && h->graph_layer == layer) return;
-    for (hipGraphExec_t *ge : {&h->graph, &h->graph_quiet})
-        if (*ge) {
-            HIP_OK(hipGraphExecDestroy(*ge));
-            *ge = nullptr;
-        }
-    for (bool nucleate : {true, false}) {
-        hipGraph_t g;
-        HIP_OK(hipStreamBeginCapture(h->stream, hipStreamCaptureModeThreadLocal));
-        for (int k = 0; k < kGraphSteps; k++) {
-            const int p = k & 1;
-            if (nucleate) exaca::launch_nucleation(h->dv, p, layer, h->stream);
-            exaca::launch_capture(h->dv, p, h->blocks, h->stream);
-        }
-        HIP_OK(hipStreamEndCapture(h->stream, &g));
-        HIP_OK(hipGraphInstantiate(nucleate ? &h->graph : &h->graph_quiet, g, nullptr, nullptr, 0));
-        HIP_OK(hipGraphDestroy(g));
-    }
-    h->graph_layer = layer;
-}
-
-void run_steps(exaca_state *h, int layer, int n, bool use_graph) {
+// n steps: a team's in one launch; else each step's own launches, the nucleation kernel only where a
+// site is due. (Replays of captured 50-step graphs run that kernel on every step of a graph with one
+// site due: 31.2 us a step at 256^3 against 30.1, 43.0 against 41.7 at 400^3, 114 against 112 at 800^3,
+// cycles 1-3000.)
+void run_steps(exaca_state *h, int layer, int n) {
     if (n <= 0) return;
     if (h->team) {
         exaca::launch_steps(h->dv, h->parity, layer, n, true, h->team, h->stream);
@@ -442,27 +411,11 @@ void run_steps(exaca_state *h, int layer, int n, bool use_graph) {
         h->nuc_through = h->cycle;
         return;
     }
-    while (n > 0) {
-        if (use_graph && h->parity == 0 && n >= kGraphSteps) {
-            ensure_graph(h, layer);
-            const int last = h->cycle + kGraphSteps;
-            const bool nucleate = nucleation_due(h, last);
-            HIP_OK(hipGraphLaunch(nucleate ? h->graph : h->graph_quiet, h->stream));
-            if (nucleate) h->nuc_through = last;
-            h->cycle = last;
-            n -= kGraphSteps;
-        }
-        else {
-            const bool nucleate = nucleation_due(h, h->cycle + 1);
-            if (nucleate) {
-                step_nucleation(h, layer);
-                h->nuc_through = h->cycle + 1;
-            }
-            step_capture(h);
-            h->parity ^= 1;
-            h->cycle += 1;
-            n -= 1;
-        }
+    for (; n > 0; n--) {
+        step_nucleation(h, layer, h->cycle + 1);
+        step_capture(h);
+        h->parity ^= 1;
+        h->cycle += 1;
     }
     finish_steps(h);
 }
@@ -517,7 +470,6 @@ void run_layer(exaca_state *h, int layer, int max_cycles, int verbose, int *out_
     if (h->pending >= 0) throw StateError("run_layer called between nucleation and capture");
     if (layer != h->layer) throw StateError("layer " + std::to_string(layer) + " is not the current layer " +
                                             std::to_string(h->layer) + " (exaca_next_layer moves on)");
-    const bool graphs = std::getenv("EXACA_NO_GRAPHS") == nullptr;
     hipEvent_t e0, e1;
     HIP_OK(hipEventCreate(&e0));
     HIP_OK(hipEventCreate(&e1));
@@ -526,7 +478,7 @@ void run_layer(exaca_state *h, int layer, int max_cycles, int verbose, int *out_
     do {
         int target = (h->cycle / 1000 + 1) * 1000;
         if (max_cycles > 0 && target > max_cycles) target = max_cycles;
-        run_steps(h, layer, target - h->cycle, graphs);
+        run_steps(h, layer, target - h->cycle);
         if (h->cycle % 1000 == 0) {
             int c = h->cycle;
             device_check(h, &c, layer, nullptr, &xswitch, verbose);
@@ -777,10 +729,9 @@ void nucleation_call(exaca_state *h, int cycle, int layer) {
     if (h->pending >= 0) throw StateError("nucleation called twice without capture");
     if (layer != h->layer) throw StateError("layer " + std::to_string(layer) + " is not the current layer");
     set_next_cycle(h, cycle);
-    step_nucleation(h, layer);
+    step_nucleation(h, layer, cycle);
     HIP_OK(hipGetLastError());
     h->pending = cycle;
-    h->nuc_through = cycle;
 }
 
 int exaca_nucleation(exaca_state *h, int cycle, int layer) {

@@ -77,7 +77,7 @@ int exaca_cell_capture(exaca_state *h, int cycle, int layer);
 int exaca_check(exaca_state *h, int *cycle, int layer, uint64_t counts[5], int *xswitch, int verbose);
 
 /* The layer's do-while loop of RunProgram_Reduced (src/runCA.cpp:290-342) on the device:
- * Nucleation + CellCapture every step (replayed from captured HIP graphs), the check every 1000
+ * Nucleation + CellCapture every step (small domains many steps in one launch), the check every 1000
  * steps. Stops at completion or after max_cycles steps (<= 0: no limit). *cycle receives the
  * final cycle; *gpu_ms (may be NULL) the device time of the loop. */
 int exaca_run_layer(exaca_state *h, int layer, int max_cycles, int verbose, int *cycle, double *gpu_ms);
@@ -179,7 +179,7 @@ int exaca_ensemble_destroy(exaca_ensemble *e);
 const char *exaca_last_error(void);
 
 /* Timed stepping (no reference counterpart): runs nsteps further steps of `layer` like
- * exaca_run_layer, without graphs, with HIP events on the handle's stream around every kernel.
+ * exaca_run_layer, one kernel after another, with HIP events on the handle's stream around every kernel.
  * ms[0..2] receive the summed device time of the nucleation, claim and apply kernels; counts
  * [0..4] the frontier-size sum, captures, solidifications, kernel launches per kind and the number
  * of steps executed (checks and cycle jumps are applied as in exaca_run_layer). */
