@@ -186,11 +186,12 @@ enum StepCount : int {
     kCntMask,  // liquid masks built
     kStepCounts
 };
-// Running counters since the last booking, one slot per workgroup (part[row * nparts + workgroup]), two
-// rows per kind of event: their number, and the sum of the serials of their steps. Every workgroup
-// adds to its own slot, and the booking sums the rows. Same-address atomics from thousands of
-// workgroups would serialise.
+// Running counters since the last booking, a 128-byte line per workgroup (part[workgroup * kPartRows +
+// row]), two rows per kind of event: their number, and the sum of the serials of their steps. Every
+// workgroup adds to its own line, and the booking sums them. Same-address atomics from thousands of
+// workgroups would serialise, and stores to one line from several XCDs take as long.
 constexpr int kPartRows = 2 * kStepCounts;
+constexpr uint32_t kCountStride = 32;  // words between the workgroups' claim counts: a line each
 
 // Unsigned division by a constant of the domain as a multiply-high and shifts (the round-up method;
 // exact for every 32-bit dividend). Made on the host: its two 64-bit divisions take a wave a
@@ -231,7 +232,7 @@ struct DomainView {
     Octa *octa;             // octahedron records (centre, critical lengths)
     uint32_t *claim_cell;   // cells with claims in the current step, each capture-pass workgroup's in
     uint32_t *claim_bits;   //   a region of its own, and the neighbours each claimed
-    uint32_t *claim_count;  // entries of each workgroup's region
+    uint32_t *claim_count;  // entries of each workgroup's region, kCountStride apart
     int32_t nnuclei;
     const int32_t *nloc;    // the layer's nucleation sites in ascending order of their times
     const int32_t *ntime;   // NucleationTimes
@@ -241,12 +242,13 @@ struct DomainView {
     const double *grow;     // growth increment after k executed steps below the liquidus
     const uint32_t *grow_sums;  // rows of sums of the increments' deltas (growth_sums), of ksat + 2 entries
     uint32_t sums_usable;   // the rows that hold
-    int32_t ngrow;          // table length; the last entry holds for every larger k
+    double gsat;            // the last entry, which holds for every larger k
+    int32_t layer, jump0, njumps;  // the layer being solidified, its first cycle jump and the jumps so far
     int32_t ksat;           // from this k on every increment is the last entry (the 0.045 cap or the
                             // 210 K saturation)
     StepCtl *ctl;
     StepStats *stats;
-    unsigned long long *part;  // kPartRows x nparts per-workgroup counters
+    unsigned long long *part;  // nparts x kPartRows per-workgroup counters
     uint32_t nparts;
     uint32_t *alarms;       // kAlarmSlots bitmaps of one bit per cell: process the cell at the step
                             // whose serial is the bitmap's slot (mod kAlarmSlots)

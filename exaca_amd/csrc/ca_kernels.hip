@@ -367,14 +367,11 @@ __device__ __forceinline__ bool is_unclaimed_liquid(unsigned long long lm) {
 // (pass 1 visits the window only and accumulates only while LayerID <= layer, and the undercooling
 // is never reset between layers; src/CAupdate.cpp:217-237, src/runCA.cpp:283-418). 0 while the cell
 // waits for its liquidus time or its layer.
-// The layer and its cycle jumps, read once.
+// The layer and its cycle jumps.
 struct LayerAt {
     int layer, j0, j1;
 };
-__device__ __forceinline__ LayerAt layer_at(const StepCtl *c) {
-    const int L = c->layer;
-    return LayerAt{L, c->layer_jump0[L], c->njumps};
-}
+__device__ __forceinline__ LayerAt layer_at(const DomainView &d) { return LayerAt{d.layer, d.jump0, d.njumps}; }
 __device__ __forceinline__ int growth_index(const DomainView &d, const LayerAt &at, int cts, int lid, uint32_t q, int cycle) {
     const StepCtl *c = d.ctl;
     if (lid > at.layer) return 0;
@@ -412,7 +409,7 @@ struct Growth {
     }
 };
 __device__ __forceinline__ Growth growth_of(const DomainView &d) {
-    return Growth{d.grow, d.grow_sums, nullptr, d.ksat, 0, d.grow[d.ngrow - 1], d.sums_usable};
+    return Growth{d.grow, d.grow_sums, nullptr, d.ksat, 0, d.gsat, d.sums_usable};
 }
 // Copies as many rows of the sums as fit to the workgroup's LDS buffer of N entries. Every thread of the
 // workgroup calls it.
@@ -421,7 +418,11 @@ __device__ __forceinline__ void stage_sums(const DomainView &d, Growth &g, uint3
     const int len = d.ksat + 2;
     g.staged = (const __attribute__((address_space(3))) uint32_t *)lds;
     g.nstaged = N / len < kSumRows ? N / len : kSumRows;
-    for (int i = threadIdx.x; i < g.nstaged * len; i += BLOCK) lds[i] = d.grow_sums[i];
+    const int n = g.nstaged * len;
+    const uint4 *src = reinterpret_cast<const uint4 *>(d.grow_sums);
+    uint4 *dst = reinterpret_cast<uint4 *>(lds);
+    for (int i = threadIdx.x; i < n / 4; i += BLOCK) dst[i] = src[i];
+    for (int i = n / 4 * 4 + threadIdx.x; i < n; i += BLOCK) lds[i] = d.grow_sums[i];
     __syncthreads();
 }
 
@@ -466,8 +467,10 @@ struct Tally {
     // to workgroup b's running totals
     __device__ __forceinline__ void put(const DomainView &d, uint32_t b) {
         if (threadIdx.x >= kStepCounts || !n) return;
-        d.part[static_cast<size_t>(2 * threadIdx.x) * d.nparts + b] += n;
-        d.part[static_cast<size_t>(2 * threadIdx.x + 1) * d.nparts + b] += at;
+        // (an atomic, though nothing else writes the line: it need not wait for the old value)
+        unsigned long long *p = d.part + static_cast<size_t>(b) * kPartRows + 2 * threadIdx.x;
+        atomicAdd(p, n);
+        atomicAdd(p + 1, at);
         n = at = 0;
     }
 };
@@ -558,7 +561,7 @@ __device__ __forceinline__ int nucleate_body(const DomainView &d, int cycle, uin
                     const CellWords w = load_cell(d.cells + r);
                     if ((w.ct & kTypeMask) != kActive || !(cycle > w.cts && w.lid <= layer)) continue;
                     if (!(w.flags & kCounted)) nent++;
-                    solidify(d, growth_of(d), r, w, growth_index(d, layer_at(d.ctl), w.cts, w.lid, r, cycle));
+                    solidify(d, growth_of(d), r, w, growth_index(d, layer_at(d), w.cts, w.lid, r, cycle));
                     d.cells[r].flags = (w.flags & ~kFresh) | kCounted;
                     nsol++;
                 }
@@ -677,10 +680,12 @@ __device__ __forceinline__ uint32_t claim_region(const DomainView &d, uint32_t n
 // BLOCK cells at a time in a uniform loop (has: the lane has one). The due cells are gathered in LDS
 // (`list`, CAP entries) over as many rounds of units as fit and then processed together, so that the
 // lanes are full; a round that does not fit is read again for the rest. With CLEAR the bits of a
-// finished round are cleared for the slot's next use, 64 steps on.
-template <int BLOCK, uint32_t CAP, bool CLEAR, typename F>
+// finished round are cleared for the slot's next use, 64 steps on. meanwhile() is called, by every
+// thread, while the first words are on their way; false: there is nothing to do after all.
+template <int BLOCK, uint32_t CAP, bool CLEAR, typename G, typename F>
 __device__ __forceinline__ void for_due(const DomainView &d, uint32_t serial, uint32_t b, uint32_t nb, uint32_t *list,
-                                        uint32_t *tot, F &&visit) {
+                                        uint32_t *tot, G &&meanwhile, F &&visit) {
+    bool first_words = true;
     constexpr uint32_t kWaves = BLOCK / 64;
     const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const UnitRange r = unit_range<BLOCK>(d, nb);
@@ -699,6 +704,8 @@ __device__ __forceinline__ void for_due(const DomainView &d, uint32_t serial, ui
             w[e] = 0;
             if (e < turns) w[e] = bits[word(e) < end ? word(e) : end - 1];
         }
+        if (first_words && !meanwhile()) return;
+        first_words = false;
 #pragma unroll
         for (uint32_t e = 0; e < kUnitsPerLane; e++) {
             w[e] = word(e) < end ? w[e] : 0u;
@@ -799,12 +806,13 @@ __device__ __forceinline__ uint32_t liquid_neighbours(const DomainView &d, const
 // neighbour's capture or nucleation empties its mask. A new active cell starts at thr = 0.
 // Cells with claims are numbered by an LDS counter (no global atomics) and handed to put(number, cell,
 // claimed neighbours).
-template <int BLOCK, uint32_t CAP, typename F>
+template <int BLOCK, uint32_t CAP, typename G, typename F>
 __device__ __forceinline__ void claim_body(const DomainView &d, const Grid &gr, const Growth &g, const LayerAt &at,
                                            int cycle, uint32_t serial, bool follows, uint32_t b, uint32_t nb,
-                                           uint32_t *list, uint32_t *tot, uint32_t *cnt, uint32_t *nclaim, F &&put) {
+                                           uint32_t *list, uint32_t *tot, uint32_t *cnt, uint32_t *nclaim,
+                                           G &&meanwhile, F &&put) {
     const int layer = at.layer;
-    for_due<BLOCK, CAP, true>(d, serial, b, nb, list, tot, [&](bool has, uint32_t j, const CellWords &w) {
+    for_due<BLOCK, CAP, true>(d, serial, b, nb, list, tot, meanwhile, [&](bool has, uint32_t j, const CellWords &w) {
         uint32_t claimed = 0;
         bool entered = false, sol = false, late = false, eval = false, mask = false;
         if (has && (w.ct & kTypeMask) == kActive) {
@@ -1006,11 +1014,12 @@ __device__ __forceinline__ void place_capture(const DomainView &d, const Neighbo
 
 // The range of active cells widened by a workgroup's new ones: those of nucleation in lohi (LDS) and
 // the captures' least and greatest index per thread. Every thread calls it. The range rarely grows: most
-// workgroups need no atomic.
+// workgroups need no atomic (elo, ehi: it as it was).
 struct NewCells {
     uint32_t lo = 0xFFFFFFFFu, hi = 0;
 };
-__device__ __forceinline__ void widen_range(const DomainView &d, uint32_t *lohi, const NewCells &n = NewCells{}) {
+__device__ __forceinline__ void widen_range(const DomainView &d, uint32_t *lohi, const NewCells &n, uint32_t elo,
+                                            uint32_t ehi) {
     const uint32_t lo = ~wave_max(~n.lo), hi = wave_max(n.hi);  // in lane 63
     if ((threadIdx.x & 63) == 63 && lo <= hi) {
         atomicMin(&lohi[0], lo);
@@ -1018,9 +1027,12 @@ __device__ __forceinline__ void widen_range(const DomainView &d, uint32_t *lohi,
     }
     __syncthreads();
     if (threadIdx.x == 0 && lohi[0] <= lohi[1]) {
-        if (lohi[0] < d.ctl->elo) atomicMin(&d.ctl->elo, lohi[0]);
-        if (lohi[1] > d.ctl->ehi) atomicMax(&d.ctl->ehi, lohi[1]);
+        if (lohi[0] < elo) atomicMin(&d.ctl->elo, lohi[0]);
+        if (lohi[1] > ehi) atomicMax(&d.ctl->ehi, lohi[1]);
     }
+}
+__device__ __forceinline__ void widen_range(const DomainView &d, uint32_t *lohi, const NewCells &n = NewCells{}) {
+    widen_range(d, lohi, n, d.ctl->elo, d.ctl->ehi);
 }
 
 // Pass B over the claimants that claimant(k, cell, bits) gives. A claim whose word holds the claimant's
@@ -1121,7 +1133,7 @@ template <int BLOCK, uint32_t CAP>
 __device__ __forceinline__ void settle_body(const DomainView &d, const Growth &g, const LayerAt &at, int next_cycle,
                                             uint32_t next_serial, uint32_t b, uint32_t nb, uint32_t *list, uint32_t *tot,
                                             uint32_t *cnt) {
-    for_due<BLOCK, CAP, false>(d, next_serial, b, nb, list, tot, [&](bool has, uint32_t j, const CellWords &w) {
+    for_due<BLOCK, CAP, false>(d, next_serial, b, nb, list, tot, [] { return true; }, [&](bool has, uint32_t j, const CellWords &w) {
         const bool late = has && (w.ct & kTypeMask) == kActive && solid_since_last(w, next_serial, next_cycle, at.layer);
         if (late) solidify(d, g, j, w, growth_index(d, at, w.cts, w.lid, j, next_cycle - 1));
         count_event(late, &cnt[kCntLate]);
@@ -1137,19 +1149,20 @@ __device__ __forceinline__ void settle_body(const DomainView &d, const Growth &g
 template <int BLOCK>
 __device__ __forceinline__ void book_totals(const DomainView &d, uint32_t serial_now, unsigned long long *red) {
     StepCtl *ctl = d.ctl;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    for (int r = wave; r < kPartRows; r += BLOCK / 64) {
-        unsigned long long *row = d.part + static_cast<size_t>(r) * d.nparts;
-        unsigned long long v = 0;
-        for (uint32_t i = lane; i < d.nparts; i += 64) {
-            const unsigned long long x = row[i];
-            v += x;
-            if (x) row[i] = 0;
-        }
-#pragma unroll
-        for (int o = 32; o > 0; o >>= 1) v += __shfl_down(v, o, 64);
-        if (lane == 0) red[r] = v;
+    // a workgroup's line is read by 16 lanes
+    static_assert(kPartRows == 16, "a line of 16 counters per workgroup");
+    unsigned long long v0 = 0;
+    for (uint32_t i = threadIdx.x; i < d.nparts * kPartRows; i += BLOCK) {
+        const unsigned long long x = d.part[i];
+        v0 += x;
+        if (x) d.part[i] = 0;
     }
+    v0 += __shfl_down(v0, 32, 64);
+    v0 += __shfl_down(v0, 16, 64);
+    if ((threadIdx.x & 63) < kPartRows) red[(threadIdx.x >> 6) * kPartRows + (threadIdx.x & 63)] = v0;
+    __syncthreads();
+    if (threadIdx.x < kPartRows)
+        for (int w = 1; w < BLOCK / 64; w++) red[threadIdx.x] += red[w * kPartRows + threadIdx.x];
     __syncthreads();
     if (threadIdx.x != 0) return;
     const unsigned long long S = serial_now, n = S - ctl->serial_booked;
@@ -1293,71 +1306,79 @@ __device__ __forceinline__ bool follows_last(const StepCtl *ctl, int cycle) {
     return cycle > 1 && ctl->last_cycle == cycle - 1;
 }
 constexpr uint32_t kDueStage = 1024;  // due cells of a turn staged in LDS
-constexpr int kClaimSums = 2048;      // entries of the growth sums staged in LDS by every claim workgroup
+constexpr int kClaimSums = 8192;      // entries of the growth sums staged in LDS by every claim workgroup
 
-__device__ __forceinline__ void nucleate_step(const DomainView &d, int p, int layer, uint32_t b, uint32_t nb) {
+// A step's kernels get its cycle and serial as arguments: a kernel's first loads find cold caches, and each
+// one that others wait for costs 1.5 us of every step. What else they need first is asked for together:
+// the claim pass reads its calendar words while it stages the growth sums (all the rows of a
+// coarse time step: a row read from memory costs the cells on it that time for every probe), the apply pass its
+// claimants before it knows how many there are. us a step without and with: 256^3 29.7, 26.0; 400^3 41.5,
+// 37.1; 800^3 (cycles 6006-6025) 161, 155.
+__device__ __forceinline__ void nucleate_step(const DomainView &d, int cycle, uint32_t serial, uint32_t b, uint32_t nb) {
     __shared__ StepTally t;
     StepCtl *ctl = d.ctl;
     if (ctl->done) return;
-    const int cycle = ctl->cycle[p];
-    const uint32_t serial = ctl->serial[p];
     const int from = ctl->nuc_at;
     clear_tally(t);
-    const int m = nucleate_body<kBlock>(d, cycle, serial, layer, from, b, nb, t.cnt, t.lohi);
+    const int m = nucleate_body<kBlock>(d, cycle, serial, d.layer, from, b, nb, t.cnt, t.lohi);
     if (b == 0 && threadIdx.x == 0) ctl->nuc_next = from + m;
     if (!m) return;
     widen_range(d, t.lohi);
     add_parts(d, b, t.cnt, serial);
 }
-__device__ __forceinline__ void claim_step(const DomainView &d, int p, uint32_t b, uint32_t nb) {
+__device__ __forceinline__ void claim_step(const DomainView &d, int cycle, uint32_t serial, bool follows, uint32_t b,
+                                           uint32_t nb) {
     __shared__ StepTally t;
     __shared__ uint32_t nclaim;
-    __shared__ uint32_t gsums[kClaimSums];
+    __shared__ __attribute__((aligned(16))) uint32_t gsums[kClaimSums];
     __shared__ uint32_t list[kDueStage], tot[kBlock / 64];
-    StepCtl *ctl = d.ctl;
-    if (ctl->done) return;
+    const int done = d.ctl->done;
     if (threadIdx.x == 0) nclaim = 0;
     clear_tally(t);
     Growth g = growth_of(d);
-    stage_sums<kBlock>(d, g, gsums);
-    const int cycle = ctl->cycle[p];
-    const uint32_t serial = ctl->serial[p];
-    if (b == 0 && threadIdx.x == 0) {
-        // the next step's control words (read only by the kernels after this one)
-        ctl->cycle[1 - p] = cycle + 1;
-        ctl->serial[1 - p] = serial + 1;
-        ctl->nuc_at = max(ctl->nuc_at, ctl->nuc_next);
-    }
     const uint32_t region = place_of(b, nb) * claim_region(d, nb);
-    claim_body<kBlock, kDueStage>(d, grid_of(d), g, layer_at(ctl), cycle, serial, follows_last(ctl, cycle), b, nb, list,
-                                  tot, t.cnt, &nclaim, [&](uint32_t k, uint32_t j, uint32_t claimed) {
-                                      d.claim_cell[region + k] = j;
-                                      d.claim_bits[region + k] = claimed;
-                                  });
+    claim_body<kBlock, kDueStage>(
+        d, grid_of(d), g, layer_at(d), cycle, serial, follows, b, nb, list, tot, t.cnt, &nclaim,
+        [&] {
+            stage_sums<kBlock>(d, g, gsums);
+            return !done;
+        },
+        [&](uint32_t k, uint32_t j, uint32_t claimed) {
+            d.claim_cell[region + k] = j;
+            d.claim_bits[region + k] = claimed;
+        });
     __syncthreads();
-    if (threadIdx.x == 0) d.claim_count[b] = nclaim;
+    if (threadIdx.x == 0) d.claim_count[b * kCountStride] = nclaim;
     add_parts(d, b, t.cnt, serial);
 }
-__device__ __forceinline__ void apply_step(const DomainView &d, int p, uint32_t a, uint32_t nbc) {
+__device__ __forceinline__ void apply_step(const DomainView &d, int cycle, uint32_t serial, int p, uint32_t a, uint32_t nbc) {
     __shared__ StepTally t;
     __shared__ ApplyLds<kBlock> s;
     StepCtl *ctl = d.ctl;
-    if (ctl->done) return;
-    const uint32_t serial = ctl->serial[p];
-    if (a == 0 && threadIdx.x == 0) ctl->last_cycle = ctl->cycle[p];
-    const uint32_t n = d.claim_count[a];
     const uint32_t region = place_of(a, nbc) * claim_region(d, nbc);
+    // (a region has room for more claimants than a workgroup has threads; a workgroup without units has
+    // neither claimants nor a region)
+    const uint32_t early = (place_of(a, nbc) < d.units ? region : 0u) + threadIdx.x;
+    const uint32_t n = d.claim_count[a * kCountStride], cell0 = d.claim_cell[early], bits0 = d.claim_bits[early], elo = ctl->elo, ehi = ctl->ehi;
+    if (ctl->done) return;
     clear_tally(t);
     NewCells made;
     apply_body<kBlock>(
         d, grid_of(d), serial, n,
         [&](uint32_t k, uint32_t &j, uint32_t &bits) {
-            j = d.claim_cell[region + k];
-            bits = d.claim_bits[region + k];
+            j = k < kBlock ? cell0 : d.claim_cell[region + k];
+            bits = k < kBlock ? bits0 : d.claim_bits[region + k];
         },
         s, t.cnt, made);
-    widen_range(d, t.lohi, made);
+    widen_range(d, t.lohi, made, elo, ehi);
     add_parts(d, a, t.cnt, serial);
+    if (a == 0 && threadIdx.x == 0) {
+        // control words for the kernels that read them there
+        ctl->last_cycle = cycle;
+        ctl->cycle[1 - p] = cycle + 1;
+        ctl->serial[1 - p] = serial + 1;
+        ctl->nuc_at = max(ctl->nuc_at, ctl->nuc_next);
+    }
 }
 __device__ __forceinline__ void settle_step(const DomainView &d, int p_next, uint32_t b, uint32_t nb) {
     __shared__ StepTally t;
@@ -1366,12 +1387,12 @@ __device__ __forceinline__ void settle_step(const DomainView &d, int p_next, uin
     if (ctl->done || !follows_last(ctl, ctl->cycle[p_next])) return;
     clear_tally(t);
     const uint32_t serial = ctl->serial[p_next];
-    settle_body<kBlock, kDueStage>(d, growth_of(d), layer_at(ctl), ctl->cycle[p_next], serial, b, nb, list, tot, t.cnt);
+    settle_body<kBlock, kDueStage>(d, growth_of(d), layer_at(d), ctl->cycle[p_next], serial, b, nb, list, tot, t.cnt);
     __syncthreads();
     add_parts(d, b, t.cnt, serial);
 }
 __device__ __forceinline__ void book_step(const DomainView &d, int p_next) {
-    __shared__ unsigned long long red[kPartRows];
+    __shared__ unsigned long long red[kPartRows * (kBlock / 64)];
     if (d.ctl->done) return;
     book_totals<kBlock>(d, d.ctl->serial[p_next], red);
     if (threadIdx.x == 0) end_domain(d, d.ctl->last_cycle);
@@ -1422,14 +1443,14 @@ constexpr uint32_t kTeamDue = 2048;     // due cells of a turn staged in LDS
 constexpr uint32_t kTeamClaims = 512;   // claimants staged in LDS; the rest go to the claim lists
 
 struct TeamLds {
-    uint32_t sums[kTeamSums];
+    __attribute__((aligned(16))) uint32_t sums[kTeamSums];
     ApplyLds<kTeamBlock> apply;
     uint32_t list[kTeamDue];
     uint32_t claim_cell[kTeamClaims], claim_bits[kTeamClaims];
     uint32_t tot[kTeamBlock / 64];
     uint32_t nclaim;
     StepTally tally[2];
-    unsigned long long red[kPartRows];
+    unsigned long long red[kPartRows * (kTeamBlock / 64)];
 };
 
 // nsteps steps of one domain (nucleate: their nucleation too), settled and booked at the end. Two
@@ -1452,7 +1473,7 @@ __device__ __forceinline__ void steps_body(const DomainView &d, int p, int layer
     const uint32_t region = place_of(b, nb) * claim_region(d, nb);
     const bool whole = scans_all<kTeamBlock>(d, nb);
     const Grid gr = grid_of(d);
-    const LayerAt at = layer_at(ctl);
+    const LayerAt at = layer_at(d);
     clear_tally(s.tally[0]);
     clear_tally(s.tally[1]);
     Tally acc;
@@ -1474,7 +1495,7 @@ __device__ __forceinline__ void steps_body(const DomainView &d, int p, int layer
             if (threadIdx.x == 0) s.nclaim = 0;
             __syncthreads();
             claim_body<kTeamBlock, kTeamDue>(d, gr, g, at, cycle, serial, follows, b, nb, s.list, s.tot, t.cnt, &s.nclaim,
-                                             [&](uint32_t k, uint32_t j, uint32_t claimed) {
+                                             [] { return true; }, [&](uint32_t k, uint32_t j, uint32_t claimed) {
                                                  if (k < kTeamClaims) {
                                                      s.claim_cell[k] = j;
                                                      s.claim_bits[k] = claimed;
@@ -1529,14 +1550,14 @@ __device__ __forceinline__ void steps_body(const DomainView &d, int p, int layer
 }
 
 // Plain launches: one domain, passed by value.
-__global__ __launch_bounds__(kBlock) void k_nucleate(DomainView d, int p, int layer) {
-    nucleate_step(d, p, layer, blockIdx.x, gridDim.x);
+__global__ __launch_bounds__(kBlock) void k_nucleate(DomainView d, int cycle, uint32_t serial) {
+    nucleate_step(d, cycle, serial, blockIdx.x, gridDim.x);
 }
-__global__ __launch_bounds__(kBlock) void k_claim(DomainView d, int p) {
-    claim_step(d, p, blockIdx.x, gridDim.x);
+__global__ __launch_bounds__(kBlock) void k_claim(DomainView d, int cycle, uint32_t serial, int follows) {
+    claim_step(d, cycle, serial, follows != 0, blockIdx.x, gridDim.x);
 }
-__global__ __launch_bounds__(kBlock) void k_apply(DomainView d, int p, int nbc) {
-    apply_step(d, p, blockIdx.x, static_cast<uint32_t>(nbc));
+__global__ __launch_bounds__(kBlock) void k_apply(DomainView d, int cycle, uint32_t serial, int p) {
+    apply_step(d, cycle, serial, p, blockIdx.x, gridDim.x);
 }
 __global__ __launch_bounds__(kBlock) void k_settle(DomainView d, int p_next) {
     settle_step(d, p_next, blockIdx.x, gridDim.x);
@@ -1769,7 +1790,7 @@ __global__ __launch_bounds__(kBlock) void k_extract(DomainView d, int field, voi
         case kFieldDiagonal: {  // float, with the growth of the steps since the cell was last looked at
             float dl = c.dl;
             if ((c.ct & kTypeMask) == kActive && !(c.lm & kLmUnknown) && !(c.flags & kFresh))
-                dl = replay_growth(growth_of(d), dl, static_cast<int>(c.win), growth_index(d, layer_at(d.ctl), c.cts, c.lid, static_cast<uint32_t>(q), d.ctl->last_cycle));
+                dl = replay_growth(growth_of(d), dl, static_cast<int>(c.win), growth_index(d, layer_at(d), c.cts, c.lid, static_cast<uint32_t>(q), d.ctl->last_cycle));
             static_cast<float *>(out)[q] = dl;
             break;
         }
@@ -1864,12 +1885,12 @@ int claim_per_cu() {
 size_t claim_entries(const DomainView &d, uint32_t most_blocks) {
     return static_cast<size_t>(d.units + std::min(d.units, most_blocks)) * kUnitCells;
 }
-void launch_nucleation(const DomainView &d, int parity, int layer, hipStream_t s) {
-    k_nucleate<<<nucleation_blocks(d), kBlock, 0, s>>>(d, parity, layer);
+void launch_nucleation(const DomainView &d, const StepAt &at, hipStream_t s) {
+    k_nucleate<<<nucleation_blocks(d), kBlock, 0, s>>>(d, at.cycle, at.serial);
 }
-void launch_capture(const DomainView &d, int parity, int blocks, hipStream_t s) {
-    k_claim<<<blocks, kBlock, 0, s>>>(d, parity);
-    k_apply<<<blocks, kBlock, 0, s>>>(d, parity, blocks);
+void launch_capture(const DomainView &d, const StepAt &at, int blocks, hipStream_t s) {
+    k_claim<<<blocks, kBlock, 0, s>>>(d, at.cycle, at.serial, at.follows);
+    k_apply<<<blocks, kBlock, 0, s>>>(d, at.cycle, at.serial, at.parity);
 }
 void launch_settle(const DomainView &d, int parity_next, int blocks, hipStream_t s) {
     k_settle<<<blocks, kBlock, 0, s>>>(d, parity_next);
@@ -1888,17 +1909,17 @@ void launch_layer_setup(const DomainView &d, int parity_next, hipStream_t s) {
 void launch_rewake(const DomainView &d, int parity_next, int blocks, hipStream_t s) {
     k_rewake<<<blocks, kBlock, 0, s>>>(d, parity_next);
 }
-void launch_step_timed(const DomainView &d, int parity, int layer, int blocks, hipStream_t s, hipEvent_t *ev) {
+void launch_step_timed(const DomainView &d, const StepAt &at, int blocks, hipStream_t s, hipEvent_t *ev) {
     int e = 0;
     auto rec = [&]() { (void)hipEventRecord(ev[e++], s); };
     rec();
-    k_nucleate<<<nucleation_blocks(d), kBlock, 0, s>>>(d, parity, layer);
+    k_nucleate<<<nucleation_blocks(d), kBlock, 0, s>>>(d, at.cycle, at.serial);
     rec();
     rec();
-    k_claim<<<blocks, kBlock, 0, s>>>(d, parity);
+    k_claim<<<blocks, kBlock, 0, s>>>(d, at.cycle, at.serial, at.follows);
     rec();
     rec();
-    k_apply<<<blocks, kBlock, 0, s>>>(d, parity, blocks);
+    k_apply<<<blocks, kBlock, 0, s>>>(d, at.cycle, at.serial, at.parity);
     rec();
 }
 void launch_steps_n(const DomainView *views, const TeamPlace *places, uint32_t workgroups, int steps, int layer,

@@ -8,15 +8,22 @@ namespace exaca {
 
 constexpr int kBlock = 256;  // four wave64s per workgroup
 
+// A step as its kernels are told of it: the cycle, the steps executed before it, whether the step before
+// ran just before it (no cycle jump, same layer), and its parity in the control block.
+struct StepAt {
+    int cycle;
+    uint32_t serial;
+    int follows, parity;
+};
 // Nucleation (src/CAupdate.cpp:67-200). A step may leave it out when no site's time falls in the
 // steps since nucleation last ran (it would examine nothing).
-void launch_nucleation(const DomainView &d, int parity, int layer, hipStream_t s);
+void launch_nucleation(const DomainView &d, const StepAt &at, hipStream_t s);
 // Its workgroups (each adds to its own slot of the nucleation counter rows).
 int nucleation_blocks(const DomainView &d);
 // CellCapture (src/CAupdate.cpp:204-728) in two kernels: the liquidus-time gate, growth, neighbour
 // scan and claims of the cells due this step (also prepares the control slot of the next step);
 // then claims decided and winners' captures.
-void launch_capture(const DomainView &d, int parity, int blocks, hipStream_t s);
+void launch_capture(const DomainView &d, const StepAt &at, int blocks, hipStream_t s);
 // The solidifications the last step left to the next one, and the counters booked: before the state
 // or the statistics are looked at. parity_next is the parity of the next step.
 void launch_settle(const DomainView &d, int parity_next, int blocks, hipStream_t s);
@@ -47,7 +54,7 @@ void launch_seed_init(const DomainView &d, const uint32_t *cells, uint32_t n, hi
 // One step with an event pair around each kernel: nucleation, claim and apply. ev holds
 // 2 * kTimedKernels events.
 constexpr int kTimedKernels = 3;
-void launch_step_timed(const DomainView &d, int parity, int layer, int blocks, hipStream_t s, hipEvent_t *ev);
+void launch_step_timed(const DomainView &d, const StepAt &at, int blocks, hipStream_t s, hipEvent_t *ev);
 // Initial cell records from compact device arrays (CellType with the seed bit, LayerID, GrainID,
 // CritTimeStep), and one field back out of the records (FieldKind layout).
 void launch_pack(const DomainView &d, const uint8_t *ct, const int8_t *lid, const int32_t *gid, const int32_t *cts,

@@ -155,7 +155,9 @@ struct exaca_state {
     std::vector<void *> buffers;
     size_t bytes = 0;
     int parity = 0;        // parity of the next step
-    int cycle = 0;         // last executed step
+    int cycle = 0;         // the cycle before the next step's
+    int last_cycle = 0;    // last executed step of the layer
+    uint32_t serial = 0;   // steps executed
     int pending = -1;      // cycle whose nucleation ran but whose capture has not
     int blocks = 2048;     // workgroups of the frontier kernels
     int team = 0;          // workgroups of the resident kernel that runs many steps (0: two launches a step)
@@ -259,7 +261,7 @@ void build_device_state(exaca_state *h) {
     d.octa = h->alloc<Octa>(n);
     d.claim_cell = h->alloc<uint32_t>(claim_entries(d, static_cast<uint32_t>(std::max(h->blocks, kMaxTeam))));
     d.claim_bits = h->alloc<uint32_t>(claim_entries(d, static_cast<uint32_t>(std::max(h->blocks, kMaxTeam))));
-    d.claim_count = h->alloc<uint32_t>(h->blocks);
+    d.claim_count = h->alloc<uint32_t>(static_cast<size_t>(h->blocks) * kCountStride);
     d.alarms = h->alloc<uint32_t>(kAlarmSlots * alarm_stride(d.ncell));
     h->nloc = h->alloc<int32_t>(hd.nloc.size());
     h->ntime = h->alloc<int32_t>(hd.ntime.size());
@@ -272,7 +274,7 @@ void build_device_state(exaca_state *h) {
     if (grow.size() >= (1u << 25)) throw std::runtime_error("undercooling never saturates within 2^25 steps");
     double *grow_d = h->alloc<double>(grow.size());
     d.grow = grow_d;
-    d.ngrow = static_cast<int32_t>(grow.size());
+    d.gsat = grow.back();
     d.ksat = growth_plateau(grow);
     const GrowthSums sums = growth_sums(grow, d.ksat);
     uint32_t *sums_d = h->alloc<uint32_t>(sums.sums.size());
@@ -316,6 +318,7 @@ void set_next_cycle(exaca_state *h, int next) {
     HIP_OK(hipMemcpyAsync(&c->jump_from[slot], &from, 4, hipMemcpyHostToDevice, h->stream));
     HIP_OK(hipMemcpyAsync(&c->jump_to[slot], &to, 4, hipMemcpyHostToDevice, h->stream));
     h->njumps++;
+    h->dv.njumps = h->njumps;
     HIP_OK(hipMemcpyAsync(&c->njumps, &h->njumps, 4, hipMemcpyHostToDevice, h->stream));
     HIP_OK(hipMemcpyAsync(&c->cycle[h->parity], &next, 4, hipMemcpyHostToDevice, h->stream));
     // The calendar counts executed steps and waits for liquidus times in cycles: every active cell
@@ -355,6 +358,8 @@ void next_layer(exaca_state *h, int layer_done, int verbose) {
     }
     h->dv.zlo = zlo;
     h->dv.nzA = zhigh + 1;
+    h->dv.layer = layer_done + 1;
+    h->dv.jump0 = h->njumps;
     // the layer's record, the new layer's first cycle, and fresh counts of the active cells
     StepCtl *c = h->ctl;
     const int32_t end = h->cycle, j0 = h->njumps, layer = layer_done + 1, one = 1, zero = 0;
@@ -379,24 +384,35 @@ void next_layer(exaca_state *h, int layer_done, int verbose) {
     HIP_OK(hipStreamSynchronize(h->stream));  // host values above are stack temporaries
     h->layer = layer;
     h->cycle = 0;
+    h->last_cycle = 0;
 }
 
-void step_capture(exaca_state *h) {
-    exaca::launch_capture(h->dv, h->parity, h->blocks, h->stream);
-}
 // After the last step of a call: its state and statistics complete.
 void finish_steps(exaca_state *h) {
     exaca::launch_settle(h->dv, h->parity, h->blocks, h->stream);
     HIP_OK(hipGetLastError());
 }
+// The step at `cycle`, the next one; and the host's account of a step executed.
+exaca::StepAt next_step(const exaca_state *h, int cycle) {
+    return exaca::StepAt{cycle, h->serial, cycle > 1 && h->last_cycle == cycle - 1, h->parity};
+}
+void stepped(exaca_state *h, int n) {
+    h->cycle += n;
+    h->last_cycle = h->cycle;
+    h->serial += static_cast<uint32_t>(n);
+    h->parity ^= n & 1;
+}
 // The nucleation of the step at `cycle`, where a site is due.
-void step_nucleation(exaca_state *h, int layer, int cycle) {
+void step_nucleation(exaca_state *h, int cycle) {
     const auto it = std::upper_bound(h->nuc_times.begin(), h->nuc_times.end(), h->nuc_through);
     if (h->nuc_skip && (it == h->nuc_times.end() || *it > cycle)) return;
-    exaca::launch_nucleation(h->dv, h->parity, layer, h->stream);
+    exaca::launch_nucleation(h->dv, next_step(h, cycle), h->stream);
     h->nuc_through = cycle;
 }
 
+void step_capture(exaca_state *h, int cycle) {
+    exaca::launch_capture(h->dv, next_step(h, cycle), h->blocks, h->stream);
+}
 // n steps: a team's in one launch; else each step's own launches, the nucleation kernel only where a
 // site is due. (Replays of captured 50-step graphs run that kernel on every step of a graph with one
 // site due: 31.2 us a step at 256^3 against 30.1, 43.0 against 41.7 at 400^3, 114 against 112 at 800^3,
@@ -406,16 +422,14 @@ void run_steps(exaca_state *h, int layer, int n) {
     if (h->team) {
         exaca::launch_steps(h->dv, h->parity, layer, n, true, h->team, h->stream);
         HIP_OK(hipGetLastError());
-        h->cycle += n;
-        h->parity ^= n & 1;
+        stepped(h, n);
         h->nuc_through = h->cycle;
         return;
     }
     for (; n > 0; n--) {
-        step_nucleation(h, layer, h->cycle + 1);
-        step_capture(h);
-        h->parity ^= 1;
-        h->cycle += 1;
+        step_nucleation(h, h->cycle + 1);
+        step_capture(h, h->cycle + 1);
+        stepped(h, 1);
     }
     finish_steps(h);
 }
@@ -537,9 +551,8 @@ void profile(exaca_state *h, int layer, int nsteps, double *ms, int64_t counts[5
         const int batch = std::min(per_batch, nsteps - done);
         int k = 0;
         for (; k < batch; k++) {
-            exaca::launch_step_timed(h->dv, h->parity, layer, h->blocks, h->stream, &ev[2 * kTimedKernels * k]);
-            h->parity ^= 1;
-            h->cycle += 1;
+            exaca::launch_step_timed(h->dv, next_step(h, h->cycle + 1), h->blocks, h->stream, &ev[2 * kTimedKernels * k]);
+            stepped(h, 1);
             h->nuc_through = h->cycle;
             if (h->cycle % 1000 == 0) {
                 k++;
@@ -729,7 +742,7 @@ void nucleation_call(exaca_state *h, int cycle, int layer) {
     if (h->pending >= 0) throw StateError("nucleation called twice without capture");
     if (layer != h->layer) throw StateError("layer " + std::to_string(layer) + " is not the current layer");
     set_next_cycle(h, cycle);
-    step_nucleation(h, layer, cycle);
+    step_nucleation(h, cycle);
     HIP_OK(hipGetLastError());
     h->pending = cycle;
 }
@@ -745,14 +758,14 @@ int exaca_nucleation_nn(exaca_state *h, int cycle, int layer, int32_t *nn) {
         // the count booked by the steps before, plus this step's per-workgroup counts (the capture
         // pass books them at the end of the step)
         const int nb = exaca::nucleation_blocks(h->dv);
-        std::vector<unsigned long long> row(static_cast<size_t>(nb));
+        std::vector<unsigned long long> lines(static_cast<size_t>(nb) * exaca::kPartRows);
         exaca::StepStats st;
-        HIP_OK(hipMemcpyAsync(row.data(), h->dv.part + static_cast<size_t>(2 * exaca::kCntNn) * h->dv.nparts,
-                              row.size() * sizeof(unsigned long long), hipMemcpyDeviceToHost, h->stream));
+        HIP_OK(hipMemcpyAsync(lines.data(), h->dv.part, lines.size() * sizeof(unsigned long long), hipMemcpyDeviceToHost,
+                              h->stream));
         HIP_OK(hipMemcpyAsync(&st, h->stats, sizeof st, hipMemcpyDeviceToHost, h->stream));
         HIP_OK(hipStreamSynchronize(h->stream));
         unsigned long long total = st.nucleated;
-        for (unsigned long long v : row) total += v;
+        for (int b = 0; b < nb; b++) total += lines[static_cast<size_t>(b) * exaca::kPartRows + 2 * exaca::kCntNn];
         *nn = static_cast<int32_t>(total);
     });
 }
@@ -764,14 +777,13 @@ int exaca_cell_capture(exaca_state *h, int cycle, int layer) {
         if (h->team) {
             exaca::launch_steps(h->dv, h->parity, layer, 1, false, h->team, h->stream);
             HIP_OK(hipGetLastError());
-            h->parity ^= 1;
+            stepped(h, 1);
         }
         else {
-            step_capture(h);
-            h->parity ^= 1;
+            step_capture(h, cycle);
+            stepped(h, 1);
             finish_steps(h);
         }
-        h->cycle = cycle;
         h->pending = -1;
     });
 }

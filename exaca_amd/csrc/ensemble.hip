@@ -294,7 +294,7 @@ void admit(exaca_ensemble *e, const exaca_prepared *pr, int *slot_out) {
     d.guv = e->guv;
     d.seed_cdl = e->seed_cdl;
     d.grow = grow;
-    d.ngrow = static_cast<int32_t>(pr->grow.size());
+    d.gsat = pr->grow.back();
     d.ksat = pr->ksat;
     d.grow_sums = sums;
     d.sums_usable = pr->sums.usable;
