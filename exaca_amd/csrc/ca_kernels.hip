@@ -976,24 +976,37 @@ __device__ __forceinline__ bool has_neighbour(const DomainView &d, const Neighbo
     const int x = c.x + n.dx, y = c.y + n.dy, z = c.z + n.dz;
     return n.l < 26 && x >= 0 && x < d.X && y >= 0 && y < d.Y && z >= 0 && z < d.nzA;
 }
-__device__ __forceinline__ void place_capture(const DomainView &d, const NeighbourLane &n, uint32_t serial,
-                                              const Capture &m, const Coord &c, bool valid, unsigned long long word) {
-    const uint32_t q = m.q, nb = q + n.off, low = static_cast<uint32_t>(word), bit = 1u << n.back;
+// A half-wave takes two captures at a time through the three steps (take, write, wake), so that two atomics
+// and two sets of next words are in flight: each trip to memory takes 1-2 us at the wide fronts, whose
+// cells are far apart. k_apply at 800^3 (cycles 6006-6025, 63 K captures a step) 72 -> 68 us; us a step: 256^3
+// 26.0 -> 25.5, 400^3 37.1 -> 36.4, 800x800x40 40.0 -> 39.6, 100^3 14.5 -> 14.3.
+struct Placing {
+    Coord c;
+    unsigned long long word;
+    uint32_t liquid, old;
+    bool has, valid, need;
+};
+__device__ __forceinline__ void take_place(const DomainView &d, const NeighbourLane &n, uint32_t serial, const Capture &m,
+                                           Placing &a) {
+    const uint32_t nb = m.q + n.off, low = static_cast<uint32_t>(a.word), bit = 1u << n.back;
     // The new cell's mask: its liquid neighbours at its first visit are those liquid now and not claimed
     // in this step (every claimed cell is captured in this step, and the claims are final). Until it is
     // stored, the new cell's own words read as a claimed liquid cell, which no other capture counts.
-    const unsigned long long ballot = __ballot(valid && is_unclaimed_liquid(word));
-    const uint32_t liquid = static_cast<uint32_t>(threadIdx.x & 32u ? ballot >> 32 : ballot);
-    const bool need = valid && (low & (kMaskUnknown | bit)) == bit;
-    uint32_t old = 0;
+    const unsigned long long ballot = __ballot(a.valid && is_unclaimed_liquid(a.word));
+    a.liquid = static_cast<uint32_t>(threadIdx.x & 32u ? ballot >> 32 : ballot);
+    a.need = a.valid && (low & (kMaskUnknown | bit)) == bit;
     uint32_t *words = reinterpret_cast<uint32_t *>(&d.cells[nb].lm);
-    if (need) {
-        old = atomicAnd(words, ~bit);
+    if (a.need) {
+        a.old = atomicAnd(words, ~bit);
         // a neighbour at or below the claimant's index still had q liquid at its visit in the reference's
         // index order: its keep word gets this step's tag (every writer of a step writes the same value)
         if (nb <= m.from) words[1] = serial + 1;
     }
-    const double xp = (c.x + d.xoff) + 0.5, yp = (c.y + d.yoff) + 0.5, zp = c.z + 0.5;
+}
+__device__ __forceinline__ void write_place(const DomainView &d, const NeighbourLane &n, uint32_t serial, const Capture &m,
+                                            const Placing &a) {
+    const uint32_t q = m.q;
+    const double xp = (a.c.x + d.xoff) + 0.5, yp = (a.c.y + d.yoff) + 0.5, zp = a.c.z + 0.5;
     const float len = critical_length(faces_of(m.gv), xp, yp, zp, m.cx, m.cy, m.cz, n.dx, n.dy, n.dz);
     const uint32_t i = n.l < 26 ? 0u : static_cast<uint32_t>(n.l - 26);
     const double centre = i < 2 ? m.cx : (i < 4 ? m.cy : m.cz);
@@ -1002,14 +1015,18 @@ __device__ __forceinline__ void place_capture(const DomainView &d, const Neighbo
     reinterpret_cast<uint32_t *>(&d.octa[q])[n.l] = n.l < 26 ? __float_as_uint(len) : half;
     // The new cell's record, whole: nothing else writes it in this pass.
     if (n.l >= 26 && n.l < 30) {
-        unsigned long long w = liquid;  // lm (lane 28)
-        if (n.l == 26) w = (word & 0xFFFFFFFFull) | static_cast<unsigned long long>(static_cast<uint32_t>(m.gid)) << 32;  // cts, gid
-        if (n.l == 27) w = (word & 0xFFFFFFFFFFull) | static_cast<unsigned long long>(kActive) << 40 | static_cast<unsigned long long>(kFresh) << 48;  // win, lid, ct, flags
+        unsigned long long w = a.liquid;  // lm (lane 28)
+        if (n.l == 26) w = (a.word & 0xFFFFFFFFull) | static_cast<unsigned long long>(static_cast<uint32_t>(m.gid)) << 32;  // cts, gid
+        if (n.l == 27) w = (a.word & 0xFFFFFFFFFFull) | static_cast<unsigned long long>(kActive) << 40 | static_cast<unsigned long long>(kFresh) << 48;  // win, lid, ct, flags
         if (n.l == 29) w = __float_as_uint(m.dl);  // dl, thr
         reinterpret_cast<unsigned long long *>(d.cells + q)[n.l < 28 ? n.l - 24 : n.l - 28] = w;
     }
     if (n.l == 30) set_alarm(d, serial + 1, q);
-    if (need && (old & (kMaskUnknown | kMaskNow)) == bit) set_alarm(d, serial + 1, nb);
+}
+__device__ __forceinline__ void wake_emptied(const DomainView &d, const NeighbourLane &n, uint32_t serial, const Capture &m,
+                                             const Placing &a) {
+    const uint32_t bit = 1u << n.back;
+    if (a.need && (a.old & (kMaskUnknown | kMaskNow)) == bit) set_alarm(d, serial + 1, m.q + n.off);
 }
 
 // The range of active cells widened by a workgroup's new ones: those of nucleation in lohi (LDS) and
@@ -1089,17 +1106,22 @@ __device__ __forceinline__ void apply_body(const DomainView &d, const Grid &gr, 
             if (all && k0 + BLOCK < nclaimants) continue;  // with the next round's
             // the neighbours' words of a half-wave's first capture are on their way while the octahedra
             // are built, and those of its next one while it places one
+            constexpr uint32_t kHalves = BLOCK / 32;
             uint32_t i = threadIdx.x >> 5;
-            Coord at{};
-            bool valid = false;
-            unsigned long long word = 0;
+            Placing next[2];
             auto fetch = [&]() {
-                if (i >= turn) return;
-                const uint32_t q = s.from[i] + gr.offset(static_cast<int>(s.which[i]));
-                at = decode(q, gr);
-                valid = has_neighbour(d, n, at);
-                const unsigned long long *p = &d.cells[n.l < 26 ? q + n.off : q].lm + (n.l < 26 ? 0 : n.l - 24);
-                if (valid || n.l == 26 || n.l == 27) word = *p;
+#pragma unroll
+                for (int u = 0; u < 2; u++) {
+                    const uint32_t iu = i + u * kHalves;
+                    next[u].has = iu < turn;
+                    next[u].valid = false;
+                    if (iu >= turn) continue;
+                    const uint32_t q = s.from[iu] + gr.offset(static_cast<int>(s.which[iu]));
+                    next[u].c = decode(q, gr);
+                    next[u].valid = has_neighbour(d, n, next[u].c);
+                    const unsigned long long *p = &d.cells[n.l < 26 ? q + n.off : q].lm + (n.l < 26 ? 0 : n.l - 24);
+                    if (next[u].valid || n.l == 26 || n.l == 27) next[u].word = *p;
+                }
             };
             fetch();
             if (threadIdx.x < turn)
@@ -1111,15 +1133,20 @@ __device__ __forceinline__ void apply_body(const DomainView &d, const Grid &gr, 
             }
             __syncthreads();
             while (i < turn) {
-                const Capture &m = s.made[i];
-                const Coord c0 = at;
-                const bool ok = valid;
-                const unsigned long long w = word;
-                made.lo = m.q < made.lo ? m.q : made.lo;
-                made.hi = m.q > made.hi ? m.q : made.hi;
-                i += BLOCK / 32;
+                Placing now[2] = {next[0], next[1]};
+                const Capture &m0 = s.made[i], &m1 = s.made[now[1].has ? i + kHalves : i];
+                made.lo = m0.q < made.lo ? m0.q : made.lo;
+                made.hi = m0.q > made.hi ? m0.q : made.hi;
+                made.lo = m1.q < made.lo ? m1.q : made.lo;
+                made.hi = m1.q > made.hi ? m1.q : made.hi;
+                take_place(d, n, serial, m0, now[0]);
+                if (now[1].has) take_place(d, n, serial, m1, now[1]);
+                i += 2 * kHalves;
                 fetch();
-                place_capture(d, n, serial, m, c0, ok, w);
+                write_place(d, n, serial, m0, now[0]);
+                if (now[1].has) write_place(d, n, serial, m1, now[1]);
+                wake_emptied(d, n, serial, m0, now[0]);
+                if (now[1].has) wake_emptied(d, n, serial, m1, now[1]);
             }
             __syncthreads();
         }
