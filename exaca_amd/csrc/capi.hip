@@ -194,23 +194,25 @@ namespace {
 
 // Workgroups of the team that steps a domain in one launch, by the cross-section that its front
 // spreads over (X * Y; of a spot melt, one spot's: the spots solidify after one another, and about
-// 1.5 radius^2 cells are due together). 0: two launches a step over the whole device are faster. Measured,
-// us a step, with teams of 1, 8, 16, 32, 64 workgroups and two launches (-: not run):
-//   24^3 7.4, 9.5, 10.0, -, -, 13.1      44^3 17.8, 13.1, 13.5, 13.9, 15.1, 17.9
-//   56^3 31.6, 15.5, 15.4, 15.8, 16.9, 19.9      64^3 29.8, 13.6, 13.3, 13.8, 15.5, 16.5
-//   100^3 84.6, 20.8, 16.4, 15.3, 16.5, 17.9     150^3 -, -, 26.4, 20.2, 19.6, 21.6
-//   176^3 -, -, 40.2, 26.4, 22.3, 23.8           200^3 -, 55.5, 35.0, 26.1, 23.9, 23.6
-//   256^3 -, 168, 91.5, 55.0, 36.3, 31.1
-//   spots of radius 20 8.4, 9.2, 9.5, 10.0, -, 11.6; 25 5.1, 5.2, 5.4, 5.4, -, 6.2; 50 49.4, 15.3,
-//   13.0, 13.0, 14.9, 14.7; 6 x 6 of radius 75 (456 x 456 cells) -, -, 32.4, 23.4, 20.5, 18.6
+// 1.5 radius^2 cells are due together). 0: two launches a step over the whole device are faster: a
+// team's barriers cost 2 to 3 us each and its few workgroups take a wide front in turns. Measured, us a
+// step, with teams of 1, 8, 16, 32, 64 workgroups and two launches (-: not run):
+//   24^3 7.1, 9.2, 9.6, -, -, 12.1               32^3 9.3, 10.5, 10.9, -, -, 13.7
+//   38^3 13.1, 11.2, 11.8, -, -, 14.7            44^3 17.0, 12.4, 12.8, 13.2, -, 15.9
+//   56^3 31.1, 14.3, 14.5, 14.8, -, 17.5         64^3 -, 12.6, 12.6, 13.2, -, 14.9
+//   80^3 -, 16.0, 14.9, 15.2, 16.6, 17.1         100^3 -, 19.8, 15.5, 14.4, 15.8, 15.9
+//   128^3 -, -, 21.6, 17.5, 17.8, 18.0           150^3 -, -, 25.3, 18.9, 17.9, 17.8
+//   176^3 -, -, -, 25.1, 20.6, 19.0              200^3 -, -, -, 24.5, 21.8, 20.9
+//   256^3 -, -, -, -, 34.4, 25.2
+//   spots of radius 20 6.9, 8.4, 8.8, -, -, 11.1; 50 50.6, 14.9, 12.5, 12.6, 14.0, 13.8; 6 x 6 of
+//   radius 75 (456 x 456 cells) -, -, 32.5, 22.9, 19.3, 16.5
 int team_size(const exaca::Deck &deck, const exaca::HostDomain &hd) {
     const long long plane = static_cast<long long>(hd.X) * hd.Y;
-    if (plane > 190 * 190) return 0;
+    if (plane > 140 * 140) return 0;
     const double area = deck.sim_type == "S" ? 1.5 * deck.spot_radius * deck.spot_radius : static_cast<double>(plane);
     if (area <= 34 * 34) return 1;
     if (area <= 60 * 60) return 8;
-    if (area <= 84 * 84) return 16;
-    return area <= 150 * 150 ? 32 : 64;
+    return area <= 84 * 84 ? 16 : 32;
 }
 
 // The layer's nucleation sites to the device; its steps start with none decided. Synchronises the
@@ -238,11 +240,13 @@ void build_device_state(exaca_state *h) {
     h->device = dev;
     hipDeviceProp_t prop;
     HIP_OK(hipGetDeviceProperties(&prop, dev));
-    // Frontier kernels: up to 4 workgroups per CU (the capture pass is then resident in one round;
-    // measured at 800^3: 2, 3, 4, 6, 8 per CU give 110, 101, 96, 102, 118 us), fewer for small
-    // domains (the frontier never exceeds the cell count, and a slice is at least one workgroup of
-    // cells).
-    const int per_cu = std::min(4, exaca::claim_per_cu());
+    // Two-launch steps: up to 4 workgroups per CU, all resident at once, and 2 where the front's plane is
+    // narrow, so that a workgroup's start-up serves more cells. Measured, us a step with 1, 2, 3, 4, 6, 8
+    // per CU: 128^3 -, 18.0, -, 18.7, -, -; 200^3 -, 20.5, -, 21.2, -, -; 256^3 26.7, 25.2, 25.6, 25.6, 35.3,
+    // 37.7; 400^3 44.1, 37.9, 37.0, 36.1, 45.4, 46.7; 800x800x40 47.5, 40.4, 38.3, 39.2, 46.7, 49.6; 800^3
+    // (cycles 6006-6025) 215, 164, 157, 147, 164, 152. Fewer for domains of few cells.
+    const int most = static_cast<long long>(hd.X) * hd.Y <= 300 * 300 ? 2 : 4;
+    const int per_cu = std::min(most, exaca::claim_per_cu());
     const long long cap = std::min<long long>(2048, ((prop.multiProcessorCount * per_cu + 7) / 8) * 8);
     const long long want = ((hd.ncell / 4096 + 7) / 8) * 8;
     h->blocks = static_cast<int>(std::max<long long>(8, std::min(cap, want)));

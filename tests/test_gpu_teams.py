@@ -1,6 +1,6 @@
 """GPU: the kernel that runs many steps of a domain in one launch, at the cross-sections where the
-number of its workgroups changes (the last of a size and the first of the next, to the first domain
-that takes two launches a step), against the oracle, cell for cell. One workgroup also gets a
+number of its workgroups changes (the last of a size and the first of the next, to the first domains
+that take two launches a step), against the oracle, cell for cell. One workgroup also gets a
 domain where a third of the cells are nuclei: about 740 captures a step, more claimants than it
 stages in LDS. Each domain is run three
 ways: in one call, in calls of odd lengths (each settles and books its own last step), and through
@@ -23,6 +23,8 @@ CASES = {
     "59x59x7": dict(n=7, nx=59, ny=59, density=1000, fraction=0.05),
     "82x82x5": dict(n=5, nx=82, ny=82, density=1000, fraction=0.05),
     "83x83x5": dict(n=5, nx=83, ny=83, density=500, fraction=0.05),
+    "138x138x4": dict(n=4, nx=138, ny=138, density=500, fraction=0.05),
+    "139x139x4": dict(n=4, nx=139, ny=139, density=500, fraction=0.05),
     "148x148x4": dict(n=4, nx=148, ny=148, density=500, fraction=0.05),
     "149x149x4": dict(n=4, nx=149, ny=149, density=200, fraction=0.05),
     "188x188x4": dict(n=4, nx=188, ny=188, density=200, fraction=0.05),
