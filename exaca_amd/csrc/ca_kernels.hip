@@ -13,12 +13,15 @@
 // A cell whose liquid neighbours were all taken by lower-indexed cells in a step turns solid in that
 // step: the claim pass of the next step finds it due and gives it that step's state, and k_settle does
 // so when the caller looks at the state in between; k_book then sums the steps' counters.
-// What bounds a step of a small domain is not its work but what a launch costs before and between
-// its loads (5-14 us a kernel for a few dozen cells: caches and code are cold after each kernel
-// boundary), so a step has as few launches as its grid-wide dependences allow: claims before winners,
+// What bounds a step of all but the widest domains is not its work but what a launch costs before and
+// between its loads (5-14 us a kernel for a few dozen cells: caches and code are cold after each kernel
+// boundary), so a step has as few phases as its domain-wide dependences allow: claims before winners,
 // captures before the next step's claims. With separate kernels for the winners, the settling and the
-// list of due cells: 28.8, 40.5, 66.4, 76.4 us a step at 24^3, 100^3, 256^3, 400^3; with two kernels
-// 18.8, 26.4, 49.5, 60.8 us; at 800^3 (cycles 6006-6025) 0.198 and 0.180 ms.
+// list of due cells a step took 28.8, 40.5, 66.4, 76.4 us at 24^3, 100^3, 256^3, 400^3; with two kernels
+// it takes 12.1, 15.9, 25.2, 36.4 us; at 800^3 (cycles 6006-6025) 0.198 and 0.151 ms.
+// A narrow domain takes its steps in k_steps, many in a launch: a team of 1 to 64 workgroups with a
+// barrier between the phases of a step (7.1 us a step at 24^3, 14.3 at 100^3); k_steps_n does so for
+// every domain of an ensemble.
 // A cell is due when something can happen to it: it is new, its liquidus time has passed, or its
 // half-diagonal reaches the least critical length of its liquid neighbours; a neighbour's capture
 // or nucleation that empties its mask is handled where it happens. Between those steps its growth
