@@ -1438,18 +1438,28 @@ __device__ __forceinline__ void book_step(const DomainView &d, int p_next) {
 // Teams are small enough that their workgroups always find room beside each other (kMaxTeam); the wait
 // is bounded all the same, by the 100 MHz clock: false (with error 16) past it, for every thread.
 constexpr unsigned long long kTeamWait = 2000000000ull;  // 20 s
+// Waits until this wave's stores and atomics, and its write-back or invalidation of a cache, have been
+// done. The compiler leaves such a wait out where it counts nothing outstanding, and it doesn't count a
+// write-back: without this one the barrier's word was stored right behind the write-back's start
+// (`buffer_wbl2`), and another XCD could see the word while records were still dirty in this one's L2.
+__device__ __forceinline__ void drain() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
 struct Team {
     uint32_t b, nb;
     uint32_t number;  // of the last barrier passed
 };
 __device__ __forceinline__ bool team_sync(const DomainView &d, Team &t) {
+    if (t.nb == 1) {
+        __syncthreads();
+        return true;
+    }
+    drain();  // every wave its own: the release below waits for its wave's alone
     __syncthreads();
-    if (t.nb == 1) return true;
     t.number++;
     bool late = false;
     if (threadIdx.x < 64) {
         if (threadIdx.x == 0) {
             __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+            drain();
             __hip_atomic_store(d.sync + t.b, t.number, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
         if (threadIdx.x < t.nb) {
@@ -1464,6 +1474,7 @@ __device__ __forceinline__ bool team_sync(const DomainView &d, Team &t) {
             }
         }
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+        drain();  // the other waves' loads follow the invalidation, not just this one's
     }
     return !__syncthreads_or(late);
 }
