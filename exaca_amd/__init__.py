@@ -46,6 +46,7 @@ _SIGNATURES = {
                                        ctypes.POINTER(ctypes.c_int), ctypes.POINTER(ctypes.c_double)]),
     "exaca_download": (ctypes.c_int, [ctypes.c_void_p, ctypes.c_int, ctypes.c_void_p, ctypes.c_size_t]),
     "exaca_query": (ctypes.c_int, [ctypes.c_void_p, _I64P]),
+    "exaca_team_query": (ctypes.c_int, [ctypes.c_void_p, _I64P]),
     "exaca_destroy": (ctypes.c_int, [ctypes.c_void_p]),
     "exaca_run_program": (ctypes.c_int, [ctypes.c_int, ctypes.c_int, ctypes.c_char_p]),
     "exaca_host_state": (ctypes.c_int, [ctypes.c_char_p, ctypes.c_char_p, ctypes.c_int, ctypes.c_void_p,
@@ -377,6 +378,12 @@ class Solver:
                 "solidified", "waiting", "list_len", "list_cap", "device_bytes", "evaluated", "masks", "layers",
                 "layer"]
         return dict(zip(keys, list(out)))
+
+    def team(self) -> dict:
+        """How the steps are launched (exaca_team_query)."""
+        out = (ctypes.c_int64 * 4)()
+        self._ok(self._lib.exaca_team_query(self._h, out))
+        return dict(zip(["workgroups", "launches", "alone"], list(out)))
 
     def profile_steps(self, nsteps: int, layer: int = 0) -> dict:
         """Runs nsteps more steps with per-kernel HIP events; summed kernel times in ms."""

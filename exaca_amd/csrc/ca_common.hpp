@@ -56,10 +56,15 @@ constexpr uint32_t kAlarmSlots = 64;
 constexpr size_t alarm_stride(long long ncell) {
     return ((static_cast<size_t>(ncell) + 31) / 32 + 7) & ~static_cast<size_t>(7);
 }
-// Workgroups of a team that steps a domain in one launch. A CU holds one of them, so the teams of the
-// four hardware queues a process has always find room beside each other in 256 CUs, however their
-// workgroups are dispatched: no team waits for one of its own that waits for room.
+// Workgroups of a team that steps a domain in one launch (meet.hpp: how they make sure that all of them run).
+// A CU holds one of them.
 constexpr int kMaxTeam = 64;
+// Words of a domain's `sync`: each workgroup's last barrier, each one's last launch, the decision (two words).
+constexpr int kSyncReport = kMaxTeam, kSyncDecision = 2 * kMaxTeam, kSyncWords = 2 * kMaxTeam + 2;
+// How long a team's workgroups wait for one another at the start of a launch, in us: longer than the domains
+// before it in a crowded ensemble's launch mostly take (1000 steps of 10 to 100 us), and not much longer
+// than one workgroup alone takes for a middle domain's.
+constexpr long kMeetWait = 1000000;
 constexpr int kMaxJumps = 4096;
 constexpr int kMaxLayers = 256;
 
@@ -103,6 +108,7 @@ struct StepCtl {
     uint32_t serial[2];   // steps executed before the step of parity p (its calendar slot)
     uint32_t elo, ehi;    // cell-index range [elo, ehi] holding every active cell (elo > ehi: none)
     int32_t njumps;       // cycle jumps taken so far (spot-melt problems)
+    uint32_t alone;       // launches that a team left to one workgroup
     int32_t error;        // flags: 2 invalid grain, 16 a barrier wait past its bound
     int32_t done;         // set by the device when a domain finishes or raised an error
     int32_t final_cycle;  // the check cycle at which it finished
@@ -252,7 +258,8 @@ struct DomainView {
     uint32_t nparts;
     uint32_t *alarms;       // kAlarmSlots bitmaps of one bit per cell: process the cell at the step
                             // whose serial is the bitmap's slot (mod kAlarmSlots)
-    uint32_t *sync;         // the team barrier's words, one per workgroup
+    uint32_t *sync;         // the team's words (kSyncWords)
+    uint32_t meet_wait;     // ticks of the 100 MHz clock that its workgroups wait for one another at the start
     int32_t autostop;       // end the domain on the device at the first check with no liquid left
     long long liquid0;      // liquid cells of the layer at the start
     int32_t *status;        // where the device reports the final cycle of an autostopped domain

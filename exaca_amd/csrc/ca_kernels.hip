@@ -39,6 +39,7 @@
 
 #include "ca_kernels.hpp"
 #include "growth.hpp"
+#include "meet.hpp"
 #include "threshold.hpp"
 
 namespace exaca {
@@ -1435,8 +1436,8 @@ __device__ __forceinline__ void book_step(const DomainView &d, int p_next) {
 // against 2.0 and 2.7 us with a workgroup that gathers and releases). What the team wrote before it
 // is visible to the team after it (agent-scope release and acquire by one wave, ordered with the rest
 // of the workgroup by its own barriers). A team of one needs the workgroup's barrier alone.
-// Teams are small enough that their workgroups always find room beside each other (kMaxTeam); the wait
-// is bounded all the same, by the 100 MHz clock: false (with error 16) past it, for every thread.
+// All of the team's workgroups run (they met before), so every wait ends; it is bounded all the same, by the
+// 100 MHz clock: false (with error 16) past it, for every thread.
 constexpr unsigned long long kTeamWait = 2000000000ull;  // 20 s
 // Waits until this wave's stores and atomics, and its write-back or invalidation of a cache, have been
 // done. The compiler leaves such a wait out where it counts nothing outstanding, and it doesn't count a
@@ -1479,6 +1480,54 @@ __device__ __forceinline__ bool team_sync(const DomainView &d, Team &t) {
     return !__syncthreads_or(late);
 }
 
+// A team's meeting (meet.hpp), by one wave of each workgroup; every lane calls and gets the same.
+struct MeetWords {
+    const DomainView &d;
+    uint32_t b, nb, launch;
+    unsigned long long t0;
+    __device__ __forceinline__ void report() const {
+        if (threadIdx.x == 0)
+            __hip_atomic_store(d.sync + kSyncReport + b, launch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    __device__ __forceinline__ unsigned long long *word() const {
+        return reinterpret_cast<unsigned long long *>(d.sync + kSyncDecision);
+    }
+    __device__ __forceinline__ static uint64_t first_lane(unsigned long long v) {
+        const uint32_t lo = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(v));
+        return static_cast<uint64_t>(__builtin_amdgcn_readfirstlane(static_cast<uint32_t>(v >> 32))) << 32 | lo;
+    }
+    __device__ __forceinline__ uint64_t decision() const {
+        return first_lane(__hip_atomic_load(word(), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+    }
+    __device__ __forceinline__ bool all_reported() const {
+        const uint32_t *r = d.sync + kSyncReport + (threadIdx.x < nb ? threadIdx.x : 0);
+        return __all(__hip_atomic_load(r, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == launch);
+    }
+    __device__ __forceinline__ bool expired() const { return static_cast<unsigned long long>(wall_clock64()) - t0 >= d.meet_wait; }
+    __device__ __forceinline__ uint64_t settle(uint64_t from, uint64_t to) const {
+        unsigned long long found = from;
+        if (threadIdx.x == 0)
+            __hip_atomic_compare_exchange_strong(word(), &found, static_cast<unsigned long long>(to), __ATOMIC_RELAXED,
+                                                 __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        return first_lane(found);
+    }
+};
+// Whether this workgroup takes part in the launch; the team is then all of it, or this one alone. role: LDS.
+__device__ __forceinline__ bool team_meets(const DomainView &d, Team &t, uint32_t launch, uint32_t &role) {
+    if (t.nb == 1) return true;
+    if (threadIdx.x < 64) {
+        const MeetWords w{d, t.b, t.nb, launch, static_cast<unsigned long long>(wall_clock64())};
+        const Meet m = meet(w, t.b, launch);
+        if (threadIdx.x == 0) role = static_cast<uint32_t>(m);
+    }
+    __syncthreads();
+    if (role == static_cast<uint32_t>(Meet::kAlone)) {
+        t.nb = 1;
+        if (threadIdx.x == 0) d.ctl->alone++;
+    }
+    return role != static_cast<uint32_t>(Meet::kLeave);
+}
+
 constexpr int kTeamSums = 12288;        // entries of the growth sums staged in LDS
 constexpr uint32_t kTeamDue = 2048;     // due cells of a turn staged in LDS
 constexpr uint32_t kTeamClaims = 512;   // claimants staged in LDS; the rest go to the claim lists
@@ -1489,7 +1538,7 @@ struct TeamLds {
     uint32_t list[kTeamDue];
     uint32_t claim_cell[kTeamClaims], claim_bits[kTeamClaims];
     uint32_t tot[kTeamBlock / 64];
-    uint32_t nclaim;
+    uint32_t nclaim, role;
     StepTally tally[2];
     unsigned long long red[kPartRows * (kTeamBlock / 64)];
 };
@@ -1499,10 +1548,12 @@ struct TeamLds {
 // cells; a step with a nucleation site due has one more. Control words and counters stay in registers
 // and LDS, the growth table in LDS, and caches and code stay warm from step to step.
 __device__ __forceinline__ void steps_body(const DomainView &d, int p, int layer, int nsteps, bool nucleate, uint32_t b,
-                                           uint32_t nb, TeamLds &s) {
+                                           uint32_t team_size, uint32_t launch, TeamLds &s) {
     StepCtl *ctl = d.ctl;
     if (ctl->done) return;
-    Team team{b, nb, ctl->barrier};
+    Team team{b, team_size, ctl->barrier};
+    if (!team_meets(d, team, launch, s.role)) return;
+    const uint32_t nb = team.nb;
     int cycle = ctl->cycle[p];
     uint32_t serial = ctl->serial[p];
     bool follows = follows_last(ctl, cycle);
@@ -1604,9 +1655,10 @@ __global__ __launch_bounds__(kBlock) void k_settle(DomainView d, int p_next) {
     settle_step(d, p_next, blockIdx.x, gridDim.x);
 }
 __global__ __launch_bounds__(kBlock) void k_book(DomainView d, int p_next) { book_step(d, p_next); }
-__global__ __launch_bounds__(kTeamBlock) void k_steps(DomainView d, int p, int layer, int nsteps, int nucleate) {
+__global__ __launch_bounds__(kTeamBlock) void k_steps(DomainView d, int p, int layer, int nsteps, int nucleate,
+                                                      uint32_t launch) {
     __shared__ TeamLds s;
-    steps_body(d, p, layer, nsteps, nucleate != 0, blockIdx.x, gridDim.x, s);
+    steps_body(d, p, layer, nsteps, nucleate != 0, blockIdx.x, gridDim.x, launch, s);
 }
 
 // Ensemble launches: workgroup i is workgroup b of the team of nb that serves the domain of one slot
@@ -1639,11 +1691,11 @@ __device__ __forceinline__ DomainView load_view(const DomainView *views, uint32_
     return d;
 }
 __global__ __launch_bounds__(kTeamBlock) void k_steps_n(const DomainView *views, const TeamPlace *places, int layer,
-                                                        int nsteps) {
+                                                        int nsteps, uint32_t launch) {
     __shared__ TeamLds s;
     const TeamPlace at = load_constant(places, blockIdx.x);
     const DomainView d = load_view(views, at.slot);
-    steps_body(d, 0, layer, nsteps, true, at.b, at.nb, s);
+    steps_body(d, 0, layer, nsteps, true, at.b, at.nb, launch, s);
 }
 
 __global__ __launch_bounds__(kBlock) void k_check(DomainView d, int cycle, int layer, CheckResult *out) {
@@ -1952,8 +2004,9 @@ void launch_settle(const DomainView &d, int parity_next, int blocks, hipStream_t
     k_settle<<<blocks, kBlock, 0, s>>>(d, parity_next);
     k_book<<<1, kBlock, 0, s>>>(d, parity_next);
 }
-void launch_steps(const DomainView &d, int parity, int layer, int steps, bool nucleate, int team, hipStream_t s) {
-    k_steps<<<team, kTeamBlock, 0, s>>>(d, parity, layer, steps, nucleate ? 1 : 0);
+void launch_steps(const DomainView &d, int parity, int layer, int steps, bool nucleate, int team, uint32_t launch,
+                  hipStream_t s) {
+    k_steps<<<team, kTeamBlock, 0, s>>>(d, parity, layer, steps, nucleate ? 1 : 0, launch);
 }
 void launch_layer_bounds(const DomainView &d, int next_layer, int *out, hipStream_t s) {
     k_layer_bounds<<<grid_for(d.ncell, 4096), kBlock, 0, s>>>(d, next_layer, out);
@@ -1979,8 +2032,8 @@ void launch_step_timed(const DomainView &d, const StepAt &at, int blocks, hipStr
     rec();
 }
 void launch_steps_n(const DomainView *views, const TeamPlace *places, uint32_t workgroups, int steps, int layer,
-                    hipStream_t s) {
-    k_steps_n<<<workgroups, kTeamBlock, 0, s>>>(views, places, layer, steps);
+                    uint32_t launch, hipStream_t s) {
+    k_steps_n<<<workgroups, kTeamBlock, 0, s>>>(views, places, layer, steps, launch);
 }
 void launch_check(const DomainView &d, int cycle, int layer, CheckResult *out, hipStream_t s) {
     k_check<<<grid_for(d.ncell, 4096), kBlock, 0, s>>>(d, cycle, layer, out);

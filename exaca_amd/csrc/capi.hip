@@ -158,6 +158,7 @@ struct exaca_state {
     int cycle = 0;         // the cycle before the next step's
     int last_cycle = 0;    // last executed step of the layer
     uint32_t serial = 0;   // steps executed
+    uint32_t launches = 0; // of the team
     int pending = -1;      // cycle whose nucleation ran but whose capture has not
     int blocks = 2048;     // workgroups of the frontier kernels
     int team = 0;          // workgroups of the resident kernel that runs many steps (0: two launches a step)
@@ -284,7 +285,8 @@ void build_device_state(exaca_state *h) {
     uint32_t *sums_d = h->alloc<uint32_t>(sums.sums.size());
     d.grow_sums = sums_d;
     d.sums_usable = sums.usable;
-    d.sync = h->alloc<uint32_t>(kMaxTeam);
+    d.sync = h->alloc<uint32_t>(kSyncWords);
+    d.meet_wait = meet_wait_ticks();
     h->ctl = h->alloc<StepCtl>(1);
     h->stats = h->alloc<StepStats>(1);
     h->check = h->alloc<CheckResult>(1);
@@ -306,7 +308,7 @@ void build_device_state(exaca_state *h) {
     StepCtl c = initial_ctl(hd);
     HIP_OK(hipMemcpyAsync(h->ctl, &c, sizeof c, hipMemcpyHostToDevice, s));
     HIP_OK(hipMemsetAsync(h->stats, 0, sizeof(StepStats), s));
-    HIP_OK(hipMemsetAsync(d.sync, 0, 4 * kMaxTeam, s));
+    HIP_OK(hipMemsetAsync(d.sync, 0, 4 * kSyncWords, s));
     HIP_OK(hipMemsetAsync(d.part, 0, 8ull * kPartRows * d.nparts, s));
     HIP_OK(hipStreamSynchronize(s));
 }
@@ -417,6 +419,13 @@ void step_nucleation(exaca_state *h, int cycle) {
 void step_capture(exaca_state *h, int cycle) {
     exaca::launch_capture(h->dv, next_step(h, cycle), h->blocks, h->stream);
 }
+// n steps of a team, in one launch.
+void step_team(exaca_state *h, int layer, int n, bool nucleate) {
+    h->launches = std::max(h->launches + 1, 1u);
+    exaca::launch_steps(h->dv, h->parity, layer, n, nucleate, h->team, h->launches, h->stream);
+    HIP_OK(hipGetLastError());
+    stepped(h, n);
+}
 // n steps: a team's in one launch; else each step's own launches, the nucleation kernel only where a
 // site is due. (Replays of captured 50-step graphs run that kernel on every step of a graph with one
 // site due: 31.2 us a step at 256^3 against 30.1, 43.0 against 41.7 at 400^3, 114 against 112 at 800^3,
@@ -424,9 +433,7 @@ void step_capture(exaca_state *h, int cycle) {
 void run_steps(exaca_state *h, int layer, int n) {
     if (n <= 0) return;
     if (h->team) {
-        exaca::launch_steps(h->dv, h->parity, layer, n, true, h->team, h->stream);
-        HIP_OK(hipGetLastError());
-        stepped(h, n);
+        step_team(h, layer, n, true);
         h->nuc_through = h->cycle;
         return;
     }
@@ -779,9 +786,7 @@ int exaca_cell_capture(exaca_state *h, int cycle, int layer) {
         if (!h) throw std::invalid_argument("null handle");
         if (h->pending != cycle) throw StateError("capture requires nucleation of the same cycle first");
         if (h->team) {
-            exaca::launch_steps(h->dv, h->parity, layer, 1, false, h->team, h->stream);
-            HIP_OK(hipGetLastError());
-            stepped(h, 1);
+            step_team(h, layer, 1, false);
         }
         else {
             step_capture(h, cycle);
@@ -934,6 +939,19 @@ int exaca_query(const exaca_state *h, int64_t out[20]) {
         out[17] = static_cast<int64_t>(st.masks);
         out[18] = h->deck.num_layers;
         out[19] = h->layer;
+    });
+}
+
+int exaca_team_query(const exaca_state *h, int64_t out[4]) {
+    return guarded([&] {
+        if (!h || !out) throw std::invalid_argument("null argument");
+        exaca::StepCtl c;
+        HIP_OK(hipStreamSynchronize(h->stream));
+        HIP_OK(hipMemcpy(&c, h->ctl, sizeof c, hipMemcpyDeviceToHost));
+        out[0] = h->team;
+        out[1] = h->launches;
+        out[2] = c.alone;
+        out[3] = 0;
     });
 }
 

@@ -91,7 +91,7 @@ size_t domain_bytes(const exaca::HostDomain &h, size_t ngrow, size_t nsums) {
     exaca::set_geometry(v, h.X, h.Y, h.nz, h.nzA);
     size_t b = 0;
     b += up(sizeof(exaca::Cell) * n) + up(sizeof(exaca::Octa) * n);  // cell records
-    b += 2 * up(4 * exaca::claim_entries(v, exaca::kMaxTeam)) + up(4 * exaca::kMaxTeam);  // claim lists, barrier words
+    b += 2 * up(4 * exaca::claim_entries(v, exaca::kMaxTeam)) + up(4 * exaca::kSyncWords);  // claim lists, team words
     b += 2 * up(4 * std::max<size_t>(h.nloc.size(), 1)) + up(8 * ngrow) + up(4 * nsums);
     b += up(sizeof(exaca::StepCtl)) + up(sizeof(exaca::StepStats)) + up(8ull * exaca::kPartRows * exaca::kMaxTeam);
     b += up(4 * exaca::kAlarmSlots * exaca::alarm_stride(h.ncell));  // calendar
@@ -133,6 +133,8 @@ struct exaca_ensemble {
     size_t places_cap = 0;
     bool dirty = true;
     long long steps = 0;
+    uint32_t launches = 0;
+    uint32_t meet_wait = 0;  // ticks
 
     ~exaca_ensemble() {
         if (arena.base) (void)hipFree(arena.base);
@@ -243,7 +245,9 @@ void launch(exaca_ensemble *e, int steps) {
     if (e->places.empty()) return;
     for (int n; steps > 0; steps -= n) {
         n = std::min(steps, kMaxLaunch);
-        exaca::launch_steps_n(e->views_d, e->places_d, static_cast<uint32_t>(e->places.size()), n, 0, e->stream);
+        e->launches = std::max(e->launches + 1, 1u);
+        exaca::launch_steps_n(e->views_d, e->places_d, static_cast<uint32_t>(e->places.size()), n, 0, e->launches,
+                              e->stream);
         HIP_OK(hipGetLastError());
     }
 }
@@ -278,7 +282,7 @@ void admit(exaca_ensemble *e, const exaca_prepared *pr, int *slot_out) {
     d.octa = reinterpret_cast<Octa *>(carve(sizeof(Octa) * n));
     d.claim_cell = reinterpret_cast<uint32_t *>(carve(4 * exaca::claim_entries(d, exaca::kMaxTeam)));
     d.claim_bits = reinterpret_cast<uint32_t *>(carve(4 * exaca::claim_entries(d, exaca::kMaxTeam)));
-    d.sync = reinterpret_cast<uint32_t *>(carve(4 * kMaxTeam));
+    d.sync = reinterpret_cast<uint32_t *>(carve(4 * kSyncWords));
     int32_t *nloc = reinterpret_cast<int32_t *>(carve(4 * std::max<size_t>(hd.nloc.size(), 1)));
     int32_t *ntime = reinterpret_cast<int32_t *>(carve(4 * std::max<size_t>(hd.nloc.size(), 1)));
     double *grow = reinterpret_cast<double *>(carve(8 * pr->grow.size()));
@@ -286,6 +290,7 @@ void admit(exaca_ensemble *e, const exaca_prepared *pr, int *slot_out) {
     d.alarms = reinterpret_cast<uint32_t *>(carve(4 * kAlarmSlots * alarm_stride(d.ncell)));
     d.ctl = reinterpret_cast<StepCtl *>(carve(sizeof(StepCtl)));
     d.stats = reinterpret_cast<StepStats *>(carve(sizeof(StepStats)));
+    d.meet_wait = e->meet_wait;
     d.nparts = kMaxTeam;
     d.part = reinterpret_cast<unsigned long long *>(carve(8ull * kPartRows * kMaxTeam));
     d.nnuclei = static_cast<int32_t>(loc.size());
@@ -316,7 +321,7 @@ void admit(exaca_ensemble *e, const exaca_prepared *pr, int *slot_out) {
     HIP_OK(hipMemcpyAsync(d.ctl, &c, sizeof c, hipMemcpyHostToDevice, s));
     HIP_OK(hipMemsetAsync(d.stats, 0, sizeof(StepStats), s));
     HIP_OK(hipMemsetAsync(d.part, 0, 8ull * kPartRows * kMaxTeam, s));
-    HIP_OK(hipMemsetAsync(d.sync, 0, 4 * kMaxTeam, s));
+    HIP_OK(hipMemsetAsync(d.sync, 0, 4 * kSyncWords, s));
     const int32_t zero = 0;
     HIP_OK(hipMemcpyAsync(e->status_d + slot, &zero, 4, hipMemcpyHostToDevice, s));
     HIP_OK(hipMemcpyAsync(e->status_d + e->slots + slot, &zero, 4, hipMemcpyHostToDevice, s));
@@ -421,6 +426,7 @@ int exaca_ensemble_create(int slots, size_t arena_bytes, exaca_ensemble **out) {
         *out = nullptr;
         auto e = std::make_unique<exaca_ensemble>();
         e->slots = slots;
+        e->meet_wait = exaca::meet_wait_ticks();
         HIP_OK(hipStreamCreateWithFlags(&e->stream, hipStreamNonBlocking));
         HIP_OK(hipMalloc(&e->arena.base, arena_bytes));
         e->arena.bytes = arena_bytes;

@@ -47,6 +47,20 @@ inline int frontier_blocks_override() {
     return static_cast<int>(v);
 }
 
+// How long a team's workgroups wait for one another at the start of a launch (meet.hpp), in ticks of the
+// 100 MHz clock: EXACA_MEET_US (0 .. 10^7 us), read when a handle or ensemble is created, overrides the
+// default. Tests set 0, so that most launches are left to one workgroup.
+inline uint32_t meet_wait_ticks() {
+    long us = kMeetWait;
+    if (const char *env = std::getenv("EXACA_MEET_US")) {
+        char *end = nullptr;
+        us = std::strtol(env, &end, 10);
+        if (end == env || *end || us < 0 || us > 10000000)
+            throw std::invalid_argument("EXACA_MEET_US must be 0 .. 10000000");
+    }
+    return static_cast<uint32_t>(us * 100);
+}
+
 template <typename F>
 int guarded(F &&f) {
     try {

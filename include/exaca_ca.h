@@ -93,6 +93,11 @@ int exaca_download(exaca_state *h, int field, void *dst, size_t dst_bytes);
  * evaluations, liquid-neighbour masks built, number of layers, current layer. */
 int exaca_query(const exaca_state *h, int64_t out[20]);
 
+/* How the steps are launched (no reference counterpart). out[0..3]: workgroups of the team that takes a
+ * launch's steps (0: two launches a step), launches of the team so far, those of them left to one
+ * workgroup because not all of the team could run at once, 0. */
+int exaca_team_query(const exaca_state *h, int64_t out[4]);
+
 /* The transition after layer `layer` (src/runCA.cpp:343-418): DomainShiftAndResize and LayerSetup
  * (src/CAinitialize.cpp:2772-2982) on the resident state, and the cycle count restarting at 0.
  * Call it when exaca_run_layer (or the check) has ended the layer; then run layer + 1. */
