@@ -65,6 +65,8 @@ constexpr int kSyncReport = kMaxTeam, kSyncDecision = 2 * kMaxTeam, kSyncWords =
 // before it in a crowded ensemble's launch mostly take (1000 steps of 10 to 100 us), and not much longer
 // than one workgroup alone takes for a middle domain's.
 constexpr long kMeetWait = 1000000;
+// The bound of a team's barriers, in us.
+constexpr long kBarrierWait = 20000000;
 constexpr int kMaxJumps = 4096;
 constexpr int kMaxLayers = 256;
 
@@ -260,6 +262,7 @@ struct DomainView {
                             // whose serial is the bitmap's slot (mod kAlarmSlots)
     uint32_t *sync;         // the team's words (kSyncWords)
     uint32_t meet_wait;     // ticks of the 100 MHz clock that its workgroups wait for one another at the start
+    uint32_t barrier_wait;  // and at a barrier, at most
     int32_t autostop;       // end the domain on the device at the first check with no liquid left
     long long liquid0;      // liquid cells of the layer at the start
     int32_t *status;        // where the device reports the final cycle of an autostopped domain

@@ -1225,17 +1225,19 @@ __device__ __forceinline__ void book_totals(const DomainView &d, uint32_t serial
 // multiple of 1000) with no liquid left: liquid cells only ever leave the liquid state by capture
 // or nucleation, so the reference's superheated + undercooled count (src/CAupdate.cpp:738-783) is
 // the initial liquid count minus both.
+__device__ __forceinline__ void stop_domain(const DomainView &d, int cycle, int32_t err) {
+    d.ctl->done = 1;
+    d.ctl->final_cycle = cycle;
+    if (err && d.status_err) *d.status_err = err;
+    if (d.status) *d.status = cycle;
+}
 __device__ __forceinline__ void end_domain(const DomainView &d, int cycle) {
     StepCtl *ctl = d.ctl;
     const int32_t err = ctl->error;
     const bool finished = d.autostop && cycle % 1000 == 0 &&
                           d.liquid0 - static_cast<long long>(d.stats->captures) -
                                   static_cast<long long>(d.stats->activated) == 0;
-    if (!err && !finished) return;
-    ctl->done = 1;
-    ctl->final_cycle = cycle;
-    if (err && d.status_err) *d.status_err = err;
-    if (d.status) *d.status = cycle;
+    if (err || finished) stop_domain(d, cycle, err);
 }
 
 // Every active cell of the window due at the next step (after a cycle jump, whose skipped steps the
@@ -1436,9 +1438,10 @@ __device__ __forceinline__ void book_step(const DomainView &d, int p_next) {
 // against 2.0 and 2.7 us with a workgroup that gathers and releases). What the team wrote before it
 // is visible to the team after it (agent-scope release and acquire by one wave, ordered with the rest
 // of the workgroup by its own barriers). A team of one needs the workgroup's barrier alone.
-// All of the team's workgroups run (they met before), so every wait ends; it is bounded all the same, by the
-// 100 MHz clock: false (with error 16) past it, for every thread.
-constexpr unsigned long long kTeamWait = 2000000000ull;  // 20 s
+// All of the team's workgroups run (they met before), so every wait ends; it is bounded all the same
+// (d.barrier_wait): past it the domain is stopped with error 16 at the step that was being taken, and
+// false returned to every thread. Nothing else of that launch is undone or completed: the barrier's number,
+// the cycle and the serial stay those of the launch's start, and no later launch takes the domain up.
 // Waits until this wave's stores and atomics, and its write-back or invalidation of a cache, have been
 // done. The compiler leaves such a wait out where it counts nothing outstanding, and it doesn't count a
 // write-back: without this one the barrier's word was stored right behind the write-back's start
@@ -1448,7 +1451,7 @@ struct Team {
     uint32_t b, nb;
     uint32_t number;  // of the last barrier passed
 };
-__device__ __forceinline__ bool team_sync(const DomainView &d, Team &t) {
+__device__ __forceinline__ bool team_sync(const DomainView &d, Team &t, int cycle) {
     if (t.nb == 1) {
         __syncthreads();
         return true;
@@ -1467,8 +1470,7 @@ __device__ __forceinline__ bool team_sync(const DomainView &d, Team &t) {
             const unsigned long long t0 = wall_clock64();
             while (static_cast<int32_t>(__hip_atomic_load(d.sync + threadIdx.x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) -
                                         t.number) < 0) {
-                if (wall_clock64() - t0 > kTeamWait) {
-                    atomicOr(&d.ctl->error, 16);
+                if (wall_clock64() - t0 > d.barrier_wait) {
                     late = true;
                     break;
                 }
@@ -1477,7 +1479,9 @@ __device__ __forceinline__ bool team_sync(const DomainView &d, Team &t) {
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
         drain();  // the other waves' loads follow the invalidation, not just this one's
     }
-    return !__syncthreads_or(late);
+    if (!__syncthreads_or(late)) return true;
+    if (threadIdx.x == 0) stop_domain(d, cycle, atomicOr(&d.ctl->error, 16) | 16);
+    return false;
 }
 
 // A team's meeting (meet.hpp), by one wave of each workgroup; every lane calls and gets the same.
@@ -1582,7 +1586,7 @@ __device__ __forceinline__ void steps_body(const DomainView &d, int p, int layer
                 site += nucleate_body<kTeamBlock>(d, cycle, serial, layer, site, b, nb, t.cnt, t.lohi);
                 next_site = site < d.nnuclei ? d.ntime[site] : 0x7FFFFFFF;
                 if (!whole) widen_range(d, t.lohi);
-                if (!team_sync(d, team)) return;
+                if (!team_sync(d, team, cycle)) return;
             }
             if (threadIdx.x == 0) s.nclaim = 0;
             __syncthreads();
@@ -1597,7 +1601,7 @@ __device__ __forceinline__ void steps_body(const DomainView &d, int p, int layer
                                                      d.claim_bits[region + k] = claimed;
                                                  }
                                              });
-            if (!team_sync(d, team)) return;
+            if (!team_sync(d, team, cycle)) return;
             if (threadIdx.x < kStepCounts) before.cnt[threadIdx.x] = 0;
             apply_body<kTeamBlock>(
                 d, gr, serial, s.nclaim,
@@ -1607,7 +1611,7 @@ __device__ __forceinline__ void steps_body(const DomainView &d, int p, int layer
                 },
                 s.apply, t.cnt, made);
             if (!whole) widen_range(d, t.lohi, made);
-            if (!team_sync(d, team)) return;
+            if (!team_sync(d, team, cycle)) return;
             acc.add(t.cnt, serial);
             follows = true;
             cycle++;
@@ -1619,7 +1623,7 @@ __device__ __forceinline__ void steps_body(const DomainView &d, int p, int layer
         widen_range(d, before.lohi);
         acc.add(t.cnt, serial);
         acc.put(d, b);
-        if (!team_sync(d, team)) return;
+        if (!team_sync(d, team, cycle)) return;
         clear_tally(s.tally[0]);
         clear_tally(s.tally[1]);
         if (b == 0) {
@@ -1635,7 +1639,7 @@ __device__ __forceinline__ void steps_body(const DomainView &d, int p, int layer
         }
         follows = false;  // settled
         if (nsteps > 0) {
-            if (!team_sync(d, team)) return;
+            if (!team_sync(d, team, cycle)) return;
             if (ctl->done) return;
         }
     }

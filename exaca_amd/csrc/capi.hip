@@ -287,6 +287,7 @@ void build_device_state(exaca_state *h) {
     d.sums_usable = sums.usable;
     d.sync = h->alloc<uint32_t>(kSyncWords);
     d.meet_wait = meet_wait_ticks();
+    d.barrier_wait = barrier_wait_ticks();
     h->ctl = h->alloc<StepCtl>(1);
     h->stats = h->alloc<StepStats>(1);
     h->check = h->alloc<CheckResult>(1);

@@ -134,7 +134,7 @@ struct exaca_ensemble {
     bool dirty = true;
     long long steps = 0;
     uint32_t launches = 0;
-    uint32_t meet_wait = 0;  // ticks
+    uint32_t meet_wait = 0, barrier_wait = 0;  // ticks
 
     ~exaca_ensemble() {
         if (arena.base) (void)hipFree(arena.base);
@@ -291,6 +291,7 @@ void admit(exaca_ensemble *e, const exaca_prepared *pr, int *slot_out) {
     d.ctl = reinterpret_cast<StepCtl *>(carve(sizeof(StepCtl)));
     d.stats = reinterpret_cast<StepStats *>(carve(sizeof(StepStats)));
     d.meet_wait = e->meet_wait;
+    d.barrier_wait = e->barrier_wait;
     d.nparts = kMaxTeam;
     d.part = reinterpret_cast<unsigned long long *>(carve(8ull * kPartRows * kMaxTeam));
     d.nnuclei = static_cast<int32_t>(loc.size());
@@ -427,6 +428,7 @@ int exaca_ensemble_create(int slots, size_t arena_bytes, exaca_ensemble **out) {
         auto e = std::make_unique<exaca_ensemble>();
         e->slots = slots;
         e->meet_wait = exaca::meet_wait_ticks();
+        e->barrier_wait = exaca::barrier_wait_ticks();
         HIP_OK(hipStreamCreateWithFlags(&e->stream, hipStreamNonBlocking));
         HIP_OK(hipMalloc(&e->arena.base, arena_bytes));
         e->arena.bytes = arena_bytes;

@@ -47,19 +47,21 @@ inline int frontier_blocks_override() {
     return static_cast<int>(v);
 }
 
-// How long a team's workgroups wait for one another at the start of a launch (meet.hpp), in ticks of the
-// 100 MHz clock: EXACA_MEET_US (0 .. 10^7 us), read when a handle or ensemble is created, overrides the
-// default. Tests set 0, so that most launches are left to one workgroup.
-inline uint32_t meet_wait_ticks() {
-    long us = kMeetWait;
-    if (const char *env = std::getenv("EXACA_MEET_US")) {
+// How long a team's workgroups wait for one another, in ticks of the 100 MHz clock: at the start of a launch
+// (meet.hpp; EXACA_MEET_US) and at a barrier, at most (EXACA_BARRIER_US). The variables, 0 .. 40000000 us, are
+// read when a handle or ensemble is created. Tests set 0: most launches are then left to one workgroup; the
+// first barrier ends the domain with error 16.
+inline uint32_t wait_ticks(const char *name, long us) {
+    if (const char *env = std::getenv(name)) {
         char *end = nullptr;
         us = std::strtol(env, &end, 10);
-        if (end == env || *end || us < 0 || us > 10000000)
-            throw std::invalid_argument("EXACA_MEET_US must be 0 .. 10000000");
+        if (end == env || *end || us < 0 || us > 40000000)
+            throw std::invalid_argument(std::string(name) + " must be 0 .. 40000000");
     }
-    return static_cast<uint32_t>(us * 100);
+    return static_cast<uint32_t>(us) * 100u;
 }
+inline uint32_t meet_wait_ticks() { return wait_ticks("EXACA_MEET_US", kMeetWait); }
+inline uint32_t barrier_wait_ticks() { return wait_ticks("EXACA_BARRIER_US", kBarrierWait); }
 
 template <typename F>
 int guarded(F &&f) {

@@ -38,7 +38,7 @@ def test_domain_left_to_one_workgroup_matches_the_oracle(tmp_path, monkeypatch, 
 
 def test_bad_waits_are_refused(tmp_path, monkeypatch):
     deck = c_deck(tmp_path / "d.txt", 8)
-    for bad in ("-1", "x", "", "10000001"):
+    for bad in ("-1", "x", "", "40000001"):
         monkeypatch.setenv("EXACA_MEET_US", bad)
         with pytest.raises(ea.ExacaError, match="EXACA_MEET_US"):
             ea.Solver(deck)
