@@ -113,6 +113,7 @@ struct StepCtl {
     uint32_t alone;       // launches that a team left to one workgroup
     int32_t error;        // flags: 2 invalid grain, 16 a barrier wait past its bound
     int32_t done;         // set by the device when a domain finishes or raised an error
+    int32_t halted;       // an error ended the steps of two launches; not yet settled and booked
     int32_t final_cycle;  // the check cycle at which it finished
     int32_t last_cycle;   // the last executed step
     int32_t nuc_at;       // nucleation sites of the layer decided so far (they lie in order of time)

@@ -1220,8 +1220,8 @@ __device__ __forceinline__ void book_totals(const DomainView &d, uint32_t serial
     ctl->serial_booked = serial_now;
 }
 
-// The end of a domain: stopped by an error flag (its later steps would work on a broken state; the
-// host learns of it at its next check or poll), or, with autostop, at a check step (cycle a
+// The end of a domain: stopped by an error flag, at the end of the step that raised it (its later steps would
+// work on a broken state; the host learns of it at its next check or poll), or, with autostop, at a check step (cycle a
 // multiple of 1000) with no liquid left: liquid cells only ever leave the liquid state by capture
 // or nucleation, so the reference's superheated + undercooled count (src/CAupdate.cpp:738-783) is
 // the initial liquid count minus both.
@@ -1350,7 +1350,7 @@ constexpr int kClaimSums = 8192;      // entries of the growth sums staged in LD
 __device__ __forceinline__ void nucleate_step(const DomainView &d, int cycle, uint32_t serial, uint32_t b, uint32_t nb) {
     __shared__ StepTally t;
     StepCtl *ctl = d.ctl;
-    if (ctl->done) return;
+    if (ctl->done | ctl->halted) return;
     const int from = ctl->nuc_at;
     clear_tally(t);
     const int m = nucleate_body<kBlock>(d, cycle, serial, d.layer, from, b, nb, t.cnt, t.lohi);
@@ -1365,7 +1365,7 @@ __device__ __forceinline__ void claim_step(const DomainView &d, int cycle, uint3
     __shared__ uint32_t nclaim;
     __shared__ __attribute__((aligned(16))) uint32_t gsums[kClaimSums];
     __shared__ uint32_t list[kDueStage], tot[kBlock / 64];
-    const int done = d.ctl->done;
+    const int done = d.ctl->done | d.ctl->halted;
     if (threadIdx.x == 0) nclaim = 0;
     clear_tally(t);
     Growth g = growth_of(d);
@@ -1393,6 +1393,8 @@ __device__ __forceinline__ void apply_step(const DomainView &d, int cycle, uint3
     // neither claimants nor a region)
     const uint32_t early = (place_of(a, nbc) < d.units ? region : 0u) + threadIdx.x;
     const uint32_t n = d.claim_count[a * kCountStride], cell0 = d.claim_cell[early], bits0 = d.claim_bits[early], elo = ctl->elo, ehi = ctl->ehi;
+    // (an error of this step's claims, or of an earlier step, after which nothing is claimed; see steps_body)
+    const int32_t err = ctl->error, halted = ctl->halted;
     if (ctl->done) return;
     clear_tally(t);
     NewCells made;
@@ -1405,12 +1407,17 @@ __device__ __forceinline__ void apply_step(const DomainView &d, int cycle, uint3
         s, t.cnt, made);
     widen_range(d, t.lohi, made, elo, ehi);
     add_parts(d, a, t.cnt, serial);
-    if (a == 0 && threadIdx.x == 0) {
+    if (a == 0 && threadIdx.x == 0 && !halted) {
         // control words for the kernels that read them there
         ctl->last_cycle = cycle;
         ctl->cycle[1 - p] = cycle + 1;
         ctl->serial[1 - p] = serial + 1;
         ctl->nuc_at = max(ctl->nuc_at, ctl->nuc_next);
+        if (err) {  // the last step: of whatever parity the host goes on to, it is settled and booked
+            ctl->halted = 1;
+            ctl->cycle[p] = cycle + 1;
+            ctl->serial[p] = serial + 1;
+        }
     }
 }
 __device__ __forceinline__ void settle_step(const DomainView &d, int p_next, uint32_t b, uint32_t nb) {
@@ -1543,6 +1550,7 @@ struct TeamLds {
     uint32_t claim_cell[kTeamClaims], claim_bits[kTeamClaims];
     uint32_t tot[kTeamBlock / 64];
     uint32_t nclaim, role;
+    int32_t broken;
     StepTally tally[2];
     unsigned long long red[kPartRows * (kTeamBlock / 64)];
 };
@@ -1602,6 +1610,11 @@ __device__ __forceinline__ void steps_body(const DomainView &d, int p, int layer
                                                  }
                                              });
             if (!team_sync(d, team, cycle)) return;
+            // A domain whose claims raised an error stops at the end of this step. (A capture can raise one only
+            // where its claim did, in this step or before: every workgroup reads the same now as later. The
+            // value is wanted after the captures; it is on its way meanwhile.)
+            const int32_t broken =
+                threadIdx.x == 0 ? __hip_atomic_load(&ctl->error, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0;
             if (threadIdx.x < kStepCounts) before.cnt[threadIdx.x] = 0;
             apply_body<kTeamBlock>(
                 d, gr, serial, s.nclaim,
@@ -1611,11 +1624,16 @@ __device__ __forceinline__ void steps_body(const DomainView &d, int p, int layer
                 },
                 s.apply, t.cnt, made);
             if (!whole) widen_range(d, t.lohi, made);
+            if (threadIdx.x == 0) s.broken = broken;
             if (!team_sync(d, team, cycle)) return;
             acc.add(t.cnt, serial);
             follows = true;
             cycle++;
             serial++;
+            if (s.broken) {
+                nsteps = 0;
+                break;
+            }
         }
         StepTally &t = s.tally[serial & 1], &before = s.tally[(serial & 1) ^ 1];
         settle_body<kTeamBlock, kTeamDue>(d, g, at, cycle, serial, b, nb, s.list, s.tot, t.cnt);
