@@ -615,7 +615,9 @@ __device__ uint32_t evaluate_claims(const DomainView &d, const Grid &gr, uint32_
     cdl[25] = v2.y;
     // In integer and min/max operations on the lengths, a neighbour that is not liquid (or, for the
     // threshold, reached) counting as infinitely far: conditions of 26 neighbours at once would need
-    // more scalar registers than there are. dlj - len has its sign bit set exactly when dlj < len.
+    // more scalar registers than there are. So does one whose length is NaN (of an orientation that the
+    // file did not give), which no half-diagonal reaches: a length is not negative, and as an integer a NaN of
+    // either sign is greater than infinity. dlj - len then has its sign bit set exactly when dlj < len.
     constexpr uint32_t kInf = 0x7F800000u;
     uint32_t beyond = 0;
     float next = __builtin_inff(), next2 = __builtin_inff();
@@ -623,7 +625,7 @@ __device__ uint32_t evaluate_claims(const DomainView &d, const Grid &gr, uint32_
 #pragma unroll
     for (int l = 0; l < 26; l++) {
         const uint32_t liq = static_cast<uint32_t>(static_cast<int32_t>(liquid << (31 - l)) >> 31);
-        const uint32_t len = (__float_as_uint(cdl[l]) & liq) | (kInf & ~liq);
+        const uint32_t len = min(__float_as_uint(cdl[l]) | ~liq, kInf);
         const uint32_t sign = __float_as_uint(dlj - __uint_as_float(len));
         beyond |= (sign >> 31) << l;
         const uint32_t open = static_cast<uint32_t>(static_cast<int32_t>(sign) >> 31);
