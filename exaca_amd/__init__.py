@@ -383,7 +383,7 @@ class Solver:
         """How the steps are launched (exaca_team_query)."""
         out = (ctypes.c_int64 * 4)()
         self._ok(self._lib.exaca_team_query(self._h, out))
-        return dict(zip(["workgroups", "launches", "alone"], list(out)))
+        return dict(zip(["workgroups", "launches", "alone", "spilled"], list(out)))
 
     def profile_steps(self, nsteps: int, layer: int = 0) -> dict:
         """Runs nsteps more steps with per-kernel HIP events; summed kernel times in ms."""

@@ -59,6 +59,7 @@ constexpr size_t alarm_stride(long long ncell) {
 // Workgroups of a team that steps a domain in one launch (meet.hpp: how they make sure that all of them run).
 // A CU holds one of them.
 constexpr int kMaxTeam = 64;
+constexpr uint32_t kTeamClaims = 512;  // claimants that a workgroup stages in LDS; the rest go to the claim lists
 // Words of a domain's `sync`: each workgroup's last barrier, each one's last launch, the decision (two words).
 constexpr int kSyncReport = kMaxTeam, kSyncDecision = 2 * kMaxTeam, kSyncWords = 2 * kMaxTeam + 2;
 // How long a team's workgroups wait for one another at the start of a launch, in us: longer than the domains
@@ -111,6 +112,7 @@ struct StepCtl {
     uint32_t elo, ehi;    // cell-index range [elo, ehi] holding every active cell (elo > ehi: none)
     int32_t njumps;       // cycle jumps taken so far (spot-melt problems)
     uint32_t alone;       // launches that a team left to one workgroup
+    uint32_t spilled;     // steps of a team's workgroup whose claimants did not all fit in LDS
     int32_t error;        // flags: 2 invalid grain, 16 a barrier wait past its bound
     int32_t done;         // set by the device when a domain finishes or raised an error
     int32_t halted;       // an error ended the steps of two launches; not yet settled and booked
@@ -264,6 +266,7 @@ struct DomainView {
     uint32_t *sync;         // the team's words (kSyncWords)
     uint32_t meet_wait;     // ticks of the 100 MHz clock that its workgroups wait for one another at the start
     uint32_t barrier_wait;  // and at a barrier, at most
+    uint32_t claim_stage;   // claimants that a team's workgroup stages in LDS (at most kTeamClaims)
     int32_t autostop;       // end the domain on the device at the first check with no liquid left
     long long liquid0;      // liquid cells of the layer at the start
     int32_t *status;        // where the device reports the final cycle of an autostopped domain

@@ -1543,7 +1543,6 @@ __device__ __forceinline__ bool team_meets(const DomainView &d, Team &t, uint32_
 
 constexpr int kTeamSums = 12288;        // entries of the growth sums staged in LDS
 constexpr uint32_t kTeamDue = 2048;     // due cells of a turn staged in LDS
-constexpr uint32_t kTeamClaims = 512;   // claimants staged in LDS; the rest go to the claim lists
 
 struct TeamLds {
     __attribute__((aligned(16))) uint32_t sums[kTeamSums];
@@ -1602,7 +1601,7 @@ __device__ __forceinline__ void steps_body(const DomainView &d, int p, int layer
             __syncthreads();
             claim_body<kTeamBlock, kTeamDue>(d, gr, g, at, cycle, serial, follows, b, nb, s.list, s.tot, t.cnt, &s.nclaim,
                                              [] { return true; }, [&](uint32_t k, uint32_t j, uint32_t claimed) {
-                                                 if (k < kTeamClaims) {
+                                                 if (k < d.claim_stage) {
                                                      s.claim_cell[k] = j;
                                                      s.claim_bits[k] = claimed;
                                                  }
@@ -1617,12 +1616,13 @@ __device__ __forceinline__ void steps_body(const DomainView &d, int p, int layer
             // value is wanted after the captures; it is on its way meanwhile.)
             const int32_t broken =
                 threadIdx.x == 0 ? __hip_atomic_load(&ctl->error, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0;
+            if (threadIdx.x == 0 && s.nclaim > d.claim_stage) atomicAdd(&ctl->spilled, 1u);
             if (threadIdx.x < kStepCounts) before.cnt[threadIdx.x] = 0;
             apply_body<kTeamBlock>(
                 d, gr, serial, s.nclaim,
                 [&](uint32_t k, uint32_t &j, uint32_t &bits) {
-                    j = k < kTeamClaims ? s.claim_cell[k] : d.claim_cell[region + k];
-                    bits = k < kTeamClaims ? s.claim_bits[k] : d.claim_bits[region + k];
+                    j = k < d.claim_stage ? s.claim_cell[k] : d.claim_cell[region + k];
+                    bits = k < d.claim_stage ? s.claim_bits[k] : d.claim_bits[region + k];
                 },
                 s.apply, t.cnt, made);
             if (!whole) widen_range(d, t.lohi, made);

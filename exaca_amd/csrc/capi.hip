@@ -286,6 +286,7 @@ void build_device_state(exaca_state *h) {
     d.grow_sums = sums_d;
     d.sums_usable = sums.usable;
     d.sync = h->alloc<uint32_t>(kSyncWords);
+    d.claim_stage = claim_stage();
     d.meet_wait = meet_wait_ticks();
     d.barrier_wait = barrier_wait_ticks();
     h->ctl = h->alloc<StepCtl>(1);
@@ -952,7 +953,7 @@ int exaca_team_query(const exaca_state *h, int64_t out[4]) {
         out[0] = h->team;
         out[1] = h->launches;
         out[2] = c.alone;
-        out[3] = 0;
+        out[3] = c.spilled;
     });
 }
 

@@ -255,6 +255,7 @@ void launch(exaca_ensemble *e, int steps) {
 void admit(exaca_ensemble *e, const exaca_prepared *pr, int *slot_out) {
     using namespace exaca;
     ensure_tables(e, pr->host, pr->deck.orientation_file);
+    const uint32_t stage = exaca::claim_stage();  // refused before anything is taken
     int slot = -1;
     for (int s = 0; s < e->slots; s++)
         if (!e->used[s]) {
@@ -290,6 +291,7 @@ void admit(exaca_ensemble *e, const exaca_prepared *pr, int *slot_out) {
     d.alarms = reinterpret_cast<uint32_t *>(carve(4 * kAlarmSlots * alarm_stride(d.ncell)));
     d.ctl = reinterpret_cast<StepCtl *>(carve(sizeof(StepCtl)));
     d.stats = reinterpret_cast<StepStats *>(carve(sizeof(StepStats)));
+    d.claim_stage = stage;
     d.meet_wait = e->meet_wait;
     d.barrier_wait = e->barrier_wait;
     d.nparts = kMaxTeam;

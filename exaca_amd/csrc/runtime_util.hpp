@@ -3,6 +3,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdlib>
 #include <stdexcept>
 #include <string>
@@ -47,6 +48,16 @@ inline int frontier_blocks_override() {
     return static_cast<int>(v);
 }
 
+// Claimants of a step that a team's workgroup stages in LDS: kTeamClaims, or fewer when EXACA_CAND_STAGE
+// (1 .. 2048, read when a handle or an ensemble's slot is created) asks for it, so that tests can drive the
+// path of those that do not fit on small domains.
+inline uint32_t claim_stage() {
+    const char *env = std::getenv("EXACA_CAND_STAGE");
+    if (!env) return kTeamClaims;
+    const long v = std::strtol(env, nullptr, 10);
+    if (v < 1 || v > 2048) throw std::invalid_argument("EXACA_CAND_STAGE must be 1 .. 2048");
+    return std::min(static_cast<uint32_t>(v), kTeamClaims);
+}
 // How long a team's workgroups wait for one another, in ticks of the 100 MHz clock: at the start of a launch
 // (meet.hpp; EXACA_MEET_US) and at a barrier, at most (EXACA_BARRIER_US). The variables, 0 .. 40000000 us, are
 // read when a handle or ensemble is created. Tests set 0: most launches are then left to one workgroup; the

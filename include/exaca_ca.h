@@ -95,7 +95,8 @@ int exaca_query(const exaca_state *h, int64_t out[20]);
 
 /* How the steps are launched (no reference counterpart). out[0..3]: workgroups of the team that takes a
  * launch's steps (0: two launches a step), launches of the team so far, those of them left to one
- * workgroup because not all of the team could run at once, 0. */
+ * workgroup because not all of the team could run at once, and steps of a workgroup whose claimants did not
+ * all fit in its LDS stage. */
 int exaca_team_query(const exaca_state *h, int64_t out[4]);
 
 /* The transition after layer `layer` (src/runCA.cpp:343-418): DomainShiftAndResize and LayerSetup
