@@ -41,7 +41,7 @@ using exaca::guarded;
 
 constexpr int kChunk = 50;         // steps are rounded up to this (even: parity 0 at launch boundaries)
 constexpr int kMaxLaunch = 1000;   // most steps of one launch (a multiple of kChunk)
-constexpr int kMaxBlocks = 256;    // largest workgroups-per-slot setting
+constexpr int kMaxBlocks = 256;    // largest workgroups-per-slot setting (above kMaxTeam: as kMaxTeam)
 constexpr size_t kAlign = 256;
 
 size_t up(size_t n) { return (n + kAlign - 1) / kAlign * kAlign; }
@@ -495,8 +495,9 @@ int exaca_ensemble_autotune(exaca_ensemble *e, int chunks_per_candidate, int *ch
         if (!e || !chosen || chunks_per_candidate <= 0) throw std::invalid_argument("bad argument");
         // Online tuning on the live ensemble: the workgroup count per slot changes only the
         // schedule, never the result, so candidates are tried on consecutive chunks and scored by
-        // device time per active-cell update.
-        const int candidates[] = {16, 32, 64, 128, 256};
+        // device time per active-cell update. A team never has more than kMaxTeam workgroups, so larger
+        // settings are the same as that one.
+        const int candidates[] = {16, 32, exaca::kMaxTeam};
         double best = 1e300;
         int best_b = candidates[0];
         hipEvent_t e0, e1;

@@ -123,7 +123,7 @@ def run_served(requests, *, slots: int = 256, arena_bytes: int = 200 << 30, chun
                 raise RuntimeError(f"served ensemble exceeded {max_steps} steps with {len(running)} domains running")
             if autotune and tuned is None and len(running) >= tune_at:
                 tuned = ens.autotune(1)
-                steps += 5 * chunk
+                steps += 3 * 50  # a chunk of 50 steps per candidate
             ens.advance(chunk)
             steps += chunk
             st, err = ens.poll_errors()

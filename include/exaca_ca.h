@@ -168,11 +168,11 @@ int exaca_ensemble_advance(exaca_ensemble *e, int steps);
  * flags of exaca_last_error's device messages; 0: none). A domain that raises one is stopped on
  * the device at the end of that step: its final cycle is then that step and its result is void. */
 int exaca_ensemble_poll(exaca_ensemble *e, int32_t *final_cycles, int32_t *errors);
-/* Workgroups per slot, at most (multiple of 8, 8..256; the device shares its compute units out among
- * the running domains by their size). */
+/* Workgroups per slot, at most (multiple of 8, 8..256, above 64 the same as 64; the device shares its compute
+ * units out among the running domains by their size). */
 int exaca_ensemble_set_blocks(exaca_ensemble *e, int blocks);
-/* Online autotuner: runs chunks_per_candidate chunks per workgroup-count candidate on the live
- * ensemble and keeps the one with the least device time per active-cell update. */
+/* Online autotuner: runs chunks_per_candidate chunks of 50 steps per workgroup-count candidate (16, 32, 64) on
+ * the live ensemble and keeps the one with the least device time per active-cell update. */
 int exaca_ensemble_autotune(exaca_ensemble *e, int chunks_per_candidate, int *chosen);
 /* out[0..7]: final cycle (0 while running), nucleation events, frontier-size sum, captures,
  * solidifications, device error flag, free arena bytes, steps enqueued so far. */
