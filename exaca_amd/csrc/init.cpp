@@ -504,12 +504,16 @@ std::vector<float> read_orientations(const std::string &path) {
     std::vector<float> guv(9 * kNumOrientations, 0.0f);
     std::ifstream in(path, std::ios::binary);
     if (!in.is_open()) throw std::runtime_error("Could not locate/open Substrate file");
-    in.seekg(0, std::ios::end);
-    const std::streamoff size = in.tellg();
-    std::string text(size > 0 ? static_cast<size_t>(size) : 0, '\0');
-    in.seekg(0);
-    in.read(&text[0], static_cast<std::streamsize>(text.size()));
-    const char *p = text.data(), *end = p + std::max<std::streamsize>(in.gcount(), 0);
+    // by pieces to the end, since a pipe has no size to ask for
+    std::string text;
+    constexpr std::streamsize kPiece = 1 << 20;
+    do {
+        const size_t had = text.size();
+        text.resize(had + kPiece);
+        in.read(&text[had], kPiece);
+        text.resize(had + static_cast<size_t>(std::max<std::streamsize>(in.gcount(), 0)));
+    } while (in);
+    const char *p = text.data(), *end = p + text.size();
     auto line_end = [&] {
         const void *q = p < end ? std::memchr(p, '\n', static_cast<size_t>(end - p)) : nullptr;
         return q ? static_cast<const char *>(q) : end;
