@@ -161,7 +161,11 @@ struct exaca_state {
     uint32_t launches = 0; // of the team
     int pending = -1;      // cycle whose nucleation ran but whose capture has not
     int blocks = 2048;     // workgroups of the frontier kernels
-    int team = 0;          // workgroups of the resident kernel that runs many steps (0: two launches a step)
+    int team = 0;          // workgroups of the team that takes single steps in one launch (0: two launches a step)
+    int run_team = 0;      // the same of many steps at a time
+    int most_team = 0;     // at most
+    uint32_t counted_serial = 0;       // steps and evaluations up to the check that last set run_team
+    unsigned long long counted = 0;
     int njumps = 0;
     // The layer's nucleation times in ascending order, and the last step whose nucleation kernel
     // ran: a step may leave the kernel out when no time falls after that step and up to it (every
@@ -193,27 +197,47 @@ struct exaca_state {
 
 namespace {
 
-// Workgroups of the team that steps a domain in one launch, by the cross-section that its front
-// spreads over (X * Y; of a spot melt, one spot's: the spots solidify after one another, and about
-// 1.5 radius^2 cells are due together). 0: two launches a step over the whole device are faster: a
-// team's barriers cost 2 to 3 us each and its few workgroups take a wide front in turns. Measured, us a
-// step, with teams of 1, 8, 16, 32, 64 workgroups and two launches (-: not run):
-//   24^3 7.1, 9.2, 9.6, -, -, 12.1               32^3 9.3, 10.5, 10.9, -, -, 13.7
-//   38^3 13.1, 11.2, 11.8, -, -, 14.7            44^3 17.0, 12.4, 12.8, 13.2, -, 15.9
-//   56^3 31.1, 14.3, 14.5, 14.8, -, 17.5         64^3 -, 12.6, 12.6, 13.2, -, 14.9
-//   80^3 -, 16.0, 14.9, 15.2, 16.6, 17.1         100^3 -, 19.8, 15.5, 14.4, 15.8, 15.9
-//   128^3 -, -, 21.6, 17.5, 17.8, 18.0           150^3 -, -, 25.3, 18.9, 17.9, 17.8
-//   176^3 -, -, -, 25.1, 20.6, 19.0              200^3 -, -, -, 24.5, 21.8, 20.9
-//   256^3 -, -, -, -, 34.4, 25.2
-//   spots of radius 20 6.9, 8.4, 8.8, -, -, 11.1; 50 50.6, 14.9, 12.5, 12.6, 14.0, 13.8; 6 x 6 of
-//   radius 75 (456 x 456 cells) -, -, 32.5, 22.9, 19.3, 16.5
-int team_size(const exaca::Deck &deck, const exaca::HostDomain &hd) {
+// Workgroups of the team that steps a domain in one launch; 0: two launches a step over the whole device are
+// faster, since a team's barriers cost 2 to 3 us each and its few workgroups take a wide front in turns.
+// Before a domain has run, by the cross-section that its front spreads over: X * Y; of a spot melt, one
+// spot's (the spots solidify after one another). Measured, us a step (over 2000 to 3000 cycles) with teams of
+// 1, 8, 16, 32, 64 workgroups and two launches (-: not run):
+//   24^3 7.1, 10.0, 10.4, 10.7, 12.9, 11.9       32^3 9.6, 11.5, 11.9, 12.3, 14.1, 13.6
+//   38^3 13.1, 12.4, 12.8, 13.1, 14.5, 14.6      44^3 17.7, 13.4, 14.0, 14.4, 15.7, 15.8
+//   56^3 32.7, 15.5, 15.6, 16.1, 17.2, 17.3      64^3 45.4, 16.8, 16.2, 16.6, 18.1, 17.4
+//   80^3 70.9, 18.5, 17.1, 17.2, 18.7, 18.0      90^3 91.7, 21.7, 17.8, 17.7, 19.3, 18.4
+//   100^3 138, 27.6, 21.0, 18.7, 19.9, 19.1      112^3 183, 33.6, 23.1, 19.8, 20.8, 19.7
+//   128^3 246, 41.0, 26.5, 21.2, 21.6, 20.4      150^3 340, 54.0, 33.6, 24.2, 22.9, 21.3
+//   spots of radius 20 8.4, 10.2, 10.6, 11.1, -, 12.0; 25 10.4, 10.7, 11.2, 11.7, -, 12.4; 27 12.1, 10.1,
+//   10.4, 10.9, 12.9, 11.3; 35 20.1, 11.6, 11.6, 11.9, 14.0, 12.3; 50 51.1, 18.2, 15.0, 14.5, 17.0, 14.6
+int team_by_size(const exaca::Deck &deck, const exaca::HostDomain &hd) {
     const long long plane = static_cast<long long>(hd.X) * hd.Y;
-    if (plane > 140 * 140) return 0;
-    const double area = deck.sim_type == "S" ? 1.5 * deck.spot_radius * deck.spot_radius : static_cast<double>(plane);
-    if (area <= 34 * 34) return 1;
-    if (area <= 60 * 60) return 8;
-    return area <= 84 * 84 ? 16 : 32;
+    const bool spots = deck.sim_type == "S";
+    // dense nuclei start fronts of their own at every plane (N steps to one): with 0.25 sites a cell, 30 x 30 cells
+    // take 75.6, 26.4, 23.5, 23.4, 24.1, 24.8 at N = 1 and 54.7, 31.9, 31.3, 31.0, 31.9, 31.5 at N = 4
+    const double sites = static_cast<double>(hd.nloc.size()) / static_cast<double>(hd.ncell);
+    const double nuclei = std::max(1.0, 30.0 * sites / std::max(deck.nratio, 1));
+    const double area = nuclei * (spots ? 2.5 * deck.spot_radius * deck.spot_radius : static_cast<double>(plane));
+    if (area > 116 * 116 || (spots && plane > 140 * 140)) return 0;
+    if (area <= 40 * 40) return 1;
+    if (area <= 61 * 61) return 8;
+    return area <= 92 * 92 ? 16 : 32;
+}
+// Afterwards, where steps are asked for many at a time, more if the cells that were evaluated a step since the
+// last check ask for them: the cross-section says nothing of a tall domain whose nuclei grow all over its depth.
+// (Not fewer: the mean says too little of a front that comes and goes; four spots of radius 44 take 13.6 us a step
+// with the 32 workgroups of their cross-section, and 21.7 with the 8 of their mean of 226.) Measured, us a step
+// with 1, 8, 16, 32 workgroups and two launches, by evaluations a step:
+//   104 9.6, 11.5, 11.9, 12.3, 13.6 (32^3)       171 13.1, 12.4, 12.8, 13.1, 14.6 (38^3)
+//   553 32.7, 15.5, 15.6, 16.1, 17.3 (56^3)      1700 91.7, 21.7, 17.8, 17.7, 18.4 (90^3)
+//   3435 183, 33.6, 23.1, 19.8, 19.7 (112^3); domains of 300 planes with 0.25 sites a cell, one or four steps a
+//   plane: 212 31.3, 21.5, 21.5, 21.0, 23.1; 677 75.6, 26.4, 23.5, 23.4, 24.8; 884 134, 44.9, 36.7, 34.6, 35.2;
+//   2228 227, 51.9, 35.1, 29.8, 26.7; 4455 440, 80.8, 53.7, 36.7, 29.7
+int team_by_due(double evaluated) {
+    if (evaluated > 3200) return 0;
+    if (evaluated <= 120) return 1;
+    if (evaluated <= 560) return 8;
+    return evaluated <= 1700 ? 16 : 32;
 }
 
 // The layer's nucleation sites to the device; its steps start with none decided. Synchronises the
@@ -251,11 +275,13 @@ void build_device_state(exaca_state *h) {
     const long long cap = std::min<long long>(2048, ((prop.multiProcessorCount * per_cu + 7) / 8) * 8);
     const long long want = ((hd.ncell / 4096 + 7) / 8) * 8;
     h->blocks = static_cast<int>(std::max<long long>(8, std::min(cap, want)));
-    h->team = std::min(team_size(h->deck, hd), prop.multiProcessorCount / 4);
+    h->most_team = std::min(kMaxTeam, prop.multiProcessorCount / 4);
+    h->team = std::min(team_by_size(h->deck, hd), h->most_team);
     if (const int forced = exaca::frontier_blocks_override()) {
         h->blocks = forced;
         h->team = 0;
     }
+    h->run_team = h->team;
 
     DomainView &d = h->dv;
     set_geometry(d, hd.X, hd.Y, hd.nz, hd.nzA);
@@ -422,9 +448,9 @@ void step_capture(exaca_state *h, int cycle) {
     exaca::launch_capture(h->dv, next_step(h, cycle), h->blocks, h->stream);
 }
 // n steps of a team, in one launch.
-void step_team(exaca_state *h, int layer, int n, bool nucleate) {
+void step_team(exaca_state *h, int layer, int n, bool nucleate, int team) {
     h->launches = std::max(h->launches + 1, 1u);
-    exaca::launch_steps(h->dv, h->parity, layer, n, nucleate, h->team, h->launches, h->stream);
+    exaca::launch_steps(h->dv, h->parity, layer, n, nucleate, team, h->launches, h->stream);
     HIP_OK(hipGetLastError());
     stepped(h, n);
 }
@@ -434,8 +460,8 @@ void step_team(exaca_state *h, int layer, int n, bool nucleate) {
 // cycles 1-3000.)
 void run_steps(exaca_state *h, int layer, int n) {
     if (n <= 0) return;
-    if (h->team) {
-        step_team(h, layer, n, true);
+    if (h->run_team) {
+        step_team(h, layer, n, true, h->run_team);
         h->nuc_through = h->cycle;
         return;
     }
@@ -465,6 +491,13 @@ void device_check(exaca_state *h, int *cycle, int layer, uint64_t counts[5], int
     HIP_OK(hipMemcpyAsync(&err, &h->ctl->error, 4, hipMemcpyDeviceToHost, h->stream));
     HIP_OK(hipStreamSynchronize(h->stream));
     if (err) throw DeviceError(exaca::device_error_text(err));
+    const uint32_t steps = h->serial - h->counted_serial;
+    if (h->team && steps >= 500) {
+        const int due = std::min(team_by_due(static_cast<double>(st.evaluated - h->counted) / steps), h->most_team);
+        h->run_team = due ? std::max(due, h->team) : 0;
+        h->counted_serial = h->serial;
+        h->counted = st.evaluated;
+    }
     if (counts)
         for (int k = 0; k < 5; k++) counts[k] = r.counts[k];
     // The range of active cells only widens between checks; narrow it to the cells active now.
@@ -788,7 +821,7 @@ int exaca_cell_capture(exaca_state *h, int cycle, int layer) {
         if (!h) throw std::invalid_argument("null handle");
         if (h->pending != cycle) throw StateError("capture requires nucleation of the same cycle first");
         if (h->team) {
-            step_team(h, layer, 1, false);
+            step_team(h, layer, 1, false, h->team);
         }
         else {
             step_capture(h, cycle);
@@ -950,7 +983,7 @@ int exaca_team_query(const exaca_state *h, int64_t out[4]) {
         exaca::StepCtl c;
         HIP_OK(hipStreamSynchronize(h->stream));
         HIP_OK(hipMemcpy(&c, h->ctl, sizeof c, hipMemcpyDeviceToHost));
-        out[0] = h->team;
+        out[0] = h->run_team;
         out[1] = h->launches;
         out[2] = c.alone;
         out[3] = c.spilled;

@@ -93,10 +93,10 @@ int exaca_download(exaca_state *h, int field, void *dst, size_t dst_bytes);
  * evaluations, liquid-neighbour masks built, number of layers, current layer. */
 int exaca_query(const exaca_state *h, int64_t out[20]);
 
-/* How the steps are launched (no reference counterpart). out[0..3]: workgroups of the team that takes a
- * launch's steps (0: two launches a step), launches of the team so far, those of them left to one
- * workgroup because not all of the team could run at once, and steps of a workgroup whose claimants did not
- * all fit in its LDS stage. */
+/* How the steps are launched (no reference counterpart). out[0..3]: workgroups of the team that takes the
+ * next exaca_run_layer's steps in one launch (0: two launches a step; a check changes it with the cells
+ * evaluated a step), launches of teams so far, those of them left to one workgroup because not all of the
+ * team could run at once, and steps of a workgroup whose claimants did not all fit in its LDS stage. */
 int exaca_team_query(const exaca_state *h, int64_t out[4]);
 
 /* The transition after layer `layer` (src/runCA.cpp:343-418): DomainShiftAndResize and LayerSetup

@@ -1,5 +1,5 @@
 """GPU: EXACA_CAND_STAGE narrows the LDS stage of a team's claimants, so that most of them take the lists in
-memory; values it never took are refused. One domain outgrows the full stage."""
+memory; values it never took are refused."""
 import numpy as np
 import pytest
 
@@ -27,15 +27,14 @@ def test_bad_stages_are_refused(tmp_path, monkeypatch, bad):
 CASES = [
     (dict(n=24, nx=20, ny=20, density=3000, fraction=0.1), 1, 1),
     (dict(n=16, nx=44, ny=44, density=2000, fraction=0.1), 2, 8),
-    # a third of the cells nuclei, one workgroup: more claimants a step than the whole stage
-    (dict(n=60, nx=30, ny=30, density=300000, fraction=1.0, N=1, G=1e5), None, 1),
+    # a quarter of the cells nuclei: hundreds of claimants a step
+    (dict(n=60, nx=30, ny=30, density=300000, fraction=1.0, N=1, G=1e5), 16, 32),
 ]
 
 
 @pytest.mark.parametrize("deck,stage,workgroups", CASES)
 def test_claimants_beyond_the_stage_match_the_oracle(tmp_path, monkeypatch, deck, stage, workgroups):
-    if stage:
-        monkeypatch.setenv("EXACA_CAND_STAGE", str(stage))
+    monkeypatch.setenv("EXACA_CAND_STAGE", str(stage))
     k = dict(deck)
     path = c_deck(tmp_path / "d.txt", k.pop("n"), **k)
     osim = orc.OracleSim(path, DATA)

@@ -1,0 +1,113 @@
+"""GPU: the cross-sections at which the number of workgroups that step a domain changes (the last of a
+size and the first of the next: arrays are four cells wider than the deck's domain), a team of eight on a
+domain too large for it to scan whole, and a tall domain whose team grows to two launches a step as nuclei
+grow all over its depth, each against the oracle."""
+import numpy as np
+import pytest
+
+import exaca_amd as ea
+import oracle as orc
+from conftest import DATA, c_deck, s_deck
+
+pytestmark = pytest.mark.gpu
+
+
+def _same(sol, osim, tag):
+    q, d = sol.query(), osim.dims()
+    for key in ("nn", "captures", "solidified", "frontier"):
+        assert q[key] == d[key], (tag, key, q[key], d[key])
+    ct = sol.field(ea.FIELD_CELLTYPE)
+    assert np.array_equal(ct, osim.field(orc.CELLTYPE)), f"{tag}: CellType"
+    assert np.array_equal(sol.field(ea.FIELD_GRAINID), osim.field(orc.GRAINID)), f"{tag}: GrainID"
+    act = np.flatnonzero(ct == 2)
+    assert np.array_equal(sol.field(ea.FIELD_DIAGONAL)[act], osim.field(orc.DIAGLEN)[act]), f"{tag}: DiagonalLength"
+
+
+def _both(deck, cycles, workgroups):
+    osim = orc.OracleSim(deck, DATA)
+    osim.run(max_cycles=cycles)
+    with ea.Solver(deck) as sol:
+        assert sol.team()["workgroups"] == workgroups
+        sol.run(max_cycles=cycles)
+        _same(sol, osim, "one call")
+    with ea.Solver(deck) as sol:
+        for c in (1, 2, 5, 68, 131, 132, cycles - 1, cycles):
+            sol.run(max_cycles=c)
+        _same(sol, osim, "calls of odd lengths")
+    with ea.Solver(deck) as sol:
+        for c in range(1, cycles + 1):
+            sol.step(c)
+            if c % 140 == 0:
+                sol.check(c)
+        _same(sol, osim, "time-step functions")
+
+
+@pytest.mark.parametrize("array,n,workgroups", [(40, 8, 1), (41, 8, 8), (61, 6, 8), (62, 6, 16), (92, 5, 16), (93, 5, 32),
+                                                (116, 4, 32), (117, 4, 0)])
+def test_cross_sections_where_the_team_changes(tmp_path, array, n, workgroups):
+    deck = c_deck(tmp_path / "d.txt", n, nx=array - 4, ny=array - 4, density=1500, fraction=0.15)
+    print(f"[sizes] {array}", flush=True)
+    _both(deck, 300, workgroups)
+
+
+@pytest.mark.parametrize("radius,workgroups", [(25, 1), (26, 8)])
+def test_spots_where_the_team_changes(tmp_path, radius, workgroups):
+    deck = s_deck(tmp_path / "s.txt", nsx=1, nsy=1, offset=radius, radius=radius, density=300, spacing=8, N=2)
+    osim = orc.OracleSim(deck, DATA)
+    osim.run(max_cycles=400)
+    with ea.Solver(deck) as sol:
+        assert sol.team()["workgroups"] == workgroups
+        sol.run(max_cycles=400)
+        q, d = sol.query(), osim.dims()
+        for key in ("nn", "captures", "solidified", "frontier"):
+            assert q[key] == d[key], (key, q[key], d[key])
+        assert np.array_equal(sol.field(ea.FIELD_CELLTYPE), osim.field(orc.CELLTYPE))
+        assert np.array_equal(sol.field(ea.FIELD_GRAINID), osim.field(orc.GRAINID))
+
+
+def test_team_that_scans_the_active_range(tmp_path):
+    """41 x 41 x 642 cells are 527 units, more than the 512 that eight workgroups hold at once: they scan the range
+    of active cells, which each other's captures and nuclei widen within the launch."""
+    deck = c_deck(tmp_path / "d.txt", 640, nx=37, ny=37, density=20000, fraction=0.3, N=2, G=1e5)
+    assert 41 * 41 * 642 > 512 * 2048
+    print("[sizes] 41 x 41 x 642", flush=True)
+    _both(deck, 420, 8)
+
+
+@pytest.mark.parametrize("side,density,N,workgroups", [(36, 100000, 4, 1), (18, 300000, 1, 8), (36, 300000, 2, 16),
+                                                       (36, 300000, 1, 32)])
+def test_dense_nuclei_make_the_team_larger(tmp_path, side, density, N, workgroups):
+    deck = c_deck(tmp_path / "d.txt", 20, nx=side, ny=side, density=density, N=N)
+    _both(deck, 150, workgroups)
+
+
+@pytest.mark.parametrize("side,first,later", [(26, 1, 16), (52, 8, 0)])
+def test_team_follows_the_cells_evaluated(tmp_path, monkeypatch, side, first, later):
+    """The smaller domain against the oracle, the larger one (33 s there) against two launches a step throughout."""
+    deck = c_deck(tmp_path / "d.txt", 400, nx=side, ny=side, density=20000, fraction=1.0, N=1, G=2e4, R=1e5)
+    if later:
+        ref = orc.OracleSim(deck, DATA)
+    else:
+        monkeypatch.setenv("EXACA_BLOCKS", "256")
+        ref = ea.Solver(deck)
+        assert ref.team()["workgroups"] == 0
+        monkeypatch.delenv("EXACA_BLOCKS")
+    sizes = []
+    with ea.Solver(deck) as sol:
+        sizes.append(sol.team()["workgroups"])
+        for cycle in (1000, 1500, 2000, 3000):
+            end, _ = sol.run(max_cycles=cycle)
+            rend, _ = ref.run(max_cycles=cycle)
+            assert end == rend
+            if later:
+                _same(sol, ref, f"cycle {end}")
+            else:
+                q, d = sol.query(), ref.query()
+                for key in ("nn", "captures", "solidified", "frontier", "evaluated", "waiting"):
+                    assert q[key] == d[key], (end, key)
+                for f in (ea.FIELD_CELLTYPE, ea.FIELD_GRAINID, ea.FIELD_DIAGONAL):
+                    assert np.array_equal(sol.field(f), ref.field(f)), (end, f)
+            sizes.append(sol.team()["workgroups"])
+            print(f"[sizes] cycle {end}: {sizes[-1]} workgroups", flush=True)
+    ref.close()
+    assert sizes[0] == first and later in sizes[1:]
