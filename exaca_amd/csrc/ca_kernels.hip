@@ -582,6 +582,12 @@ __device__ __forceinline__ int nucleate_body(const DomainView &d, int cycle, uin
     return m;
 }
 
+// An active cell without a grain: the domain ends with this step (broken: in LDS, or null).
+__device__ __forceinline__ void raise(const DomainView &d, uint32_t *broken) {
+    atomicOr(&d.ctl->error, 2);
+    if (broken) *broken = 1;
+}
+
 // Critical lengths of the liquid neighbours of frontier cell j (half-diagonal dlj): claims on
 // those reached. thr becomes the least length of the others (the caller stores it), hint the
 // record's note of which neighbour that is and of the next-least length (threshold_hint), and
@@ -590,12 +596,12 @@ __device__ __forceinline__ int nucleate_body(const DomainView &d, int cycle, uin
 // table. They are compared all at once and the claims issued after, so a lane's work does not
 // depend on its liquid count.
 __device__ uint32_t evaluate_claims(const DomainView &d, const Grid &gr, uint32_t j, float dlj, uint32_t liquid,
-                                    int32_t gid, uint8_t ct, float &thr, uint16_t &hint) {
+                                    int32_t gid, uint8_t ct, float &thr, uint16_t &hint, uint32_t *broken) {
     const float *row = d.octa[j].cdl;
     if (ct & kSeedBit) {
         int o = orientation_of(gid);
         if (o < 0) {
-            atomicOr(&d.ctl->error, 2);
+            raise(d, broken);
             o = 0;
         }
         row = d.seed_cdl + static_cast<size_t>(kCdlStride) * o;
@@ -816,7 +822,7 @@ template <int BLOCK, uint32_t CAP, typename G, typename F>
 __device__ __forceinline__ void claim_body(const DomainView &d, const Grid &gr, const Growth &g, const LayerAt &at,
                                            int cycle, uint32_t serial, bool follows, uint32_t b, uint32_t nb,
                                            uint32_t *list, uint32_t *tot, uint32_t *cnt, uint32_t *nclaim,
-                                           G &&meanwhile, F &&put) {
+                                           uint32_t *broken, G &&meanwhile, F &&put) {
     const int layer = at.layer;
     for_due<BLOCK, CAP, true>(d, serial, b, nb, list, tot, meanwhile, [&](bool has, uint32_t j, const CellWords &w) {
         uint32_t claimed = 0;
@@ -873,7 +879,7 @@ __device__ __forceinline__ void claim_body(const DomainView &d, const Grid &gr, 
                         }
                         else {
                             uint16_t hint = 0;
-                            claimed = evaluate_claims(d, gr, j, dl, liquid, w.gid, w.ct, thr, hint);
+                            claimed = evaluate_claims(d, gr, j, dl, liquid, w.gid, w.ct, thr, hint, broken);
                             flags = (flags & ~kHintMask) | hint;
                             eval = true;
                         }
@@ -923,13 +929,14 @@ struct ApplyLds {
 };
 
 // The octahedron of the winner jc's capture of its neighbour l (src/CAupdate.cpp:353-515).
-__device__ __forceinline__ void build_capture(const DomainView &d, const Grid &gr, uint32_t jc, int l, int h, Capture &m) {
+__device__ __forceinline__ void build_capture(const DomainView &d, const Grid &gr, uint32_t jc, int l, int h, Capture &m,
+                                              uint32_t *broken) {
     const Octa &e = d.octa[jc];
     // the winner's centre, float as the capture uses it
     const float wcx = static_cast<float>(e.x), wcy = static_cast<float>(e.y), wcz = static_cast<float>(e.z);
     int o = orientation_of(h);
     if (o < 0) {
-        atomicOr(&d.ctl->error, 2);
+        raise(d, broken);
         o = 0;
     }
     float gv[9];
@@ -1068,7 +1075,7 @@ __device__ __forceinline__ void widen_range(const DomainView &d, uint32_t *lohi,
 // step, the pass takes 72 us against 83 us.
 template <int BLOCK, typename F>
 __device__ __forceinline__ void apply_body(const DomainView &d, const Grid &gr, uint32_t serial, uint32_t nclaimants,
-                                           F &&claimant, ApplyLds<BLOCK> &s, uint32_t *cnt, NewCells &made) {
+                                           F &&claimant, ApplyLds<BLOCK> &s, uint32_t *cnt, NewCells &made, uint32_t *broken) {
     const uint32_t lane = threadIdx.x & 63;
     const NeighbourLane n = neighbour_lane(gr);
     if (threadIdx.x == 0) s.n = 0;
@@ -1132,7 +1139,7 @@ __device__ __forceinline__ void apply_body(const DomainView &d, const Grid &gr, 
             fetch();
             if (threadIdx.x < turn)
                 build_capture(d, gr, s.from[threadIdx.x], static_cast<int>(s.which[threadIdx.x]), s.gid[threadIdx.x],
-                              s.made[threadIdx.x]);
+                              s.made[threadIdx.x], broken);
             if (threadIdx.x == 0) {
                 cnt[kCntCap] += turn;
                 s.n = 0;
@@ -1373,7 +1380,7 @@ __device__ __forceinline__ void claim_step(const DomainView &d, int cycle, uint3
     Growth g = growth_of(d);
     const uint32_t region = place_of(b, nb) * claim_region(d, nb);
     claim_body<kBlock, kDueStage>(
-        d, grid_of(d), g, layer_at(d), cycle, serial, follows, b, nb, list, tot, t.cnt, &nclaim,
+        d, grid_of(d), g, layer_at(d), cycle, serial, follows, b, nb, list, tot, t.cnt, &nclaim, nullptr,
         [&] {
             stage_sums<kBlock>(d, g, gsums);
             return !done;
@@ -1406,7 +1413,7 @@ __device__ __forceinline__ void apply_step(const DomainView &d, int cycle, uint3
             j = k < kBlock ? cell0 : d.claim_cell[region + k];
             bits = k < kBlock ? bits0 : d.claim_bits[region + k];
         },
-        s, t.cnt, made);
+        s, t.cnt, made, nullptr);
     widen_range(d, t.lohi, made, elo, ehi);
     add_parts(d, a, t.cnt, serial);
     if (a == 0 && threadIdx.x == 0 && !halted) {
@@ -1451,6 +1458,10 @@ __device__ __forceinline__ void book_step(const DomainView &d, int p_next) {
 // (d.barrier_wait): past it the domain is stopped with error 16 at the step that was being taken, and
 // false returned to every thread. Nothing else of that launch is undone or completed: the barrier's number,
 // the cycle and the serial stay those of the launch's start, and no later launch takes the domain up.
+// broken (LDS): whether an error was raised. After a step's claims (claims) every workgroup learns of every
+// other's, so that all stop after the same step. A word read there may already be the next barrier's, of the same
+// step: its bit was set by that step's claims or by a capture, whose error a claim of the same step raised
+// before it. The other barriers don't look: a word read there may be of the next step.
 // Waits until this wave's stores and atomics, and its write-back or invalidation of a cache, have been
 // done. The compiler leaves such a wait out where it counts nothing outstanding, and it doesn't count a
 // write-back: without this one the barrier's word was stored right behind the write-back's start
@@ -1458,32 +1469,36 @@ __device__ __forceinline__ void book_step(const DomainView &d, int p_next) {
 __device__ __forceinline__ void drain() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
 struct Team {
     uint32_t b, nb;
-    uint32_t number;  // of the last barrier passed
+    uint32_t number;  // of the last barrier passed, twice; bit 0 of a posted word: an error was raised
 };
-__device__ __forceinline__ bool team_sync(const DomainView &d, Team &t, int cycle) {
+__device__ __forceinline__ bool team_sync(const DomainView &d, Team &t, int cycle, uint32_t &broken,
+                                          bool claims = false) {
     if (t.nb == 1) {
         __syncthreads();
         return true;
     }
     drain();  // every wave its own: the release below waits for its wave's alone
     __syncthreads();
-    t.number++;
+    t.number += 2;
     bool late = false;
     if (threadIdx.x < 64) {
         if (threadIdx.x == 0) {
             __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
             drain();
-            __hip_atomic_store(d.sync + t.b, t.number, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            __hip_atomic_store(d.sync + t.b, t.number | broken, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
         if (threadIdx.x < t.nb) {
             const unsigned long long t0 = wall_clock64();
-            while (static_cast<int32_t>(__hip_atomic_load(d.sync + threadIdx.x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) -
+            uint32_t word;
+            while (static_cast<int32_t>((word = __hip_atomic_load(d.sync + threadIdx.x, __ATOMIC_RELAXED,
+                                                                  __HIP_MEMORY_SCOPE_AGENT)) -
                                         t.number) < 0) {
                 if (wall_clock64() - t0 > d.barrier_wait) {
                     late = true;
                     break;
                 }
             }
+            if (claims && (word & 1u)) broken = 1;
         }
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
         drain();  // the other waves' loads follow the invalidation, not just this one's
@@ -1551,7 +1566,7 @@ struct TeamLds {
     uint32_t claim_cell[kTeamClaims], claim_bits[kTeamClaims];
     uint32_t tot[kTeamBlock / 64];
     uint32_t nclaim, role;
-    int32_t broken;
+    uint32_t broken;  // an error was raised, here or by the time of the last barrier elsewhere in the team
     StepTally tally[2];
     unsigned long long red[kPartRows * (kTeamBlock / 64)];
 };
@@ -1579,6 +1594,7 @@ __device__ __forceinline__ void steps_body(const DomainView &d, int p, int layer
     const bool whole = scans_all<kTeamBlock>(d, nb);
     const Grid gr = grid_of(d);
     const LayerAt at = layer_at(d);
+    if (threadIdx.x == 0) s.broken = 0;
     clear_tally(s.tally[0]);
     clear_tally(s.tally[1]);
     Tally acc;
@@ -1595,28 +1611,23 @@ __device__ __forceinline__ void steps_body(const DomainView &d, int p, int layer
                 site += nucleate_body<kTeamBlock>(d, cycle, serial, layer, site, b, nb, t.cnt, t.lohi);
                 next_site = site < d.nnuclei ? d.ntime[site] : 0x7FFFFFFF;
                 if (!whole) widen_range(d, t.lohi);
-                if (!team_sync(d, team, cycle)) return;
+                if (!team_sync(d, team, cycle, s.broken)) return;
             }
             if (threadIdx.x == 0) s.nclaim = 0;
             __syncthreads();
             claim_body<kTeamBlock, kTeamDue>(d, gr, g, at, cycle, serial, follows, b, nb, s.list, s.tot, t.cnt, &s.nclaim,
-                                             [] { return true; }, [&](uint32_t k, uint32_t j, uint32_t claimed) {
+                                             &s.broken, [] { return true; }, [&](uint32_t k, uint32_t j, uint32_t claimed) {
                                                  if (k < d.claim_stage) {
                                                      s.claim_cell[k] = j;
                                                      s.claim_bits[k] = claimed;
                                                  }
                                                  else {
+                                                     if (k == d.claim_stage) atomicAdd(&ctl->spilled, 1u);
                                                      d.claim_cell[region + k] = j;
                                                      d.claim_bits[region + k] = claimed;
                                                  }
                                              });
-            if (!team_sync(d, team, cycle)) return;
-            // A domain whose claims raised an error stops at the end of this step. (A capture can raise one only
-            // where its claim did, in this step or before: every workgroup reads the same now as later. The
-            // value is wanted after the captures; it is on its way meanwhile.)
-            const int32_t broken =
-                threadIdx.x == 0 ? __hip_atomic_load(&ctl->error, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0;
-            if (threadIdx.x == 0 && s.nclaim > d.claim_stage) atomicAdd(&ctl->spilled, 1u);
+            if (!team_sync(d, team, cycle, s.broken, true)) return;
             if (threadIdx.x < kStepCounts) before.cnt[threadIdx.x] = 0;
             apply_body<kTeamBlock>(
                 d, gr, serial, s.nclaim,
@@ -1624,15 +1635,14 @@ __device__ __forceinline__ void steps_body(const DomainView &d, int p, int layer
                     j = k < d.claim_stage ? s.claim_cell[k] : d.claim_cell[region + k];
                     bits = k < d.claim_stage ? s.claim_bits[k] : d.claim_bits[region + k];
                 },
-                s.apply, t.cnt, made);
+                s.apply, t.cnt, made, &s.broken);
             if (!whole) widen_range(d, t.lohi, made);
-            if (threadIdx.x == 0) s.broken = broken;
-            if (!team_sync(d, team, cycle)) return;
+            if (!team_sync(d, team, cycle, s.broken)) return;
             acc.add(t.cnt, serial);
             follows = true;
             cycle++;
             serial++;
-            if (s.broken) {
+            if (s.broken) {  // an error: the domain stops at the end of this step
                 nsteps = 0;
                 break;
             }
@@ -1643,7 +1653,7 @@ __device__ __forceinline__ void steps_body(const DomainView &d, int p, int layer
         widen_range(d, before.lohi);
         acc.add(t.cnt, serial);
         acc.put(d, b);
-        if (!team_sync(d, team, cycle)) return;
+        if (!team_sync(d, team, cycle, s.broken)) return;
         clear_tally(s.tally[0]);
         clear_tally(s.tally[1]);
         if (b == 0) {
@@ -1654,12 +1664,12 @@ __device__ __forceinline__ void steps_body(const DomainView &d, int p, int layer
                 end_domain(d, cycle - 1);
                 ctl->cycle[p_end] = cycle;
                 ctl->serial[p_end] = serial;
-                ctl->barrier = team.number + (nsteps > 0);  // with the barrier below
+                ctl->barrier = team.number + 2 * (nsteps > 0);  // with the barrier below
             }
         }
         follows = false;  // settled
         if (nsteps > 0) {
-            if (!team_sync(d, team, cycle)) return;
+            if (!team_sync(d, team, cycle, s.broken)) return;
             if (ctl->done) return;
         }
     }
