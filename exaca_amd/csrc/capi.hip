@@ -234,10 +234,10 @@ int team_by_size(const exaca::Deck &deck, const exaca::HostDomain &hd) {
 //   plane: 212 31.3, 21.5, 21.5, 21.0, 23.1; 677 75.6, 26.4, 23.5, 23.4, 24.8; 884 134, 44.9, 36.7, 34.6, 35.2;
 //   2228 227, 51.9, 35.1, 29.8, 26.7; 4455 440, 80.8, 53.7, 36.7, 29.7
 int team_by_due(double evaluated) {
-    if (evaluated > 3200) return 0;
-    if (evaluated <= 120) return 1;
-    if (evaluated <= 560) return 8;
-    return evaluated <= 1700 ? 16 : 32;
+    if (evaluated > 3800) return 0;
+    if (evaluated <= 220) return 1;
+    if (evaluated <= 700) return 8;
+    return evaluated <= 2000 ? 16 : 32;
 }
 
 // The layer's nucleation sites to the device; its steps start with none decided. Synchronises the
