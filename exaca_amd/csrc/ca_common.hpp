@@ -60,8 +60,8 @@ constexpr size_t alarm_stride(long long ncell) {
 // A CU holds one of them.
 constexpr int kMaxTeam = 64;
 constexpr uint32_t kTeamClaims = 512;  // claimants that a workgroup stages in LDS; the rest go to the claim lists
-// Words of a domain's `sync`: each workgroup's last barrier, each one's last launch, the decision (two words).
-constexpr int kSyncReport = kMaxTeam, kSyncDecision = 2 * kMaxTeam, kSyncWords = 2 * kMaxTeam + 2;
+// Words of a domain's `sync`: each workgroup's last barrier, and its report for a launch (meet.hpp; two words).
+constexpr int kSyncReports = kMaxTeam, kSyncWords = 3 * kMaxTeam;
 // How long a team's workgroups wait for one another at the start of a launch, in us: longer than the domains
 // before it in a crowded ensemble's launch mostly take (1000 steps of 10 to 100 us), and not much longer
 // than one workgroup alone takes for a middle domain's.

@@ -1508,44 +1508,44 @@ __device__ __forceinline__ bool team_sync(const DomainView &d, Team &t, int cycl
     return false;
 }
 
-// A team's meeting (meet.hpp), by one wave of each workgroup; every lane calls and gets the same.
+// A team's meeting (meet.hpp), by one wave of each workgroup, a lane to a word; every lane calls and gets the
+// same. Two trips to memory where all run.
 struct MeetWords {
     const DomainView &d;
-    uint32_t b, nb, launch;
-    unsigned long long t0;
+    uint32_t b, nb;
+    unsigned long long launch, t0, seen;  // seen: what this lane's word held
+    __device__ __forceinline__ unsigned long long *word(uint32_t i) const {
+        return reinterpret_cast<unsigned long long *>(d.sync + kSyncReports) + i;
+    }
     __device__ __forceinline__ void report() const {
         if (threadIdx.x == 0)
-            __hip_atomic_store(d.sync + kSyncReport + b, launch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            (void)__hip_atomic_fetch_max(word(b), static_cast<unsigned long long>(meet_reported(launch)), __ATOMIC_RELAXED,
+                                         __HIP_MEMORY_SCOPE_AGENT);
     }
-    __device__ __forceinline__ unsigned long long *word() const {
-        return reinterpret_cast<unsigned long long *>(d.sync + kSyncDecision);
+    __device__ __forceinline__ Met look() {
+        seen = __hip_atomic_load(word(threadIdx.x < nb ? threadIdx.x : b), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        return Met{__all(seen == meet_reported(launch)) != 0, __any(seen == meet_refused(launch)) != 0};
     }
-    __device__ __forceinline__ static uint64_t first_lane(unsigned long long v) {
-        const uint32_t lo = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(v));
-        return static_cast<uint64_t>(__builtin_amdgcn_readfirstlane(static_cast<uint32_t>(v >> 32))) << 32 | lo;
+    __device__ __forceinline__ bool expired() const {
+        return static_cast<unsigned long long>(wall_clock64()) - t0 >= d.meet_wait;
     }
-    __device__ __forceinline__ uint64_t decision() const {
-        return first_lane(__hip_atomic_load(word(), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
-    }
-    __device__ __forceinline__ bool all_reported() const {
-        const uint32_t *r = d.sync + kSyncReport + (threadIdx.x < nb ? threadIdx.x : 0);
-        return __all(__hip_atomic_load(r, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == launch);
-    }
-    __device__ __forceinline__ bool expired() const { return static_cast<unsigned long long>(wall_clock64()) - t0 >= d.meet_wait; }
-    __device__ __forceinline__ uint64_t settle(uint64_t from, uint64_t to) const {
-        unsigned long long found = from;
-        if (threadIdx.x == 0)
-            __hip_atomic_compare_exchange_strong(word(), &found, static_cast<unsigned long long>(to), __ATOMIC_RELAXED,
-                                                 __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        return first_lane(found);
+    __device__ __forceinline__ void refuse() const {
+        unsigned long long was = seen;
+        if (threadIdx.x < nb && seen < meet_reported(launch))
+            (void)__hip_atomic_compare_exchange_strong(word(threadIdx.x), &was,
+                                                       static_cast<unsigned long long>(meet_refused(launch)),
+                                                       __ATOMIC_RELAXED, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
 };
 // Whether this workgroup takes part in the launch; the team is then all of it, or this one alone. role: LDS.
-__device__ __forceinline__ bool team_meets(const DomainView &d, Team &t, uint32_t launch, uint32_t &role) {
+__device__ __forceinline__ bool team_meets(const DomainView &d, Team &t, unsigned long long launch, uint32_t &role) {
     if (t.nb == 1) return true;
     if (threadIdx.x < 64) {
-        const MeetWords w{d, t.b, t.nb, launch, static_cast<unsigned long long>(wall_clock64())};
-        const Meet m = meet(w, t.b, launch);
+        Meet m = t.b == 0 ? Meet::kAlone : Meet::kLeave;  // (given no time at all)
+        if (d.meet_wait) {
+            MeetWords w{d, t.b, t.nb, launch, static_cast<unsigned long long>(wall_clock64()), 0};
+            m = meet(w, t.b);
+        }
         if (threadIdx.x == 0) role = static_cast<uint32_t>(m);
     }
     __syncthreads();
@@ -1576,7 +1576,7 @@ struct TeamLds {
 // cells; a step with a nucleation site due has one more. Control words and counters stay in registers
 // and LDS, the growth table in LDS, and caches and code stay warm from step to step.
 __device__ __forceinline__ void steps_body(const DomainView &d, int p, int layer, int nsteps, bool nucleate, uint32_t b,
-                                           uint32_t team_size, uint32_t launch, TeamLds &s) {
+                                           uint32_t team_size, unsigned long long launch, TeamLds &s) {
     StepCtl *ctl = d.ctl;
     if (ctl->done) return;
     Team team{b, team_size, ctl->barrier};
@@ -1690,7 +1690,7 @@ __global__ __launch_bounds__(kBlock) void k_settle(DomainView d, int p_next) {
 }
 __global__ __launch_bounds__(kBlock) void k_book(DomainView d, int p_next) { book_step(d, p_next); }
 __global__ __launch_bounds__(kTeamBlock) void k_steps(DomainView d, int p, int layer, int nsteps, int nucleate,
-                                                      uint32_t launch) {
+                                                      unsigned long long launch) {
     __shared__ TeamLds s;
     steps_body(d, p, layer, nsteps, nucleate != 0, blockIdx.x, gridDim.x, launch, s);
 }
@@ -1725,7 +1725,7 @@ __device__ __forceinline__ DomainView load_view(const DomainView *views, uint32_
     return d;
 }
 __global__ __launch_bounds__(kTeamBlock) void k_steps_n(const DomainView *views, const TeamPlace *places, int layer,
-                                                        int nsteps, uint32_t launch) {
+                                                        int nsteps, unsigned long long launch) {
     __shared__ TeamLds s;
     const TeamPlace at = load_constant(places, blockIdx.x);
     const DomainView d = load_view(views, at.slot);
@@ -2038,7 +2038,7 @@ void launch_settle(const DomainView &d, int parity_next, int blocks, hipStream_t
     k_settle<<<blocks, kBlock, 0, s>>>(d, parity_next);
     k_book<<<1, kBlock, 0, s>>>(d, parity_next);
 }
-void launch_steps(const DomainView &d, int parity, int layer, int steps, bool nucleate, int team, uint32_t launch,
+void launch_steps(const DomainView &d, int parity, int layer, int steps, bool nucleate, int team, uint64_t launch,
                   hipStream_t s) {
     k_steps<<<team, kTeamBlock, 0, s>>>(d, parity, layer, steps, nucleate ? 1 : 0, launch);
 }
@@ -2066,7 +2066,7 @@ void launch_step_timed(const DomainView &d, const StepAt &at, int blocks, hipStr
     rec();
 }
 void launch_steps_n(const DomainView *views, const TeamPlace *places, uint32_t workgroups, int steps, int layer,
-                    uint32_t launch, hipStream_t s) {
+                    uint64_t launch, hipStream_t s) {
     k_steps_n<<<workgroups, kTeamBlock, 0, s>>>(views, places, layer, steps, launch);
 }
 void launch_check(const DomainView &d, int cycle, int layer, CheckResult *out, hipStream_t s) {

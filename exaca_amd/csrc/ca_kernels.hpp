@@ -28,10 +28,10 @@ void launch_capture(const DomainView &d, const StepAt &at, int blocks, hipStream
 // or the statistics are looked at. parity_next is the parity of the next step.
 void launch_settle(const DomainView &d, int parity_next, int blocks, hipStream_t s);
 // `steps` steps in one launch of a team of workgroups (at most kMaxTeam), settled and booked;
-// nucleate: with their nucleation (else none of their sites may be due). launch: a number that none of the
-// domain's launches before had, nor 0.
+// nucleate: with their nucleation (else none of their sites may be due). launch: a number greater than 0 and
+// those of the domain's launches before.
 constexpr int kTeamBlock = 512;
-void launch_steps(const DomainView &d, int parity, int layer, int steps, bool nucleate, int team, uint32_t launch,
+void launch_steps(const DomainView &d, int parity, int layer, int steps, bool nucleate, int team, uint64_t launch,
                   hipStream_t s);
 // Capture-pass workgroups that a CU holds at once.
 int claim_per_cu();
@@ -48,7 +48,7 @@ void launch_layer_setup(const DomainView &d, int parity_next, hipStream_t s);
 // `steps` steps (an even number, from parity 0) of the domains of a device-resident table of views,
 // settled and booked: one workgroup per entry of `places`.
 void launch_steps_n(const DomainView *views, const TeamPlace *places, uint32_t workgroups, int steps, int layer,
-                    uint32_t launch, hipStream_t s);
+                    uint64_t launch, hipStream_t s);
 // IntermediateOutputAndCheck's reduction (src/CAupdate.cpp:738-758, 792-808).
 void launch_check(const DomainView &d, int cycle, int layer, CheckResult *out, hipStream_t s);
 // Octahedra of the initially active cells (src/CAinitialize.cpp:1936-2043).

@@ -158,7 +158,7 @@ struct exaca_state {
     int cycle = 0;         // the cycle before the next step's
     int last_cycle = 0;    // last executed step of the layer
     uint32_t serial = 0;   // steps executed
-    uint32_t launches = 0; // of the team
+    uint64_t launches = 0; // of teams
     int pending = -1;      // cycle whose nucleation ran but whose capture has not
     int blocks = 2048;     // workgroups of the frontier kernels
     int team = 0;          // workgroups of the team that takes single steps in one launch (0: two launches a step)
@@ -449,8 +449,7 @@ void step_capture(exaca_state *h, int cycle) {
 }
 // n steps of a team, in one launch.
 void step_team(exaca_state *h, int layer, int n, bool nucleate, int team) {
-    h->launches = std::max(h->launches + 1, 1u);
-    exaca::launch_steps(h->dv, h->parity, layer, n, nucleate, team, h->launches, h->stream);
+    exaca::launch_steps(h->dv, h->parity, layer, n, nucleate, team, ++h->launches, h->stream);
     HIP_OK(hipGetLastError());
     stepped(h, n);
 }
@@ -984,7 +983,7 @@ int exaca_team_query(const exaca_state *h, int64_t out[4]) {
         HIP_OK(hipStreamSynchronize(h->stream));
         HIP_OK(hipMemcpy(&c, h->ctl, sizeof c, hipMemcpyDeviceToHost));
         out[0] = h->run_team;
-        out[1] = h->launches;
+        out[1] = static_cast<int64_t>(h->launches);
         out[2] = c.alone;
         out[3] = c.spilled;
     });

@@ -133,7 +133,7 @@ struct exaca_ensemble {
     size_t places_cap = 0;
     bool dirty = true;
     long long steps = 0;
-    uint32_t launches = 0;
+    uint64_t launches = 0;
     uint32_t meet_wait = 0, barrier_wait = 0;  // ticks
 
     ~exaca_ensemble() {
@@ -245,8 +245,7 @@ void launch(exaca_ensemble *e, int steps) {
     if (e->places.empty()) return;
     for (int n; steps > 0; steps -= n) {
         n = std::min(steps, kMaxLaunch);
-        e->launches = std::max(e->launches + 1, 1u);
-        exaca::launch_steps_n(e->views_d, e->places_d, static_cast<uint32_t>(e->places.size()), n, 0, e->launches,
+        exaca::launch_steps_n(e->views_d, e->places_d, static_cast<uint32_t>(e->places.size()), n, 0, ++e->launches,
                               e->stream);
         HIP_OK(hipGetLastError());
     }

@@ -60,7 +60,7 @@ inline uint32_t claim_stage() {
 }
 // How long a team's workgroups wait for one another, in ticks of the 100 MHz clock: at the start of a launch
 // (meet.hpp; EXACA_MEET_US) and at a barrier, at most (EXACA_BARRIER_US). The variables, 0 .. 40000000 us, are
-// read when a handle or ensemble is created. Tests set 0: most launches are then left to one workgroup; the
+// read when a handle or ensemble is created. Tests set 0: every launch is then left to one workgroup; the
 // first barrier ends the domain with error 16.
 inline uint32_t wait_ticks(const char *name, long us) {
     if (const char *env = std::getenv(name)) {

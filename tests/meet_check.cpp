@@ -16,27 +16,37 @@
 using exaca::Meet;
 
 struct Words {
-    std::atomic<uint32_t> report[64];
-    std::atomic<uint64_t> decision;
+    std::atomic<uint64_t> word[64];
 };
 struct Group {
     Words &words;
-    uint32_t b, nb, launch;
-    mutable int looks;  // until the wait expires (negative: never)
-    void report() const { words.report[b].store(launch, std::memory_order_relaxed); }
-    uint64_t decision() const {
+    uint32_t b, nb;
+    uint64_t launch;
+    int looks;  // until the wait expires (negative: never)
+    uint64_t seen[64] = {};
+    void report() {
+        uint64_t v = words.word[b].load();
+        while (v < exaca::meet_reported(launch) &&
+               !words.word[b].compare_exchange_weak(v, exaca::meet_reported(launch), std::memory_order_relaxed)) {
+        }
+    }
+    exaca::Met look() {
         std::this_thread::yield();
-        return words.decision.load(std::memory_order_relaxed);
+        exaca::Met m{true, false};
+        for (uint32_t i = 0; i < nb; i++) {
+            seen[i] = words.word[i].load(std::memory_order_relaxed);
+            m.all = m.all && seen[i] == exaca::meet_reported(launch);
+            m.refused = m.refused || seen[i] == exaca::meet_refused(launch);
+        }
+        return m;
     }
-    bool all_reported() const {
+    bool expired() { return looks >= 0 && (looks == 0 || looks-- == 0); }
+    void refuse() {
         for (uint32_t i = 0; i < nb; i++)
-            if (words.report[i].load(std::memory_order_relaxed) != launch) return false;
-        return true;
-    }
-    bool expired() const { return looks >= 0 && looks-- == 0; }
-    uint64_t settle(uint64_t from, uint64_t to) const {
-        words.decision.compare_exchange_strong(from, to, std::memory_order_relaxed);
-        return from;
+            if (seen[i] < exaca::meet_reported(launch)) {
+                uint64_t was = seen[i];
+                words.word[i].compare_exchange_strong(was, exaca::meet_refused(launch), std::memory_order_relaxed);
+            }
     }
 };
 
@@ -61,8 +71,8 @@ int main() {
                 std::vector<std::thread> run;
                 for (uint32_t i = part; i < (part ? nb : first); i++)
                     run.emplace_back([&, b = order[i]] {
-                        const Group g{words, b, nb, static_cast<uint32_t>(launch), looks[b]};
-                        role[b] = exaca::meet(g, b, static_cast<uint32_t>(launch));
+                        Group g{words, b, nb, static_cast<uint64_t>(launch), looks[b]};
+                        role[b] = exaca::meet(g, b);
                     });
                 for (std::thread &t : run) t.join();
                 if (first == nb) break;

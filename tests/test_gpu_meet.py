@@ -1,6 +1,6 @@
-"""GPU: launches of a team whose workgroups do not all run at once. With no time to meet, most launches
-are left to one workgroup of the team: a domain stepped by both kinds of launches equals the oracle, and an
-ensemble equals one whose teams meet. Two ensembles that each fill the compute units and a solver, stepped
+"""GPU: launches of a team whose workgroups do not all run at once. With no time to meet, every launch is left
+to one workgroup of the team; with 1 us, some are: a domain stepped so equals the oracle, and an ensemble
+equals one whose teams meet. Two ensembles that each fill the compute units and a solver, stepped
 from three threads at once, all end, with the results they have alone."""
 import threading
 
@@ -14,9 +14,10 @@ from conftest import DATA, c_deck
 pytestmark = pytest.mark.gpu
 
 
+@pytest.mark.parametrize("wait", [0, 1])
 @pytest.mark.parametrize("side,workgroups", [(44, 8), (70, 16), (96, 32)])
-def test_domain_left_to_one_workgroup_matches_the_oracle(tmp_path, monkeypatch, side, workgroups):
-    monkeypatch.setenv("EXACA_MEET_US", "0")
+def test_domain_left_to_one_workgroup_matches_the_oracle(tmp_path, monkeypatch, side, workgroups, wait):
+    monkeypatch.setenv("EXACA_MEET_US", str(wait))
     deck = c_deck(tmp_path / "d.txt", 8, nx=side, ny=side, density=1000, fraction=0.2)
     osim = orc.OracleSim(deck, DATA)
     osim.run(max_cycles=300)
@@ -25,7 +26,8 @@ def test_domain_left_to_one_workgroup_matches_the_oracle(tmp_path, monkeypatch, 
             sol.run(max_cycles=c)
         team = sol.team()
         print(f"[meet] {side}: {team}", flush=True)
-        assert team["workgroups"] == workgroups and team["launches"] == 9 and 0 < team["alone"] <= 9
+        assert team["workgroups"] == workgroups and team["launches"] == 9
+        assert team["alone"] == 9 if wait == 0 else 0 <= team["alone"] <= 9
         q, d = sol.query(), osim.dims()
         for key in ("nn", "captures", "solidified", "frontier"):
             assert q[key] == d[key], (key, q[key], d[key])
@@ -79,9 +81,10 @@ def _domains(tmp_path, tag, count, seed):
 def test_ensemble_left_to_single_workgroups(tmp_path, monkeypatch):
     preps = _domains(tmp_path, "e", 24, 5)
     met = _solve_all(preps, 400)
-    monkeypatch.setenv("EXACA_MEET_US", "0")
-    print("[meet] ensemble without meeting", flush=True)
-    _same(_solve_all(preps, 400), met)
+    for wait in ("0", "1", "3"):
+        monkeypatch.setenv("EXACA_MEET_US", wait)
+        print(f"[meet] ensemble with {wait} us to meet", flush=True)
+        _same(_solve_all(preps, 400), met)
 
 
 def test_ensembles_and_a_solver_at_once(tmp_path):
