@@ -218,7 +218,10 @@ int team_by_size(const exaca::Deck &deck, const exaca::HostDomain &hd) {
     const double sites = static_cast<double>(hd.nloc.size()) / static_cast<double>(hd.ncell);
     const double nuclei = std::max(1.0, 30.0 * sites / std::max(deck.nratio, 1));
     const double area = nuclei * (spots ? 2.5 * deck.spot_radius * deck.spot_radius : static_cast<double>(plane));
-    if (area > 116 * 116 || (spots && plane > 140 * 140)) return 0;
+    // finer time steps have fewer cells due in each: 130^3 takes 20.8, 17.4, 17.0 with 8, 16, 32 workgroups and
+    // 18.6 with two launches at N = 25; 13.5, 13.6, 13.9 and 14.3 at N = 50; 44.3, 27.9, 21.4 and 18.6 at N = 5
+    const int widest = spots || deck.nratio > 15 ? 140 : 116;
+    if (area > widest * widest || plane > 140 * 140) return 0;
     if (area <= 40 * 40) return 1;
     if (area <= 61 * 61) return 8;
     return area <= 92 * 92 ? 16 : 32;

@@ -50,6 +50,12 @@ def test_cross_sections_where_the_team_changes(tmp_path, array, n, workgroups):
     _both(deck, 300, workgroups)
 
 
+@pytest.mark.parametrize("array,N,workgroups", [(117, 15, 0), (117, 16, 32), (140, 25, 32), (141, 25, 0)])
+def test_fine_time_steps_keep_a_team_longer(tmp_path, array, N, workgroups):
+    deck = c_deck(tmp_path / "d.txt", 4, nx=array - 4, ny=array - 4, density=500, fraction=0.15, N=N)
+    _both(deck, 300, workgroups)
+
+
 @pytest.mark.parametrize("radius,workgroups", [(25, 1), (26, 8)])
 def test_spots_where_the_team_changes(tmp_path, radius, workgroups):
     deck = s_deck(tmp_path / "s.txt", nsx=1, nsy=1, offset=radius, radius=radius, density=300, spacing=8, N=2)
