@@ -40,8 +40,10 @@ CXX_FLAGS = ["-O2", "-std=c++17", "-fPIC", "-ffp-contract=off", "-Wall", "-Wextr
 HIP_SOURCES = ["ca_kernels.hip", "capi.hip", "ensemble.hip"]
 CXX_SOURCES = ["deck.cpp", "init.cpp", "output.cpp"]
 # The initial state's random draws (a block Mersenne Twister) vectorise at -O3; no flag here
-# relaxes IEEE arithmetic, so the state stays bit-identical.
-CXX_OPT = {"init.cpp": "-O3"}
+# relaxes IEEE arithmetic, so the state stays bit-identical. Their loops fill whole cache lines: without the
+# alignment an edit anywhere before them in the file or the link moves the time of a 310^3 domain between 48 and
+# 60 ms.
+CXX_OPT = {"init.cpp": ["-O3", "-falign-functions=64"]}
 
 
 def _run(cmd: list[str], verbose: bool) -> None:
@@ -62,7 +64,7 @@ def build(verbose: bool = False) -> Path:
     objs = []
     for src in CXX_SOURCES:
         obj = OUT / (src + ".o")
-        flags = [CXX_OPT.get(src, f) if f == "-O2" else f for f in CXX_FLAGS]
+        flags = CXX_OPT.get(src, ["-O2"]) + CXX_FLAGS[1:]
         _run([CXX, *flags, "-c", str(CSRC / src), "-o", str(obj)], verbose)
         objs.append(str(obj))
     host_objs = list(objs)
