@@ -1628,6 +1628,9 @@ __device__ __forceinline__ void steps_body(const DomainView &d, int p, int layer
                                                  }
                                              });
             if (!team_sync(d, team, cycle, s.broken, true)) return;
+            // (0: an error, and the domain stops at the end of this step. Read with the number of claimants, and no
+            // branch out of the loop: with one, 24^3 cells take 6.98 us a step instead of 6.84)
+            const int go = 1 - __builtin_amdgcn_readfirstlane(static_cast<int>(s.broken));
             if (threadIdx.x < kStepCounts) before.cnt[threadIdx.x] = 0;
             apply_body<kTeamBlock>(
                 d, gr, serial, s.nclaim,
@@ -1642,11 +1645,9 @@ __device__ __forceinline__ void steps_body(const DomainView &d, int p, int layer
             follows = true;
             cycle++;
             serial++;
-            if (s.broken) {  // an error: the domain stops at the end of this step
-                nsteps = 0;
-                break;
-            }
+            n *= go;
         }
+        if (s.broken) nsteps = 0;
         StepTally &t = s.tally[serial & 1], &before = s.tally[(serial & 1) ^ 1];
         settle_body<kTeamBlock, kTeamDue>(d, g, at, cycle, serial, b, nb, s.list, s.tot, t.cnt);
         widen_range(d, t.lohi, made);
