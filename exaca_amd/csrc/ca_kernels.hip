@@ -18,9 +18,9 @@
 // boundary), so a step has as few phases as its domain-wide dependences allow: claims before winners,
 // captures before the next step's claims. With separate kernels for the winners, the settling and the
 // list of due cells a step took 28.8, 40.5, 66.4, 76.4 us at 24^3, 100^3, 256^3, 400^3; with two kernels
-// it takes 12.1, 15.9, 25.2, 36.4 us; at 800^3 (cycles 6006-6025) 0.198 and 0.151 ms.
+// it takes 12.1, 15.9, 25.2, 36.4 us; at 800^3 (cycles 6006-6025) 0.198 and 0.155 ms.
 // A narrow domain takes its steps in k_steps, many in a launch: a team of 1 to 64 workgroups with a
-// barrier between the phases of a step (7.1 us a step at 24^3, 14.3 at 100^3); k_steps_n does so for
+// barrier between the phases of a step (6.9 us a step at 24^3, 15.5 at 100^3); k_steps_n does so for
 // every domain of an ensemble.
 // A cell is due when something can happen to it: it is new, its liquidus time has passed, or its
 // half-diagonal reaches the least critical length of its liquid neighbours; a neighbour's capture
@@ -1071,7 +1071,7 @@ __device__ __forceinline__ void widen_range(const DomainView &d, uint32_t *lohi,
 // lanes of a half-wave, so that the words of three consecutive neighbours are read together, its
 // lengths are one store of one line, and its chain is one length and one mask long instead of 26.
 // One lane per capture took 242 registers (two waves a SIMD) and about 10 000 cycles for one
-// capture, this 123 registers and half the cycles (24^3 9.3 -> 7.4 us a step); at 800^3, 63 000 captures a
+// capture, this 121 registers and half the cycles (24^3 9.3 -> 7.4 us a step); at 800^3, 63 000 captures a
 // step, the pass takes 72 us against 83 us.
 template <int BLOCK, typename F>
 __device__ __forceinline__ void apply_body(const DomainView &d, const Grid &gr, uint32_t serial, uint32_t nclaimants,
@@ -1450,8 +1450,8 @@ __device__ __forceinline__ void book_step(const DomainView &d, int p_next) {
 // ---- A team of workgroups that runs many steps of one domain in one launch. ----
 
 // The team's barrier: every workgroup posts the barrier's number in its own word and waits for all
-// the others' words (each polls all of them: one hop, 1.7 us for 8 workgroups and 2.6 us for 32,
-// against 2.0 and 2.7 us with a workgroup that gathers and releases). What the team wrote before it
+// the others' words (each polls all of them: one hop. With the waits below and a wave's stores to write back
+// 1.7, 2.1, 2.6, 4.5 us for 8, 16, 32, 64 workgroups; with none 1.4, 1.7, 1.9, 4.0). What the team wrote before it
 // is visible to the team after it (agent-scope release and acquire by one wave, ordered with the rest
 // of the workgroup by its own barriers). A team of one needs the workgroup's barrier alone.
 // All of the team's workgroups run (they met before), so every wait ends; it is bounded all the same

@@ -270,9 +270,9 @@ void build_device_state(exaca_state *h) {
     HIP_OK(hipGetDeviceProperties(&prop, dev));
     // Two-launch steps: up to 4 workgroups per CU, all resident at once, and 2 where the front's plane is
     // narrow, so that a workgroup's start-up serves more cells. Measured, us a step with 1, 2, 3, 4, 6, 8
-    // per CU: 128^3 -, 18.0, -, 18.7, -, -; 200^3 -, 20.5, -, 21.2, -, -; 256^3 26.7, 25.2, 25.6, 25.6, 35.3,
-    // 37.7; 400^3 44.1, 37.9, 37.0, 36.1, 45.4, 46.7; 800x800x40 47.5, 40.4, 38.3, 39.2, 46.7, 49.6; 800^3
-    // (cycles 6006-6025) 215, 164, 157, 147, 164, 152. Fewer for domains of few cells.
+    // per CU, over 3000 cycles: 128^3 19.5, 20.2, 20.5, 20.8, 28.1, 30.7; 200^3 23.8, 23.8, 24.1, 24.5, 34.1,
+    // 36.4; 256^3 29.0, 27.1, 27.7, 27.8, 38.0, 40.5; 400^3 45.8, 40.8, 39.8, 39.6, 50.1, 52.5; 800x800x40 (1000)
+    // 55.7, 47.5, 45.0, 46.1, 55.7, 60.0; 800^3 (6006-6025) 216, 169, 156, 152, 161, 157. Fewer for few cells.
     const int most = static_cast<long long>(hd.X) * hd.Y <= 300 * 300 ? 2 : 4;
     const int per_cu = std::min(most, exaca::claim_per_cu());
     const long long cap = std::min<long long>(2048, ((prop.multiProcessorCount * per_cu + 7) / 8) * 8);

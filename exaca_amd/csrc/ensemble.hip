@@ -3,7 +3,7 @@
 // Each domain occupies one slot: its state lives in a sub-range of a single device arena, and its
 // DomainView sits in a device-resident slot table. A launch runs many steps of every domain: a team of
 // workgroups takes each domain through them on its own (k_steps_n), so no domain waits for another
-// within a launch, and the larger a domain, the larger its team (share_out). Every domain keeps its
+// once its team has met (meet.hpp), and the larger a domain, the larger its team (share_out). Every domain keeps its
 // own cycle, control block and calendar, and stops itself on the device at the first 1000-step check
 // with no liquid left, so each one evolves exactly as it would alone on the plain path. The host
 // admits new domains into free slots between launches (continuous batching) and polls the
@@ -166,9 +166,9 @@ void ensure_tables(exaca_ensemble *e, const exaca::HostDomain &h, const std::str
 
 // Estimated time of a step (us) of a domain with that cross-section and team: a chain that grows
 // with the team's barriers, and the front's cells by the team, dearer in a large domain, whose records
-// the caches don't hold. Single domains measured, us: 24^3 7.4
-// with 1 workgroup, 44^3 17.8 with 1 and 13.1 with 8, 100^3 84.6 with 1, 20.8 with 8 and 15.3 with 32,
-// 256^3 168 with 8 and 36.3 with 64.
+// the caches don't hold. Single domains measured, us: 24^3 7.1
+// with 1 workgroup, 44^3 17.7 with 1 and 13.4 with 8, 100^3 138 with 1, 27.6 with 8 and 18.7 with 32, 150^3 54.0
+// with 8 and 22.9 with 64.
 double step_estimate(const exaca::DomainView &d, int team) {
     const double chain = team == 1 ? 3.0 : 7.0 + std::log2(static_cast<double>(team));
     const double per_cell = 0.0075 + 0.0125 * std::min(1.0, static_cast<double>(d.ncell) / 1.6e7);
@@ -182,9 +182,8 @@ double step_estimate(const exaca::DomainView &d, int team) {
 // it gains from it; beyond the CUs only while it would take half as long again as its share of them
 // (its larger team costs the others time). The largest teams come first, so that the small domains
 // fill in behind them. Measured, ms for all solves (at most 32 workgroups a slot) within the CUs only,
-// beyond them while the estimate of the launch falls, and by this rule: 256 domains of sides 32-256
-// 4892, 3016, 3491; 64 of 32-64 254, 267, 252; 16 of 64-192 303, 329, 302. (Every slot's row of the same
-// number of workgroups, with kernel boundaries between the passes: 5872, 1045, 738.)
+// beyond them with a factor of 2, this 1.5, 1.1 and 1: 256 domains of sides 32-256 3562, 2380, 2094, 1918, 1963;
+// 256 of 32-64 203, 203, 204, 216, 216; 64 of 32-64 92, 92, 92, 104, 110; 16 of 64-192 185, 184, 185, 184, 192.
 void share_out(exaca_ensemble *e) {
     if (!e->dirty) return;
     std::vector<std::pair<double, int>> running;  // estimate, slot

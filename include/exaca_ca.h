@@ -184,8 +184,9 @@ int exaca_ensemble_destroy(exaca_ensemble *e);
 /* Message of the last failure on this thread. */
 const char *exaca_last_error(void);
 
-/* Timed stepping (no reference counterpart): runs nsteps further steps of `layer` like
- * exaca_run_layer, one kernel after another, with HIP events on the handle's stream around every kernel.
+/* Timed stepping (no reference counterpart): runs nsteps further steps of `layer`, to the results of
+ * exaca_run_layer, by the kernels of two launches a step one after another, whatever exaca_run_layer would
+ * launch for the domain (exaca_team_query), with HIP events on the handle's stream around every kernel.
  * ms[0..2] receive the summed device time of the nucleation, claim and apply kernels; counts
  * [0..4] the frontier-size sum, captures, solidifications, kernel launches per kind and the number
  * of steps executed (checks and cycle jumps are applied as in exaca_run_layer). */
